@@ -2,12 +2,11 @@
 //
 // In the reference's attention layer the rotation of Q and K runs as its own
 // launch immediately before the cache write, on the same K tensor. Here a
-// workgroup owns a run of 16-byte work items of ONE token (so position, cos/sin
-// row and cache slot are workgroup-uniform): it stages the token's cos/sin row
-// in LDS as fp32, rotates Q and K in fp32 with a single rounding to the storage
-// type, and, when a cache is given, stores the rotated K and the V row straight
-// into the token's slot. K is read once and V never takes a separate launch.
-// Without a cache the kernel is the plain rotation.
+// workgroup belongs to ONE token (so position, cos/sin row and cache slot are
+// workgroup-uniform): its lanes rotate Q and K in fp32 with a single rounding
+// to the storage type and, when a cache is given, store the rotated K and the V
+// row straight into the token's slot. K is read once and V never takes a
+// separate launch. Without a cache the kernel is the plain rotation.
 //
 // Vectors are 16 bytes (8 bf16/fp16 or 4 fp32 elements); a "pair-vector" is the
 // x half and the y half of the same rotation lanes of one head.
@@ -64,39 +63,37 @@ struct F32 {
   static constexpr int kBytes = 4;
 };
 
-// unpack / pack one 16-byte vector to fp32 lanes
+// one 16-byte pair-vector in fp32 with one rounding: ox = x cos - y sin, oy = y cos + x sin
 template <typename T>
 struct Vec {
-  static constexpr int kElems = 16 / T::kBytes;
-  static __device__ __forceinline__ void unpack(u32x4 v, float* out) {
+  static __device__ __forceinline__ void rotate(u32x4 x, u32x4 y, u32x4 cx, u32x4 cy, u32x4 sx, u32x4 sy,
+                                                u32x4& ox, u32x4& oy) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      out[2 * i] = T::load((uint16_t)(v[i] & 0xffffu));
-      out[2 * i + 1] = T::load((uint16_t)(v[i] >> 16));
-    }
-  }
-  static __device__ __forceinline__ u32x4 pack(const float* in) {
-    u32x4 v;
+      float o[2][2];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      v[i] = T::store2(in[2 * i], in[2 * i + 1]);
-    return v;
+      for (int w = 0; w < 2; ++w) {
+        const auto f = [&](u32x4 v) { return T::load((uint16_t)(w ? v[i] >> 16 : v[i] & 0xffffu)); };
+        o[0][w] = f(x) * f(cx) - f(y) * f(sx);
+        o[1][w] = f(y) * f(cy) + f(x) * f(sy);
+      }
+      ox[i] = T::store2(o[0][0], o[0][1]);
+      oy[i] = T::store2(o[1][0], o[1][1]);
+    }
   }
   static __device__ __forceinline__ float load1(const char* p) { return T::load(*(const uint16_t*)p); }
   static __device__ __forceinline__ void store1(char* p, float f) { *(uint16_t*)p = T::store(f); }
 };
 template <>
 struct Vec<F32> {
-  static constexpr int kElems = 4;
-  static __device__ __forceinline__ void unpack(u32x4 v, float* out) {
+  static __device__ __forceinline__ void rotate(u32x4 x, u32x4 y, u32x4 cx, u32x4 cy, u32x4 sx, u32x4 sy,
+                                                u32x4& ox, u32x4& oy) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) out[i] = __uint_as_float(v[i]);
-  }
-  static __device__ __forceinline__ u32x4 pack(const float* in) {
-    u32x4 v;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = __float_as_uint(in[i]);
-    return v;
+    for (int i = 0; i < 4; ++i) {
+      const auto f = [&](u32x4 v) { return __uint_as_float(v[i]); };
+      ox[i] = __float_as_uint(f(x) * f(cx) - f(y) * f(sx));
+      oy[i] = __float_as_uint(f(y) * f(cy) + f(x) * f(sy));
+    }
   }
   static __device__ __forceinline__ float load1(const char* p) { return *(const float*)p; }
   static __device__ __forceinline__ void store1(char* p, float f) { *(float*)p = f; }
@@ -129,237 +126,287 @@ struct RopeArgs {
   int64_t cache_block_stride, cache_slot_stride;  // bytes
   int64_t num_cache_blocks;
   uint32_t groups_per_token;  // workgroups per token
-  int pv_shift;               // log2(pair-vectors per head) or -1
-  int cs_vector;              // cos/sin rows are 16-byte aligned runs of whole vectors
+  // vector kernel
+  uint32_t lanes_per_token;   // lanes that have work
+  uint32_t pairs_per_head;    // pair-vectors of one head
+  uint32_t pairs_magic;       // ceil(2^32 / pairs_per_head): lane / pairs_per_head = mulhi(lane, magic)
+  uint32_t pairs_one;         // all ones where pairs_per_head is 1 (magic is then 0)
+  uint32_t v_items;           // 16-byte vectors of the token's V row (0 without a cache)
 };
 
-// Work items of one token, in this order: rotation pair-vectors of the Q heads
-// then the K heads, pass-through vectors beyond rotary_dim, V vectors. A
-// workgroup takes IPL * blockDim.x consecutive items of one token, IPL per lane
-// (item = first + j * blockDim.x, so the lanes of a wavefront stay on
-// consecutive vectors): all of the lane's global loads are issued first, the
-// cos/sin row is staged in LDS while they are in flight, then the lane computes
-// and stores.
+// How a token finds its cache slot: not at all (plain rotation), through a slot
+// mapping, or through the page table.
+enum Addressing : int { kNoCache, kSlots, kPages };
+
+// Entry t of an int32 or int64 array (width in bytes). Two loads side by side and no
+// branch: a branch on the width makes the scalar unit wait for the value inside it.
+__device__ __forceinline__ int64_t index_of(const void* array, int width, uint32_t t) {
+  const int32_t words = width >> 2;
+  const int32_t* p = reinterpret_cast<const int32_t*>(array) + (int64_t)t * words;
+  const int32_t lo = p[0], hi = p[words - 1];
+  return ((int64_t)(words == 2 ? hi : lo >> 31) << 32) | (uint32_t)lo;
+}
+
+// Byte offset of token t's slot from the start of a cache plane, or -1 where the
+// write skips the token. Uniform over the workgroup: scalar loads. POW2: the block
+// size is a power of two (the other form carries 64-bit divisions).
+template <Addressing ADDR, bool POW2>
+__device__ __forceinline__ int64_t slot_offset(const RopeArgs& a, uint32_t t, int64_t pos) {
+  if constexpr (ADDR == kNoCache) return -1;
+  int64_t blk = -1, off = 0;
+  if constexpr (ADDR == kPages) {
+    const int64_t b = a.batch_indices[t];
+    if (b >= 0 && b < a.batch_size) {
+      const int64_t pg = POW2 ? (pos >> a.bs_shift) : pos / a.block_size;
+      off = pos - (POW2 ? pg << a.bs_shift : pg * a.block_size);
+      const int64_t it = (int64_t)a.kv_indptr[b] + pg;
+      if (it >= 0 && it < (int64_t)a.kv_indptr[b + 1] && it < a.num_kv_indices) blk = a.kv_indices[it];
+    }
+  } else {
+    const int64_t s = index_of(a.slot_mapping, a.slot_bytes, t);
+    if (s >= 0) {
+      blk = POW2 ? (s >> a.bs_shift) : s / a.block_size;
+      off = s - (POW2 ? blk << a.bs_shift : blk * a.block_size);
+    }
+  }
+  if (blk < 0 || blk >= a.num_cache_blocks) return -1;
+  return blk * a.cache_block_stride + off * a.cache_slot_stride;
+}
+
 template <bool NT>
 __device__ __forceinline__ u32x4 ld16(const char* p) {
   if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
   else return *reinterpret_cast<const u32x4*>(p);
 }
+template <bool NT>
+__device__ __forceinline__ void st16(char* p, u32x4 v) {
+  if constexpr (NT) __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
+  else *reinterpret_cast<u32x4*>(p) = v;
+}
 
-// NTL: non-temporal loads, bit 0 for the K and V rows, bit 1 for the Q rows.
-template <typename T, bool VECTOR, int IPL, int NTL>
-__global__ __launch_bounds__(kThreads) void rope_cache_kernel(RopeArgs a) {
+// 16-byte path. A lane owns ONE pair-vector of one Q or K head and carries
+// pass-through vectors (V, then the lanes beyond rotary_dim) along, so a token is
+// as few wavefronts as its pair-vectors need (a V row of its own lanes costs
+// 8 heads x 128 a sixth wavefront, 4 heads a fifth). blockIdx = (group, token).
+// What bounds it: at decode sizes the chain launch -> position -> cos/sin row ->
+// store and the instructions on it; at prefill sizes HBM. Hence
+//   - the lane's own four 16-byte pieces of the cos/sin row go straight to
+//     registers; staging the row in LDS as fp32 for all heads puts an LDS write, a
+//     barrier and 32 LDS words per lane on that chain. Two and four heads per lane
+//     share the pieces and lose more in wavefronts in flight (3.3 and 3.9 us where
+//     one head takes 2.8; 8.5 and 8.4 where it takes 7.7);
+//   - nothing waits for the position before the Q, K and V loads are issued;
+//   - an instantiation holds only the code its launch needs: with every addressing
+//     form, 64-bit divisions and the tails in one kernel a decode launch takes 3.9
+//     instead of 3.4 us.
+// Per launch, 8 launches to a graph, before (LDS, V on lanes of its own) and now:
+// 2 tokens x 40 heads x 64 3.37 -> 2.84 us, 256 x 40 x 128 4.03 -> 3.41, 2048 x 32 x
+// 128 8.87 -> 7.65 (4.9 TB/s), 8192 x 72 x 128 60.1 -> 56.8 (5.9 TB/s).
+// TAIL: up to two pass-through vectors per lane, from V and from the heads'
+// unrotated lanes; without it at most one, from V.
+// NTL: non-temporal loads, bit 0 for the K and V rows, bit 1 for the Q rows. NTQ: non-temporal stores of
+// query_out (by its size, see the launch).
+template <typename T, Addressing ADDR, bool POW2, bool TAIL, int NTL, bool NTQ>
+__global__ __launch_bounds__(kThreads) void rope_vector_kernel(RopeArgs a) {
   using VT = Vec<T>;
-  constexpr int EV = VECTOR ? VT::kElems : 1;
-  constexpr int E = T::kBytes;
-  __shared__ float cs[2 * kMaxRotaryDim];  // cos[0, rd) | sin[0, rd)
+  constexpr uint32_t E = T::kBytes;
+  const uint32_t t = blockIdx.y;
+  const uint32_t lane = blockIdx.x * blockDim.x + threadIdx.x;
+  if (lane >= a.lanes_per_token) return;
+  const int64_t pos = index_of(a.positions, a.pos_bytes, t);
 
-  const uint32_t t = blockIdx.x / a.groups_per_token;
-  const uint32_t group = blockIdx.x - t * a.groups_per_token;
-  const int64_t pos = a.pos_bytes == 8 ? reinterpret_cast<const int64_t*>(a.positions)[t]
-                                       : (int64_t) reinterpret_cast<const int32_t*>(a.positions)[t];
-  if (pos < 0 || pos >= a.max_position) return;  // no cos/sin row: the token is left alone
-  const uint32_t rd = a.rotary_dim;
-  const uint32_t half = rd >> 1;
-  const uint32_t D = a.head_dim;
+  const uint32_t half = (a.rotary_dim >> 1) * E;  // bytes
+  const uint32_t h = __umulhi(lane, a.pairs_magic) + (lane & a.pairs_one);
+  const uint32_t pv = (lane - h * a.pairs_per_head) * 16;
   const uint32_t heads = a.num_heads + a.num_kv_heads;
-  const uint32_t pv_per_head = half / EV;
-  const uint32_t rot_items = heads * pv_per_head;
-  const uint32_t tail_per_head = (D - rd) / EV;
-  const uint32_t tail_items = heads * tail_per_head;
-  const uint32_t v_items = a.key_cache ? a.num_kv_heads * D / EV : 0;
-
-  // ---- this lane's items and their loads ----
-  enum : int { kNone, kRotate, kTail, kValue };
-  int kind[IPL];
-  bool is_k[IPL];
-  uint32_t e0[IPL];     // first lane inside the head (rotation / tail)
-  int64_t in_off[IPL];  // byte offset of the item inside its source row == inside its out row
-  u32x4 rx[IPL], ry[IPL];  // 16-byte path: x half and y half (or the one pass-through vector)
-  float sx[IPL], sy[IPL];  // element path
-  const uint32_t first = group * (IPL * blockDim.x) + threadIdx.x;
-#pragma unroll
-  for (int j = 0; j < IPL; ++j) {
-    const uint32_t item = first + j * blockDim.x;
-    kind[j] = kNone;
-    is_k[j] = false;
-    e0[j] = 0;
-    in_off[j] = 0;
-    sx[j] = sy[j] = 0.f;
-    if (item < rot_items) {
-      kind[j] = kRotate;
-      const uint32_t h = a.pv_shift >= 0 ? item >> a.pv_shift : item / pv_per_head;
-      e0[j] = (item - h * pv_per_head) * EV;
-      is_k[j] = h >= a.num_heads;
-      const uint32_t hh = is_k[j] ? h - a.num_heads : h;
-      in_off[j] = (int64_t)hh * D * E;
-      const char* in = (is_k[j] ? a.key + (int64_t)t * a.k_token_stride
-                                : a.query + (int64_t)t * a.q_token_stride) + in_off[j];
-      if constexpr (VECTOR) {
-        if (is_k[j]) {
-          rx[j] = ld16<(NTL & 1) != 0>(in + (int64_t)e0[j] * E);
-          ry[j] = ld16<(NTL & 1) != 0>(in + (int64_t)(half + e0[j]) * E);
-        } else {
-          rx[j] = ld16<(NTL & 2) != 0>(in + (int64_t)e0[j] * E);
-          ry[j] = ld16<(NTL & 2) != 0>(in + (int64_t)(half + e0[j]) * E);
-        }
+  const bool rotates = !TAIL || (a.pairs_per_head != 0 && h < heads);
+  const bool is_k = h >= a.num_heads;
+  const uint32_t head_off = (is_k ? h - a.num_heads : h) * a.head_dim * E + pv;
+  u32x4 x, y;
+  if (rotates) {
+    if (NTL == 1 || NTL == 2) {
+      if (is_k) {
+        const char* in = a.key + (int64_t)t * a.k_token_stride + head_off;
+        x = ld16<(NTL & 1) != 0>(in);
+        y = ld16<(NTL & 1) != 0>(in + half);
       } else {
-        sx[j] = VT::load1(in + (int64_t)e0[j] * E);
-        sy[j] = VT::load1(in + (int64_t)(half + e0[j]) * E);
-      }
-    } else if (item < rot_items + tail_items) {
-      kind[j] = kTail;
-      const uint32_t it = item - rot_items;
-      const uint32_t h = it / tail_per_head;
-      e0[j] = rd + (it - h * tail_per_head) * EV;
-      is_k[j] = h >= a.num_heads;
-      const uint32_t hh = is_k[j] ? h - a.num_heads : h;
-      in_off[j] = ((int64_t)hh * D + e0[j]) * E;
-      const char* in = (is_k[j] ? a.key + (int64_t)t * a.k_token_stride
-                                : a.query + (int64_t)t * a.q_token_stride) + in_off[j];
-      if constexpr (VECTOR) rx[j] = is_k[j] ? ld16<(NTL & 1) != 0>(in) : ld16<(NTL & 2) != 0>(in);
-      else sx[j] = VT::load1(in);
-    } else if (item < rot_items + tail_items + v_items) {
-      kind[j] = kValue;
-      in_off[j] = (int64_t)(item - rot_items - tail_items) * EV * E;
-      const char* in = a.value + (int64_t)t * a.v_token_stride + in_off[j];
-      if constexpr (VECTOR) rx[j] = ld16<(NTL & 1) != 0>(in);
-      else sx[j] = VT::load1(in);
-    }
-  }
-
-  // ---- cos/sin row of this position: issue the loads (first vector of each lane) ----
-  const char* cs_row = a.cos_sin_cache + pos * (int64_t)(2 * rd) * E;
-  constexpr int CV = VT::kElems;  // whole 16-byte vectors when the row is aligned and a multiple of them
-  const uint32_t cs_vecs = 2 * rd / CV;
-  u32x4 cs_first = {0, 0, 0, 0};
-  if (a.cs_vector && threadIdx.x < cs_vecs)
-    cs_first = *reinterpret_cast<const u32x4*>(cs_row + (int64_t)threadIdx.x * 16);
-
-  // ---- slot of this token (workgroup-uniform) ----
-  // Placed after every vector load has been issued and before the first wait on
-  // them: the chain of dependent scalar loads runs while they are in flight.
-  char* kc_row = nullptr;
-  char* vc_row = nullptr;
-  if (a.key_cache) {
-    int64_t blk = -1, off = 0;
-    if (a.batch_indices) {
-      const int64_t b = a.batch_indices[t];
-      if (b >= 0 && b < a.batch_size) {
-        const int64_t pg = a.bs_shift >= 0 ? (pos >> a.bs_shift) : pos / a.block_size;
-        off = pos - pg * a.block_size;
-        const int64_t it = (int64_t)a.kv_indptr[b] + pg;
-        if (it >= 0 && it < (int64_t)a.kv_indptr[b + 1] && it < a.num_kv_indices) blk = a.kv_indices[it];
+        const char* in = a.query + (int64_t)t * a.q_token_stride + head_off;
+        x = ld16<(NTL & 2) != 0>(in);
+        y = ld16<(NTL & 2) != 0>(in + half);
       }
     } else {
-      const int64_t s = a.slot_bytes == 8 ? reinterpret_cast<const int64_t*>(a.slot_mapping)[t]
-                                          : (int64_t) reinterpret_cast<const int32_t*>(a.slot_mapping)[t];
-      if (s >= 0) {
-        blk = a.bs_shift >= 0 ? (s >> a.bs_shift) : s / a.block_size;
-        off = s - blk * a.block_size;
+      const char* in = (is_k ? a.key + (int64_t)t * a.k_token_stride : a.query + (int64_t)t * a.q_token_stride) + head_off;
+      x = ld16<NTL != 0>(in);
+      y = ld16<NTL != 0>(in + half);
+    }
+  }
+  // pass-through vectors of this lane: V first, then the tails of the heads
+  constexpr int kExtra = TAIL ? 2 : (ADDR == kNoCache ? 0 : 1);
+  u32x4 ev[kExtra + 1];
+  uint32_t eoff[kExtra + 1];  // byte offset inside the row it comes from == inside the row it goes to
+  int ekind[kExtra + 1];      // 0 none, 1 V, 2 tail of a Q head, 3 tail of a K head
+#pragma unroll
+  for (int j = 0; j < kExtra; ++j) {
+    const uint32_t e = lane + j * a.lanes_per_token;
+    ekind[j] = 0;
+    if (ADDR != kNoCache && e < a.v_items) {
+      ekind[j] = 1;
+      eoff[j] = e * 16;
+      ev[j] = ld16<(NTL & 1) != 0>(a.value + (int64_t)t * a.v_token_stride + eoff[j]);
+    } else if (TAIL) {
+      const uint32_t tail_per_head = (a.head_dim - a.rotary_dim) * E / 16;
+      if (e < a.v_items + heads * tail_per_head) {
+        const uint32_t i = e - a.v_items;
+        const uint32_t th = i / tail_per_head;
+        const bool tk = th >= a.num_heads;
+        ekind[j] = tk ? 3 : 2;
+        eoff[j] = ((tk ? th - a.num_heads : th) * a.head_dim + a.rotary_dim) * E + (i - th * tail_per_head) * 16;
+        ev[j] = tk ? ld16<(NTL & 1) != 0>(a.key + (int64_t)t * a.k_token_stride + eoff[j])
+                   : ld16<(NTL & 2) != 0>(a.query + (int64_t)t * a.q_token_stride + eoff[j]);
       }
     }
-    if (blk >= 0 && blk < a.num_cache_blocks) {
-      const int64_t slot_off = blk * a.cache_block_stride + off * a.cache_slot_stride;
-      kc_row = a.key_cache + slot_off;
-      vc_row = a.value_cache + slot_off;
-    }
   }
-  // ---- cos/sin row into LDS as fp32, shared by all heads ----
-  if (a.cs_vector) {
-    for (uint32_t i = threadIdx.x; i < cs_vecs; i += blockDim.x) {
-      float f[CV];
-      VT::unpack(i == threadIdx.x ? cs_first : *reinterpret_cast<const u32x4*>(cs_row + (int64_t)i * 16), f);
-#pragma unroll
-      for (int e = 0; e < CV; ++e) cs[i * CV + e] = f[e];
-    }
-  } else {
-    for (uint32_t i = threadIdx.x; i < 2 * rd; i += blockDim.x) cs[i] = VT::load1(cs_row + (int64_t)i * E);
-  }
-  __syncthreads();
 
-  // ---- compute and store ----
-  char* qo_row = a.query_out + (int64_t)t * a.qo_token_stride;
-  char* ko_row = a.key_out ? a.key_out + (int64_t)t * a.ko_token_stride : nullptr;
-#pragma unroll
-  for (int j = 0; j < IPL; ++j) {
-    // outs[0]: the rotated tensor handed back (read again by attention right away);
-    // outs[1]: the cache row of a K item (not read again by this step: non-temporal)
-    char* outs[2] = {is_k[j] ? ko_row : qo_row, is_k[j] ? kc_row : nullptr};
-    if (kind[j] == kRotate) {
-      float x[EV], y[EV], ox[EV], oy[EV];
-      if constexpr (VECTOR) {
-        VT::unpack(rx[j], x);
-        VT::unpack(ry[j], y);
-      } else {
-        x[0] = sx[j];
-        y[0] = sy[j];
+  if (pos < 0 || pos >= a.max_position) return;  // no cos/sin row: the token is left alone
+  u32x4 cos_x, cos_y, sin_x, sin_y;
+  if (rotates) {
+    const char* row = a.cos_sin_cache + pos * (int64_t)(4 * half) + pv;
+    cos_x = ld16<false>(row);
+    cos_y = ld16<false>(row + half);
+    sin_x = ld16<false>(row + 2 * half);
+    sin_y = ld16<false>(row + 3 * half);
+  }
+  const int64_t slot = slot_offset<ADDR, POW2>(a, t, pos);
+
+  if (rotates) {
+    u32x4 ox, oy;
+    VT::rotate(x, y, cos_x, cos_y, sin_x, sin_y, ox, oy);
+    if (!is_k) {  // read again by attention right away
+      char* out = a.query_out + (int64_t)t * a.qo_token_stride + head_off;
+      st16<NTQ>(out, ox);
+      st16<NTQ>(out + half, oy);
+    } else {
+      if (a.key_out) {
+        char* out = a.key_out + (int64_t)t * a.ko_token_stride + head_off;
+        st16<false>(out, ox);
+        st16<false>(out + half, oy);
       }
-#pragma unroll
-      for (int i = 0; i < EV; ++i) {
-        const float cos_x = cs[e0[j] + i], cos_y = cs[half + e0[j] + i];
-        const float sin_x = cs[rd + e0[j] + i], sin_y = cs[rd + half + e0[j] + i];
-        ox[i] = x[i] * cos_x - y[i] * sin_x;
-        oy[i] = y[i] * cos_y + x[i] * sin_y;
+      if (ADDR != kNoCache && slot >= 0) {  // the cache row is not read again by this step
+        char* out = a.key_cache + slot + head_off;
+        st16<true>(out, ox);
+        st16<true>(out + half, oy);
       }
+    }
+  }
 #pragma unroll
-      for (int o = 0; o < 2; ++o) {
-        if (!outs[o]) continue;
-        char* out = outs[o] + in_off[j];
-        if constexpr (VECTOR) {
-          u32x4* px = reinterpret_cast<u32x4*>(out + (int64_t)e0[j] * E);
-          u32x4* py = reinterpret_cast<u32x4*>(out + (int64_t)(half + e0[j]) * E);
-          if (o == 1) {
-            __builtin_nontemporal_store(VT::pack(ox), px);
-            __builtin_nontemporal_store(VT::pack(oy), py);
-          } else {
-            *px = VT::pack(ox);
-            *py = VT::pack(oy);
-          }
-        } else {
-          VT::store1(out + (int64_t)e0[j] * E, ox[0]);
-          VT::store1(out + (int64_t)(half + e0[j]) * E, oy[0]);
-        }
-      }
-    } else if (kind[j] == kTail) {
-      // lanes beyond rotary_dim pass through unchanged (partial rotary)
-#pragma unroll
-      for (int o = 0; o < 2; ++o) {
-        if (!outs[o]) continue;
-        if constexpr (VECTOR) *reinterpret_cast<u32x4*>(outs[o] + in_off[j]) = rx[j];
-        else VT::store1(outs[o] + in_off[j], sx[j]);
-      }
-    } else if (kind[j] == kValue && vc_row) {
-      // the V row goes to the cache as it is
-      if constexpr (VECTOR) __builtin_nontemporal_store(rx[j], reinterpret_cast<u32x4*>(vc_row + in_off[j]));
-      else VT::store1(vc_row + in_off[j], sx[j]);
+  for (int j = 0; j < kExtra; ++j) {
+    if (ekind[j] == 1) {
+      if (slot >= 0) st16<true>(a.value_cache + slot + eoff[j], ev[j]);
+    } else if (TAIL && ekind[j] == 2) {
+      st16<NTQ>(a.query_out + (int64_t)t * a.qo_token_stride + eoff[j], ev[j]);
+    } else if (TAIL && ekind[j] == 3) {
+      if (a.key_out) st16<false>(a.key_out + (int64_t)t * a.ko_token_stride + eoff[j], ev[j]);
+      if (ADDR != kNoCache && slot >= 0) st16<true>(a.key_cache + slot + eoff[j], ev[j]);
     }
   }
 }
 
-// One item per lane is what runs: 2 and 4 items per lane were measured from
-// 6 MiB to 324 MiB per launch and never gained (the launch is either latency-bound
-// or already has enough workgroups in flight).
-template <typename T, bool VECTOR>
-void launch_rope_ipl(const RopeArgs& a, dim3 grid, dim3 block, hipStream_t s) {
-  if constexpr (VECTOR) {
-    switch (kvc::g_rope_tune.nt & 3) {
-      case 1: hipLaunchKernelGGL((rope_cache_kernel<T, true, 1, 1>), grid, block, 0, s, a); break;
-      case 2: hipLaunchKernelGGL((rope_cache_kernel<T, true, 1, 2>), grid, block, 0, s, a); break;
-      case 3: hipLaunchKernelGGL((rope_cache_kernel<T, true, 1, 3>), grid, block, 0, s, a); break;
-      default: hipLaunchKernelGGL((rope_cache_kernel<T, true, 1, 0>), grid, block, 0, s, a); break;
+// Element path: rows that are no whole number of aligned 16-byte vectors. One
+// rotation pair or one pass-through element per lane, in this order: pairs of the
+// Q heads then the K heads, elements beyond rotary_dim, V.
+template <typename T>
+__global__ __launch_bounds__(kThreads) void rope_element_kernel(RopeArgs a) {
+  using VT = Vec<T>;
+  constexpr int E = T::kBytes;
+  const uint32_t t = blockIdx.x / a.groups_per_token;
+  const uint32_t item = (blockIdx.x - t * a.groups_per_token) * blockDim.x + threadIdx.x;
+  const int64_t pos = index_of(a.positions, a.pos_bytes, t);
+  if (pos < 0 || pos >= a.max_position) return;  // no cos/sin row: the token is left alone
+  const uint32_t rd = a.rotary_dim, half = rd >> 1, D = a.head_dim;
+  const uint32_t heads = a.num_heads + a.num_kv_heads;
+  const uint32_t rot_items = heads * half, tail_per_head = D - rd, tail_items = heads * tail_per_head;
+  const int64_t slot = !a.key_cache ? -1 : a.batch_indices ? slot_offset<kPages, false>(a, t, pos)
+                                                         : slot_offset<kSlots, false>(a, t, pos);
+  const char* cs = a.cos_sin_cache + pos * (int64_t)(2 * rd) * E;
+  if (item < rot_items + tail_items) {
+    const bool pair = item < rot_items;
+    const uint32_t i = pair ? item : item - rot_items;
+    const uint32_t h = pair ? i / half : i / tail_per_head;
+    const uint32_t e = pair ? i - h * half : rd + (i - h * tail_per_head);
+    const bool is_k = h >= a.num_heads;
+    const int64_t off = ((int64_t)(is_k ? h - a.num_heads : h) * D + e) * E;
+    const char* in = (is_k ? a.key + (int64_t)t * a.k_token_stride : a.query + (int64_t)t * a.q_token_stride) + off;
+    char* outs[2] = {is_k ? (a.key_out ? a.key_out + (int64_t)t * a.ko_token_stride + off : nullptr)
+                          : a.query_out + (int64_t)t * a.qo_token_stride + off,
+                     is_k && slot >= 0 ? a.key_cache + slot + off : nullptr};
+    float ox = VT::load1(in), oy = 0.f;
+    if (pair) {
+      const float x = ox, y = VT::load1(in + (int64_t)half * E);
+      const float cos_x = VT::load1(cs + (int64_t)e * E), cos_y = VT::load1(cs + (int64_t)(half + e) * E);
+      const float sin_x = VT::load1(cs + (int64_t)(rd + e) * E), sin_y = VT::load1(cs + (int64_t)(rd + half + e) * E);
+      ox = x * cos_x - y * sin_x;
+      oy = y * cos_y + x * sin_y;
     }
-  } else {
-    hipLaunchKernelGGL((rope_cache_kernel<T, false, 1, 0>), grid, block, 0, s, a);
+#pragma unroll
+    for (int o = 0; o < 2; ++o) {
+      if (!outs[o]) continue;
+      VT::store1(outs[o], ox);
+      if (pair) VT::store1(outs[o] + (int64_t)half * E, oy);
+    }
+  } else if (a.key_cache && item < rot_items + tail_items + a.num_kv_heads * D) {
+    const int64_t off = (int64_t)(item - rot_items - tail_items) * E;
+    if (slot >= 0) VT::store1(a.value_cache + slot + off, VT::load1(a.value + (int64_t)t * a.v_token_stride + off));
+  }
+}
+
+template <typename T, Addressing ADDR, bool POW2, bool TAIL, int NTL>
+void launch_vector_ntq(const RopeArgs& a, bool ntq, dim3 grid, dim3 block, hipStream_t s) {
+  if (ntq) hipLaunchKernelGGL((rope_vector_kernel<T, ADDR, POW2, TAIL, NTL, true>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((rope_vector_kernel<T, ADDR, POW2, TAIL, NTL, false>), grid, block, 0, s, a);
+}
+
+template <typename T, Addressing ADDR>
+void launch_vector(const RopeArgs& a, bool pow2, bool tail, bool ntq, dim3 grid, dim3 block, hipStream_t s) {
+  switch (kvc::g_rope_tune.nt & 3) {
+    case 0:
+      if (pow2 && !tail) launch_vector_ntq<T, ADDR, true, false, 0>(a, ntq, grid, block, s);
+      else if (pow2) launch_vector_ntq<T, ADDR, true, true, 0>(a, ntq, grid, block, s);
+      else launch_vector_ntq<T, ADDR, false, true, 0>(a, ntq, grid, block, s);
+      break;
+    case 1: launch_vector_ntq<T, ADDR, false, true, 1>(a, ntq, grid, block, s); break;
+    case 2: launch_vector_ntq<T, ADDR, false, true, 2>(a, ntq, grid, block, s); break;
+    default: launch_vector_ntq<T, ADDR, false, true, 3>(a, ntq, grid, block, s); break;
   }
 }
 
 template <typename T>
-void launch_rope(const RopeArgs& a, int64_t num_tokens, bool vector, unsigned threads,
-                 hipStream_t s) {
-  const dim3 grid((unsigned)(num_tokens * a.groups_per_token)), block(threads);
-  if (vector) launch_rope_ipl<T, true>(a, grid, block, s);
-  else launch_rope_ipl<T, false>(a, grid, block, s);
+int launch_rope(RopeArgs a, int64_t num_tokens, bool vector, bool tail, bool ntq, unsigned threads,
+                hipStream_t s) {
+  if (!vector) {
+    hipLaunchKernelGGL((rope_element_kernel<T>), dim3((unsigned)(num_tokens * a.groups_per_token)), dim3(threads),
+                       0, s, a);
+    KVC_HIP(hipGetLastError());
+    return KVC_OK;
+  }
+  const bool pow2 = a.bs_shift >= 0;
+  constexpr int64_t kMaxY = 65535;  // tokens of one launch
+  const int64_t slot_step = a.slot_bytes, pos_step = a.pos_bytes;
+  for (int64_t t0 = 0; t0 < num_tokens; t0 += kMaxY) {
+    const dim3 grid(a.groups_per_token, (unsigned)std::min(kMaxY, num_tokens - t0)), block(threads);
+    if (!a.key_cache) launch_vector<T, kNoCache>(a, true, tail, ntq, grid, block, s);
+    else if (a.batch_indices) launch_vector<T, kPages>(a, pow2, tail, ntq, grid, block, s);
+    else launch_vector<T, kSlots>(a, pow2, tail, ntq, grid, block, s);
+    KVC_HIP(hipGetLastError());
+    a.query += kMaxY * a.q_token_stride;
+    a.key += kMaxY * a.k_token_stride;
+    if (a.value) a.value += kMaxY * a.v_token_stride;
+    a.query_out += kMaxY * a.qo_token_stride;
+    if (a.key_out) a.key_out += kMaxY * a.ko_token_stride;
+    a.positions = (const char*)a.positions + kMaxY * pos_step;
+    if (a.slot_mapping) a.slot_mapping = (const char*)a.slot_mapping + kMaxY * slot_step;
+    if (a.batch_indices) a.batch_indices += kMaxY;
+  }
+  return KVC_OK;
 }
 
 struct RopeGeom {
@@ -470,36 +517,61 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
              (uint64_t)a.v_token_stride | (uint64_t)a.cache_block_stride |
              (uint64_t)a.cache_slot_stride;
   }
-  // 16-byte vectors need aligned rows and halves that hold whole vectors
+  // 16-byte vectors need aligned rows and halves that hold whole vectors (and offsets inside a row that fit
+  // 32 bits)
   const int ev = 16 / E;
-  const bool vector = (align % 16 == 0) && ((g.rotary_dim / 2) % ev == 0) &&
+  align |= (uintptr_t)cos_sin_cache;
+  const bool vector = (align % 16 == 0) && (g.num_heads + g.num_kv_heads) * g.head_dim * E <= (int64_t(1) << 29) && ((g.rotary_dim / 2) % ev == 0) &&
                       ((g.head_dim - g.rotary_dim) % ev == 0) && (g.head_dim % ev == 0);
-  const int64_t ev_used = vector ? ev : 1;
   const int64_t heads = g.num_heads + g.num_kv_heads;
-  const int64_t items = heads * ((g.rotary_dim / 2) / ev_used) +
-                        heads * ((g.head_dim - g.rotary_dim) / ev_used) +
-                        (c ? g.num_kv_heads * g.head_dim / ev_used : 0);
-  a.pv_shift = log2_exact((g.rotary_dim / 2) / ev_used);
-  a.cs_vector = ((uintptr_t)a.cos_sin_cache % 16 == 0) && ((2 * g.rotary_dim * E) % 16 == 0) ? 1 : 0;
-  // Lanes per workgroup, from graph-timed sweeps (64 to 8192 tokens): the plain
-  // rotation runs the same with 64 or 128 lanes and slower with 256; with the
-  // cache write fused in, one wavefront per workgroup is 3-9 % faster than two
-  // (the barrier then costs nothing, and a workgroup whose slot chain is late
-  // holds back fewer lanes).
   unsigned threads = (unsigned)kvc::g_rope_tune.threads;
-  if (threads != 64 && threads != 128 && threads != 256) threads = c ? 64 : 128;
-  a.groups_per_token = (uint32_t)std::max<int64_t>(1, (items + threads - 1) / threads);
+  const bool fixed = threads == 64 || threads == 128 || threads == 192 || threads == 256;
+  bool tail = false, ntq = false;
+  if (vector) {
+    const int64_t pairs = heads * ((g.rotary_dim / 2) / ev);
+    const int64_t v_items = c ? g.num_kv_heads * g.head_dim / ev : 0;
+    const int64_t extras = heads * ((g.head_dim - g.rotary_dim) / ev) + v_items;
+    const int64_t lanes = std::max(pairs, (extras + 1) / 2);  // at most two pass-through vectors per lane
+    tail = g.rotary_dim < g.head_dim || v_items > pairs;
+    a.v_items = (uint32_t)v_items;
+    a.lanes_per_token = (uint32_t)lanes;
+    a.pairs_per_head = (uint32_t)((g.rotary_dim / 2) / ev);
+    // exact for every lane: lanes * pairs_per_head < 2^32 (lanes < 2^25, at most 64 pair-vectors per head)
+    a.pairs_magic = a.pairs_per_head > 1 ? (uint32_t)(((uint64_t(1) << 32) + a.pairs_per_head - 1) / a.pairs_per_head) : 0;
+    a.pairs_one = a.pairs_per_head == 1 ? ~0u : 0u;
+    // The largest workgroup that cuts a token into an ODD number of workgroups. They are dealt round-robin to
+    // the 8 XCDs; with an even number every second XCD gets only first halves (with the V vectors), the others
+    // only the short last ones: 40 heads x 128 (5 wavefronts), 2048 tokens, as 3 x 128 lanes 9.5 us, as 5 x 64
+    // 9.7, as 2 x 192 10.5, as 2 x 256 11.3; 40 heads x 64 (3 wavefronts) as 1 x 256 6.3, as 2 x 128 7.0.
+    const int64_t waves = (lanes + 63) / 64;
+    if (!fixed) {
+      threads = 256;
+      for (unsigned w = 4; w >= 1; --w)
+        if ((waves + w - 1) / w % 2 == 1) {
+          threads = 64 * w;
+          break;
+        }
+    }
+    a.groups_per_token = (uint32_t)std::max<int64_t>(1, (lanes + threads - 1) / threads);
+    // query_out past the caches: from 48 MiB on it no longer fits the L2s (8 x 4 MiB) beside what else the
+    // launch moves. A rotation followed by a kernel that reads query_out: 134 MB 77.6 us against 79.6,
+    // 67 MB 46.7 against 47.8, 59 MB 37.4 against 38.3; at 33 MB 26.7 against 26.2 and below it costs more.
+    ntq = g.num_tokens * g.num_heads * g.head_dim * E >= (int64_t(48) << 20);
+  } else {
+    const int64_t items = heads * (g.rotary_dim / 2) + heads * (g.head_dim - g.rotary_dim) +
+                          (c ? g.num_kv_heads * g.head_dim : 0);
+    if (!fixed) threads = 128;
+    a.groups_per_token = (uint32_t)std::max<int64_t>(1, (items + threads - 1) / threads);
+  }
   if (g.num_tokens * (int64_t)a.groups_per_token > 0x7fffffffll)
     return fail(KVC_ERR_UNSUPPORTED, "%s: launch of %lld workgroups is too large", fn,
                 (long long)(g.num_tokens * (int64_t)a.groups_per_token));
   hipStream_t s = (hipStream_t)stream;
   switch (g.dtype) {
-    case KVC_DTYPE_BF16: launch_rope<BF16>(a, g.num_tokens, vector, threads, s); break;
-    case KVC_DTYPE_F16: launch_rope<F16>(a, g.num_tokens, vector, threads, s); break;
-    default: launch_rope<F32>(a, g.num_tokens, vector, threads, s); break;
+    case KVC_DTYPE_BF16: return launch_rope<BF16>(a, g.num_tokens, vector, tail, ntq, threads, s);
+    case KVC_DTYPE_F16: return launch_rope<F16>(a, g.num_tokens, vector, tail, ntq, threads, s);
+    default: return launch_rope<F32>(a, g.num_tokens, vector, tail, ntq, threads, s);
   }
-  KVC_HIP(hipGetLastError());
-  return KVC_OK;
 }
 
 }  // namespace

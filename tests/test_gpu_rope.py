@@ -469,3 +469,45 @@ def test_distance_to_the_reference_kernels_possible_roundings(gpu, name, T, Hq, 
     # observed: never more than ONE such ulp, with 70-83 % of the lanes bit-identical; the
     # analytic bound above is the guarantee
     assert max(worst.values()) <= 1.0, worst
+
+
+@pytest.mark.parametrize("T,Hq,Hkv,D,rd,dtype,bs", [
+    (5, 3, 1, 16, 16, torch.bfloat16, 16),       # one pair-vector per head
+    (37, 5, 3, 96, 96, torch.float16, 16),       # six: no power of two; a last wavefront of partly idle lanes
+    (33, 2, 6, 64, 64, torch.bfloat16, 16),      # more V vectors than pair-vectors
+    (29, 4, 2, 80, 32, torch.float16, 16),       # two pass-through vectors per lane, from V and from the tails
+    (29, 4, 2, 72, 16, torch.float32, 16),
+    (40, 4, 2, 64, 64, torch.bfloat16, 12),      # block size that is no power of two
+    (65537, 1, 1, 16, 16, torch.bfloat16, 16),   # one token more than a launch holds
+    (6144, 32, 1, 128, 128, torch.bfloat16, 16),  # query_out of 48 MiB: stored past the caches
+])
+def test_shapes_at_the_edges_of_the_vector_kernel(gpu, T, Hq, Hkv, D, rd, dtype, bs):
+    """Rotation against the float64 formula (half an ulp), rows and their places in the cache bit for bit, through
+    the slot mapping and through the page table, and with a table that is not 16-byte aligned (element path)."""
+    q, k, v, pos, cs = (t.to(gpu) for t in _case(gpu, T, Hq, Hkv, D, rd, dtype, max_pos=T + bs, seed=T + D))
+    pos = torch.arange(T, device=gpu, dtype=torch.int32)      # one request whose tokens are positions 0..T-1
+    nb = T // bs + 3
+    pages = torch.from_numpy(np.random.default_rng(T).permutation(nb)[:T // bs + 1].astype(np.int32)).to(gpu)
+    slots = pages.long()[(pos // bs).long()] * bs + pos.long() % bs
+    slots[0] = -1                                             # skipped by the write, rotated all the same
+    pool = torch.zeros(nb, 2, bs, Hkv, D, dtype=dtype, device=gpu)
+    q_out, k_out = kvc.rotary_pos_emb_and_cache(q, k, v, pos, cs, D, pool, slots)
+    want = torch.zeros_like(pool)
+    b, e = slots[1:] // bs, slots[1:] % bs
+    want[b, 0, e] = k_out[1:].view(-1, Hkv, D)
+    want[b, 1, e] = v[1:].view(-1, Hkv, D)
+    assert torch.equal(pool, want)
+    some = slice(0, T, max(1, T // 500))
+    for got, x, name in ((q_out, q, "query"), (k_out, k, "key")):
+        _check_rotation(got[some].cpu(), x[some].cpu(), pos[some].cpu(), cs.cpu(), D, dtype, name)
+    indptr = torch.tensor([0, pages.numel()], dtype=torch.int32, device=gpu)
+    last = torch.tensor([(T - 1) % bs + 1], dtype=torch.int32, device=gpu)
+    owner = torch.zeros(T, dtype=torch.int32, device=gpu)
+    owner[0] = -1
+    paged = torch.zeros_like(pool)
+    q_paged, k_paged = kvc.rotary_pos_emb_and_append_paged(q, k, v, owner, pos, cs, D, paged, pages, indptr, last)
+    assert torch.equal(paged, want) and torch.equal(q_paged, q_out) and torch.equal(k_paged, k_out)
+    odd = torch.empty(cs.numel() + 1, dtype=dtype, device=gpu)[1:].view(cs.shape)
+    odd.copy_(cs)
+    q_odd, k_odd = kvc.rotary_pos_emb(q, k, pos, odd, D)
+    assert torch.equal(q_odd, q_out) and torch.equal(k_odd, k_out)

@@ -107,6 +107,30 @@ int kvc_write_runs_layers(const void* key, const void* value,
                           int elem_bytes, void* stream);
 
 /*
+ * A step's inputs without a copy command. kvc_staging_acquire hands out one of the
+ * calling thread's pinned buffers (at least `bytes`, 16-byte aligned), to be filled by
+ * the caller; the next of the two calls below on the same thread launches a kernel that
+ * reads it over the link, and the buffer is reused by itself once the kernel has. An
+ * acquired buffer that no launch follows is handed out again. kvc_thread_release frees
+ * them. Not under stream capture (KVC_ERR_UNSUPPORTED): a replay would read what the
+ * buffer holds by then. No counterpart in the reference, which uploads six tensors per
+ * step (runtime/worker/llm_worker/model_worker.py:399-423).
+ *
+ * kvc_staging_upload copies the first `bytes` (whole 16-byte vectors) to dst.
+ * kvc_build_write_index_staged is kvc_build_write_index on a buffer that holds, as
+ * int32, input_lens | context_lens | num_blocks (batch_size each, then padded to a
+ * multiple of four words) | the concatenated block tables; kv_indices, 16-byte aligned,
+ * receives the tables. batch_size >= 1; slot_mapping may be NULL.
+ */
+int kvc_staging_acquire(int64_t bytes, void** out);
+int kvc_staging_upload(void* dst, int64_t bytes, void* stream);
+int kvc_build_write_index_staged(int64_t batch_size, int64_t num_kv_indices, int64_t page_size,
+                                 int64_t nnz, int32_t* cu_seqlens_q, int32_t* kv_indptr,
+                                 int32_t* kv_last_page_len, int32_t* kv_indices,
+                                 int32_t* batch_indices, int32_t* positions,
+                                 int64_t* slot_mapping, void* stream);
+
+/*
  * Do two streams feed the same hardware queue? The runtime maps every stream of
  * a process onto a few hardware queues (4 unless GPU_MAX_HW_QUEUES says
  * otherwise). Kernels of streams that share one run one after the other, and a

@@ -103,6 +103,9 @@ SIGNATURES = {
     "kvc_get_batch_indices_positions": (c_int, [_P, _P, _I64, _I64, _P, _P, _P]),
     "kvc_build_write_index": (c_int, [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _P, _P, _P, _P, _P, _P,
                                       _P, _P, _P, _I64, _P]),
+    "kvc_staging_acquire": (c_int, [_I64, ctypes.POINTER(_P)]),
+    "kvc_staging_upload": (c_int, [_P, _I64, _P]),
+    "kvc_build_write_index_staged": (c_int, [_I64, _I64, _I64, _I64, _P, _P, _P, _P, _P, _P, _P, _P]),
     "kvc_slot_runs": (c_int, [_P, c_int, _I64, _I64, _P, _P, _I64, _P]),
     "kvc_streams_share_hw_queue": (c_int, [_P, _P, _P]),
     "kvc_write_runs_layers": (c_int, [_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64,

@@ -619,17 +619,23 @@ __global__ void batch_indices_positions_kernel(const int32_t* append_indptr,
   }
 }
 
-// Whole index preparation of a step in one launch (one workgroup): prefix sums
-// of the per-request new-token counts, block counts and block-run counts, the
-// last-page fill, and for every new token its request, absolute position and
-// slot. The per-token outputs are CAPACITY-bound: entries from the step's token
-// count up to `nnz` are filled with -1 (a request index, position and slot every
-// write kernel skips), so a launch recorded once for `nnz` tokens serves steps
-// of any smaller size.
+// Whole index preparation of a step in one launch: prefix sums of the per-request
+// new-token counts, block counts and block-run counts, the last-page fill, and for
+// every new token its request, absolute position and slot. The per-token outputs
+// are CAPACITY-bound: entries from the step's token count up to `nnz` are filled
+// with -1 (a request index, position and slot every write kernel skips), so a
+// launch recorded once for `nnz` tokens serves steps of any smaller size.
 // A block run is a maximal range of a request's new tokens that falls into one
 // block: consecutive tokens on the source side, consecutive cache entries on
 // the other. Its descriptor is four int32: first token, block id, first entry,
 // token count. The first token of every run writes it.
+// The inputs may lie in pinned host memory: the launch then is the upload too
+// (`ids_out`, `words`: the block tables go to the device on the way, 16 bytes a
+// lane, read before the scans and stored after them so that the two waits on the
+// link overlap).
+// Bound: latency. Every workgroup scans the (at most 1024) requests for itself and
+// takes its share of the tokens and of the tables; one workgroup for all of them
+// walked 8192 tokens in 8 rounds of dependent loads (12.7 us; 6.3 at 2048).
 constexpr int kPrepThreads = 1024;
 
 // Inclusive scan of three values over the workgroup's 1024 lanes: shuffles inside
@@ -659,50 +665,84 @@ __device__ __forceinline__ void scan3(int32_t& q, int32_t& n, int32_t& r, int32_
   }
 }
 
-__global__ __launch_bounds__(kPrepThreads) void build_write_index_kernel(
-    const int32_t* input_lens, const int32_t* context_lens, const int32_t* num_blocks,
-    const int32_t* kv_indices, int32_t batch_size, int64_t num_kv_indices, int32_t page_size,
-    int64_t nnz, int32_t* cu_seqlens_q, int32_t* kv_indptr, int32_t* kv_last_page_len,
-    int32_t* batch_indices, int32_t* positions, int64_t* slot_mapping, int32_t* run_indptr,
-    int32_t* runs, int32_t* num_runs, int64_t max_runs) {
+struct IndexArgs {
+  const int32_t *input_lens, *context_lens, *num_blocks, *kv_indices;  // device or pinned host memory
+  int32_t batch_size, page_size;
+  int64_t num_kv_indices, nnz;
+  int32_t *cu_seqlens_q, *kv_indptr, *kv_last_page_len, *batch_indices, *positions;
+  int64_t* slot_mapping;
+  int32_t *run_indptr, *runs, *num_runs;
+  int64_t max_runs;
+  int32_t* ids_out;      // copy of kv_indices on the device, or null
+  uint32_t* read_flags;  // one word per workgroup in host memory, or null:
+  uint32_t flag_value;   // set to this once the workgroup has read its inputs
+};
+
+// One word per workgroup tells the host that the workgroup is done with a staging
+// buffer. Relaxed is enough: whatever a lane read from the buffer it has stored or
+// branched on before the barrier, so those loads have returned; a release at system
+// scope would write the L2 back first.
+__device__ __forceinline__ void tell_host(uint32_t* flags, uint32_t value) {
+  __syncthreads();
+  if (threadIdx.x == 0)
+    __hip_atomic_store(flags + blockIdx.x, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__global__ __launch_bounds__(kPrepThreads) void build_write_index_kernel(IndexArgs a) {
   __shared__ int32_t carry[3];
   __shared__ int32_t wave_sums[kPrepThreads / 64][3];
   // prefix sums of a batch that fits one chunk stay in LDS for the per-token part
   __shared__ int32_t lds_cu[kPrepThreads + 1], lds_indptr[kPrepThreads + 1], lds_runptr[kPrepThreads + 1];
+  __shared__ int32_t lds_ctx[kPrepThreads];
   const int tid = threadIdx.x;
-  const bool in_lds = batch_size <= kPrepThreads;
+  const bool first_wg = blockIdx.x == 0;
+  const int32_t page_size = a.page_size;
+  const int64_t lane0 = (int64_t)blockIdx.x * kPrepThreads + tid, lanes = (int64_t)gridDim.x * kPrepThreads;
+  // the lane's first 16 bytes of the block tables
+  const int64_t words4 = a.ids_out ? a.num_kv_indices / 4 : 0;
+  const bool has_ids = lane0 < words4;
+  int4 ids = make_int4(0, 0, 0, 0);
+  if (has_ids) ids = reinterpret_cast<const int4*>(a.kv_indices)[lane0];
+  // a batch beyond one chunk keeps its prefix sums in the outputs and is launched as one workgroup
+  const bool in_lds = a.batch_size <= kPrepThreads;
   if (tid == 0) {
     carry[0] = carry[1] = carry[2] = 0;
-    cu_seqlens_q[0] = 0;
-    kv_indptr[0] = 0;
-    if (run_indptr) run_indptr[0] = 0;
     lds_cu[0] = lds_indptr[0] = lds_runptr[0] = 0;
+    if (first_wg) {
+      a.cu_seqlens_q[0] = 0;
+      a.kv_indptr[0] = 0;
+      if (a.run_indptr) a.run_indptr[0] = 0;
+    }
   }
   // every descriptor starts out empty: a run whose first token lies beyond `nnz` is never written
-  if (runs)
-    for (int64_t r = tid; r < max_runs; r += kPrepThreads)
-      reinterpret_cast<int4*>(runs)[r] = make_int4(0, -1, 0, 0);
+  // (a launch with descriptors is one workgroup: the barrier orders this before the tokens)
+  if (a.runs)
+    for (int64_t r = tid; r < a.max_runs; r += kPrepThreads)
+      reinterpret_cast<int4*>(a.runs)[r] = make_int4(0, -1, 0, 0);
   __syncthreads();
-  for (int32_t base = 0; base < batch_size; base += kPrepThreads) {
+  for (int32_t base = 0; base < a.batch_size; base += kPrepThreads) {
     const int32_t b = base + tid;
-    int32_t q = b < batch_size ? input_lens[b] : 0;
-    int32_t n = b < batch_size ? num_blocks[b] : 0;
-    const int32_t ctx = b < batch_size ? context_lens[b] : 0;
+    int32_t q = b < a.batch_size ? a.input_lens[b] : 0;
+    int32_t n = b < a.batch_size ? a.num_blocks[b] : 0;
+    const int32_t ctx = b < a.batch_size ? a.context_lens[b] : 0;
     // runs of the request: the blocks its new positions [ctx - q, ctx) touch
     int32_t nr = (q > 0 && ctx >= q) ? (ctx - 1) / page_size - (ctx - q) / page_size + 1 : 0;
     scan3(q, n, nr, wave_sums);
     q += carry[0];
     n += carry[1];
     nr += carry[2];
-    if (b < batch_size) {
-      cu_seqlens_q[b + 1] = q;
-      kv_indptr[b + 1] = n;
-      if (run_indptr) run_indptr[b + 1] = nr;
-      kv_last_page_len[b] = ctx > 0 ? (ctx - 1) % page_size + 1 : 0;
+    if (b < a.batch_size) {
+      if (first_wg) {
+        a.cu_seqlens_q[b + 1] = q;
+        a.kv_indptr[b + 1] = n;
+        if (a.run_indptr) a.run_indptr[b + 1] = nr;
+        a.kv_last_page_len[b] = ctx > 0 ? (ctx - 1) % page_size + 1 : 0;
+      }
       if (in_lds) {
         lds_cu[b + 1] = q;
         lds_indptr[b + 1] = n;
         lds_runptr[b + 1] = nr;
+        lds_ctx[b] = ctx;
       }
     }
     __syncthreads();  // everyone has read the carry
@@ -713,23 +753,24 @@ __global__ __launch_bounds__(kPrepThreads) void build_write_index_kernel(
     }
     __syncthreads();
   }
-  if (tid == 0 && num_runs) *num_runs = (int32_t)(carry[2] < max_runs ? carry[2] : max_runs);
+  if (first_wg && tid == 0 && a.num_runs) *a.num_runs = (int32_t)(carry[2] < a.max_runs ? carry[2] : a.max_runs);
   // per token: find its request by bisection over the prefix sums just written
   // (visible to the whole workgroup after the barrier above); the request's new
   // tokens occupy positions [context - input, context)
-  const int32_t* cu = in_lds ? lds_cu : cu_seqlens_q;
-  const int32_t* indptr = in_lds ? lds_indptr : kv_indptr;
-  const int32_t* runptr = in_lds ? lds_runptr : run_indptr;
+  const int32_t* cu = in_lds ? lds_cu : a.cu_seqlens_q;
+  const int32_t* indptr = in_lds ? lds_indptr : a.kv_indptr;
+  const int32_t* runptr = in_lds ? lds_runptr : a.run_indptr;
+  const int32_t* context = in_lds ? lds_ctx : a.context_lens;
   const int64_t total = carry[0];
-  const int64_t limit = total < nnz ? total : nnz;
-  for (int64_t out = tid; out < nnz; out += kPrepThreads) {
+  const int64_t limit = total < a.nnz ? total : a.nnz;
+  for (int64_t out = lane0; out < a.nnz; out += lanes) {
     if (out >= limit) {  // beyond this step's tokens: entries every write kernel skips
-      batch_indices[out] = -1;
-      positions[out] = -1;
-      if (slot_mapping) slot_mapping[out] = -1;
+      a.batch_indices[out] = -1;
+      a.positions[out] = -1;
+      if (a.slot_mapping) a.slot_mapping[out] = -1;
       continue;
     }
-    int32_t lo = 0, hi = batch_size;  // invariant: cu[lo] <= out < cu[hi]
+    int32_t lo = 0, hi = a.batch_size;  // invariant: cu[lo] <= out < cu[hi]
     while (hi - lo > 1) {
       const int32_t mid = (lo + hi) >> 1;
       if (cu[mid] <= out) lo = mid;
@@ -739,26 +780,42 @@ __global__ __launch_bounds__(kPrepThreads) void build_write_index_kernel(
     const int32_t begin = cu[b];
     const int32_t n_new = cu[b + 1] - begin;
     const int32_t j = (int32_t)(out - begin);
-    const int32_t ctx = context_lens[b];
+    const int32_t ctx = context[b];
     const int32_t pos = ctx - n_new + j;
-    batch_indices[out] = b;
-    positions[out] = pos;
+    a.batch_indices[out] = b;
+    a.positions[out] = pos;
     const int64_t it = (int64_t)indptr[b] + pos / page_size;
-    const int64_t table_end = indptr[b + 1] < num_kv_indices ? indptr[b + 1] : num_kv_indices;
+    const int64_t table_end = indptr[b + 1] < a.num_kv_indices ? indptr[b + 1] : a.num_kv_indices;
     const bool in_table = pos >= 0 && it >= 0 && it < table_end;
-    const int32_t block = in_table ? kv_indices[it] : -1;
-    if (slot_mapping) slot_mapping[out] = in_table ? (int64_t)block * page_size + pos % page_size : -1;
-    if (runs && pos >= 0 && ctx >= n_new && (j == 0 || pos % page_size == 0)) {
+    const int32_t block = in_table ? a.kv_indices[it] : -1;
+    if (a.slot_mapping) a.slot_mapping[out] = in_table ? (int64_t)block * page_size + pos % page_size : -1;
+    if (a.runs && pos >= 0 && ctx >= n_new && (j == 0 || pos % page_size == 0)) {
       const int32_t first_pos = ctx - n_new;
       const int64_t r = (int64_t)runptr[b] + (pos / page_size - first_pos / page_size);
-      if (r >= 0 && r < max_runs) {
+      if (r >= 0 && r < a.max_runs) {
         int64_t count = page_size - pos % page_size;
         if (count > n_new - j) count = n_new - j;
-        if (count > nnz - out) count = nnz - out;
-        reinterpret_cast<int4*>(runs)[r] = make_int4((int32_t)out, block, pos % page_size, (int32_t)count);
+        if (count > a.nnz - out) count = a.nnz - out;
+        reinterpret_cast<int4*>(a.runs)[r] = make_int4((int32_t)out, block, pos % page_size, (int32_t)count);
       }
     }
   }
+  if (a.ids_out) {
+    if (has_ids) reinterpret_cast<int4*>(a.ids_out)[lane0] = ids;
+    for (int64_t i = lane0 + lanes; i < words4; i += lanes)
+      reinterpret_cast<int4*>(a.ids_out)[i] = reinterpret_cast<const int4*>(a.kv_indices)[i];
+    const int64_t i = 4 * words4 + lane0;  // the last words
+    if (i < a.num_kv_indices) a.ids_out[i] = a.kv_indices[i];
+  }
+  if (a.read_flags) tell_host(a.read_flags, a.flag_value);
+}
+
+// Staging buffer (pinned host memory) -> device buffer, 16 bytes a lane.
+__global__ __launch_bounds__(kThreads) void upload_kernel(const int4* src, int4* dst, int64_t words4,
+                                                          uint32_t* read_flags, uint32_t flag_value) {
+  for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < words4; i += (int64_t)gridDim.x * kThreads)
+    dst[i] = src[i];
+  tell_host(read_flags, flag_value);
 }
 
 // Block runs of an arbitrary slot mapping (one workgroup): token t opens a run
@@ -1767,6 +1824,118 @@ int run_swap(const char* fn, bool out, char* pool, char* host_pool, const int64_
   return KVC_OK;
 }
 
+// --------------------------- staging of a step's inputs ----------------------
+// A ring of pinned buffers per thread in which a binding assembles what a small
+// kernel then reads over the link itself: no copy command, no event (a recorded
+// event costs 3 us of host time here, a launch 3). Each workgroup of the reading
+// kernel sets a word in the buffer's head when it has read its share; a buffer is
+// handed out again once all have. Bounded: kStageSlots buffers of the largest size
+// asked for (rounded up to a power of two); kvc_thread_release gives them back.
+constexpr int kStageSlots = 4;
+constexpr int kStageMaxWgs = 64;
+constexpr int64_t kStageHead = kStageMaxWgs * (int64_t)sizeof(uint32_t);
+
+struct StageRing {
+  char* base = nullptr;
+  int64_t slot_bytes = 0;  // head included
+  int next = 0;
+  uint32_t seq = 0;
+  uint32_t used_seq[kStageSlots] = {};
+  int used_wgs[kStageSlots] = {};  // workgroups of the last kernel that read the slot, 0 = none
+  int64_t acquired = -1;           // bytes of the slot that is being filled, -1 = none
+};
+thread_local StageRing g_stage;
+
+// Wait until the last reader of slot i is through. It normally has been for several
+// calls; a reader that is still queued behind long work is waited for like an event.
+int stage_wait(StageRing& r, int i) {
+  if (!r.used_wgs[i]) return KVC_OK;
+  const uint32_t* flags = reinterpret_cast<const uint32_t*>(r.base + i * r.slot_bytes);
+  const auto read = [&] {
+    for (int w = 0; w < r.used_wgs[i]; ++w)
+      if (__atomic_load_n(flags + w, __ATOMIC_ACQUIRE) != r.used_seq[i]) return false;
+    return true;
+  };
+  for (int spin = 0; spin < 20000; ++spin)
+    if (read()) {
+      r.used_wgs[i] = 0;
+      return KVC_OK;
+    }
+  KVC_HIP(hipDeviceSynchronize());
+  r.used_wgs[i] = 0;
+  return KVC_OK;
+}
+
+int stage_release() {
+  StageRing& r = g_stage;
+  if (!r.base) return KVC_OK;
+  for (int i = 0; i < kStageSlots; ++i) {
+    const int rc = stage_wait(r, i);
+    if (rc != KVC_OK) return rc;
+  }
+  char* base = r.base;
+  r = StageRing{};
+  KVC_HIP(hipHostFree(base));
+  return KVC_OK;
+}
+
+int stage_acquire(int64_t bytes, void** out) {
+  StageRing& r = g_stage;
+  *out = nullptr;
+  r.acquired = -1;
+  if (kStageHead + bytes > r.slot_bytes) {
+    int64_t slot = 64 << 10;
+    while (slot < kStageHead + bytes) slot *= 2;
+    const int rc = stage_release();
+    if (rc != KVC_OK) return rc;
+    KVC_HIP(hipHostMalloc((void**)&r.base, kStageSlots * slot, hipHostMallocPortable));
+    r.slot_bytes = slot;
+    for (int i = 0; i < kStageSlots; ++i) std::memset(r.base + i * slot, 0, kStageHead);
+  }
+  const int rc = stage_wait(r, r.next);
+  if (rc != KVC_OK) return rc;
+  r.acquired = bytes;
+  *out = r.base + r.next * r.slot_bytes + kStageHead;
+  return KVC_OK;
+}
+
+// The acquired slot's flags and value for a kernel of `wgs` workgroups that reads it; the slot counts as in use
+// from here on.
+int stage_hand_over(const char* fn, int64_t bytes, int wgs, void* stream, uint32_t** flags, uint32_t* value) {
+  StageRing& r = g_stage;
+  if (r.acquired < bytes)
+    return fail(KVC_ERR_STAGING, "%s: %lld bytes wanted of a staging buffer of %lld (kvc_staging_acquire comes first)",
+                fn, (long long)bytes, (long long)r.acquired);
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  KVC_HIP(hipStreamIsCapturing((hipStream_t)stream, &capturing));
+  if (capturing != hipStreamCaptureStatusNone)
+    return fail(KVC_ERR_UNSUPPORTED, "%s: the staging buffer of a recorded launch would be overwritten before a replay", fn);
+  const int i = r.next;
+  if (++r.seq == 0) r.seq = 1;
+  r.used_seq[i] = *value = r.seq;
+  r.used_wgs[i] = wgs;
+  *flags = reinterpret_cast<uint32_t*>(r.base + i * r.slot_bytes);
+  r.next = (i + 1) % kStageSlots;
+  r.acquired = -1;
+  return KVC_OK;
+}
+
+// Workgroups of the index build: a batch that fits one scan chunk is scanned by each
+// of them, so a round of 1024 tokens, or of 4096 block ids to upload, gets its own.
+unsigned index_grid(int64_t batch_size, int64_t nnz, int64_t upload_ids) {
+  if (batch_size > kPrepThreads) return 1;
+  const int64_t want = std::max((nnz + kPrepThreads - 1) / kPrepThreads,
+                                (upload_ids + 4 * kPrepThreads - 1) / (4 * kPrepThreads));
+  return (unsigned)std::min<int64_t>(kStageMaxWgs, std::max<int64_t>(1, want));
+}
+
+// shared driver of the two index-build entry points
+int launch_build_index(IndexArgs a, void* stream, unsigned grid) {
+  hipLaunchKernelGGL(build_write_index_kernel, dim3(grid), dim3(kPrepThreads), 0, (hipStream_t)stream, a);
+  KVC_HIP(hipGetLastError());
+  return KVC_OK;
+}
+
 // --------------------------- swap that allocates nothing ---------------------
 // The id lists of a direct swap live in a static device array instead of a
 // caller-provided workspace, and reach it as kernel arguments instead of through
@@ -2101,13 +2270,58 @@ int kvc_build_write_index(const int32_t* input_lens, const int32_t* context_lens
     num_runs = nullptr;
     max_runs = 0;
   }
-  hipLaunchKernelGGL(build_write_index_kernel, dim3(1), dim3(kPrepThreads), 0, (hipStream_t)stream,
-                     input_lens, context_lens, num_blocks, kv_indices, (int32_t)batch_size,
-                     num_kv_indices, (int32_t)page_size, nnz, cu_seqlens_q, kv_indptr,
-                     kv_last_page_len, batch_indices, positions, slot_mapping, run_indptr, runs,
-                     num_runs, max_runs);
+  const IndexArgs a{input_lens, context_lens, num_blocks, kv_indices, (int32_t)batch_size, (int32_t)page_size,
+                    num_kv_indices, nnz, cu_seqlens_q, kv_indptr, kv_last_page_len, batch_indices, positions,
+                    slot_mapping, run_indptr, runs, num_runs, max_runs, nullptr, nullptr, 0};
+  return launch_build_index(a, stream, runs ? 1 : index_grid(batch_size, nnz, 0));
+}
+
+int kvc_staging_acquire(int64_t bytes, void** out) {
+  if (!out || bytes < 0 || bytes > (int64_t(1) << 30))
+    return fail(KVC_ERR_INVALID_ARG, "kvc_staging_acquire: %lld bytes", (long long)bytes);
+  return stage_acquire(bytes, out);
+}
+
+int kvc_staging_upload(void* dst, int64_t bytes, void* stream) {
+  const char* fn = "kvc_staging_upload";
+  if (bytes < 0 || bytes % 16 || (bytes > 0 && (!dst || (uintptr_t)dst % 16)))
+    return fail(KVC_ERR_INVALID_ARG, "%s: %lld bytes to %p (whole 16-byte vectors, aligned)", fn, (long long)bytes, dst);
+  if (bytes == 0) return KVC_OK;
+  const int64_t words4 = bytes / 16;
+  const int grid = (int)std::min<int64_t>(kStageMaxWgs, (words4 + kThreads - 1) / kThreads);
+  uint32_t *flags = nullptr, value = 0;
+  const int rc = stage_hand_over(fn, bytes, grid, stream, &flags, &value);
+  if (rc != KVC_OK) return rc;
+  const char* src = reinterpret_cast<const char*>(flags) + kStageHead;
+  hipLaunchKernelGGL(upload_kernel, dim3(grid), dim3(kThreads), 0, (hipStream_t)stream,
+                     reinterpret_cast<const int4*>(src), (int4*)dst, words4, flags, value);
   KVC_HIP(hipGetLastError());
   return KVC_OK;
+}
+
+int kvc_build_write_index_staged(int64_t batch_size, int64_t num_kv_indices, int64_t page_size, int64_t nnz,
+                                 int32_t* cu_seqlens_q, int32_t* kv_indptr, int32_t* kv_last_page_len,
+                                 int32_t* kv_indices, int32_t* batch_indices, int32_t* positions,
+                                 int64_t* slot_mapping, void* stream) {
+  const char* fn = "kvc_build_write_index_staged";
+  if (batch_size <= 0 || nnz < 0 || num_kv_indices < 0 || page_size <= 0 || batch_size > 0x7fffffffll ||
+      page_size > 0x7fffffffll || nnz > 0x7fffffffll)
+    return fail(KVC_ERR_INVALID_ARG, "%s: batch_size=%lld nnz=%lld page_size=%lld", fn, (long long)batch_size,
+                (long long)nnz, (long long)page_size);
+  if (!cu_seqlens_q || !kv_indptr || !kv_last_page_len || (num_kv_indices > 0 && !kv_indices) ||
+      (nnz > 0 && (!batch_indices || !positions)))
+    return fail(KVC_ERR_INVALID_ARG, "%s: null output", fn);
+  if ((uintptr_t)kv_indices % 16) return fail(KVC_ERR_INVALID_ARG, "%s: kv_indices must be 16-byte aligned", fn);
+  const int64_t ids_at = round_up(3 * batch_size, 4);
+  const unsigned grid = index_grid(batch_size, nnz, num_kv_indices);
+  uint32_t *flags = nullptr, value = 0;
+  const int rc = stage_hand_over(fn, (ids_at + num_kv_indices) * (int64_t)sizeof(int32_t), (int)grid, stream, &flags, &value);
+  if (rc != KVC_OK) return rc;
+  const int32_t* staged = reinterpret_cast<const int32_t*>(reinterpret_cast<const char*>(flags) + kStageHead);
+  const IndexArgs a{staged, staged + batch_size, staged + 2 * batch_size, staged + ids_at, (int32_t)batch_size,
+                    (int32_t)page_size, num_kv_indices, nnz, cu_seqlens_q, kv_indptr, kv_last_page_len,
+                    batch_indices, positions, slot_mapping, nullptr, nullptr, nullptr, 0, kv_indices, flags, value};
+  return launch_build_index(a, stream, grid);
 }
 
 int kvc_streams_share_hw_queue(void* stream_x, void* stream_y, int* shared) {
@@ -2397,7 +2611,11 @@ int kvc_swap_in_prepared(void* pool, const void* host_pool, const int64_t* host_
                   staging, staging_bytes, mode, true, kernel_stream, copy_stream);
 }
 
-int kvc_thread_release(void) { return swap_ctx_release(); }
+int kvc_thread_release(void) {
+  const int rc = stage_release();
+  const int rc_swap = swap_ctx_release();
+  return rc != KVC_OK ? rc : rc_swap;
+}
 
 int kvc_swap_noalloc(int to_host, void* pool, void* host_pool, const int64_t* gpu_ids,
                      const int64_t* host_ids, int64_t n, int64_t num_layers,

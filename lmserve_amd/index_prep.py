@@ -155,8 +155,25 @@ def to_device_one_launch(inputs: Sequence[InferInput], page_size: int, device="c
     host only packs four small arrays (new-token count, context length and
     block-table length per request, and the concatenated block tables); prefix
     sums, positions, request indices and slots are computed on the device in a
-    single launch. Requests are ordered as `make_kv_index_inputs` orders them."""
+    single launch, which also brings the arrays over: the packing happens in
+    native code, straight into the pinned buffer that launch reads. Requests are
+    ordered as `make_kv_index_inputs` orders them. The tensors share one allocation."""
+    from . import _lib
     from .paged import build_write_index
+
+    fast = _lib.fast_entry("build_index")
+    if fast is not None:
+        dev = torch.device(device)
+        if dev.type == "cuda":
+            index = torch.cuda.current_device() if dev.index is None else dev.index
+            # 1 = requests (or a device, or a recording stream) it does not handle: the path below does
+            got = fast(inputs, page_size, bool(with_slot_mapping), index, torch._C._cuda_getCurrentRawStream(index))
+            if type(got) is tuple:
+                cu, indptr, last, kv_indices, batch_indices, positions, slots, prefill_input_len = got
+                return DeviceKVIndexInputs(positions, cu, prefill_input_len, batch_indices, positions, kv_indices,
+                                           indptr, last, slots)
+            if got < 0:
+                _lib.check(got)
 
     order = sorted(range(len(inputs)), key=lambda i: -inputs[i].input_len)
     reqs = [inputs[i] for i in order]

@@ -30,6 +30,7 @@ from typing import Optional, Sequence
 import numpy as np
 import torch
 
+from . import _lib
 from .index_prep import InferInput
 from .paged import BlockRuns, PagedKVWritePlan, build_write_index, max_block_runs
 from .rotary import PagedRotaryWritePlan
@@ -58,15 +59,16 @@ class KVWriteStep:
             raise ValueError("capacities must be positive")
         B, T, N = self.max_requests, self.max_tokens, self.max_block_ids
         # one device buffer and one pinned mirror: [input_lens | context_lens | num_blocks | kv_indices]
-        self._packed = torch.zeros(3 * B + N, dtype=torch.int32, device=self.device)
-        self._host = torch.zeros(3 * B + N, dtype=torch.int32, pin_memory=True)
+        words = (3 * B + N + 3) // 4 * 4      # uploads come in whole 16-byte vectors
+        self._packed = torch.zeros(words, dtype=torch.int32, device=self.device)
+        self._host = torch.zeros(words, dtype=torch.int32, pin_memory=True)
         self._host_np = self._host.numpy()
         self._uploaded = torch.cuda.Event()
         self._upload_pending = False
         self.input_lens = self._packed[0:B]
         self.context_lens = self._packed[B:2 * B]
         self.num_blocks = self._packed[2 * B:3 * B]
-        self.kv_indices = self._packed[3 * B:]
+        self.kv_indices = self._packed[3 * B:3 * B + N]
         i32 = dict(dtype=torch.int32, device=self.device)
         self.cu_seqlens_q = torch.zeros(B + 1, **i32)
         self.kv_indptr = torch.zeros(B + 1, **i32)
@@ -132,7 +134,20 @@ class KVWriteStep:
     def set_requests(self, inputs: Sequence[InferInput]) -> list:
         """`set_arrays` from the scheduler's requests (proto/worker.proto:40-47),
         ordered by decreasing new-token count as the reference orders them
-        (model_worker.py:326-328). Returns that order (indices into `inputs`)."""
+        (model_worker.py:326-328). Returns that order (indices into `inputs`). Packed
+        in native code into a pinned buffer that a small launch on the current
+        stream uploads."""
+        fast = _lib.fast_entry("upload_requests")
+        if fast is not None:
+            index = self._packed.device.index
+            # 1 = not what it reads, or beyond a capacity: the path below handles it or says why
+            got = fast(inputs, self.max_requests, self.max_tokens, self.max_block_ids, self._packed.data_ptr(), index,
+                       torch._C._cuda_getCurrentRawStream(index))
+            if type(got) is tuple:
+                order, self.num_requests, self.num_tokens = got
+                return order
+            if got < 0:
+                _lib.check(got)
         order = sorted(range(len(inputs)), key=lambda i: -inputs[i].input_len)
         reqs = [inputs[i] for i in order]
         tables: list = []

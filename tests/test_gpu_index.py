@@ -119,3 +119,38 @@ def test_one_launch_index_build_marks_positions_outside_the_table(gpu):
     _, _, _, _, pos, slots = kvc.build_write_index(
         _up([1, 1], gpu), _up([20, 5], gpu), _up([1, 1], gpu), _up([7, 3], gpu), 16, 2)
     assert pos.tolist() == [19, 4] and slots.tolist() == [-1, 3 * 16 + 4]
+
+
+@pytest.mark.parametrize("sizes", [
+    [1], [1] * 1024, [1] * 1025,                     # one scan chunk, and one request beyond it
+    [1024], [1025], [700, 324, 1], [2048, 1, 1],     # a round of 1024 tokens per workgroup, and one token more
+    [5000, 3, 2, 1],                                 # 20 000 block ids: several workgroups upload them
+], ids=str)
+def test_index_from_requests_at_the_edges_of_its_launch(gpu, sizes):
+    """Requests packed into the staging ring, against the oracle's statement of the index: every remainder of
+    the 16-byte upload, more calls in flight than the ring has buffers, on two streams."""
+    rng = np.random.default_rng(len(sizes) + sizes[0])
+    ps = 4
+    calls = []
+    for k in range(9):
+        reqs = []
+        for i, n in enumerate(sizes[:len(sizes) - (k % 2 if len(sizes) > 1 else 0)]):
+            filled = int(rng.integers(0, 50))
+            blocks = (filled + n + ps - 1) // ps + (k if i == 0 else 0)    # tables may be longer than needed
+            blocks += 20000 if n == 5000 else 0
+            reqs.append(kvc.InferInput(i, [], n, filled, filled + n, rng.integers(0, 1 << 20, blocks).tolist()))
+        calls.append([reqs[i] for i in rng.permutation(len(reqs))])
+    streams = [torch.cuda.current_stream(gpu), torch.cuda.Stream(gpu)]
+    got = []
+    for k, reqs in enumerate(calls):
+        with torch.cuda.stream(streams[k % 2]):
+            got.append(kvc.to_device_one_launch(reqs, ps, gpu))
+    torch.cuda.synchronize()
+    for reqs, dev in zip(calls, got):
+        ordered = sorted(reqs, key=lambda r: -r.input_len)
+        ids = [b for r in ordered for b in r.block_ids]
+        want = orc.build_write_index_np([r.input_len for r in ordered], [r.context_len for r in ordered],
+                                        [len(r.block_ids) for r in ordered], ids, ps)
+        for g, w in zip((dev.cu_seqlens_q, dev.kv_block_indptrs, dev.kv_last_block_lens, dev.batch_indices,
+                         dev.positions, dev.slot_mapping, dev.kv_block_indices), list(want) + [np.asarray(ids)]):
+            assert np.array_equal(g.cpu().numpy(), w)

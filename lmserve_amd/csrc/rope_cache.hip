@@ -553,10 +553,16 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
         }
     }
     a.groups_per_token = (uint32_t)std::max<int64_t>(1, (lanes + threads - 1) / threads);
-    // query_out past the caches: from 48 MiB on it no longer fits the L2s (8 x 4 MiB) beside what else the
-    // launch moves. A rotation followed by a kernel that reads query_out: 134 MB 77.6 us against 79.6,
-    // 67 MB 46.7 against 47.8, 59 MB 37.4 against 38.3; at 33 MB 26.7 against 26.2 and below it costs more.
-    ntq = g.num_tokens * g.num_heads * g.head_dim * E >= (int64_t(48) << 20);
+    // query_out by non-temporal stores from 4 MiB on where a half head is whole 128-byte lines: plain stores sit
+    // dirty in the L2s until the kernel's end writes them all back. Measured alone, and with a kernel behind it
+    // that reads query_out (us a pair; plain -> non-temporal): 8 MiB of 32 heads x 128 5.6 -> 5.1, 8.9 -> 8.3;
+    // 14 MiB of 28 heads 8.7 -> 6.9, 11.2 -> 11.2; 16 MiB of 64 heads 8.3 -> 7.9, 12.1 -> 12.4; 32 MiB of 64 heads
+    // 17.5 -> 14.0, 23.3 -> 23.3; 67 MB of 32 heads 37.8 -> 36.1, 47.8 -> 47.2. Below 4 MiB the reader loses more
+    // than the launch gains (2 MiB of 32 heads 2.73 -> 2.70, 4.9 -> 5.1). A half head of 64 bytes writes each line
+    // in two parts and gains nothing (16 MiB of 32 heads x 64 9.8 -> 10.2) before 48 MiB.
+    const int64_t query_bytes = g.num_tokens * g.num_heads * g.head_dim * E;
+    ntq = query_bytes >= (int64_t(48) << 20) ||
+          (query_bytes >= (int64_t(4) << 20) && !tail && g.rotary_dim * E % 256 == 0);
   } else {
     const int64_t items = heads * (g.rotary_dim / 2) + heads * (g.head_dim - g.rotary_dim) +
                           (c ? g.num_kv_heads * g.head_dim : 0);

@@ -1,6 +1,6 @@
 // libkvcache: paged KV-cache data movement for MI355X (gfx950, CDNA4).
 //
-// Four kernels carry the whole path; all are HBM-bound byte movers, so the
+// Five kernels carry the whole path; all are HBM-bound byte movers, so the
 // design is about coalescing and bytes in flight, not arithmetic:
 //
 //   write_rows_kernel   a workgroup owns ONE token and a run of 16-byte vectors
@@ -19,9 +19,11 @@
 //                       contiguous on both sides). A workgroup owns a chunk of
 //                       256 lanes x UNROLL x 16 bytes, issues all its loads
 //                       before its first store, and walks chunks grid-stride.
-//                       The same kernel serves copy_blocks (pool -> pool), the
-//                       swap gather/scatter (pool <-> staging ring in host
-//                       layout) and the direct swap (pool <-> mapped host pool).
+//                       Small launches, narrow vectors, and the direct swap
+//                       (pool <-> mapped host pool).
+//   stream_tiles_kernel the same for large launches: copy_blocks (pool -> pool)
+//                       and the swap gather/scatter (pool <-> staging ring in
+//                       host layout), chunks ordered per XCD.
 //   index kernels       seq_lens and (batch_indices, positions) for the paged
 //                       write; a few KiB of int32.
 //
@@ -484,6 +486,61 @@ __global__ __launch_bounds__(kThreads) void copy_tiles_kernel(TileArgs a) {
       const int64_t off = base + (int64_t)j * kThreads * VEC;
       if (off < a.tile_bytes) st<NT>(reinterpret_cast<V*>(dst + off), data[j]);
     }
+  }
+}
+
+// Large copies: one chunk of one tile per workgroup, 16-byte vectors, the order of
+// the chunks chosen per XCD. Bound: HBM, and of that the part that the spread of
+// the addresses in flight costs. Workgroups are dealt round-robin to the 8 XCDs;
+// here each XCD walks a run of `xcd_run` neighbouring chunks (a few hundred KiB)
+// instead of every eighth chunk, and the launch keeps the region in flight small:
+// either one vector per lane in workgroups of 64 lanes, or two in workgroups of 256
+// of which a CU holds 5 instead of 8 (dynamic LDS that nothing uses). TB/s, copy of
+// 1024 blocks x 32 layers of 64 KiB in a pool of 4104 blocks / in one of 16384 / a
+// gather of 256 x 80 / a scatter of them:
+//   two vectors, no runs (what ran before; the gather one)   5.2  4.9  6.3  5.3
+//   two vectors, runs of 64 chunks                           5.45 5.6  -    5.7
+//   two vectors, runs, 5 workgroups per CU                   6.05 6.05 6.45 6.35
+//   one vector, 64 lanes, runs of 64 / of 256 chunks         6.1/6.2 6.2/6.2 6.6/6.7 6.4/6.25
+struct StreamArgs {
+  const char* src_base;
+  char* dst_base;
+  const int64_t* src_ids;  // device; nullptr = identity (i)
+  const int64_t* dst_ids;
+  int id_stride;
+  uint32_t tile_bytes, chunks_per_tile, num_layers, total_chunks, xcd_run;
+  int64_t src_layer_stride, src_block_stride, dst_layer_stride, dst_block_stride;
+  int64_t num_src_blocks, num_dst_blocks;
+};
+
+template <int THREADS, int UNROLL, bool NTL, bool NTS>
+__global__ __launch_bounds__(THREADS) void stream_tiles_kernel(StreamArgs a) {
+  uint32_t w = blockIdx.x;
+  const uint32_t span = 8 * a.xcd_run;
+  const uint32_t in_span = w % span;
+  // a span that the launch does not fill stays in grid order
+  if (w - in_span + span <= a.total_chunks) w = w - in_span + (in_span & 7u) * a.xcd_run + (in_span >> 3);
+  const uint32_t tile = w / a.chunks_per_tile;
+  const uint32_t chunk = w - tile * a.chunks_per_tile;
+  const uint32_t i = tile / a.num_layers;
+  const uint32_t layer = tile - i * a.num_layers;
+  const int64_t sid = a.src_ids ? a.src_ids[(int64_t)i * a.id_stride] : i;
+  const int64_t did = a.dst_ids ? a.dst_ids[(int64_t)i * a.id_stride] : i;
+  if (sid < 0 || sid >= a.num_src_blocks || did < 0 || did >= a.num_dst_blocks) return;
+  const char* src = a.src_base + layer * a.src_layer_stride + sid * a.src_block_stride;
+  char* dst = a.dst_base + layer * a.dst_layer_stride + did * a.dst_block_stride;
+  if (src == dst) return;
+  const uint32_t base = chunk * (THREADS * UNROLL * 16) + threadIdx.x * 16;
+  u32x4 data[UNROLL];
+#pragma unroll
+  for (int j = 0; j < UNROLL; ++j) {
+    const uint32_t off = base + j * (THREADS * 16);
+    if (off < a.tile_bytes) data[j] = ld<NTL>(reinterpret_cast<const u32x4*>(src + off));
+  }
+#pragma unroll
+  for (int j = 0; j < UNROLL; ++j) {
+    const uint32_t off = base + j * (THREADS * 16);
+    if (off < a.tile_bytes) st<NTS>(reinterpret_cast<u32x4*>(dst + off), data[j]);
   }
 }
 
@@ -1345,16 +1402,57 @@ void launch_tiles_nt(const TileArgs& a, unsigned grid, hipStream_t s, bool nt) {
   else hipLaunchKernelGGL((copy_tiles_kernel<VEC, UNROLL, false>), dim3(grid), dim3(kThreads), 0, s, a);
 }
 
+// What a launch copies between: blocks of a pool, or a dense buffer on one side.
+enum class TileSides { kPools, kGather, kScatter };
+
+// The stream kernel for a launch of `n` tiles per layer. The dense side of a gather or
+// scatter is kept in, or taken from, the 256 MiB last-level cache while it fits (plain
+// accesses): a scatter right behind the gather of the same buffer then moves 7.0
+// instead of 6.5 TB/s for both (256 blocks of 1 MiB and 128 of 2 MiB), and 3 % less
+// where the buffer was not in the cache after all. Beyond that size plain accesses
+// cost 10 %.
+int launch_stream(const TileArgs& t, TileSides sides, int64_t n, hipStream_t s) {
+  StreamArgs a{};
+  a.src_base = t.src_base; a.dst_base = t.dst_base;
+  a.src_ids = t.src_ids; a.dst_ids = t.dst_ids; a.id_stride = t.id_stride;
+  a.tile_bytes = (uint32_t)t.tile_bytes;
+  a.num_layers = t.num_layers;
+  a.src_layer_stride = t.src_layer_stride; a.src_block_stride = t.src_block_stride;
+  a.dst_layer_stride = t.dst_layer_stride; a.dst_block_stride = t.dst_block_stride;
+  a.num_src_blocks = t.num_src_blocks; a.num_dst_blocks = t.num_dst_blocks;
+  // a gather streams best one vector per lane (6.6 against 6.45 TB/s), a copy and a scatter no worse with two
+  const bool gather = sides == TileSides::kGather;
+  const uint32_t threads = gather ? 64 : 256, unroll = gather ? 1 : 2, chunk = threads * unroll * 16;
+  a.chunks_per_tile = (a.tile_bytes + chunk - 1) / chunk;
+  a.total_chunks = (uint32_t)(n * a.num_layers * a.chunks_per_tile);
+  a.xcd_run = gather ? 256 : 64;
+  const bool dense_cached = n * (int64_t)a.num_layers * t.tile_bytes <= (int64_t(256) << 20);
+  const bool plain_load = sides == TileSides::kScatter && dense_cached;
+  const bool plain_store = gather && dense_cached;
+  const dim3 grid(a.total_chunks), block(threads);
+  constexpr unsigned kFivePerCu = 160 * 1024 / 5;
+  if (gather && plain_store) hipLaunchKernelGGL((stream_tiles_kernel<64, 1, true, false>), grid, block, 0, s, a);
+  else if (gather) hipLaunchKernelGGL((stream_tiles_kernel<64, 1, true, true>), grid, block, 0, s, a);
+  else if (plain_load) hipLaunchKernelGGL((stream_tiles_kernel<256, 2, false, true>), grid, block, kFivePerCu, s, a);
+  else hipLaunchKernelGGL((stream_tiles_kernel<256, 2, true, true>), grid, block, kFivePerCu, s, a);
+  g_last = LastLaunch{KVC_KERNEL_COPY_TILES, 16, (int64_t)unroll, (int64_t)threads, (int64_t)a.total_chunks,
+                      plain_load || plain_store ? 0 : 1};
+  KVC_HIP(hipGetLastError());
+  return KVC_OK;
+}
+
 template <int VEC>
-int launch_tiles_vec(TileArgs a, int unroll, int max_wgs, hipStream_t s, bool nt, int64_t n, int large) {
+int launch_tiles_vec(TileArgs a, int unroll, int max_wgs, hipStream_t s, bool nt, int64_t n, TileSides sides) {
   if (unroll <= 0) {
     // By size, from sweeps of copy_blocks (1 to 4096 pairs x 32 layers x 64 KiB):
     // a launch that fits a quarter of the resident workgroups runs best as few,
     // deep workgroups (the smallest depth that gets it there; up to a whole tile
     // per workgroup while that stays within half the resident set): 6-8 % faster
     // than 4 vectors per lane from 32 to 128 MiB (a gather: 12-15 % faster than
-    // with 1). Larger launches stream best with `large` vectors per lane: 2, or 1
-    // when the scattered side is the one being read (gather).
+    // with 1). Larger launches go through the stream kernel; what it does not take
+    // (narrow vectors, tiles below 8 KiB, a capped grid, more than 2^31 chunks, plain copies or another
+    // tile order by request) runs with 2 vectors per lane, or 1 when the scattered
+    // side is the one being read (gather).
     const int64_t resident = resident_workgroups();
     const auto chunks = [&](int u) {
       const int64_t c = (int64_t)kThreads * VEC * u;
@@ -1363,7 +1461,16 @@ int launch_tiles_vec(TileArgs a, int unroll, int max_wgs, hipStream_t s, bool nt
     unroll = 0;
     for (int u = 1; u <= 16 && !unroll; u *= 2)
       if (chunks(u) <= resident / 4) unroll = u;
-    if (!unroll) unroll = chunks(16) <= resident / 2 ? 16 : large;
+    if (!unroll && chunks(16) <= resident / 2) unroll = 16;
+    if (!unroll) {
+      // (a tile below one chunk would leave lanes of every workgroup without work)
+      const int64_t one_chunk = sides == TileSides::kGather ? 1024 : 8192;
+      if (VEC == 16 && max_wgs <= 0 && nt && !g_tune.copy_order && a.tile_bytes >= one_chunk &&
+          a.tile_bytes <= (int64_t(1) << 30) &&
+          n * (int64_t)a.num_layers * ((a.tile_bytes + 1023) / 1024) <= 0x7fffffffll)
+        return launch_stream(a, sides, n, s);
+      unroll = sides == TileSides::kGather ? 1 : 2;
+    }
   }
   // do not carry more vectors per lane than the tile can fill
   while (unroll > 1 && (int64_t)kThreads * VEC * (unroll / 2) >= a.tile_bytes) unroll /= 2;
@@ -1387,22 +1494,22 @@ int launch_tiles_vec(TileArgs a, int unroll, int max_wgs, hipStream_t s, bool nt
   return KVC_OK;
 }
 
-// unroll > 0: fixed; 0: the copy_unroll knob (by size unless set); gather: the gather_unroll knob
-int launch_tiles(const TileArgs& a, int64_t n, int max_wgs, hipStream_t s, bool gather = false) {
+// vectors per lane: the gather_unroll knob for a gather, else copy_unroll; by size unless set
+int launch_tiles(const TileArgs& a, int64_t n, int max_wgs, hipStream_t s, TileSides sides = TileSides::kPools) {
   if (n == 0 || a.num_layers == 0 || a.tile_bytes == 0) return KVC_OK;
   const int vec = common_vec({(uint64_t)(uintptr_t)a.src_base, (uint64_t)(uintptr_t)a.dst_base,
                               (uint64_t)a.src_layer_stride, (uint64_t)a.src_block_stride,
                               (uint64_t)a.dst_layer_stride, (uint64_t)a.dst_block_stride,
                               (uint64_t)a.tile_bytes});
-  int unroll = gather ? g_tune.gather_unroll : g_tune.copy_unroll;
+  int unroll = sides == TileSides::kGather ? g_tune.gather_unroll : g_tune.copy_unroll;
   if (unroll != 1 && unroll != 2 && unroll != 4 && unroll != 8 && unroll != 16) unroll = 0;  // by size
   const bool nt = g_tune.copy_nt != 0;
   switch (vec) {
-    case 16: return launch_tiles_vec<16>(a, unroll, max_wgs, s, nt, n, gather ? 1 : 2);
-    case 8: return launch_tiles_vec<8>(a, unroll, max_wgs, s, nt, n, gather ? 1 : 2);
-    case 4: return launch_tiles_vec<4>(a, unroll, max_wgs, s, nt, n, gather ? 1 : 2);
-    case 2: return launch_tiles_vec<2>(a, unroll, max_wgs, s, nt, n, gather ? 1 : 2);
-    default: return launch_tiles_vec<1>(a, unroll, max_wgs, s, nt, n, gather ? 1 : 2);
+    case 16: return launch_tiles_vec<16>(a, unroll, max_wgs, s, nt, n, sides);
+    case 8: return launch_tiles_vec<8>(a, unroll, max_wgs, s, nt, n, sides);
+    case 4: return launch_tiles_vec<4>(a, unroll, max_wgs, s, nt, n, sides);
+    case 2: return launch_tiles_vec<2>(a, unroll, max_wgs, s, nt, n, sides);
+    default: return launch_tiles_vec<1>(a, unroll, max_wgs, s, nt, n, sides);
   }
 }
 
@@ -1785,7 +1892,7 @@ int run_swap(const char* fn, bool out, char* pool, char* host_pool, const int64_
       t.dst_base = slot; t.dst_ids = nullptr;
       t.dst_layer_stride = g.block_bytes; t.dst_block_stride = width;
       t.num_dst_blocks = count;
-      rc = launch_tiles(t, count, g_tune.copy_max_wgs, ks, true);
+      rc = launch_tiles(t, count, g_tune.copy_max_wgs, ks, TileSides::kGather);
       if (rc != KVC_OK) return rc;
       if (two_streams) {
         KVC_HIP(hipEventRecord(c.filled[sl], ks));
@@ -1811,7 +1918,7 @@ int run_swap(const char* fn, bool out, char* pool, char* host_pool, const int64_
       t.dst_base = pool_l0; t.dst_ids = d_gpu_ids + done;
       t.dst_layer_stride = g.layer_stride_bytes; t.dst_block_stride = g.block_bytes;
       t.num_dst_blocks = g.num_gpu_blocks;
-      rc = launch_tiles(t, count, g_tune.copy_max_wgs, ks);
+      rc = launch_tiles(t, count, g_tune.copy_max_wgs, ks, TileSides::kScatter);
       if (rc != KVC_OK) return rc;
       if (two_streams) KVC_HIP(hipEventRecord(c.drained[sl], ks));
     }
@@ -2487,7 +2594,8 @@ static int run_gather_scatter(const char* fn, bool gather, char* pool, char* buf
     t.dst_layer_stride = layer_stride_bytes; t.dst_block_stride = block_bytes;
     t.num_dst_blocks = num_blocks;
   }
-  return launch_tiles(t, n, g_tune.copy_max_wgs, (hipStream_t)stream, gather);
+  return launch_tiles(t, n, g_tune.copy_max_wgs, (hipStream_t)stream,
+                      gather ? TileSides::kGather : TileSides::kScatter);
 }
 
 int kvc_gather_blocks(const void* pool, void* buffer, const int64_t* block_ids, int64_t n,

@@ -145,3 +145,55 @@ def test_every_launch_shape_the_size_rule_picks_matches_the_oracle(gpu, n):
     assert np.array_equal(bits_of(dense), want_dense)
     view[:, flat[0::2]] = want_dense.swapaxes(0, 1)                 # a no-op by value: dst == src content
     assert np.array_equal(bits_of(dpool), want)
+
+
+@pytest.mark.parametrize("tile_bytes,n,L", [
+    (8192, 400, 3),        # one chunk per tile
+    (8208, 400, 3),        # a second chunk of one vector
+    (20480, 350, 3),       # two and a half chunks
+    (65552, 176, 3),       # one vector past 64 KiB; a last span of chunks that is not full
+    (65536, 129, 8),       # whole spans and a remainder
+])
+def test_stream_kernel_edges(gpu, tile_bytes, n, L):
+    """Launches beyond the small regime: tiles that end inside a chunk, spans of chunks that the launch does not
+    fill, ids that are skipped; copy, gather and scatter against NumPy, dense buffers below 256 MiB."""
+    nb = 2 * n + 5
+    pool = random_pool((L, nb, tile_bytes // 2), seed=n)
+    rng = np.random.default_rng(n)
+    ids = rng.permutation(nb)
+    src, dst = ids[:n].copy(), ids[n:2 * n].copy()
+    src[3], dst[5] = nb, -1                                # outside the pool: skipped
+    dst[7] = src[7]                                        # a pair onto itself
+    want = pool.copy()
+    ok = (src < nb) & (dst >= 0)
+    want[:, dst[ok]] = pool[:, src[ok]]
+    dpool = to_bf16(pool, gpu)
+    maps = torch.from_numpy(np.stack([src, dst], 1).reshape(-1)).to(gpu)
+    kvc.copy_blocks(dpool, maps)
+    ran = _lib.last_launch()
+    assert ran["kernel"] == _lib.KVC_KERNEL_COPY_TILES and ran["per_lane"] == 2
+    assert ran["grid"] == n * L * ((tile_bytes + 8191) // 8192)
+    assert np.array_equal(bits_of(dpool), want)
+    picked = torch.from_numpy(ids[:n].copy()).to(gpu)
+    dense = kvc.gather_blocks(dpool, picked)
+    assert _lib.last_launch()["threads"] == 64 and _lib.last_launch()["per_lane"] == 1
+    assert np.array_equal(bits_of(dense), want[:, ids[:n]].swapaxes(0, 1))
+    back = torch.from_numpy(ids[5:5 + n].copy()).to(gpu)   # overlaps the blocks that were gathered
+    kvc.scatter_blocks(dpool, back, dense)
+    assert _lib.last_launch()["per_lane"] == 2
+    want[:, ids[5:5 + n]] = want[:, ids[:n]].copy()
+    assert np.array_equal(bits_of(dpool), want)
+
+
+def test_stream_kernel_dense_buffer_beyond_the_last_level_cache(gpu):
+    """Past 256 MiB the dense side is read and written non-temporally too."""
+    L, nb, n = 16, 300, 257                                # 257 MiB of dense buffer
+    pool = torch.randint(-2**15, 2**15, (L, nb, 32768), dtype=torch.int16, device=gpu)
+    ids = torch.from_numpy(np.random.default_rng(1).permutation(nb)).to(gpu)
+    dense = kvc.gather_blocks(pool, ids[:n].contiguous())
+    assert _lib.last_launch()["non_temporal"] == 1
+    assert torch.equal(dense, pool[:, ids[:n]].transpose(0, 1))
+    want = pool.clone()
+    want[:, ids[nb - n:]] = dense.transpose(0, 1)
+    kvc.scatter_blocks(pool, ids[nb - n:].contiguous(), dense)
+    assert _lib.last_launch()["non_temporal"] == 1 and torch.equal(pool, want)

@@ -508,7 +508,8 @@ struct StreamArgs {
   const int64_t* src_ids;  // device; nullptr = identity (i)
   const int64_t* dst_ids;
   int id_stride;
-  uint32_t tile_bytes, chunks_per_tile, num_layers, total_chunks, xcd_run;
+  uint32_t tile_bytes, chunks_per_tile, num_layers, num_items, total_chunks, xcd_run;
+  int layer_slowest;       // order of the tiles: 0 = layers of one block are neighbours, 1 = blocks of one layer
   int64_t src_layer_stride, src_block_stride, dst_layer_stride, dst_block_stride;
   int64_t num_src_blocks, num_dst_blocks;
 };
@@ -522,8 +523,14 @@ __global__ __launch_bounds__(THREADS) void stream_tiles_kernel(StreamArgs a) {
   if (w - in_span + span <= a.total_chunks) w = w - in_span + (in_span & 7u) * a.xcd_run + (in_span >> 3);
   const uint32_t tile = w / a.chunks_per_tile;
   const uint32_t chunk = w - tile * a.chunks_per_tile;
-  const uint32_t i = tile / a.num_layers;
-  const uint32_t layer = tile - i * a.num_layers;
+  uint32_t i, layer;
+  if (a.layer_slowest) {
+    layer = tile / a.num_items;
+    i = tile - layer * a.num_items;
+  } else {
+    i = tile / a.num_layers;
+    layer = tile - i * a.num_layers;
+  }
   const int64_t sid = a.src_ids ? a.src_ids[(int64_t)i * a.id_stride] : i;
   const int64_t did = a.dst_ids ? a.dst_ids[(int64_t)i * a.id_stride] : i;
   if (sid < 0 || sid >= a.num_src_blocks || did < 0 || did >= a.num_dst_blocks) return;
@@ -1426,6 +1433,11 @@ int launch_stream(const TileArgs& t, TileSides sides, int64_t n, hipStream_t s) 
   a.chunks_per_tile = (a.tile_bytes + chunk - 1) / chunk;
   a.total_chunks = (uint32_t)(n * a.num_layers * a.chunks_per_tile);
   a.xcd_run = gather ? 256 : 64;
+  a.num_items = (uint32_t)n;
+  // Copies of small tiles walk a layer at a time: with the layers of a block as neighbours a run of 64 chunks
+  // touches as many far-apart pages (8 KiB x 80 layers: 4000 blocks 5.05 -> 5.2 TB/s, 300 blocks 4.85 -> 5.3;
+  // from 32 KiB on it makes no difference, and a dense side wants its own order: gather 6.2 -> 5.1).
+  a.layer_slowest = sides == TileSides::kPools && t.tile_bytes < (32 << 10);
   const bool dense_cached = n * (int64_t)a.num_layers * t.tile_bytes <= (int64_t(256) << 20);
   const bool plain_load = sides == TileSides::kScatter && dense_cached;
   const bool plain_store = gather && dense_cached;

@@ -27,6 +27,7 @@
 #include <cstdint>
 
 #include <ATen/ops/empty.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/variable.h>
 
 #include <algorithm>
@@ -400,15 +401,15 @@ bool read_requests(PyObject* inputs, Requests* out) {
   out->in_order.reserve(n);
   bool sorted = true;
   for (Py_ssize_t i = 0; i < n; ++i) {
+    if (PySequence_Fast_GET_SIZE(inputs) != n) return false;  // an attribute that is a property may run anything
     PyObject* r = PySequence_Fast_GET_ITEM(inputs, i);
     Requests::One one{0, 0, 0, nullptr};
-    PyObject* ids = nullptr;
-    if (int_attr(r, s_input, &one.input_len) && int_attr(r, s_context, &one.context_len) &&
-        (ids = PyObject_GetAttr(r, s_ids)) != nullptr) {
-      one.ids = PySequence_Fast(ids, "block_ids");
-      Py_DECREF(ids);
-    }
-    if (!one.ids) {
+    Py_INCREF(r);
+    if (int_attr(r, s_input, &one.input_len) && int_attr(r, s_context, &one.context_len))
+      one.ids = PyObject_GetAttr(r, s_ids);
+    Py_DECREF(r);
+    if (!one.ids || !(PyList_Check(one.ids) || PyTuple_Check(one.ids))) {
+      Py_XDECREF(one.ids);
       PyErr_Clear();
       return false;
     }
@@ -464,6 +465,16 @@ bool pack_requests(const Requests& q, int64_t stride, int64_t ids_at, int32_t* d
   return true;
 }
 
+// A staging buffer, without the interpreter's lock: where the device is far behind this waits for one, and what
+// the device waits for may be another thread's work.
+int acquire_staging(int64_t bytes, void** out) {
+  int rc;
+  Py_BEGIN_ALLOW_THREADS
+  rc = kvc_staging_acquire(bytes, out);
+  Py_END_ALLOW_THREADS
+  return rc;
+}
+
 bool stream_is_capturing(void* stream) {
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing((hipStream_t)stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone;
@@ -481,6 +492,7 @@ PyObject* piece(const at::Tensor& of, at::ScalarType type, int64_t n, int64_t of
  * kv_last_page_len, kv_indices, batch_indices, positions, slot_mapping | None, prefill tokens):
  * requests packed into a staging buffer, kvc_build_write_index_staged into one allocation */
 PyObject* fast_build_index(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS  // an allocation that fails is a Python exception
   int64_t page_size, with_slots, device;
   void* stream;
   if (nargs != 5) {
@@ -497,7 +509,7 @@ PyObject* fast_build_index(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const int64_t B = (int64_t)q.in_order.size(), N = q.ids, T = q.tokens;
   const int64_t ids_at = (3 * B + 3) / 4 * 4;
   void* staged = nullptr;
-  int rc = kvc_staging_acquire((ids_at + N + 4) * 4, &staged);
+  int rc = acquire_staging((ids_at + N + 4) * 4, &staged);
   if (rc < 0) return PyLong_FromLong(rc);
   if (!pack_requests(q, B, ids_at, (int32_t*)staged)) return PyLong_FromLong(NOT_FAST);
   // one allocation, every piece 16-byte aligned: slots first (8 bytes an element), then int32 pieces
@@ -516,11 +528,13 @@ PyObject* fast_build_index(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   return Py_BuildValue("(NNNNNNNL)", piece(buf, at::kInt, B + 1, o_cu), piece(buf, at::kInt, B + 1, o_ptr),
                        piece(buf, at::kInt, B, o_last), piece(buf, at::kInt, N, o_ids), piece(buf, at::kInt, T, o_bi),
                        piece(buf, at::kInt, T, o_pos), slots, (long long)q.prefill_tokens);
+  END_HANDLE_TH_ERRORS
 }
 
 /* upload_requests(requests, max_requests, max_tokens, max_ids, dst, device, stream) -> an int (1, or a negative
  * kvc_status), or (order, requests, tokens): packed as a KVWriteStep holds them and uploaded to its buffer */
 PyObject* fast_upload_requests(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS  // an allocation that fails is a Python exception
   int64_t max_requests, max_tokens, max_ids, device;
   void *dst, *stream;
   if (nargs != 7) {
@@ -536,7 +550,7 @@ PyObject* fast_upload_requests(PyObject*, PyObject* const* args, Py_ssize_t narg
   if (n > max_requests || q.tokens > max_tokens || q.ids > max_ids) return PyLong_FromLong(NOT_FAST);
   void* staged = nullptr;
   const int64_t bytes = (ids_at + q.ids + 3) / 4 * 16;
-  int rc = kvc_staging_acquire(bytes, &staged);
+  int rc = acquire_staging(bytes, &staged);
   if (rc < 0) return PyLong_FromLong(rc);
   if (!pack_requests(q, max_requests, ids_at, (int32_t*)staged)) return PyLong_FromLong(NOT_FAST);
   rc = kvc_staging_upload(dst, bytes, stream);
@@ -545,6 +559,7 @@ PyObject* fast_upload_requests(PyObject*, PyObject* const* args, Py_ssize_t narg
   if (!order) return nullptr;
   for (size_t i = 0; i < q.order.size(); ++i) PyList_SET_ITEM(order, i, PyLong_FromLongLong(q.order[i]));
   return Py_BuildValue("(NLL)", order, (long long)n, (long long)q.tokens);
+  END_HANDLE_TH_ERRORS
 }
 
 /* scalar_type_code(tensor) -> the integer the two calls above compare dtypes with */

@@ -154,3 +154,67 @@ def test_index_from_requests_at_the_edges_of_its_launch(gpu, sizes):
         for g, w in zip((dev.cu_seqlens_q, dev.kv_block_indptrs, dev.kv_last_block_lens, dev.batch_indices,
                          dev.positions, dev.slot_mapping, dev.kv_block_indices), list(want) + [np.asarray(ids)]):
             assert np.array_equal(g.cpu().numpy(), w)
+
+
+def _check_build(reqs, gpu):
+    want = kvc.to_device(kvc.make_kv_index_inputs(reqs, 16), 16, gpu)
+    got = kvc.to_device_one_launch(reqs, 16, gpu)
+    for name in ("cu_seqlens_q", "kv_block_indptrs", "kv_last_block_lens", "kv_block_indices", "batch_indices",
+                 "positions", "slot_mapping"):
+        assert torch.equal(getattr(got, name), getattr(want, name)), name
+
+
+def test_one_launch_index_build_reports_an_allocation_that_fails(gpu):
+    """As an exception of the interpreter; the next call works."""
+    huge = [kvc.InferInput(seq_id=0, input_ids=[], input_len=1 << 29, filled_token_len=0, context_len=1 << 29,
+                           block_ids=[0])]
+    torch.cuda.empty_cache()
+    torch.cuda.set_per_process_memory_fraction(0.01)       # below the 8 GiB of output tensors
+    try:
+        with pytest.raises(torch.cuda.OutOfMemoryError):
+            kvc.to_device_one_launch(huge, 16, gpu)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    import workloads as wl
+    _check_build(wl.decode_step(wl.LLAMA_3_8B, num_blocks=256, batch=8, max_context=100, seed=1).inputs, gpu)
+
+
+def test_index_builds_far_ahead_of_the_device_and_from_threads_that_end(gpu):
+    """More builds than staging buffers behind long work: each waits for a buffer without the interpreter's lock and
+    reads its own requests. Threads that end pass their buffers on, readers still queued included."""
+    import threading
+    import time
+    import workloads as wl
+    steps = [wl.decode_step(wl.LLAMA_3_8B, num_blocks=512, batch=8 + i, max_context=300, seed=i).inputs
+             for i in range(12)]
+    want = [kvc.to_device(kvc.make_kv_index_inputs(r, 16), 16, gpu) for r in steps]
+    torch.cuda.synchronize()
+    ticks, stop, got = [0], threading.Event(), []
+
+    def tick():
+        while not stop.is_set():
+            time.sleep(0.001)
+            ticks[0] += 1
+
+    ticker = threading.Thread(target=tick)
+    ticker.start()
+    x = torch.ones(4096, 4096, device=gpu)
+    x @ x
+    torch.cuda.synchronize()
+    before, t0 = ticks[0], time.perf_counter()
+    for _ in range(60):
+        y = x @ x                                            # about 0.1 s of queued work
+    for r in steps[:8]:
+        got.append(kvc.to_device_one_launch(r, 16, gpu))
+    waited, ticked = time.perf_counter() - t0, ticks[0] - before
+    for r in steps[8:]:
+        worker = threading.Thread(target=lambda: got.append(kvc.to_device_one_launch(r, 16, gpu)))
+        y = x @ x
+        worker.start()
+        worker.join()
+    stop.set()
+    ticker.join()
+    torch.cuda.synchronize()
+    assert ticked >= waited / 0.02 - 2
+    for g, w in zip(got, want):
+        assert torch.equal(g.slot_mapping, w.slot_mapping) and torch.equal(g.kv_block_indices, w.kv_block_indices)

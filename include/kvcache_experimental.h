@@ -132,6 +132,27 @@ int kvc_build_write_index_staged(int64_t batch_size, int64_t num_kv_indices, int
                                  int64_t* slot_mapping, void* stream);
 
 /*
+ * kvc_rotary_plan_run for several layers whose buffers are all at hand, in one launch
+ * (one for every 64 layers) where that cannot change the result: the plan has slots, rows
+ * and caches are 16-byte aligned, and nothing that one layer writes is read or written by
+ * another. Otherwise one launch per layer, in order. The layers share their strides and
+ * number of pages; key_out may be NULL. *one_launch (may be NULL): 1 where the first
+ * form ran. Model loops of the reference rotate and append layer by layer
+ * (runtime/worker/llm_worker/models/llama.py:236-242).
+ */
+typedef struct kvc_rotary_layer {
+  const void* query;
+  const void* key;
+  const void* value;
+  void* query_out;
+  void* key_out;
+  void* paged_kv_cache;
+} kvc_rotary_layer;
+int kvc_rotary_plan_run_layers(const kvc_rotary_plan* plan, int64_t num_layers, const kvc_rotary_layer* layers,
+                               int64_t q_token_stride, int64_t k_token_stride, int64_t v_token_stride,
+                               int64_t page_stride, int64_t num_pages, int* one_launch, void* stream);
+
+/*
  * Do two streams feed the same hardware queue? The runtime maps every stream of
  * a process onto a few hardware queues (4 unless GPU_MAX_HW_QUEUES says
  * otherwise). Kernels of streams that share one run one after the other, and a

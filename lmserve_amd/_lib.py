@@ -78,6 +78,7 @@ SIGNATURES = {
     "kvc_rotary_plan_create": (c_int, [_P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _P, _P, _I64,
                                        _I64, _I64, c_int, ctypes.POINTER(_P)]),
     "kvc_rotary_plan_run": (c_int, [_P, _P, _P, _P, _I64, _I64, _I64, _P, _P, _P, _I64, _I64, _P]),
+    "kvc_rotary_plan_run_layers": (c_int, [_P, _I64, _P, _I64, _I64, _I64, _I64, _I64, ctypes.POINTER(c_int), _P]),
     "kvc_rotary_plan_destroy": (c_int, [_P]),
     "kvc_rotary_plan_resolve_slots": (c_int, [_P, _P, _P]),
     "kvc_order_pairs_by_host_id": (c_int, [_P, _P, _I64]),

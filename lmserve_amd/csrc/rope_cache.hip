@@ -20,6 +20,7 @@
 
 #include "common.h"
 #include "kvcache.h"
+#include "kvcache_experimental.h"
 
 namespace kvc {
 RopeTuning g_rope_tune;
@@ -134,6 +135,12 @@ struct RopeArgs {
   uint32_t v_items;           // 16-byte vectors of the token's V row (0 without a cache)
 };
 
+// One layer's buffers, as RopeArgs names them
+struct RopeLayer {
+  const char *query, *key, *value;
+  char *query_out, *key_out, *key_cache, *value_cache;
+};
+
 // How a token finds its cache slot: not at all (plain rotation), through a slot
 // mapping, or through the page table.
 enum Addressing : int { kNoCache, kSlots, kPages };
@@ -210,7 +217,7 @@ __device__ __forceinline__ void st16(char* p, u32x4 v) {
 // NTL: non-temporal loads, bit 0 for the K and V rows, bit 1 for the Q rows. NTQ: non-temporal stores of
 // query_out (by its size, see the launch).
 template <typename T, Addressing ADDR, bool FAST, bool TAIL, int NTL, bool NTQ>
-__global__ __launch_bounds__(kThreads) void rope_vector_kernel(RopeArgs a) {
+__device__ __forceinline__ void rope_vector_lane(const RopeArgs& a, const RopeLayer p) {
   using VT = Vec<T>;
   constexpr uint32_t E = T::kBytes;
   const uint32_t t = blockIdx.y;
@@ -229,16 +236,16 @@ __global__ __launch_bounds__(kThreads) void rope_vector_kernel(RopeArgs a) {
   if (rotates) {
     if (NTL == 1 || NTL == 2) {
       if (is_k) {
-        const char* in = a.key + (int64_t)t * a.k_token_stride + head_off;
+        const char* in = p.key + (int64_t)t * a.k_token_stride + head_off;
         x = ld16<(NTL & 1) != 0>(in);
         y = ld16<(NTL & 1) != 0>(in + half);
       } else {
-        const char* in = a.query + (int64_t)t * a.q_token_stride + head_off;
+        const char* in = p.query + (int64_t)t * a.q_token_stride + head_off;
         x = ld16<(NTL & 2) != 0>(in);
         y = ld16<(NTL & 2) != 0>(in + half);
       }
     } else {
-      const char* in = (is_k ? a.key + (int64_t)t * a.k_token_stride : a.query + (int64_t)t * a.q_token_stride) + head_off;
+      const char* in = (is_k ? p.key + (int64_t)t * a.k_token_stride : p.query + (int64_t)t * a.q_token_stride) + head_off;
       x = ld16<NTL != 0>(in);
       y = ld16<NTL != 0>(in + half);
     }
@@ -255,7 +262,7 @@ __global__ __launch_bounds__(kThreads) void rope_vector_kernel(RopeArgs a) {
     if (ADDR != kNoCache && e < a.v_items) {
       ekind[j] = 1;
       eoff[j] = e * 16;
-      ev[j] = ld16<(NTL & 1) != 0>(a.value + (int64_t)t * a.v_token_stride + eoff[j]);
+      ev[j] = ld16<(NTL & 1) != 0>(p.value + (int64_t)t * a.v_token_stride + eoff[j]);
     } else if (TAIL) {
       const uint32_t tail_per_head = (a.head_dim - a.rotary_dim) * E / 16;
       if (e < a.v_items + heads * tail_per_head) {
@@ -264,8 +271,8 @@ __global__ __launch_bounds__(kThreads) void rope_vector_kernel(RopeArgs a) {
         const bool tk = th >= a.num_heads;
         ekind[j] = tk ? 3 : 2;
         eoff[j] = ((tk ? th - a.num_heads : th) * a.head_dim + a.rotary_dim) * E + (i - th * tail_per_head) * 16;
-        ev[j] = tk ? ld16<(NTL & 1) != 0>(a.key + (int64_t)t * a.k_token_stride + eoff[j])
-                   : ld16<(NTL & 2) != 0>(a.query + (int64_t)t * a.q_token_stride + eoff[j]);
+        ev[j] = tk ? ld16<(NTL & 1) != 0>(p.key + (int64_t)t * a.k_token_stride + eoff[j])
+                   : ld16<(NTL & 2) != 0>(p.query + (int64_t)t * a.q_token_stride + eoff[j]);
       }
     }
   }
@@ -285,17 +292,17 @@ __global__ __launch_bounds__(kThreads) void rope_vector_kernel(RopeArgs a) {
     u32x4 ox, oy;
     VT::rotate(x, y, cos_x, cos_y, sin_x, sin_y, ox, oy);
     if (!is_k) {  // read again by attention right away
-      char* out = a.query_out + (int64_t)t * a.qo_token_stride + head_off;
+      char* out = p.query_out + (int64_t)t * a.qo_token_stride + head_off;
       st16<NTQ>(out, ox);
       st16<NTQ>(out + half, oy);
     } else {
-      if (a.key_out) {
-        char* out = a.key_out + (int64_t)t * a.ko_token_stride + head_off;
+      if (p.key_out) {
+        char* out = p.key_out + (int64_t)t * a.ko_token_stride + head_off;
         st16<false>(out, ox);
         st16<false>(out + half, oy);
       }
       if (ADDR != kNoCache && slot >= 0) {  // the cache row is not read again by this step
-        char* out = a.key_cache + slot + head_off;
+        char* out = p.key_cache + slot + head_off;
         st16<true>(out, ox);
         st16<true>(out + half, oy);
       }
@@ -304,14 +311,38 @@ __global__ __launch_bounds__(kThreads) void rope_vector_kernel(RopeArgs a) {
 #pragma unroll
   for (int j = 0; j < kExtra; ++j) {
     if (ekind[j] == 1) {
-      if (slot >= 0) st16<true>(a.value_cache + slot + eoff[j], ev[j]);
+      if (slot >= 0) st16<true>(p.value_cache + slot + eoff[j], ev[j]);
     } else if (TAIL && ekind[j] == 2) {
-      st16<NTQ>(a.query_out + (int64_t)t * a.qo_token_stride + eoff[j], ev[j]);
+      st16<NTQ>(p.query_out + (int64_t)t * a.qo_token_stride + eoff[j], ev[j]);
     } else if (TAIL && ekind[j] == 3) {
-      if (a.key_out) st16<false>(a.key_out + (int64_t)t * a.ko_token_stride + eoff[j], ev[j]);
-      if (ADDR != kNoCache && slot >= 0) st16<true>(a.key_cache + slot + eoff[j], ev[j]);
+      if (p.key_out) st16<false>(p.key_out + (int64_t)t * a.ko_token_stride + eoff[j], ev[j]);
+      if (ADDR != kNoCache && slot >= 0) st16<true>(p.key_cache + slot + eoff[j], ev[j]);
     }
   }
+}
+
+template <typename T, Addressing ADDR, bool FAST, bool TAIL, int NTL, bool NTQ>
+__global__ __launch_bounds__(kThreads) void rope_vector_kernel(RopeArgs a) {
+  rope_vector_lane<T, ADDR, FAST, TAIL, NTL, NTQ>(
+      a, RopeLayer{a.query, a.key, a.value, a.query_out, a.key_out, a.key_cache, a.value_cache});
+}
+
+// The same for several layers of one step, blockIdx.z the layer, their pointers in the
+// kernel arguments. A recorded step has every layer's buffers at hand before it begins;
+// as one node per layer it is bound by what a node costs, not by its bytes. A replay with
+// the index build, per layer -> one launch (us): 64 tokens x 32 heads x 128 x 28 layers
+// 66.6 -> 17.8 (the index build alone 17.4), 256 x 48 heads x 32 88.9 -> 27.1, 717 tokens
+// of those 139.5 -> 91.0, 3001 x 10 heads x 80 326 -> 198 (6.2 TB/s).
+constexpr int kLayersPerLaunch = 64;  // 3.5 KiB of the 4 KiB a launch's arguments may take
+struct RopeLayersArgs {
+  RopeArgs a;
+  RopeLayer layer[kLayersPerLaunch];
+};
+static_assert(sizeof(RopeLayersArgs) <= 4096, "kernel arguments");
+
+template <typename T, bool TAIL, bool NTQ>
+__global__ __launch_bounds__(kThreads) void rope_layers_kernel(RopeLayersArgs args) {
+  rope_vector_lane<T, kSlots, true, TAIL, 0, NTQ>(args.a, args.layer[blockIdx.z]);
 }
 
 // Element path: rows that are no whole number of aligned 16-byte vectors. One
@@ -412,6 +443,25 @@ int launch_rope(RopeArgs a, int64_t num_tokens, bool vector, bool tail, bool ntq
   return KVC_OK;
 }
 
+// Several layers of slot-mapped writes, as many to a launch as the arguments hold
+template <typename T>
+int launch_rope_layers(RopeArgs a, const RopeLayer* layers, int64_t num_layers, int64_t num_tokens, bool tail,
+                       bool ntq, unsigned threads, hipStream_t s) {
+  RopeLayersArgs args{};
+  for (int64_t l0 = 0; l0 < num_layers; l0 += kLayersPerLaunch) {
+    const int64_t n = std::min<int64_t>(kLayersPerLaunch, num_layers - l0);
+    args.a = a;
+    std::copy(layers + l0, layers + l0 + n, args.layer);
+    const dim3 grid(a.groups_per_token, (unsigned)num_tokens, (unsigned)n), block(threads);
+    if (tail && ntq) hipLaunchKernelGGL((rope_layers_kernel<T, true, true>), grid, block, 0, s, args);
+    else if (tail) hipLaunchKernelGGL((rope_layers_kernel<T, true, false>), grid, block, 0, s, args);
+    else if (ntq) hipLaunchKernelGGL((rope_layers_kernel<T, false, true>), grid, block, 0, s, args);
+    else hipLaunchKernelGGL((rope_layers_kernel<T, false, false>), grid, block, 0, s, args);
+    KVC_HIP(hipGetLastError());
+  }
+  return KVC_OK;
+}
+
 struct RopeGeom {
   int64_t num_tokens, num_heads, num_kv_heads, head_dim, rotary_dim, max_position;
   int64_t q_token_stride, k_token_stride, v_token_stride, qo_token_stride, ko_token_stride;  // elements
@@ -430,9 +480,38 @@ struct CacheGeom {
   int64_t block_size, cache_block_stride, cache_slot_stride, num_cache_blocks;  // strides in elements
 };
 
+// Does a byte range that one layer writes meet anything that another layer reads or writes?
+// Then the layers depend on their order, and one launch has none. Bytes: of the rows and of a
+// layer's whole cache.
+struct LayerExtents {
+  int64_t query, key, value, query_out, key_out, cache;
+};
+bool layers_depend(const RopeLayer* layers, int64_t n, const LayerExtents& e) {
+  struct Range {
+    const char *begin, *end;
+  };
+  const auto range = [](const char* p, int64_t bytes) { return Range{p, p ? p + bytes : p}; };
+  for (int64_t i = 0; i < n; ++i) {
+    const RopeLayer& w = layers[i];
+    for (int64_t j = 0; j < n; ++j) {
+      if (j == i) continue;
+      const RopeLayer& o = layers[j];
+      for (const Range& x : {range(w.query_out, e.query_out), range(w.key_out, e.key_out), range(w.key_cache, e.cache)})
+        for (const Range& y : {range(o.query, e.query), range(o.key, e.key), range(o.value, e.value),
+                               range(o.query_out, e.query_out), range(o.key_out, e.key_out), range(o.key_cache, e.cache)})
+          if (x.begin < y.end && y.begin < x.end) return true;
+    }
+  }
+  return false;
+}
+
+constexpr int kLayerByLayer = 1;  // run_rope: nothing launched, the layers' buffers do not suit one launch
+
+// With `layers` (the first of them the buffers named before) every layer goes into one launch, or none does.
 int run_rope(const char* fn, const void* query, const void* key, const void* value,
              void* query_out, void* key_out, const void* positions, int pos_bytes,
-             const void* cos_sin_cache, const RopeGeom& g, const CacheGeom* c, void* stream) {
+             const void* cos_sin_cache, const RopeGeom& g, const CacheGeom* c, void* stream,
+             const RopeLayer* layers = nullptr, int64_t num_layers = 0) {
   int E;
   switch (g.dtype) {
     case KVC_DTYPE_BF16: case KVC_DTYPE_F16: E = 2; break;
@@ -520,6 +599,11 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
              (uint64_t)a.v_token_stride | (uint64_t)a.cache_block_stride |
              (uint64_t)a.cache_slot_stride;
   }
+  for (int64_t l = 0; l < num_layers; ++l) {
+    const RopeLayer& p = layers[l];
+    align |= (uintptr_t)p.query | (uintptr_t)p.key | (uintptr_t)p.value | (uintptr_t)p.query_out |
+             (uintptr_t)p.key_out | (uintptr_t)p.key_cache | (uintptr_t)p.value_cache;
+  }
   // 16-byte vectors need aligned rows and halves that hold whole vectors (and offsets inside a row that fit
   // 32 bits)
   const int ev = 16 / E;
@@ -563,7 +647,7 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
     // 17.5 -> 14.0, 23.3 -> 23.3; 67 MB of 32 heads 37.8 -> 36.1, 47.8 -> 47.2. Below 4 MiB the reader loses more
     // than the launch gains (2 MiB of 32 heads 2.73 -> 2.70, 4.9 -> 5.1). A half head of 64 bytes writes each line
     // in two parts and gains nothing (16 MiB of 32 heads x 64 9.8 -> 10.2) before 48 MiB.
-    const int64_t query_bytes = g.num_tokens * g.num_heads * g.head_dim * E;
+    const int64_t query_bytes = std::max<int64_t>(1, num_layers) * g.num_tokens * g.num_heads * g.head_dim * E;
     ntq = query_bytes >= (int64_t(48) << 20) ||
           (query_bytes >= (int64_t(4) << 20) && !tail && g.rotary_dim * E % 256 == 0);
   } else {
@@ -576,6 +660,16 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
     return fail(KVC_ERR_UNSUPPORTED, "%s: launch of %lld workgroups is too large", fn,
                 (long long)(g.num_tokens * (int64_t)a.groups_per_token));
   hipStream_t s = (hipStream_t)stream;
+  if (layers) {
+    if (!vector || !c->slot_mapping || c->slot_bytes != 8 || pos_bytes != 4 || a.bs_shift < 0 ||
+        (kvc::g_rope_tune.nt & 3) || g.num_tokens > 65535)
+      return kLayerByLayer;
+    switch (g.dtype) {
+      case KVC_DTYPE_BF16: return launch_rope_layers<BF16>(a, layers, num_layers, g.num_tokens, tail, ntq, threads, s);
+      case KVC_DTYPE_F16: return launch_rope_layers<F16>(a, layers, num_layers, g.num_tokens, tail, ntq, threads, s);
+      default: return launch_rope_layers<F32>(a, layers, num_layers, g.num_tokens, tail, ntq, threads, s);
+    }
+  }
   switch (g.dtype) {
     case KVC_DTYPE_BF16: return launch_rope<BF16>(a, g.num_tokens, vector, tail, ntq, threads, s);
     case KVC_DTYPE_F16: return launch_rope<F16>(a, g.num_tokens, vector, tail, ntq, threads, s);
@@ -718,6 +812,54 @@ int kvc_rotary_plan_run(const kvc_rotary_plan* plan, const void* query, const vo
       plan->rotary_dim, q_token_stride, k_token_stride, v_token_stride, query_out, key_out, q_row,
       k_row, paged_kv_cache, plan->kv_indices, plan->kv_indptr, plan->batch_size,
       plan->num_kv_indices, plan->page_size, page_stride, num_pages, plan->dtype, stream);
+}
+
+int kvc_rotary_plan_run_layers(const kvc_rotary_plan* plan, int64_t num_layers, const kvc_rotary_layer* layers,
+                               int64_t q_token_stride, int64_t k_token_stride, int64_t v_token_stride,
+                               int64_t page_stride, int64_t num_pages, int* one_launch, void* stream) {
+  constexpr const char* fn = "kvc_rotary_plan_run_layers";
+  if (one_launch) *one_launch = 0;
+  if (!plan) return fail(KVC_ERR_INVALID_ARG, "%s: null plan", fn);
+  if (num_layers < 0 || num_layers > 0xffff || (num_layers > 0 && !layers))
+    return fail(KVC_ERR_INVALID_ARG, "%s: %lld layers", fn, (long long)num_layers);
+  if (num_pages < 0 || page_stride < 0 || q_token_stride < 0 || k_token_stride < 0 || v_token_stride < 0)
+    return fail(KVC_ERR_INVALID_ARG, "%s: negative size", fn);
+  const int64_t q_row = plan->num_heads * plan->head_dim, k_row = plan->num_kv_heads * plan->head_dim;
+  const int64_t E = plan->dtype == KVC_DTYPE_F32 ? 4 : 2, nnz = plan->nnz;
+  const int64_t plane = plan->page_size * k_row;
+  bool whole = plan->slots && num_layers > 1 && nnz > 0 && num_pages > 0 && page_stride >= 2 * plane;
+  RopeLayer* const p = whole ? new (std::nothrow) RopeLayer[num_layers] : nullptr;
+  whole = p != nullptr;
+  for (int64_t l = 0; l < num_layers && whole; ++l) {
+    const kvc_rotary_layer& y = layers[l];
+    whole = y.query && y.key && y.value && y.query_out && y.paged_kv_cache;
+    p[l] = RopeLayer{(const char*)y.query, (const char*)y.key, (const char*)y.value, (char*)y.query_out, (char*)y.key_out,
+                     (char*)y.paged_kv_cache, (char*)y.paged_kv_cache + plane * E};
+  }
+  int rc = kLayerByLayer;
+  if (whole && !layers_depend(p, num_layers,
+                              {((nnz - 1) * q_token_stride + q_row) * E, ((nnz - 1) * k_token_stride + k_row) * E,
+                               ((nnz - 1) * v_token_stride + k_row) * E, nnz * q_row * E, nnz * k_row * E,
+                               ((num_pages - 1) * page_stride + 2 * plane) * E})) {
+    const RopeGeom g{nnz, plan->num_heads, plan->num_kv_heads, plan->head_dim, plan->rotary_dim, plan->max_position,
+                     q_token_stride, k_token_stride, v_token_stride, q_row, k_row, plan->dtype};
+    const CacheGeom c{p->key_cache, p->value_cache, plan->slots, 8, nullptr, nullptr, nullptr, 0, 0,
+                      plan->page_size, page_stride, k_row, num_pages};
+    rc = run_rope(fn, p->query, p->key, p->value, p->query_out, p->key_out, plan->positions, 4,
+                  plan->cos_sin_cache, g, &c, stream, p, num_layers);
+  }
+  delete[] p;
+  if (rc != kLayerByLayer) {
+    if (rc == KVC_OK && one_launch) *one_launch = 1;
+    return rc;
+  }
+  for (int64_t l = 0; l < num_layers; ++l) {
+    const kvc_rotary_layer& y = layers[l];
+    rc = kvc_rotary_plan_run(plan, y.query, y.key, y.value, q_token_stride, k_token_stride, v_token_stride, y.query_out,
+                             y.key_out, y.paged_kv_cache, page_stride, num_pages, stream);
+    if (rc != KVC_OK) return rc;
+  }
+  return KVC_OK;
 }
 
 int kvc_rotary_plan_resolve_slots(kvc_rotary_plan* plan, int64_t* slots, void* stream) {

@@ -392,6 +392,47 @@ class PagedRotaryWritePlan:
         return query_out, key_out
 
 
+    def run_layers(self, queries, keys, values, paged_kv_caches, query_outs) -> bool:
+        """`run` of several layers whose buffers are all at hand (a step to be
+        recorded): one launch for all of them where that cannot change the result
+        (a plan with slots, layers of the same strides, aligned rows, and nothing
+        one layer writes read or written by another), otherwise layer by layer, in
+        order. Every `query_outs[l]` is a buffer. Returns whether one launch did it."""
+        if not len(queries) == len(keys) == len(values) == len(query_outs) == len(paged_kv_caches):
+            raise ValueError("run_layers takes as many of each buffer as there are layers")
+        layers = list(zip(queries, keys, values, query_outs, paged_kv_caches))
+        strides = set()
+        rows = (ctypes.c_void_p * 6 * len(layers))()
+        if self.slots is not None and self.nnz and len(layers) > 1:
+            for row, (q, k, v, o, c) in zip(rows, layers):
+                if not all(isinstance(t, torch.Tensor) for t in (q, k, v, o, c)):
+                    break
+                st = c.stride()
+                if c.dtype is not self.dtype or c.device != self.device or c.dim() != 5 or c.shape[0] == 0 \
+                        or c.shape[1:] != self._cache_shape_tail or st[4] != 1 or st[3] != self.D \
+                        or st[2] != self.kv_row or st[1] != self._k_plane \
+                        or any(t.dim() not in (2, 3) for t in (q, k, v, o)):
+                    break
+                try:
+                    self._rows(o, self.q_row, "query_out", dense=True)
+                    strides.add((self._rows(q, self.q_row, "query"), self._rows(k, self.kv_row, "key"),
+                                 self._rows(v, self.kv_row, "value"),
+                                 st[0] if c.shape[0] > 1 else self._dense_page, c.shape[0]))
+                except (TypeError, ValueError):
+                    break     # `run` names what is wrong with this layer, after the ones before it
+                row[:] = q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), None, c.data_ptr()
+            else:
+                if len(strides) == 1:
+                    one = ctypes.c_int(0)
+                    _lib.check(_lib.lib().kvc_rotary_plan_run_layers(
+                        self._plan, len(layers), rows, *strides.pop(), ctypes.byref(one),
+                        self._get_stream(self._dev_index)))
+                    return bool(one.value)
+        for q, k, v, o, c in layers:
+            self.run(q, k, v, c, query_out=o)
+        return False
+
+
 class RotaryEmbedding(torch.nn.Module):
     """`RotaryEmbedding` of the reference (rotary_embedding.py:11-80): builds the
     cos/sin table from a HF-style config and rotates `(query, key)` in `forward`."""

@@ -179,12 +179,19 @@ class KVWriteStep:
     def capture(self, keys: Sequence[torch.Tensor], values: Sequence[torch.Tensor],
                 caches: Sequence[torch.Tensor], queries: Optional[Sequence[torch.Tensor]] = None,
                 query_outs: Optional[Sequence[torch.Tensor]] = None) -> "torch.cuda.CUDAGraph":
-        """Record `build_index` and one write per layer into a hipGraph. The tensors
+        """Record `build_index` and every layer's write into a hipGraph. The tensors
         are the fixed buffers the model writes its projections into before every
         replay (`max_tokens` rows each). With `queries` the fused rotation runs in
-        place of the plain write. One eager pass runs first (outside the capture)."""
+        place of the plain write, and with `query_outs` as well as one launch for all
+        layers whose buffers allow it (`PagedRotaryWritePlan.run_layers`). One eager
+        pass runs first (outside the capture)."""
         def body():
             self.build_index()
+            if queries is not None and query_outs is not None and self.rotary_plan is not None:
+                n = min(len(keys), len(values), len(caches))
+                self.rotary_plan.run_layers([queries[l] for l in range(n)], keys[:n], values[:n], caches[:n],
+                                            [query_outs[l] for l in range(n)])
+                return
             for l, (k, v, c) in enumerate(zip(keys, values, caches)):
                 if queries is None:
                     self.append(k, v, c)

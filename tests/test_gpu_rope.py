@@ -511,3 +511,60 @@ def test_shapes_at_the_edges_of_the_vector_kernel(gpu, T, Hq, Hkv, D, rd, dtype,
     odd.copy_(cs)
     q_odd, k_odd = kvc.rotary_pos_emb(q, k, pos, odd, D)
     assert torch.equal(q_odd, q_out) and torch.equal(k_odd, k_out)
+
+
+@pytest.mark.parametrize("L,T,Hq,Hkv,D,rd,dtype,bs,form", [
+    (2, 1, 32, 8, 64, 64, torch.bfloat16, 16, "one"),
+    (65, 7, 5, 3, 96, 96, torch.float16, 16, "one"),        # one layer more than a launch holds
+    (5, 29, 4, 2, 80, 32, torch.float16, 16, "one"),        # tails
+    (5, 33, 2, 6, 64, 64, torch.float32, 16, "one"),
+    (3, 700, 8, 1, 128, 128, torch.bfloat16, 16, "one"),    # query_out of 4 MiB and more in all: past the caches
+    (3, 8, 4, 2, 64, 64, torch.bfloat16, 16, "in place"),   # each layer's query_out is its own query
+    (3, 8, 4, 2, 64, 64, torch.bfloat16, 16, "chained"),    # a layer's query_out is the next one's query
+    (3, 8, 4, 2, 64, 64, torch.bfloat16, 16, "shared out"),
+    (3, 8, 4, 2, 64, 64, torch.bfloat16, 16, "interleaved caches"),
+    (3, 8, 4, 2, 64, 64, torch.bfloat16, 16, "shifted"),    # rows that are not 16-byte aligned
+    (3, 8, 4, 2, 64, 64, torch.bfloat16, 16, "other strides"),
+    (3, 8, 4, 2, 64, 64, torch.bfloat16, 12, "block size"),
+    (3, 8, 4, 2, 64, 64, torch.bfloat16, 16, "no slots"),
+])
+def test_layers_of_a_plan_in_one_launch_equal_layer_by_layer(gpu, L, T, Hq, Hkv, D, rd, dtype, bs, form):
+    """Same bytes as one `run` per layer, and one launch exactly where the layers do not depend on their order."""
+    g = torch.Generator().manual_seed(L * T)
+    nb, qw, kw = T // bs + 4, Hq * D, Hkv * D
+    cs = rotary.make_cos_sin_cache(rd, T + 9, 500000.0, dtype=dtype).to(gpu)
+    pos = torch.arange(3, T + 3, dtype=torch.int32, device=gpu)
+    pages = torch.randperm(nb, generator=g)[:(T + 2) // bs + 1].to(gpu, torch.int32)
+    indptr = torch.tensor([0, pages.numel()], dtype=torch.int32, device=gpu)
+    last = torch.tensor([(T + 2) % bs + 1], dtype=torch.int32, device=gpu)
+    owner = torch.zeros(T, dtype=torch.int32, device=gpu)
+    plan = rotary.PagedRotaryWritePlan(owner, pos, pages, indptr, last, cs, Hq, Hkv, D, bs,
+                                       resolve_slots=form != "no slots")
+    start = torch.randn(L, T, qw + 2 * kw + 8, generator=g).to(dtype).to(gpu)
+
+    def buffers():
+        shift = 1 if form == "shifted" else 0
+        x = start.clone()
+        rows = [x[l, :, shift:shift + qw + 2 * kw].split([qw, kw, kw], dim=1) for l in range(L)]
+        q, k, v = (list(t) for t in zip(*rows))
+        if form in ("in place", "chained"):
+            q = [t.contiguous() for t in q]
+        if form == "other strides":
+            k[1] = k[1].contiguous()
+        out = torch.zeros(L, T, qw, dtype=dtype, device=gpu)
+        outs = {"in place": q, "chained": q[1:] + [out[0]], "shared out": [out[0]] * L}.get(form, list(out))
+        if form == "interleaved caches":
+            pool = torch.zeros(nb, L, 2, bs, Hkv, D, dtype=dtype, device=gpu).transpose(0, 1)
+        else:
+            pool = torch.zeros(L, nb, 2, bs, Hkv, D, dtype=dtype, device=gpu)
+        return q, k, v, list(pool), outs, pool
+
+    q, k, v, caches, outs, pool = buffers()
+    for l in range(L):
+        plan.run(q[l], k[l], v[l], caches[l], query_out=outs[l])
+    want = [pool.clone()] + [t.clone() for t in outs]
+    q, k, v, caches, outs, pool = buffers()
+    assert plan.run_layers(q, k, v, caches, outs) is (form in ("one", "in place"))
+    assert all(torch.equal(a, b) for a, b in zip([pool] + outs, want))
+    with pytest.raises(ValueError):
+        plan.run_layers(q, k[1:], v, caches, outs)

@@ -153,6 +153,17 @@ int kvc_rotary_plan_run_layers(const kvc_rotary_plan* plan, int64_t num_layers, 
                                int64_t page_stride, int64_t num_pages, int* one_launch, void* stream);
 
 /*
+ * kvc_copy_blocks on a pair list in host memory, [src, dst] * num_pairs, read before the
+ * call returns; nothing waits for the device. Up to 448 pairs travel in the launch's own
+ * arguments (16-byte aligned blocks); any other list is staged as above into `scratch`
+ * (16 * num_pairs bytes of device memory, 16-byte aligned, in use until the copy has run).
+ * With a NULL scratch such a list is refused with KVC_ERR_STAGING, nothing launched.
+ */
+int kvc_copy_blocks_host_pairs(void* kv_caches, const int64_t* pairs, int64_t num_pairs, int64_t* scratch,
+                               int64_t num_layers, int64_t layer_stride_bytes, int64_t block_bytes,
+                               int64_t num_blocks, void* stream);
+
+/*
  * Do two streams feed the same hardware queue? The runtime maps every stream of
  * a process onto a few hardware queues (4 unless GPU_MAX_HW_QUEUES says
  * otherwise). Kernels of streams that share one run one after the other, and a

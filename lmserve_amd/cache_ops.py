@@ -111,6 +111,15 @@ def copy_blocks(
     if kv_caches.dim() < 2 or not kv_caches.is_contiguous():
         raise ValueError("kv_caches must be a contiguous [L, num_blocks, ...] tensor")
     num_layers, num_blocks = kv_caches.shape[0], kv_caches.shape[1]
+    fast = _lib.fast_entry("copy_blocks") if type(src_to_dst) is dict and not validate else None
+    if fast is not None:
+        # the pairs reach the device with the launch: no copy command to wait for (1 = not what it reads)
+        index = kv_caches.device.index
+        rc = fast(kv_caches, src_to_dst, index, torch._C._cuda_getCurrentRawStream(index))
+        if rc == 0:
+            return
+        if rc < 0:
+            _lib.check(rc)
     if isinstance(src_to_dst, torch.Tensor):
         block_maps_tensor = src_to_dst
         if block_maps_tensor.dtype != torch.int64 or block_maps_tensor.device != kv_caches.device \

@@ -562,6 +562,57 @@ PyObject* fast_upload_requests(PyObject*, PyObject* const* args, Py_ssize_t narg
   END_HANDLE_TH_ERRORS
 }
 
+/* copy_blocks(kv_caches, {src: [dst, ...]}, device, stream) -> 0, 1, or a negative kvc_status:
+ * kvc_copy_blocks_host_pairs on a contiguous [L, num_blocks, ...] pool */
+PyObject* fast_copy_blocks(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS  // an allocation that fails is a Python exception
+  int64_t device;
+  void* stream;
+  if (nargs != 4) {
+    PyErr_SetString(PyExc_TypeError, "copy_blocks takes 4 arguments");
+    return nullptr;
+  }
+  if (!as_i64(args[2], &device) || !as_ptr(args[3], &stream)) return nullptr;
+  const at::Tensor* c = tensor_of(args[0]);
+  if (!c || !PyDict_CheckExact(args[1]) || !c->is_cuda() || c->device().index() != device || c->dim() < 2 ||
+      !c->is_contiguous() || c->numel() == 0 || !on_current_device((int)device) || stream_is_capturing(stream))
+    return PyLong_FromLong(NOT_FAST);
+  std::vector<int64_t> pairs;
+  pairs.reserve(2 * (size_t)PyDict_GET_SIZE(args[1]));
+  PyObject *key, *value;
+  Py_ssize_t at = 0;
+  while (PyDict_Next(args[1], &at, &key, &value)) {  // nothing below runs Python code
+    int64_t src, dst;
+    if (!PyList_CheckExact(value) && !PyTuple_CheckExact(value)) return PyLong_FromLong(NOT_FAST);
+    const Py_ssize_t n = PySequence_Fast_GET_SIZE(value);
+    for (Py_ssize_t i = 0; i < n; ++i) {
+      if (!int_of(key, &src) || !int_of(PySequence_Fast_GET_ITEM(value, i), &dst)) {
+        PyErr_Clear();
+        return PyLong_FromLong(NOT_FAST);
+      }
+      pairs.push_back(src);
+      pairs.push_back(dst);
+    }
+  }
+  const int64_t n = (int64_t)pairs.size() / 2, layers = c->sizes()[0], blocks = c->sizes()[1];
+  if (n == 0) return PyLong_FromLong(0);
+  const int64_t layer_bytes = c->numel() / layers * (int64_t)c->element_size();
+  void* const pool = c->data_ptr();
+  int rc = kvc_copy_blocks_host_pairs(pool, pairs.data(), n, nullptr, layers, layer_bytes, layer_bytes / blocks, blocks,
+                                      stream);
+  if (rc == KVC_ERR_STAGING) {
+    const at::Tensor buf =
+        at::empty({2 * n}, at::TensorOptions().dtype(at::kLong).device(at::kCUDA, (c10::DeviceIndex)device));
+    int64_t* const scratch = (int64_t*)buf.data_ptr();
+    Py_BEGIN_ALLOW_THREADS  // may wait for a staging buffer
+    rc = kvc_copy_blocks_host_pairs(pool, pairs.data(), n, scratch, layers, layer_bytes, layer_bytes / blocks, blocks,
+                                    stream);
+    Py_END_ALLOW_THREADS
+  }
+  return PyLong_FromLong(rc);
+  END_HANDLE_TH_ERRORS
+}
+
 /* scalar_type_code(tensor) -> the integer the two calls above compare dtypes with */
 PyObject* scalar_type_code(PyObject*, PyObject* o) {
   const at::Tensor* t = tensor_of(o);
@@ -589,6 +640,8 @@ PyMethodDef methods[] = {
      "Requests -> the step's index tensors, one launch; 1 = not what it reads, or a negative kvc_status."},
     {"upload_requests", (PyCFunction)(void (*)(void))fast_upload_requests, METH_FASTCALL,
      "Requests -> a KVWriteStep's packed buffer; 1 = not what it reads, or a negative kvc_status."},
+    {"copy_blocks", (PyCFunction)(void (*)(void))fast_copy_blocks, METH_FASTCALL,
+     "kvc_copy_blocks_host_pairs on a pool and a dict; 0, 1 = not what it reads, or a negative kvc_status."},
     {"scalar_type_code", (PyCFunction)scalar_type_code, METH_O, "Integer code of a tensor's dtype."},
     {nullptr, nullptr, 0, nullptr}};
 

@@ -438,8 +438,28 @@ struct TileArgs {
   uint64_t total_chunks;   // n * num_layers * chunks_per_tile
 };
 
-template <int VEC, int UNROLL, bool NT>
-__global__ __launch_bounds__(kThreads) void copy_tiles_kernel(TileArgs a) {
+// A few (source, destination) pairs in the kernel's own arguments. A list in device memory costs a copy command
+// that the host waits for, and with it for everything queued before: a fork of 6 blocks of 2 MiB into two copies
+// each 24.4 us a call with it, 10.0 without. A launch's arguments may take 4 KiB; longer lists are staged (2048
+// pairs of 2 MiB 1466 -> 1420 us a call, 1730 -> 1470 where the pool is new).
+constexpr int kInlinePairs = 448;
+struct PairList {
+  int32_t id[2 * kInlinePairs];
+};
+
+struct ListIds {  // ids of the launch's i-th block, from device memory
+  const TileArgs& a;
+  __device__ __forceinline__ int64_t src(int64_t i) const { return a.src_ids ? a.src_ids[i * a.id_stride] : i; }
+  __device__ __forceinline__ int64_t dst(int64_t i) const { return a.dst_ids ? a.dst_ids[i * a.id_stride] : i; }
+};
+struct InlineIds {
+  const PairList& p;
+  __device__ __forceinline__ int64_t src(int64_t i) const { return p.id[2 * i]; }
+  __device__ __forceinline__ int64_t dst(int64_t i) const { return p.id[2 * i + 1]; }
+};
+
+template <int VEC, int UNROLL, bool NT, typename IDS>
+__device__ __forceinline__ void copy_tiles_chunks(const TileArgs& a, const IDS& ids) {
   using V = typename VecOf<VEC>::type;
   constexpr int64_t kChunk = (int64_t)kThreads * UNROLL * VEC;
   for (uint64_t w = blockIdx.x; w < a.total_chunks; w += gridDim.x) {
@@ -470,8 +490,7 @@ __global__ __launch_bounds__(kThreads) void copy_tiles_kernel(TileArgs a) {
         i = (int64_t)(tile / a.num_layers);
       }
     }
-    const int64_t sid = a.src_ids ? a.src_ids[i * a.id_stride] : i;
-    const int64_t did = a.dst_ids ? a.dst_ids[i * a.id_stride] : i;
+    const int64_t sid = ids.src(i), did = ids.dst(i);
     if (sid < 0 || sid >= a.num_src_blocks || did < 0 || did >= a.num_dst_blocks) continue;
     const char* src = a.src_base + layer * a.src_layer_stride + sid * a.src_block_stride;
     char* dst = a.dst_base + layer * a.dst_layer_stride + did * a.dst_block_stride;
@@ -489,6 +508,15 @@ __global__ __launch_bounds__(kThreads) void copy_tiles_kernel(TileArgs a) {
       if (off < a.tile_bytes) st<NT>(reinterpret_cast<V*>(dst + off), data[j]);
     }
   }
+}
+
+template <int VEC, int UNROLL, bool NT>
+__global__ __launch_bounds__(kThreads) void copy_tiles_kernel(TileArgs a) {
+  copy_tiles_chunks<VEC, UNROLL, NT>(a, ListIds{a});
+}
+template <int UNROLL>
+__global__ __launch_bounds__(kThreads) void copy_pairs_kernel(TileArgs a, PairList p) {
+  copy_tiles_chunks<16, UNROLL, true>(a, InlineIds{p});
 }
 
 // Large copies: one chunk of one tile per workgroup, 16-byte vectors, the order of
@@ -516,8 +544,8 @@ struct StreamArgs {
   int64_t num_src_blocks, num_dst_blocks;
 };
 
-template <int THREADS, int UNROLL, bool NTL, bool NTS>
-__global__ __launch_bounds__(THREADS) void stream_tiles_kernel(StreamArgs a) {
+template <int THREADS, int UNROLL, bool NTL, bool NTS, typename SRC, typename DST>
+__device__ __forceinline__ void stream_tile_chunk(const StreamArgs& a, const SRC& src_id, const DST& dst_id) {
   uint32_t w = blockIdx.x;
   const uint32_t span = 8 * a.xcd_run;
   const uint32_t in_span = w % span;
@@ -533,8 +561,7 @@ __global__ __launch_bounds__(THREADS) void stream_tiles_kernel(StreamArgs a) {
     i = tile / a.num_layers;
     layer = tile - i * a.num_layers;
   }
-  const int64_t sid = a.src_ids ? a.src_ids[(int64_t)i * a.id_stride] : i;
-  const int64_t did = a.dst_ids ? a.dst_ids[(int64_t)i * a.id_stride] : i;
+  const int64_t sid = src_id(i), did = dst_id(i);
   if (sid < 0 || sid >= a.num_src_blocks || did < 0 || did >= a.num_dst_blocks) return;
   const char* src = a.src_base + layer * a.src_layer_stride + sid * a.src_block_stride;
   char* dst = a.dst_base + layer * a.dst_layer_stride + did * a.dst_block_stride;
@@ -551,6 +578,17 @@ __global__ __launch_bounds__(THREADS) void stream_tiles_kernel(StreamArgs a) {
     const uint32_t off = base + j * (THREADS * 16);
     if (off < a.tile_bytes) st<NTS>(reinterpret_cast<u32x4*>(dst + off), data[j]);
   }
+}
+
+template <int THREADS, int UNROLL, bool NTL, bool NTS>
+__global__ __launch_bounds__(THREADS) void stream_tiles_kernel(StreamArgs a) {
+  stream_tile_chunk<THREADS, UNROLL, NTL, NTS>(
+      a, [&](uint32_t i) { return a.src_ids ? a.src_ids[(int64_t)i * a.id_stride] : (int64_t)i; },
+      [&](uint32_t i) { return a.dst_ids ? a.dst_ids[(int64_t)i * a.id_stride] : (int64_t)i; });
+}
+__global__ __launch_bounds__(kThreads) void stream_pairs_kernel(StreamArgs a, PairList p) {
+  stream_tile_chunk<kThreads, 2, true, true>(
+      a, [&](uint32_t i) { return (int64_t)p.id[2 * i]; }, [&](uint32_t i) { return (int64_t)p.id[2 * i + 1]; });
 }
 
 // ---------------------------------------------------------------------------
@@ -1420,7 +1458,7 @@ enum class TileSides { kPools, kGather, kScatter };
 // instead of 6.5 TB/s for both (256 blocks of 1 MiB and 128 of 2 MiB), and 3 % less
 // where the buffer was not in the cache after all. Beyond that size plain accesses
 // cost 10 %.
-int launch_stream(const TileArgs& t, TileSides sides, int64_t n, hipStream_t s) {
+int launch_stream(const TileArgs& t, TileSides sides, int64_t n, hipStream_t s, const PairList* pairs) {
   StreamArgs a{};
   a.src_base = t.src_base; a.dst_base = t.dst_base;
   a.src_ids = t.src_ids; a.dst_ids = t.dst_ids; a.id_stride = t.id_stride;
@@ -1445,7 +1483,8 @@ int launch_stream(const TileArgs& t, TileSides sides, int64_t n, hipStream_t s) 
   const bool plain_store = gather && dense_cached;
   const dim3 grid(a.total_chunks), block(threads);
   constexpr unsigned kFivePerCu = 160 * 1024 / 5;
-  if (gather && plain_store) hipLaunchKernelGGL((stream_tiles_kernel<64, 1, true, false>), grid, block, 0, s, a);
+  if (pairs) hipLaunchKernelGGL(stream_pairs_kernel, grid, block, kFivePerCu, s, a, *pairs);
+  else if (gather && plain_store) hipLaunchKernelGGL((stream_tiles_kernel<64, 1, true, false>), grid, block, 0, s, a);
   else if (gather) hipLaunchKernelGGL((stream_tiles_kernel<64, 1, true, true>), grid, block, 0, s, a);
   else if (plain_load) hipLaunchKernelGGL((stream_tiles_kernel<256, 2, false, true>), grid, block, kFivePerCu, s, a);
   else hipLaunchKernelGGL((stream_tiles_kernel<256, 2, true, true>), grid, block, kFivePerCu, s, a);
@@ -1456,7 +1495,8 @@ int launch_stream(const TileArgs& t, TileSides sides, int64_t n, hipStream_t s) 
 }
 
 template <int VEC>
-int launch_tiles_vec(TileArgs a, int unroll, int max_wgs, hipStream_t s, bool nt, int64_t n, TileSides sides) {
+int launch_tiles_vec(TileArgs a, int unroll, int max_wgs, hipStream_t s, bool nt, int64_t n, TileSides sides,
+                     const PairList* pairs) {
   if (unroll <= 0) {
     // By size, from sweeps of copy_blocks (1 to 4096 pairs x 32 layers x 64 KiB):
     // a launch that fits a quarter of the resident workgroups runs best as few,
@@ -1482,7 +1522,7 @@ int launch_tiles_vec(TileArgs a, int unroll, int max_wgs, hipStream_t s, bool nt
       if (VEC == 16 && max_wgs <= 0 && nt && !g_tune.copy_order && a.tile_bytes >= one_chunk &&
           a.tile_bytes <= (int64_t(1) << 30) &&
           n * (int64_t)a.num_layers * ((a.tile_bytes + 1023) / 1024) <= 0x7fffffffll)
-        return launch_stream(a, sides, n, s);
+        return launch_stream(a, sides, n, s, pairs);
       unroll = sides == TileSides::kGather ? 1 : 2;
     }
   }
@@ -1496,7 +1536,16 @@ int launch_tiles_vec(TileArgs a, int unroll, int max_wgs, hipStream_t s, bool nt
   uint64_t grid = a.total_chunks;
   if (max_wgs > 0) grid = std::min<uint64_t>(grid, (uint64_t)max_wgs);
   grid = std::min<uint64_t>(grid, 0x7fffffffull);
-  switch (unroll) {
+  if (pairs) {  // 16-byte vectors and non-temporal accesses: the caller has looked
+    const dim3 g((unsigned)grid), b(kThreads);
+    switch (unroll) {
+      case 1: hipLaunchKernelGGL((copy_pairs_kernel<1>), g, b, 0, s, a, *pairs); break;
+      case 2: hipLaunchKernelGGL((copy_pairs_kernel<2>), g, b, 0, s, a, *pairs); break;
+      case 4: hipLaunchKernelGGL((copy_pairs_kernel<4>), g, b, 0, s, a, *pairs); break;
+      case 8: hipLaunchKernelGGL((copy_pairs_kernel<8>), g, b, 0, s, a, *pairs); break;
+      default: hipLaunchKernelGGL((copy_pairs_kernel<16>), g, b, 0, s, a, *pairs); break;
+    }
+  } else switch (unroll) {
     case 1: launch_tiles_nt<VEC, 1>(a, (unsigned)grid, s, nt); break;
     case 2: launch_tiles_nt<VEC, 2>(a, (unsigned)grid, s, nt); break;
     case 4: launch_tiles_nt<VEC, 4>(a, (unsigned)grid, s, nt); break;
@@ -1508,8 +1557,11 @@ int launch_tiles_vec(TileArgs a, int unroll, int max_wgs, hipStream_t s, bool nt
   return KVC_OK;
 }
 
+constexpr int kNotInline = 1;  // launch_tiles: nothing launched, the kernels that take `pairs` do not take this copy
+
 // vectors per lane: the gather_unroll knob for a gather, else copy_unroll; by size unless set
-int launch_tiles(const TileArgs& a, int64_t n, int max_wgs, hipStream_t s, TileSides sides = TileSides::kPools) {
+int launch_tiles(const TileArgs& a, int64_t n, int max_wgs, hipStream_t s, TileSides sides = TileSides::kPools,
+                 const PairList* pairs = nullptr) {
   if (n == 0 || a.num_layers == 0 || a.tile_bytes == 0) return KVC_OK;
   const int vec = common_vec({(uint64_t)(uintptr_t)a.src_base, (uint64_t)(uintptr_t)a.dst_base,
                               (uint64_t)a.src_layer_stride, (uint64_t)a.src_block_stride,
@@ -1518,12 +1570,13 @@ int launch_tiles(const TileArgs& a, int64_t n, int max_wgs, hipStream_t s, TileS
   int unroll = sides == TileSides::kGather ? g_tune.gather_unroll : g_tune.copy_unroll;
   if (unroll != 1 && unroll != 2 && unroll != 4 && unroll != 8 && unroll != 16) unroll = 0;  // by size
   const bool nt = g_tune.copy_nt != 0;
+  if (pairs && (vec != 16 || !nt)) return kNotInline;
   switch (vec) {
-    case 16: return launch_tiles_vec<16>(a, unroll, max_wgs, s, nt, n, sides);
-    case 8: return launch_tiles_vec<8>(a, unroll, max_wgs, s, nt, n, sides);
-    case 4: return launch_tiles_vec<4>(a, unroll, max_wgs, s, nt, n, sides);
-    case 2: return launch_tiles_vec<2>(a, unroll, max_wgs, s, nt, n, sides);
-    default: return launch_tiles_vec<1>(a, unroll, max_wgs, s, nt, n, sides);
+    case 16: return launch_tiles_vec<16>(a, unroll, max_wgs, s, nt, n, sides, pairs);
+    case 8: return launch_tiles_vec<8>(a, unroll, max_wgs, s, nt, n, sides, nullptr);
+    case 4: return launch_tiles_vec<4>(a, unroll, max_wgs, s, nt, n, sides, nullptr);
+    case 2: return launch_tiles_vec<2>(a, unroll, max_wgs, s, nt, n, sides, nullptr);
+    default: return launch_tiles_vec<1>(a, unroll, max_wgs, s, nt, n, sides, nullptr);
   }
 }
 
@@ -2624,29 +2677,72 @@ int kvc_write_runs_layers(const void* key, const void* value, void* key_cache, v
                         max_runs, g, stream);
 }
 
-int kvc_copy_blocks(void* kv_caches, const int64_t* block_maps, int64_t num_pairs,
-                    int64_t num_layers, int64_t layer_stride_bytes, int64_t block_bytes,
-                    int64_t num_blocks, void* stream) {
+static int run_copy_blocks(const char* fn, void* kv_caches, const int64_t* block_maps, const PairList* pairs,
+                           int64_t num_pairs, int64_t num_layers, int64_t layer_stride_bytes, int64_t block_bytes,
+                           int64_t num_blocks, void* stream) {
   if (num_pairs < 0 || num_layers < 0 || block_bytes < 0 || num_blocks < 0 || layer_stride_bytes < 0)
-    return fail(KVC_ERR_INVALID_ARG, "kvc_copy_blocks: negative size");
+    return fail(KVC_ERR_INVALID_ARG, "%s: negative size", fn);
   if (num_pairs == 0 || num_layers == 0 || block_bytes == 0) return KVC_OK;
-  if (!kv_caches || !block_maps) return fail(KVC_ERR_INVALID_ARG, "kvc_copy_blocks: null pointer");
+  if (!kv_caches || !(block_maps || pairs)) return fail(KVC_ERR_INVALID_ARG, "%s: null pointer", fn);
   if (layer_stride_bytes < block_bytes)
-    return fail(KVC_ERR_INVALID_ARG, "kvc_copy_blocks: layer stride %lld < block bytes %lld",
+    return fail(KVC_ERR_INVALID_ARG, "%s: layer stride %lld < block bytes %lld", fn,
                 (long long)layer_stride_bytes, (long long)block_bytes);
-  if (num_layers > 0xffffffffll) return fail(KVC_ERR_UNSUPPORTED, "kvc_copy_blocks: too many layers");
+  if (num_layers > 0xffffffffll) return fail(KVC_ERR_UNSUPPORTED, "%s: too many layers", fn);
   TileArgs t{};
   t.src_base = (const char*)kv_caches;
   t.dst_base = (char*)kv_caches;
   t.src_ids = block_maps;
-  t.dst_ids = block_maps + 1;
+  t.dst_ids = block_maps ? block_maps + 1 : nullptr;
   t.id_stride = 2;
   t.src_layer_stride = t.dst_layer_stride = layer_stride_bytes;
   t.src_block_stride = t.dst_block_stride = block_bytes;
   t.num_src_blocks = t.num_dst_blocks = num_blocks;
   t.tile_bytes = block_bytes;
   t.num_layers = (uint32_t)num_layers;
-  return launch_tiles(t, num_pairs, g_tune.copy_max_wgs, (hipStream_t)stream);
+  return launch_tiles(t, num_pairs, g_tune.copy_max_wgs, (hipStream_t)stream, TileSides::kPools, pairs);
+}
+
+int kvc_copy_blocks(void* kv_caches, const int64_t* block_maps, int64_t num_pairs,
+                    int64_t num_layers, int64_t layer_stride_bytes, int64_t block_bytes,
+                    int64_t num_blocks, void* stream) {
+  return run_copy_blocks("kvc_copy_blocks", kv_caches, block_maps, nullptr, num_pairs, num_layers, layer_stride_bytes,
+                         block_bytes, num_blocks, stream);
+}
+
+int kvc_copy_blocks_host_pairs(void* kv_caches, const int64_t* pairs, int64_t num_pairs, int64_t* scratch,
+                               int64_t num_layers, int64_t layer_stride_bytes, int64_t block_bytes,
+                               int64_t num_blocks, void* stream) {
+  const char* fn = "kvc_copy_blocks_host_pairs";
+  if (num_pairs <= 0 || !pairs)
+    return num_pairs == 0 ? KVC_OK : fail(KVC_ERR_INVALID_ARG, "%s: bad pair list", fn);
+  if (num_pairs <= kInlinePairs) {
+    PairList list;
+    int64_t n = 0;
+    for (int64_t i = 0; i < num_pairs; ++i) {
+      const int64_t src = pairs[2 * i], dst = pairs[2 * i + 1];
+      // a pair with an id outside the pool (or beyond 32 bits: left to the other form) copies nothing
+      if (src < 0 || src >= num_blocks || dst < 0 || dst >= num_blocks) continue;
+      if (src > INT32_MAX || dst > INT32_MAX) { n = -1; break; }
+      list.id[2 * n] = (int32_t)src;
+      list.id[2 * n + 1] = (int32_t)dst;
+      ++n;
+    }
+    if (n >= 0) {
+      const int rc = run_copy_blocks(fn, kv_caches, nullptr, &list, n, num_layers, layer_stride_bytes, block_bytes,
+                                     num_blocks, stream);
+      if (rc != kNotInline) return rc;
+    }
+  }
+  if (!scratch) return fail(KVC_ERR_STAGING, "%s: this list needs %lld bytes of scratch", fn, (long long)(16 * num_pairs));
+  if ((uintptr_t)scratch % 16) return fail(KVC_ERR_INVALID_ARG, "%s: misaligned scratch", fn);
+  void* staged = nullptr;
+  int rc = kvc_staging_acquire(16 * num_pairs, &staged);
+  if (rc != KVC_OK) return rc;
+  memcpy(staged, pairs, 16 * num_pairs);
+  rc = kvc_staging_upload(scratch, 16 * num_pairs, stream);
+  if (rc != KVC_OK) return rc;
+  return run_copy_blocks(fn, kv_caches, scratch, nullptr, num_pairs, num_layers, layer_stride_bytes, block_bytes,
+                         num_blocks, stream);
 }
 
 // device-to-device gather / scatter between pool blocks and a dense buffer in

@@ -197,3 +197,39 @@ def test_stream_kernel_dense_buffer_beyond_the_last_level_cache(gpu):
     want[:, ids[nb - n:]] = dense.transpose(0, 1)
     kvc.scatter_blocks(pool, ids[nb - n:].contiguous(), dense)
     assert _lib.last_launch()["non_temporal"] == 1 and torch.equal(pool, want)
+
+
+@pytest.mark.parametrize("block_elems,n,L", [
+    (4096, 1, 2),
+    (4096, 447, 2),        # with the pair that is skipped a list of 448: the longest in a launch's own arguments
+    (4096, 448, 2),        # one more: staged
+    (4096, 300, 8),        # the stream kernel
+    (2051, 20, 2),         # 2-byte vectors: staged
+])
+def test_pairs_from_a_dict_reach_the_device_with_the_launch(gpu, block_elems, n, L):
+    """Lists on either side of what a launch's arguments hold, ids outside the pool skipped, back to back with
+    other lists and no synchronisation between, and from another stream; also with the call extension's place
+    taken by the list in device memory."""
+    nb = 2 * n + 6
+    pool = random_pool((L, nb, block_elems), seed=n)
+    dpool, dlist = to_bf16(pool, gpu), to_bf16(pool, gpu)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    for rep in range(7):
+        ids = np.random.default_rng(rep).permutation(nb).tolist()
+        d = {}
+        for i in range(n):
+            d.setdefault(ids[i - i % 2], []).append(ids[n + 2 + i])
+        d[ids[0]].append([nb, -1, 2**40, 1 - 2**63][rep % 4])
+        for src, dsts in d.items():
+            for dst in dsts:
+                if 0 <= dst < nb:
+                    pool[:, dst] = pool[:, src]
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side if rep == 5 else torch.cuda.current_stream()):
+            kvc.copy_blocks(dpool, d)
+        torch.cuda.current_stream().wait_stream(side)
+        kvc.copy_blocks(dlist, torch.tensor(kvc.flatten_block_maps(d), device=gpu))
+    assert np.array_equal(bits_of(dpool), pool) and np.array_equal(bits_of(dlist), pool)
+    with pytest.raises((TypeError, ValueError)):
+        kvc.copy_blocks(dpool, {0: ["x"]})

@@ -26,6 +26,10 @@
 
 #include <cstdint>
 
+#if PY_VERSION_HEX < 0x030B0000
+#include <longintrepr.h>
+#endif
+
 #include <ATen/ops/empty.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/variable.h>
@@ -270,23 +274,28 @@ bool cos_sin_table(const at::Tensor& cs, at::ScalarType type, int device) {
          cs.sizes()[1] % 2 == 0 && cs.strides()[1] == 1 && (cs.sizes()[0] <= 1 || cs.strides()[0] == cs.sizes()[1]);
 }
 
-/* rotary_pos_emb(query, key, positions, cos_sin_cache, head_dim, query_out, key_out, device, stream):
- * kvc_rotary_pos_emb on tensors; the outputs are dense [n, width] buffers of the caller */
+// A dense, uninitialised tensor of a tensor's shape, type and device.
+at::Tensor dense_like(const at::Tensor& t) {
+  return at::empty(t.sizes(), at::TensorOptions().dtype(t.scalar_type()).device(t.device()));
+}
+
+/* rotary_pos_emb(query, key, positions, cos_sin_cache, head_dim, device, stream) -> 1, a negative kvc_status, or
+ * (query_out, key_out): kvc_rotary_pos_emb on tensors into new dense ones (allocated here: through the interpreter
+ * a call takes 9.5 us, so 5.0) */
 PyObject* fast_rotary_pos_emb(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-  if (nargs != 9) {
-    PyErr_SetString(PyExc_TypeError, "rotary_pos_emb takes 9 arguments");
+  HANDLE_TH_ERRORS  // an allocation that fails is a Python exception
+  if (nargs != 7) {
+    PyErr_SetString(PyExc_TypeError, "rotary_pos_emb takes 7 arguments");
     return nullptr;
   }
   int64_t head_dim, device;
   void* stream;
-  if (!as_i64(args[4], &head_dim) || !as_i64(args[7], &device) || !as_ptr(args[8], &stream)) return nullptr;
+  if (!as_i64(args[4], &head_dim) || !as_i64(args[5], &device) || !as_ptr(args[6], &stream)) return nullptr;
   const at::Tensor* q = tensor_of(args[0]);
   const at::Tensor* k = tensor_of(args[1]);
   const at::Tensor* pos = tensor_of(args[2]);
   const at::Tensor* cs = tensor_of(args[3]);
-  const at::Tensor* qo = tensor_of(args[5]);
-  const at::Tensor* ko = tensor_of(args[6]);
-  if (!q || !k || !pos || !cs || !qo || !ko || head_dim <= 0) return PyLong_FromLong(NOT_FAST);
+  if (!q || !k || !pos || !cs || head_dim <= 0) return PyLong_FromLong(NOT_FAST);
   const int dev = (int)device;
   const at::ScalarType type = q->scalar_type();
   const int kd = kvc_dtype_of(type);
@@ -294,16 +303,22 @@ PyObject* fast_rotary_pos_emb(PyObject*, PyObject* const* args, Py_ssize_t nargs
   const bool pos64 = pos->scalar_type() == at::kLong;
   if (!index_array(*pos, dev, pos64 ? at::kLong : at::kInt)) return PyLong_FromLong(NOT_FAST);
   const int64_t n = pos->sizes()[0];
-  int64_t qw, qs, kw, ks, ow, os;
+  int64_t qw, qs, kw, ks;
   if (n == 0 || !token_rows(*q, n, type, dev, &qw, &qs) || !token_rows(*k, n, type, dev, &kw, &ks) ||
       qw % head_dim || kw % head_dim)
     return PyLong_FromLong(NOT_FAST);
-  if (!token_rows(*qo, n, type, dev, &ow, &os) || ow != qw || os != qw) return PyLong_FromLong(NOT_FAST);
-  if (!token_rows(*ko, n, type, dev, &ow, &os) || ow != kw || os != kw) return PyLong_FromLong(NOT_FAST);
-  return PyLong_FromLong(kvc_rotary_pos_emb(q->data_ptr(), k->data_ptr(), pos->data_ptr(), pos64 ? 8 : 4,
-                                            cs->data_ptr(), cs->sizes()[0], n, qw / head_dim, kw / head_dim,
-                                            head_dim, cs->sizes()[1] / 2, qs, ks, qo->data_ptr(),
-                                            ko->data_ptr(), qw, kw, kd, stream));
+  at::Tensor qo, ko;
+  {
+    pybind11::gil_scoped_release no_lock;  // the allocator may wait
+    qo = dense_like(*q);
+    ko = dense_like(*k);
+  }
+  const int rc = kvc_rotary_pos_emb(q->data_ptr(), k->data_ptr(), pos->data_ptr(), pos64 ? 8 : 4, cs->data_ptr(),
+                                    cs->sizes()[0], n, qw / head_dim, kw / head_dim, head_dim, cs->sizes()[1] / 2, qs,
+                                    ks, qo.data_ptr(), ko.data_ptr(), qw, kw, kd, stream);
+  if (rc < 0) return PyLong_FromLong(rc);
+  return Py_BuildValue("(NN)", THPVariable_Wrap(std::move(qo)), THPVariable_Wrap(std::move(ko)));
+  END_HANDLE_TH_ERRORS
 }
 
 /* rotary_append_paged(query, key, value, batch_indices, positions, cos_sin_cache, head_dim, cache,
@@ -366,6 +381,7 @@ struct Requests {
   struct One {
     int64_t input_len, context_len, num_ids;
     PyObject* ids;  // owned: a list or tuple
+    int64_t filled_len;  // where asked for
   };
   std::vector<One> in_order;     // by decreasing input_len, stable
   std::vector<int64_t> order;    // their places in the caller's list
@@ -375,8 +391,21 @@ struct Requests {
   }
 };
 
+// An int of one digit (30 bits) is read in place: a step of 34 000 block ids 181 -> 158 us.
 inline bool int_of(PyObject* o, int64_t* out) {
   if (!PyLong_Check(o)) return false;
+#if PY_VERSION_HEX >= 0x030C0000
+  if (PyUnstable_Long_IsCompact((PyLongObject*)o)) {
+    *out = PyUnstable_Long_CompactValue((PyLongObject*)o);
+    return true;
+  }
+#else
+  const Py_ssize_t digits = Py_SIZE(o);
+  if (digits == 0 || digits == 1) {
+    *out = digits ? (int64_t)((PyLongObject*)o)->ob_digit[0] : 0;
+    return true;
+  }
+#endif
   int overflow = 0;
   *out = PyLong_AsLongLongAndOverflow(o, &overflow);
   return !overflow && !(*out == -1 && PyErr_Occurred());
@@ -392,10 +421,11 @@ bool int_attr(PyObject* o, PyObject* name, int64_t* out) {
 
 // False (no Python error set) when the requests are anything but objects with integer
 // input_len and context_len and a sequence block_ids: the caller's own path then says why.
-bool read_requests(PyObject* inputs, Requests* out) {
+bool read_requests(PyObject* inputs, Requests* out, bool with_filled = false) {
   static PyObject* const s_input = PyUnicode_InternFromString("input_len");
   static PyObject* const s_context = PyUnicode_InternFromString("context_len");
   static PyObject* const s_ids = PyUnicode_InternFromString("block_ids");
+  static PyObject* const s_filled = PyUnicode_InternFromString("filled_token_len");
   if (!PyList_Check(inputs) && !PyTuple_Check(inputs)) return false;
   const Py_ssize_t n = PySequence_Fast_GET_SIZE(inputs);
   out->in_order.reserve(n);
@@ -403,9 +433,10 @@ bool read_requests(PyObject* inputs, Requests* out) {
   for (Py_ssize_t i = 0; i < n; ++i) {
     if (PySequence_Fast_GET_SIZE(inputs) != n) return false;  // an attribute that is a property may run anything
     PyObject* r = PySequence_Fast_GET_ITEM(inputs, i);
-    Requests::One one{0, 0, 0, nullptr};
+    Requests::One one{0, 0, 0, nullptr, 0};
     Py_INCREF(r);
-    if (int_attr(r, s_input, &one.input_len) && int_attr(r, s_context, &one.context_len))
+    if (int_attr(r, s_input, &one.input_len) && int_attr(r, s_context, &one.context_len) &&
+        (!with_filled || int_attr(r, s_filled, &one.filled_len)))
       one.ids = PyObject_GetAttr(r, s_ids);
     Py_DECREF(r);
     if (!one.ids || !(PyList_Check(one.ids) || PyTuple_Check(one.ids))) {
@@ -465,6 +496,8 @@ bool pack_requests(const Requests& q, int64_t stride, int64_t ids_at, int32_t* d
   return true;
 }
 
+constexpr int64_t kStagingMost = int64_t(1) << 30;  // bytes of one staging buffer; the callers' own paths take more
+
 // A staging buffer, without the interpreter's lock: where the device is far behind this waits for one, and what
 // the device waits for may be another thread's work.
 int acquire_staging(int64_t bytes, void** out) {
@@ -488,6 +521,14 @@ PyObject* piece(const at::Tensor& of, at::ScalarType type, int64_t n, int64_t of
   return THPVariable_Wrap(at::Tensor(std::move(impl)));
 }
 
+// An uninitialised buffer of whole 8-byte words on the device; the allocator may wait, so without the lock.
+at::Tensor device_bytes(int64_t bytes, int device) {
+  at::Tensor t;
+  pybind11::gil_scoped_release no_lock;
+  t = at::empty({bytes / 8}, at::TensorOptions().dtype(at::kLong).device(at::kCUDA, (c10::DeviceIndex)device));
+  return t;
+}
+
 /* build_index(requests, page_size, with_slots, device, stream) -> 1, or (cu_seqlens_q, kv_indptr,
  * kv_last_page_len, kv_indices, batch_indices, positions, slot_mapping | None, prefill tokens):
  * requests packed into a staging buffer, kvc_build_write_index_staged into one allocation */
@@ -508,6 +549,7 @@ PyObject* fast_build_index(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     return PyLong_FromLong(NOT_FAST);
   const int64_t B = (int64_t)q.in_order.size(), N = q.ids, T = q.tokens;
   const int64_t ids_at = (3 * B + 3) / 4 * 4;
+  if ((ids_at + N + 4) * 4 > kStagingMost) return PyLong_FromLong(NOT_FAST);
   void* staged = nullptr;
   int rc = acquire_staging((ids_at + N + 4) * 4, &staged);
   if (rc < 0) return PyLong_FromLong(rc);
@@ -516,7 +558,7 @@ PyObject* fast_build_index(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const auto up = [](int64_t bytes) { return (bytes + 15) / 16 * 16; };
   const int64_t o_cu = with_slots ? up(8 * T) : 0, o_ptr = o_cu + up(4 * (B + 1)), o_last = o_ptr + up(4 * (B + 1)),
                 o_ids = o_last + up(4 * B), o_bi = o_ids + up(4 * N), o_pos = o_bi + up(4 * T), end = o_pos + up(4 * T);
-  const at::Tensor buf = at::empty({end / 8}, at::TensorOptions().dtype(at::kLong).device(at::kCUDA, (c10::DeviceIndex)device));
+  const at::Tensor buf = device_bytes(end, (int)device);
   char* p = (char*)buf.data_ptr();
   rc = kvc_build_write_index_staged(B, N, page_size, T, (int32_t*)(p + o_cu), (int32_t*)(p + o_ptr),
                                     (int32_t*)(p + o_last), (int32_t*)(p + o_ids), (int32_t*)(p + o_bi),
@@ -528,6 +570,147 @@ PyObject* fast_build_index(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   return Py_BuildValue("(NNNNNNNL)", piece(buf, at::kInt, B + 1, o_cu), piece(buf, at::kInt, B + 1, o_ptr),
                        piece(buf, at::kInt, B, o_last), piece(buf, at::kInt, N, o_ids), piece(buf, at::kInt, T, o_bi),
                        piece(buf, at::kInt, T, o_pos), slots, (long long)q.prefill_tokens);
+  END_HANDLE_TH_ERRORS
+}
+
+/* host_index(requests, page_size) -> 1, or (position_ids, cu_seqlens_q, prefill tokens, kv_indices, kv_indptr,
+ * kv_last_page_len, batch_indices, positions, slots, order): the index arrays of a step as bytearrays of int32
+ * (slots: int64). 1 also where a request is inconsistent: the caller's own path names it. */
+PyObject* fast_host_index(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS  // an allocation that fails is a Python exception
+  if (nargs != 2) {
+    PyErr_SetString(PyExc_TypeError, "host_index takes 2 arguments");
+    return nullptr;
+  }
+  int64_t page_size;
+  if (!int_of(args[1], &page_size) || page_size <= 0 || page_size > INT32_MAX) return PyLong_FromLong(NOT_FAST);
+  Requests q;
+  if (!read_requests(args[0], &q, true) || q.tokens == 0 || q.ids == 0) return PyLong_FromLong(NOT_FAST);
+  for (const Requests::One& r : q.in_order)
+    if (r.filled_len < 0 || r.context_len - r.filled_len != r.input_len ||
+        r.num_ids < (r.context_len + page_size - 1) / page_size)
+      return PyLong_FromLong(NOT_FAST);
+  const int64_t B = (int64_t)q.in_order.size(), T = q.tokens;
+  const int64_t bytes[8] = {4 * T, 4 * (B + 1), 4 * q.ids, 4 * (B + 1), 4 * B, 4 * T, 4 * T, 8 * T};
+  PyObject* out[9] = {};  // eight arrays, then the order
+  bool ok = true;
+  for (int i = 0; i < 8 && ok; ++i) ok = (out[i] = PyByteArray_FromStringAndSize(nullptr, bytes[i]));
+  if (ok) ok = (out[8] = PyList_New(B));
+  bool read = ok;
+  if (ok) {
+    const auto words = [&](int i) { return (int32_t*)PyByteArray_AS_STRING(out[i]); };
+    int32_t *pos = words(0), *cu = words(1), *ids = words(2), *ptr = words(3), *last = words(4), *bi = words(5);
+    int64_t* slots = (int64_t*)PyByteArray_AS_STRING(out[7]);
+    int64_t t = 0, at = 0;
+    cu[0] = ptr[0] = 0;
+    for (int64_t b = 0; b < B && read; ++b) {
+      const Requests::One& r = q.in_order[b];
+      if (!(read = copy_ids(r.ids, r.num_ids, ids + at))) break;
+      const int64_t from = t;
+      for (int64_t p = r.filled_len; p < r.context_len;) {
+        const int64_t page = p / page_size, end = std::min(r.context_len, (page + 1) * page_size);
+        for (int64_t slot = ids[at + page] * page_size + p % page_size; p < end; ++p, ++t) {
+          pos[t] = (int32_t)p;
+          bi[t] = (int32_t)b;
+          slots[t] = slot++;
+        }
+      }
+      cu[b + 1] = cu[b] + (int32_t)(t - from);
+      at += r.num_ids;
+      ptr[b + 1] = (int32_t)at;
+      // of an empty request, (0 - 1) mod page_size + 1
+      last[b] = (int32_t)(r.context_len ? (r.context_len - 1) % page_size + 1 : page_size);
+    }
+    if (read) memcpy(PyByteArray_AS_STRING(out[6]), pos, (size_t)bytes[6]);
+    for (int64_t b = 0; b < B && ok; ++b) {
+      PyObject* o = PyLong_FromLongLong(q.order[b]);
+      if (!(ok = o != nullptr)) break;
+      PyList_SET_ITEM(out[8], b, o);
+    }
+  }
+  if (!ok || !read) {
+    for (PyObject* o : out) Py_XDECREF(o);
+    return ok ? PyLong_FromLong(NOT_FAST) : nullptr;
+  }
+  return Py_BuildValue("(NNLNNNNNNN)", out[0], out[1], (long long)q.prefill_tokens, out[2], out[3], out[4], out[5],
+                       out[6], out[7], out[8]);
+  END_HANDLE_TH_ERRORS
+}
+
+constexpr int64_t kUploadMost = 4 << 20;  // bytes of index arrays that go through the staging ring
+
+// The dense buffer of a one-dimensional array of native integers, released with the object.
+struct HostArray {
+  Py_buffer view{};
+  bool held = false;
+  ~HostArray() {
+    if (held) PyBuffer_Release(&view);
+  }
+  bool open(PyObject* o, Py_ssize_t itemsize) {
+    if (PyObject_GetBuffer(o, &view, PyBUF_C_CONTIGUOUS | PyBUF_FORMAT) != 0) {
+      PyErr_Clear();
+      return false;
+    }
+    held = true;
+    const char* f = view.format;
+    return view.ndim == 1 && view.itemsize == itemsize && view.len > 0 && f && f[1] == 0 &&
+           (f[0] == 'i' || f[0] == 'l' || f[0] == 'q');
+  }
+  int64_t size() const { return (int64_t)(view.len / view.itemsize); }
+  const int32_t* words() const { return (const int32_t*)view.buf; }
+};
+
+/* upload_index(position_ids, cu_seqlens_q, kv_indices, kv_indptr, kv_last_page_len, slots | None, page_size, device,
+ * stream) -> 1, a negative kvc_status, or (position_ids, cu_seqlens_q, kv_indices, kv_indptr, kv_last_page_len,
+ * batch_indices, positions, slots | None) on the device, in one allocation: the arrays go through a staging buffer,
+ * where a copy of each from pageable memory would wait for all work queued before it; kvc_get_seq_lens and
+ * kvc_get_batch_indices_positions follow. */
+PyObject* fast_upload_index(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS  // an allocation that fails is a Python exception
+  int64_t page_size, device;
+  void* stream;
+  if (nargs != 9) {
+    PyErr_SetString(PyExc_TypeError, "upload_index takes 9 arguments");
+    return nullptr;
+  }
+  if (!as_i64(args[7], &device) || !as_ptr(args[8], &stream)) return nullptr;
+  if (!int_of(args[6], &page_size) || page_size <= 0 || page_size > INT32_MAX || !on_current_device((int)device) ||
+      stream_is_capturing(stream))
+    return PyLong_FromLong(NOT_FAST);
+  const int arrays = args[5] == Py_None ? 5 : 6;
+  HostArray a[6];
+  for (int i = 0; i < arrays; ++i)
+    if (!a[i].open(args[i], i == 5 ? 8 : 4)) return PyLong_FromLong(NOT_FAST);
+  const int64_t B = a[4].size(), T = a[1].words()[a[1].size() - 1];
+  if (a[1].size() != B + 1 || a[3].size() != B + 1 || T <= 0) return PyLong_FromLong(NOT_FAST);
+  const auto up = [](int64_t n) { return (n + 15) / 16 * 16; };
+  int64_t at[7] = {};
+  for (int i = 0; i < arrays; ++i) at[i + 1] = at[i] + up(a[i].view.len);
+  // more is better off with the copy engine, and would leave the ring that large
+  if (at[arrays] > kUploadMost) return PyLong_FromLong(NOT_FAST);
+  const int64_t staged_bytes = at[arrays], o_bi = staged_bytes, o_pos = o_bi + up(4 * T), o_seq = o_pos + up(4 * T),
+                end = o_seq + up(4 * B);
+  void* staged = nullptr;
+  int rc = acquire_staging(staged_bytes, &staged);
+  if (rc < 0) return PyLong_FromLong(rc);
+  for (int i = 0; i < arrays; ++i) memcpy((char*)staged + at[i], a[i].view.buf, (size_t)a[i].view.len);
+  const at::Tensor buf = device_bytes(end, (int)device);
+  char* p = (char*)buf.data_ptr();
+  rc = kvc_staging_upload(p, staged_bytes, stream);
+  if (rc == KVC_OK)
+    rc = kvc_get_seq_lens((const int32_t*)(p + at[3]), (const int32_t*)(p + at[4]), B, page_size, (int32_t*)(p + o_seq),
+                          stream);
+  if (rc == KVC_OK)
+    rc = kvc_get_batch_indices_positions((const int32_t*)(p + at[1]), (const int32_t*)(p + o_seq), B, T,
+                                         (int32_t*)(p + o_bi), (int32_t*)(p + o_pos), stream);
+  if (rc < 0) return PyLong_FromLong(rc);
+  PyObject* slots;
+  if (arrays == 6) slots = piece(buf, at::kLong, a[5].size(), at[5]);
+  else Py_INCREF(slots = Py_None);
+  return Py_BuildValue("(NNNNNNNN)", piece(buf, at::kInt, a[0].size(), at[0]), piece(buf, at::kInt, B + 1, at[1]),
+                       piece(buf, at::kInt, a[2].size(), at[2]), piece(buf, at::kInt, B + 1, at[3]),
+                       piece(buf, at::kInt, B, at[4]), piece(buf, at::kInt, T, o_bi), piece(buf, at::kInt, T, o_pos),
+                       slots);
   END_HANDLE_TH_ERRORS
 }
 
@@ -550,6 +733,7 @@ PyObject* fast_upload_requests(PyObject*, PyObject* const* args, Py_ssize_t narg
   if (n > max_requests || q.tokens > max_tokens || q.ids > max_ids) return PyLong_FromLong(NOT_FAST);
   void* staged = nullptr;
   const int64_t bytes = (ids_at + q.ids + 3) / 4 * 16;
+  if (bytes > kStagingMost) return PyLong_FromLong(NOT_FAST);
   int rc = acquire_staging(bytes, &staged);
   if (rc < 0) return PyLong_FromLong(rc);
   if (!pack_requests(q, max_requests, ids_at, (int32_t*)staged)) return PyLong_FromLong(NOT_FAST);
@@ -638,6 +822,10 @@ PyMethodDef methods[] = {
      "kvc_rotary_pos_emb_and_append_paged on tensors; 0, 1 = not the fast layout, or a negative kvc_status."},
     {"build_index", (PyCFunction)(void (*)(void))fast_build_index, METH_FASTCALL,
      "Requests -> the step's index tensors, one launch; 1 = not what it reads, or a negative kvc_status."},
+    {"host_index", (PyCFunction)(void (*)(void))fast_host_index, METH_FASTCALL,
+     "Requests -> the step's index arrays in host memory; 1 = not what it reads."},
+    {"upload_index", (PyCFunction)(void (*)(void))fast_upload_index, METH_FASTCALL,
+     "Index arrays -> device tensors; 1 = not what it reads, or a negative kvc_status."},
     {"upload_requests", (PyCFunction)(void (*)(void))fast_upload_requests, METH_FASTCALL,
      "Requests -> a KVWriteStep's packed buffer; 1 = not what it reads, or a negative kvc_status."},
     {"copy_blocks", (PyCFunction)(void (*)(void))fast_copy_blocks, METH_FASTCALL,

@@ -95,17 +95,14 @@ def rotary_pos_emb(query: torch.Tensor, key: torch.Tensor, positions: torch.Tens
     """Rotate `query [T, Hq*D]` and `key [T, Hkv*D]`; returns new tensors of the
     inputs' shapes (rotary_embedding_ops.py:8-35)."""
     fast = _fast_entry("rotary_pos_emb")
-    if fast is not None and isinstance(query, torch.Tensor) and query.is_cuda and query.dim() in (2, 3) \
-            and isinstance(key, torch.Tensor) and key.dim() in (2, 3):
+    if fast is not None and isinstance(query, torch.Tensor) and query.is_cuda:
         # common layouts: checked and launched from C++ (1 = not one of them: fall through)
         dev = query.device.index
-        q_out = torch.empty(query.shape, dtype=query.dtype, device=query.device)
-        k_out = torch.empty(key.shape, dtype=key.dtype, device=key.device)
-        rc = fast(query, key, positions, cos_sin_cache, head_dim, q_out, k_out, dev, _raw_stream(dev))
-        if rc == 0:
-            return q_out, k_out
-        if rc < 0:
-            _lib.check(rc)
+        got = fast(query, key, positions, cos_sin_cache, head_dim, dev, _raw_stream(dev))
+        if type(got) is tuple:
+            return got
+        if got < 0:
+            _lib.check(got)
     q2, k2, positions, pos_bytes, kd, T = _prep(query, key, positions, cos_sin_cache, head_dim)
     q_out = torch.empty_like(q2, memory_format=torch.contiguous_format)
     k_out = torch.empty_like(k2, memory_format=torch.contiguous_format)

@@ -218,3 +218,29 @@ def test_index_builds_far_ahead_of_the_device_and_from_threads_that_end(gpu):
     assert ticked >= waited / 0.02 - 2
     for g, w in zip(got, want):
         assert torch.equal(g.slot_mapping, w.slot_mapping) and torch.equal(g.kv_block_indices, w.kv_block_indices)
+
+
+@pytest.mark.parametrize("tokens,page", [(1, 16), (3, 1), (1023, 16), (4099, 7)])
+def test_host_arrays_on_the_device_in_every_form(gpu, tokens, page):
+    """Dense arrays through the staging ring, more calls than it has buffers, on two streams; strided
+    arrays take the copies: the same tensors."""
+    rng = np.random.default_rng(tokens)
+    filled = int(rng.integers(0, 40))
+    # tables of exactly the blocks a context needs: the device derives the context from the table's length
+    reqs = [kvc.InferInput(i, [], n, filled, filled + n, rng.integers(0, 1 << 24, -(-(filled + n) // page)).tolist())
+            for i, n in enumerate([1, tokens, 2])]
+    host = kvc.make_kv_index_inputs(reqs, page)
+    strided = kvc.KVIndexInputs(**{k: np.repeat(v, 2)[::2] if isinstance(v, np.ndarray) else v
+                                   for k, v in vars(host).items()})
+    side = torch.cuda.Stream(gpu)
+    got = [kvc.to_device(h, page, gpu, slots) for h in (host, strided) for slots in (True, False)]
+    with torch.cuda.stream(side):
+        got += [kvc.to_device(host, page, gpu) for _ in range(7)]
+    torch.cuda.synchronize()
+    for dev in got:
+        for name in ("position_ids", "cu_seqlens_q", "kv_block_indices", "kv_block_indptrs", "kv_last_block_lens",
+                     "batch_indices", "positions", "slot_mapping"):
+            t, want = getattr(dev, name), getattr(host, name)
+            if t is not None:
+                assert t.is_contiguous() and t.device == gpu and np.array_equal(t.cpu().numpy(), want), name
+    assert got[1].slot_mapping is None and got[3].slot_mapping is None

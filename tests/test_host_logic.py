@@ -182,6 +182,39 @@ def test_slot_oracle_of_the_page_table_write_is_pinned():
                                                        idx.kv_block_indptrs, s.block_size), idx.slot_mapping)
 
 
+class _Requests(list):
+    """Requests that the native build refuses: `len` and `[]` are what the loop in the interpreter uses."""
+
+    def __init__(self, requests):
+        self.requests = requests
+
+    def __len__(self):
+        return len(self.requests)
+
+    def __getitem__(self, i):
+        return self.requests[i]
+
+
+@pytest.mark.parametrize("sizes,page", [([1], 16), ([1, 1, 1], 1), ([16, 1, 17], 16), ([5, 0, 33], 4), ([700, 1, 2], 7)])
+def test_make_kv_index_inputs_natively_as_in_the_interpreter(sizes, page):
+    """Block ids of one and two digits of a Python int, tables longer than needed, empty requests, ties in order."""
+    rng = np.random.default_rng(len(sizes) * page)
+    reqs = []
+    for i, n in enumerate(sizes):
+        filled = int(rng.integers(0, 3 * page + 1))
+        ids = rng.integers(0, 2**31, (filled + n + page - 1) // page + i).tolist()
+        reqs.append(InferInput(i, [], n, filled, filled + n, tuple([0, *ids]) if i % 2 else ids + [2**30, 2**30 - 1]))
+    native, plain = make_kv_index_inputs(reqs, page), make_kv_index_inputs(_Requests(reqs), page)
+    for name, want in vars(plain).items():
+        got = getattr(native, name)
+        assert type(got) is type(want)
+        if isinstance(want, np.ndarray):
+            assert got.dtype == want.dtype and np.array_equal(got, want) and got.flags.writeable, name
+        else:
+            assert got == want, name
+    assert not np.shares_memory(native.position_ids, native.positions)
+
+
 def test_make_kv_index_inputs_rejects_inconsistent_requests():
     with pytest.raises(ValueError):
         make_kv_index_inputs([InferInput(0, [1, 1], 2, 0, 3, [0])], 4)   # len mismatch

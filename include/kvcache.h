@@ -369,10 +369,11 @@ int kvc_order_pairs_by_host_id(int64_t* gpu_ids, int64_t* host_ids, int64_t n);
  *     extents, and KVC_SWAP_AUTO reads it to choose (NULL: direct). The caller
  *     orders these calls after the prepare call (same stream, or an event) and
  *     keeps `staging` untouched in between.
- * kvc_thread_release frees what the swap entry points keep per calling thread
- * (events, pinned id bounce buffers); it waits for that thread's pending id
- * uploads. Optional: a thread that never calls it keeps a few KiB of pinned
- * memory until the process ends. */
+ * kvc_thread_release frees what this library keeps per calling thread (events,
+ * pinned id bounce buffers, the staging ring of step inputs) and the staging
+ * rings of threads that have ended; it waits for their pending reads. Optional:
+ * a thread that never calls it keeps a few KiB of pinned memory until the
+ * process ends, and its staging ring goes to the next thread that needs one. */
 int kvc_swap_prepare(const int64_t* gpu_ids, const int64_t* host_ids, int64_t n,
                      int64_t num_gpu_blocks, int64_t num_host_blocks,
                      void* staging, int64_t staging_bytes, void* stream);

@@ -4,6 +4,8 @@ from __future__ import annotations
 import numpy as np
 import torch
 
+from lmserve_amd.index_prep import InferInput
+
 # bf16 bit patterns 0xFFC0..0xFFFF are NaNs with the sign bit set: values a
 # float->bf16 conversion of N(0,1) samples never produces, so a pool pre-filled
 # with them shows every written element and every stray write.
@@ -75,3 +77,62 @@ class FifoBlockIds:
             self.users[i] -= 1
             if self.users[i] == 0:
                 self.queue.append(i)
+
+
+class _Mapped(list):
+    """A sequence that maps its elements on read: what it stores is not what it holds."""
+
+    def __init__(self, items, read):
+        super().__init__(items)
+        self.read = read
+
+    def __getitem__(self, i):
+        return self.read(super().__getitem__(i))
+
+    def __iter__(self):
+        return (self.read(x) for x in super().__iter__())
+
+
+class _Lazy(list):
+    """A sequence that stores nothing and loads its elements on read."""
+
+    def __init__(self, items):
+        super().__init__()
+        self.items = items
+
+    def __len__(self):
+        return len(self.items)
+
+    def __getitem__(self, i):
+        return self.items[i]
+
+    def __iter__(self):
+        return iter(self.items)
+
+
+class _Shifted(int):
+    """An integer that converts to another than it stores."""
+
+    def __int__(self):
+        return int.__add__(self, 100)
+
+    __index__ = __int__
+
+
+def mapped_requests(form):
+    """(requests in a form that overrides how they are read, the same requests plainly): blocks 107 and 103."""
+    plain = [InferInput(0, [], 2, 1, 3, [107]), InferInput(1, [], 1, 0, 1, [103])]
+    if form == "block_ids mapped":
+        return [InferInput(0, [], 2, 1, 3, _Mapped([7], lambda x: x + 100)),
+                InferInput(1, [], 1, 0, 1, _Mapped([3], lambda x: x + 100))], plain
+    if form == "block_ids lazy":
+        return [InferInput(0, [], 2, 1, 3, _Lazy([107])), InferInput(1, [], 1, 0, 1, _Lazy([103]))], plain
+    if form == "requests mapped":
+        return _Mapped([0, 1], plain.__getitem__), plain
+    if form == "requests lazy":
+        return _Lazy(plain), plain
+    assert form == "ids converted"
+    return [InferInput(0, [], 2, 1, 3, [_Shifted(7)]), InferInput(1, [], 1, 0, 1, [_Shifted(3)])], plain
+
+
+MAPPED_FORMS = ["block_ids mapped", "block_ids lazy", "requests mapped", "requests lazy", "ids converted"]

@@ -5,6 +5,7 @@ import torch
 
 import lmserve_amd as kvc
 from oracle import kvc_oracle as orc
+from tests.helpers import MAPPED_FORMS, mapped_requests
 
 pytestmark = pytest.mark.gpu
 
@@ -244,3 +245,18 @@ def test_host_arrays_on_the_device_in_every_form(gpu, tokens, page):
             if t is not None:
                 assert t.is_contiguous() and t.device == gpu and np.array_equal(t.cpu().numpy(), want), name
     assert got[1].slot_mapping is None and got[3].slot_mapping is None
+
+
+# (a general path reads what an int subclass stores, by struct.pack: "ids converted" is the host arrays' own)
+@pytest.mark.parametrize("form", MAPPED_FORMS[:-1])
+def test_requests_are_read_as_they_read_themselves(gpu, form):
+    """Subclasses that map or load their elements on read, by both ways to the device; an empty step only
+    where the requests are empty."""
+    reqs, _ = mapped_requests(form)
+    got = kvc.to_device_one_launch(reqs, 16, gpu)
+    assert got.slot_mapping.tolist() == [107 * 16 + 1, 107 * 16 + 2, 103 * 16]
+    assert got.kv_block_indices.tolist() == [107, 103]
+    step = kvc.KVWriteStep(1, 64, 16, torch.bfloat16, gpu, max_requests=3, max_tokens=4, max_block_ids=5)
+    assert step.set_requests(reqs) == [0, 1]
+    step.build_index()
+    assert step.slot_mapping.tolist() == [107 * 16 + 1, 107 * 16 + 2, 103 * 16, -1]

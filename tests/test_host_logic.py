@@ -9,7 +9,7 @@ import lmserve_amd as kvc
 import workloads as wl
 from lmserve_amd.index_prep import InferInput, make_kv_index_inputs
 from oracle import kvc_oracle as orc
-from tests.helpers import FifoBlockIds
+from tests.helpers import MAPPED_FORMS, FifoBlockIds, mapped_requests
 
 
 def test_flatten_block_maps_keeps_dict_order_and_fans_out():
@@ -183,7 +183,7 @@ def test_slot_oracle_of_the_page_table_write_is_pinned():
 
 
 class _Requests(list):
-    """Requests that the native build refuses: `len` and `[]` are what the loop in the interpreter uses."""
+    """Requests that the native build leaves to the loop in the interpreter, which uses `len` and `[]`."""
 
     def __init__(self, requests):
         self.requests = requests
@@ -213,6 +213,15 @@ def test_make_kv_index_inputs_natively_as_in_the_interpreter(sizes, page):
         else:
             assert got == want, name
     assert not np.shares_memory(native.position_ids, native.positions)
+
+
+@pytest.mark.parametrize("form", MAPPED_FORMS)
+def test_make_kv_index_inputs_reads_subclasses_as_they_read_themselves(form):
+    reqs, plain = mapped_requests(form)
+    got, want = make_kv_index_inputs(reqs, 16), make_kv_index_inputs(plain, 16)
+    assert got.slot_mapping.tolist() == [107 * 16 + 1, 107 * 16 + 2, 103 * 16]
+    for name in ("position_ids", "kv_block_indices", "kv_block_indptrs", "batch_indices", "slot_mapping"):
+        assert np.array_equal(getattr(got, name), getattr(want, name)), name
 
 
 def test_make_kv_index_inputs_rejects_inconsistent_requests():

@@ -214,9 +214,14 @@ __device__ __forceinline__ void st16(char* p, u32x4 v) {
 // 128 8.87 -> 7.65 (4.9 TB/s), 8192 x 72 x 128 60.1 -> 56.8 (5.9 TB/s).
 // TAIL: up to two pass-through vectors per lane, from V and from the heads'
 // unrotated lanes; without it at most one, from V.
-// NTL: non-temporal loads, bit 0 for the K and V rows, bit 1 for the Q rows. NTQ: non-temporal stores of
-// query_out (by its size, see the launch).
-template <typename T, Addressing ADDR, bool FAST, bool TAIL, int NTL, bool NTQ>
+// NTL: non-temporal loads, bit 0 for the K and V rows, bit 1 for the Q rows.
+// query_out by plain stores, whatever its size: non-temporal ones take a part of this launch into the kernel that
+// reads it, and more than that part. Launch alone, then launch + a copy of query_out, then launch + the maximum of
+// every head (us; plain -> non-temporal): 8 MiB of 32 heads x 128 5.7 -> 5.1, 9.4 -> 9.8, 13.6 -> 13.4; 14 MiB of 28
+// heads 8.3 -> 7.4, 13.5 -> 14.5, 19.6 -> 19.6; 32 MiB of 64 heads 17.8 -> 14.0, 27.2 -> 29.8, 39.8 -> 41.4; 64 MiB
+// 31.5 -> 29.8, 52.2 -> 54.0, 70.6 -> 75.5; 187 MiB 85.0 -> 81.5, 159 -> 164, 203 -> 211; 80 MiB of 32 heads x 80 with
+// 32 lanes rotated 66 -> 79, 100 -> 110, 217 -> 254.
+template <typename T, Addressing ADDR, bool FAST, bool TAIL, int NTL>
 __device__ __forceinline__ void rope_vector_lane(const RopeArgs& a, const RopeLayer p) {
   using VT = Vec<T>;
   constexpr uint32_t E = T::kBytes;
@@ -293,8 +298,8 @@ __device__ __forceinline__ void rope_vector_lane(const RopeArgs& a, const RopeLa
     VT::rotate(x, y, cos_x, cos_y, sin_x, sin_y, ox, oy);
     if (!is_k) {  // read again by attention right away
       char* out = p.query_out + (int64_t)t * a.qo_token_stride + head_off;
-      st16<NTQ>(out, ox);
-      st16<NTQ>(out + half, oy);
+      st16<false>(out, ox);
+      st16<false>(out + half, oy);
     } else {
       if (p.key_out) {
         char* out = p.key_out + (int64_t)t * a.ko_token_stride + head_off;
@@ -313,7 +318,7 @@ __device__ __forceinline__ void rope_vector_lane(const RopeArgs& a, const RopeLa
     if (ekind[j] == 1) {
       if (slot >= 0) st16<true>(p.value_cache + slot + eoff[j], ev[j]);
     } else if (TAIL && ekind[j] == 2) {
-      st16<NTQ>(p.query_out + (int64_t)t * a.qo_token_stride + eoff[j], ev[j]);
+      st16<false>(p.query_out + (int64_t)t * a.qo_token_stride + eoff[j], ev[j]);
     } else if (TAIL && ekind[j] == 3) {
       if (p.key_out) st16<false>(p.key_out + (int64_t)t * a.ko_token_stride + eoff[j], ev[j]);
       if (ADDR != kNoCache && slot >= 0) st16<true>(p.key_cache + slot + eoff[j], ev[j]);
@@ -321,9 +326,9 @@ __device__ __forceinline__ void rope_vector_lane(const RopeArgs& a, const RopeLa
   }
 }
 
-template <typename T, Addressing ADDR, bool FAST, bool TAIL, int NTL, bool NTQ>
+template <typename T, Addressing ADDR, bool FAST, bool TAIL, int NTL>
 __global__ __launch_bounds__(kThreads) void rope_vector_kernel(RopeArgs a) {
-  rope_vector_lane<T, ADDR, FAST, TAIL, NTL, NTQ>(
+  rope_vector_lane<T, ADDR, FAST, TAIL, NTL>(
       a, RopeLayer{a.query, a.key, a.value, a.query_out, a.key_out, a.key_cache, a.value_cache});
 }
 
@@ -340,9 +345,9 @@ struct RopeLayersArgs {
 };
 static_assert(sizeof(RopeLayersArgs) <= 4096, "kernel arguments");
 
-template <typename T, bool TAIL, bool NTQ>
+template <typename T, bool TAIL>
 __global__ __launch_bounds__(kThreads) void rope_layers_kernel(RopeLayersArgs args) {
-  rope_vector_lane<T, kSlots, true, TAIL, 0, NTQ>(args.a, args.layer[blockIdx.z]);
+  rope_vector_lane<T, kSlots, true, TAIL, 0>(args.a, args.layer[blockIdx.z]);
 }
 
 // Element path: rows that are no whole number of aligned 16-byte vectors. One
@@ -393,30 +398,24 @@ __global__ __launch_bounds__(kThreads) void rope_element_kernel(RopeArgs a) {
   }
 }
 
-template <typename T, Addressing ADDR, bool FAST, bool TAIL, int NTL>
-void launch_vector_ntq(const RopeArgs& a, bool ntq, dim3 grid, dim3 block, hipStream_t s) {
-  if (ntq) hipLaunchKernelGGL((rope_vector_kernel<T, ADDR, FAST, TAIL, NTL, true>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((rope_vector_kernel<T, ADDR, FAST, TAIL, NTL, false>), grid, block, 0, s, a);
-}
-
 template <typename T, Addressing ADDR>
-void launch_vector(const RopeArgs& a, bool tail, bool ntq, dim3 grid, dim3 block, hipStream_t s) {
+void launch_vector(const RopeArgs& a, bool tail, dim3 grid, dim3 block, hipStream_t s) {
   const bool fast = a.pos_bytes == 4 && (ADDR == kNoCache || a.bs_shift >= 0) && (ADDR != kSlots || a.slot_bytes == 8);
+  const auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, s, a); };
   switch (kvc::g_rope_tune.nt & 3) {
     case 0:
-      if (fast && !tail) launch_vector_ntq<T, ADDR, true, false, 0>(a, ntq, grid, block, s);
-      else if (fast) launch_vector_ntq<T, ADDR, true, true, 0>(a, ntq, grid, block, s);
-      else launch_vector_ntq<T, ADDR, false, true, 0>(a, ntq, grid, block, s);
+      if (fast && !tail) launch(rope_vector_kernel<T, ADDR, true, false, 0>);
+      else if (fast) launch(rope_vector_kernel<T, ADDR, true, true, 0>);
+      else launch(rope_vector_kernel<T, ADDR, false, true, 0>);
       break;
-    case 1: launch_vector_ntq<T, ADDR, false, true, 1>(a, ntq, grid, block, s); break;
-    case 2: launch_vector_ntq<T, ADDR, false, true, 2>(a, ntq, grid, block, s); break;
-    default: launch_vector_ntq<T, ADDR, false, true, 3>(a, ntq, grid, block, s); break;
+    case 1: launch(rope_vector_kernel<T, ADDR, false, true, 1>); break;
+    case 2: launch(rope_vector_kernel<T, ADDR, false, true, 2>); break;
+    default: launch(rope_vector_kernel<T, ADDR, false, true, 3>); break;
   }
 }
 
 template <typename T>
-int launch_rope(RopeArgs a, int64_t num_tokens, bool vector, bool tail, bool ntq, unsigned threads,
-                hipStream_t s) {
+int launch_rope(RopeArgs a, int64_t num_tokens, bool vector, bool tail, unsigned threads, hipStream_t s) {
   if (!vector) {
     hipLaunchKernelGGL((rope_element_kernel<T>), dim3((unsigned)(num_tokens * a.groups_per_token)), dim3(threads),
                        0, s, a);
@@ -427,9 +426,9 @@ int launch_rope(RopeArgs a, int64_t num_tokens, bool vector, bool tail, bool ntq
   const int64_t slot_step = a.slot_bytes, pos_step = a.pos_bytes;
   for (int64_t t0 = 0; t0 < num_tokens; t0 += kMaxY) {
     const dim3 grid(a.groups_per_token, (unsigned)std::min(kMaxY, num_tokens - t0)), block(threads);
-    if (!a.key_cache) launch_vector<T, kNoCache>(a, tail, ntq, grid, block, s);
-    else if (a.batch_indices) launch_vector<T, kPages>(a, tail, ntq, grid, block, s);
-    else launch_vector<T, kSlots>(a, tail, ntq, grid, block, s);
+    if (!a.key_cache) launch_vector<T, kNoCache>(a, tail, grid, block, s);
+    else if (a.batch_indices) launch_vector<T, kPages>(a, tail, grid, block, s);
+    else launch_vector<T, kSlots>(a, tail, grid, block, s);
     KVC_HIP(hipGetLastError());
     a.query += kMaxY * a.q_token_stride;
     a.key += kMaxY * a.k_token_stride;
@@ -446,17 +445,15 @@ int launch_rope(RopeArgs a, int64_t num_tokens, bool vector, bool tail, bool ntq
 // Several layers of slot-mapped writes, as many to a launch as the arguments hold
 template <typename T>
 int launch_rope_layers(RopeArgs a, const RopeLayer* layers, int64_t num_layers, int64_t num_tokens, bool tail,
-                       bool ntq, unsigned threads, hipStream_t s) {
+                       unsigned threads, hipStream_t s) {
   RopeLayersArgs args{};
   for (int64_t l0 = 0; l0 < num_layers; l0 += kLayersPerLaunch) {
     const int64_t n = std::min<int64_t>(kLayersPerLaunch, num_layers - l0);
     args.a = a;
     std::copy(layers + l0, layers + l0 + n, args.layer);
     const dim3 grid(a.groups_per_token, (unsigned)num_tokens, (unsigned)n), block(threads);
-    if (tail && ntq) hipLaunchKernelGGL((rope_layers_kernel<T, true, true>), grid, block, 0, s, args);
-    else if (tail) hipLaunchKernelGGL((rope_layers_kernel<T, true, false>), grid, block, 0, s, args);
-    else if (ntq) hipLaunchKernelGGL((rope_layers_kernel<T, false, true>), grid, block, 0, s, args);
-    else hipLaunchKernelGGL((rope_layers_kernel<T, false, false>), grid, block, 0, s, args);
+    if (tail) hipLaunchKernelGGL((rope_layers_kernel<T, true>), grid, block, 0, s, args);
+    else hipLaunchKernelGGL((rope_layers_kernel<T, false>), grid, block, 0, s, args);
     KVC_HIP(hipGetLastError());
   }
   return KVC_OK;
@@ -613,7 +610,7 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
   const int64_t heads = g.num_heads + g.num_kv_heads;
   unsigned threads = (unsigned)kvc::g_rope_tune.threads;
   const bool fixed = threads == 64 || threads == 128 || threads == 192 || threads == 256;
-  bool tail = false, ntq = false;
+  bool tail = false;
   if (vector) {
     const int64_t pairs = heads * ((g.rotary_dim / 2) / ev);
     const int64_t v_items = c ? g.num_kv_heads * g.head_dim / ev : 0;
@@ -640,16 +637,6 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
         }
     }
     a.groups_per_token = (uint32_t)std::max<int64_t>(1, (lanes + threads - 1) / threads);
-    // query_out by non-temporal stores from 4 MiB on where a half head is whole 128-byte lines: plain stores sit
-    // dirty in the L2s until the kernel's end writes them all back. Measured alone, and with a kernel behind it
-    // that reads query_out (us a pair; plain -> non-temporal): 8 MiB of 32 heads x 128 5.6 -> 5.1, 8.9 -> 8.3;
-    // 14 MiB of 28 heads 8.7 -> 6.9, 11.2 -> 11.2; 16 MiB of 64 heads 8.3 -> 7.9, 12.1 -> 12.4; 32 MiB of 64 heads
-    // 17.5 -> 14.0, 23.3 -> 23.3; 67 MB of 32 heads 37.8 -> 36.1, 47.8 -> 47.2. Below 4 MiB the reader loses more
-    // than the launch gains (2 MiB of 32 heads 2.73 -> 2.70, 4.9 -> 5.1). A half head of 64 bytes writes each line
-    // in two parts and gains nothing (16 MiB of 32 heads x 64 9.8 -> 10.2) before 48 MiB.
-    const int64_t query_bytes = std::max<int64_t>(1, num_layers) * g.num_tokens * g.num_heads * g.head_dim * E;
-    ntq = query_bytes >= (int64_t(48) << 20) ||
-          (query_bytes >= (int64_t(4) << 20) && !tail && g.rotary_dim * E % 256 == 0);
   } else {
     const int64_t items = heads * (g.rotary_dim / 2) + heads * (g.head_dim - g.rotary_dim) +
                           (c ? g.num_kv_heads * g.head_dim : 0);
@@ -665,15 +652,15 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
         (kvc::g_rope_tune.nt & 3) || g.num_tokens > 65535)
       return kLayerByLayer;
     switch (g.dtype) {
-      case KVC_DTYPE_BF16: return launch_rope_layers<BF16>(a, layers, num_layers, g.num_tokens, tail, ntq, threads, s);
-      case KVC_DTYPE_F16: return launch_rope_layers<F16>(a, layers, num_layers, g.num_tokens, tail, ntq, threads, s);
-      default: return launch_rope_layers<F32>(a, layers, num_layers, g.num_tokens, tail, ntq, threads, s);
+      case KVC_DTYPE_BF16: return launch_rope_layers<BF16>(a, layers, num_layers, g.num_tokens, tail, threads, s);
+      case KVC_DTYPE_F16: return launch_rope_layers<F16>(a, layers, num_layers, g.num_tokens, tail, threads, s);
+      default: return launch_rope_layers<F32>(a, layers, num_layers, g.num_tokens, tail, threads, s);
     }
   }
   switch (g.dtype) {
-    case KVC_DTYPE_BF16: return launch_rope<BF16>(a, g.num_tokens, vector, tail, ntq, threads, s);
-    case KVC_DTYPE_F16: return launch_rope<F16>(a, g.num_tokens, vector, tail, ntq, threads, s);
-    default: return launch_rope<F32>(a, g.num_tokens, vector, tail, ntq, threads, s);
+    case KVC_DTYPE_BF16: return launch_rope<BF16>(a, g.num_tokens, vector, tail, threads, s);
+    case KVC_DTYPE_F16: return launch_rope<F16>(a, g.num_tokens, vector, tail, threads, s);
+    default: return launch_rope<F32>(a, g.num_tokens, vector, tail, threads, s);
   }
 }
 

@@ -479,7 +479,7 @@ def test_distance_to_the_reference_kernels_possible_roundings(gpu, name, T, Hq, 
     (29, 4, 2, 72, 16, torch.float32, 16),
     (40, 4, 2, 64, 64, torch.bfloat16, 12),      # block size that is no power of two
     (65537, 1, 1, 16, 16, torch.bfloat16, 16),   # one token more than a launch holds
-    (6144, 32, 1, 128, 128, torch.bfloat16, 16),  # query_out of 48 MiB: stored past the caches
+    (6144, 32, 1, 128, 128, torch.bfloat16, 16),  # query_out of 48 MiB
 ])
 def test_shapes_at_the_edges_of_the_vector_kernel(gpu, T, Hq, Hkv, D, rd, dtype, bs):
     """Rotation against the float64 formula (half an ulp), rows and their places in the cache bit for bit, through
@@ -518,7 +518,7 @@ def test_shapes_at_the_edges_of_the_vector_kernel(gpu, T, Hq, Hkv, D, rd, dtype,
     (65, 7, 5, 3, 96, 96, torch.float16, 16, "one"),        # one layer more than a launch holds
     (5, 29, 4, 2, 80, 32, torch.float16, 16, "one"),        # tails
     (5, 33, 2, 6, 64, 64, torch.float32, 16, "one"),
-    (3, 700, 8, 1, 128, 128, torch.bfloat16, 16, "one"),    # query_out of 4 MiB and more in all: past the caches
+    (3, 700, 8, 1, 128, 128, torch.bfloat16, 16, "one"),    # query_out of more than 4 MiB in all
     (3, 8, 4, 2, 64, 64, torch.bfloat16, 16, "in place"),   # each layer's query_out is its own query
     (3, 8, 4, 2, 64, 64, torch.bfloat16, 16, "chained"),    # a layer's query_out is the next one's query
     (3, 8, 4, 2, 64, 64, torch.bfloat16, 16, "shared out"),

@@ -483,7 +483,7 @@ def test_distance_to_the_reference_kernels_possible_roundings(gpu, name, T, Hq, 
 ])
 def test_shapes_at_the_edges_of_the_vector_kernel(gpu, T, Hq, Hkv, D, rd, dtype, bs):
     """Rotation against the float64 formula (half an ulp), rows and their places in the cache bit for bit, through
-    the slot mapping and through the page table, and with a table that is not 16-byte aligned (element path)."""
+    the slot mapping and through the page table, and with a table that is not 16-byte aligned."""
     q, k, v, pos, cs = (t.to(gpu) for t in _case(gpu, T, Hq, Hkv, D, rd, dtype, max_pos=T + bs, seed=T + D))
     pos = torch.arange(T, device=gpu, dtype=torch.int32)      # one request whose tokens are positions 0..T-1
     nb = T // bs + 3
@@ -524,6 +524,8 @@ def test_shapes_at_the_edges_of_the_vector_kernel(gpu, T, Hq, Hkv, D, rd, dtype,
     (3, 8, 4, 2, 64, 64, torch.bfloat16, 16, "shared out"),
     (3, 8, 4, 2, 64, 64, torch.bfloat16, 16, "interleaved caches"),
     (3, 8, 4, 2, 64, 64, torch.bfloat16, 16, "shifted"),    # rows that are not 16-byte aligned
+    (3, 8, 4, 2, 64, 64, torch.bfloat16, 16, "shifted table"),   # the cos/sin table alone: any element will do
+    (3, 8, 4, 2, 64, 64, torch.float32, 16, "shifted table"),
     (3, 8, 4, 2, 64, 64, torch.bfloat16, 16, "other strides"),
     (3, 8, 4, 2, 64, 64, torch.bfloat16, 12, "block size"),
     (3, 8, 4, 2, 64, 64, torch.bfloat16, 16, "no slots"),
@@ -533,6 +535,8 @@ def test_layers_of_a_plan_in_one_launch_equal_layer_by_layer(gpu, L, T, Hq, Hkv,
     g = torch.Generator().manual_seed(L * T)
     nb, qw, kw = T // bs + 4, Hq * D, Hkv * D
     cs = rotary.make_cos_sin_cache(rd, T + 9, 500000.0, dtype=dtype).to(gpu)
+    if form == "shifted table":
+        cs = torch.cat([cs.flatten()[:1], cs.flatten()])[1:].view_as(cs)
     pos = torch.arange(3, T + 3, dtype=torch.int32, device=gpu)
     pages = torch.randperm(nb, generator=g)[:(T + 2) // bs + 1].to(gpu, torch.int32)
     indptr = torch.tensor([0, pages.numel()], dtype=torch.int32, device=gpu)
@@ -564,7 +568,7 @@ def test_layers_of_a_plan_in_one_launch_equal_layer_by_layer(gpu, L, T, Hq, Hkv,
         plan.run(q[l], k[l], v[l], caches[l], query_out=outs[l])
     want = [pool.clone()] + [t.clone() for t in outs]
     q, k, v, caches, outs, pool = buffers()
-    assert plan.run_layers(q, k, v, caches, outs) is (form in ("one", "in place"))
+    assert plan.run_layers(q, k, v, caches, outs) is (form in ("one", "in place", "shifted table"))
     assert all(torch.equal(a, b) for a, b in zip([pool] + outs, want))
     with pytest.raises(ValueError):
         plan.run_layers(q, k[1:], v, caches, outs)

@@ -82,8 +82,10 @@ struct Vec {
       oy[i] = T::store2(o[1][0], o[1][1]);
     }
   }
-  static __device__ __forceinline__ float load1(const char* p) { return T::load(*(const uint16_t*)p); }
-  static __device__ __forceinline__ void store1(char* p, float f) { *(uint16_t*)p = T::store(f); }
+  // one element
+  typedef uint16_t Word;
+  static __device__ __forceinline__ float wide(Word w) { return T::load(w); }
+  static __device__ __forceinline__ Word narrow(float f) { return T::store(f); }
 };
 template <>
 struct Vec<F32> {
@@ -96,8 +98,9 @@ struct Vec<F32> {
       oy[i] = __float_as_uint(f(y) * f(cy) + f(x) * f(sy));
     }
   }
-  static __device__ __forceinline__ float load1(const char* p) { return *(const float*)p; }
-  static __device__ __forceinline__ void store1(char* p, float f) { *(float*)p = f; }
+  typedef uint32_t Word;
+  static __device__ __forceinline__ float wide(Word w) { return __uint_as_float(w); }
+  static __device__ __forceinline__ Word narrow(float f) { return __float_as_uint(f); }
 };
 
 struct RopeArgs {
@@ -360,54 +363,80 @@ __global__ __launch_bounds__(kThreads) void rope_layers_kernel(RopeLayersArgs ar
 // Element path: rows that are no whole number of aligned 16-byte vectors. One
 // rotation pair or one pass-through element per lane, in this order: pairs of the
 // Q heads then the K heads, elements beyond rotary_dim, V.
-template <typename T>
+// Bound: instructions and 2- or 4-byte accesses at prefill sizes, the chain of
+// dependent loads at decode sizes. So the rows are asked for first, the position's
+// and the slot's chains run behind them, and the lean index forms are as above. us a
+// launch with the row of cos/sin in LDS (first form), the slot's chain ahead of
+// the rows, and now: 256 tokens x 15 heads x 36 in fp32 3.77, 5.26, 3.23; 256 x 40 x
+// 128 in bf16 8.03, 7.14, 6.42; 2048 of those 40.4, 37.1, 30.0; 2048 x 32 x 80 with 20
+// lanes rotated 33.9, 29.9, 23.3. 64 and 256 lanes to a workgroup are within 8 % of
+// 128, more often slower.
+template <typename T, Addressing ADDR, bool FAST>
 __global__ __launch_bounds__(kThreads) void rope_element_kernel(RopeArgs a) {
   using VT = Vec<T>;
   constexpr int E = T::kBytes;
   const uint32_t t = blockIdx.x / a.groups_per_token;
   const uint32_t item = (blockIdx.x - t * a.groups_per_token) * blockDim.x + threadIdx.x;
-  const int64_t pos = index_of(a.positions, a.pos_bytes, t);
-  if (pos < 0 || pos >= a.max_position) return;  // no cos/sin row: the token is left alone
+  const int64_t pos = FAST ? (int64_t) reinterpret_cast<const int32_t*>(a.positions)[t] : index_of(a.positions, a.pos_bytes, t);
   const uint32_t rd = a.rotary_dim, half = rd >> 1, D = a.head_dim;
   const uint32_t heads = a.num_heads + a.num_kv_heads;
-  const uint32_t rot_items = heads * half, tail_per_head = D - rd, tail_items = heads * tail_per_head;
-  const int64_t slot = !a.key_cache ? -1 : a.batch_indices ? slot_offset<kPages, false>(a, t, pos)
-                                                         : slot_offset<kSlots, false>(a, t, pos);
-  const char* cs = a.cos_sin_cache + pos * (int64_t)(2 * rd) * E;
-  if (item < rot_items + tail_items) {
-    const bool pair = item < rot_items;
-    const uint32_t i = pair ? item : item - rot_items;
-    const uint32_t h = pair ? i / half : i / tail_per_head;
-    const uint32_t e = pair ? i - h * half : rd + (i - h * tail_per_head);
-    const bool is_k = h >= a.num_heads;
-    const int64_t off = ((int64_t)(is_k ? h - a.num_heads : h) * D + e) * E;
-    const char* in = (is_k ? a.key + (int64_t)t * a.k_token_stride : a.query + (int64_t)t * a.q_token_stride) + off;
-    char* outs[2] = {is_k ? (a.key_out ? a.key_out + (int64_t)t * a.ko_token_stride + off : nullptr)
-                          : a.query_out + (int64_t)t * a.qo_token_stride + off,
-                     is_k && slot >= 0 ? a.key_cache + slot + off : nullptr};
-    float ox = VT::load1(in), oy = 0.f;
-    if (pair) {
-      const float x = ox, y = VT::load1(in + (int64_t)half * E);
-      const float cos_x = VT::load1(cs + (int64_t)e * E), cos_y = VT::load1(cs + (int64_t)(half + e) * E);
-      const float sin_x = VT::load1(cs + (int64_t)(rd + e) * E), sin_y = VT::load1(cs + (int64_t)(rd + half + e) * E);
-      ox = x * cos_x - y * sin_x;
-      oy = y * cos_y + x * sin_y;
-    }
-#pragma unroll
-    for (int o = 0; o < 2; ++o) {
-      if (!outs[o]) continue;
-      VT::store1(outs[o], ox);
-      if (pair) VT::store1(outs[o] + (int64_t)half * E, oy);
-    }
-  } else if (a.key_cache && item < rot_items + tail_items + a.num_kv_heads * D) {
-    const int64_t off = (int64_t)(item - rot_items - tail_items) * E;
-    if (slot >= 0) VT::store1(a.value_cache + slot + off, VT::load1(a.value + (int64_t)t * a.v_token_stride + off));
+  const uint32_t rot_items = heads * half, tail_per_head = D - rd, head_items = rot_items + heads * tail_per_head;
+  const bool pair = item < rot_items;
+  const bool is_v = item >= head_items;
+  if (is_v && (ADDR == kNoCache || item >= head_items + a.num_kv_heads * D)) return;
+  const uint32_t i = pair ? item : item - rot_items;
+  const uint32_t h = is_v ? 0 : pair ? i / half : i / tail_per_head;
+  const uint32_t e = pair ? i - h * half : rd + (i - h * tail_per_head);
+  const bool is_k = h >= a.num_heads;
+  const int64_t off = is_v ? (int64_t)(item - head_items) * E : ((int64_t)(is_k ? h - a.num_heads : h) * D + e) * E;
+  const char* in = (is_v ? a.value + (int64_t)t * a.v_token_stride
+                         : is_k ? a.key + (int64_t)t * a.k_token_stride : a.query + (int64_t)t * a.q_token_stride) + off;
+  const auto at = [](const char* p) { return *reinterpret_cast<const typename VT::Word*>(p); };
+  const typename VT::Word x = at(in), y = pair ? at(in + (int64_t)half * E) : 0;
+  if (pos < 0 || pos >= a.max_position) return;  // no cos/sin row: the token is left alone
+  typename VT::Word cos_x = 0, cos_y = 0, sin_x = 0, sin_y = 0;
+  if (pair) {
+    const char* cs = a.cos_sin_cache + pos * (int64_t)(2 * rd) * E + (int64_t)e * E;
+    cos_x = at(cs);
+    cos_y = at(cs + (int64_t)half * E);
+    sin_x = at(cs + (int64_t)rd * E);
+    sin_y = at(cs + (int64_t)(rd + half) * E);
   }
+  const int64_t slot = slot_offset<ADDR, FAST>(a, t, pos);
+  typename VT::Word ox = x, oy = 0;
+  if (pair) {  // narrowed once, the products contracted by hand: the same bits in every instantiation
+    ox = VT::narrow(__builtin_fmaf(VT::wide(x), VT::wide(cos_x), -(VT::wide(y) * VT::wide(sin_x))));
+    oy = VT::narrow(__builtin_fmaf(VT::wide(y), VT::wide(cos_y), VT::wide(x) * VT::wide(sin_y)));
+  }
+  const auto put = [](char* p, typename VT::Word w) { *reinterpret_cast<typename VT::Word*>(p) = w; };
+  char* row = is_v ? nullptr : is_k ? a.key_out : a.query_out;
+  if (row) {
+    row += (int64_t)t * (is_k ? a.ko_token_stride : a.qo_token_stride) + off;
+    put(row, ox);
+    if (pair) put(row + (int64_t)half * E, oy);
+  }
+  if (ADDR != kNoCache && slot >= 0 && (is_v || is_k)) {
+    char* out = (is_v ? a.value_cache : a.key_cache) + slot + off;
+    put(out, ox);
+    if (pair) put(out + (int64_t)half * E, oy);
+  }
+}
+
+// Index types and block size that the lean instantiations take
+template <Addressing ADDR>
+bool fast_index(const RopeArgs& a) {
+  return a.pos_bytes == 4 && (ADDR == kNoCache || a.bs_shift >= 0) && (ADDR != kSlots || a.slot_bytes == 8);
+}
+
+template <typename T, Addressing ADDR>
+void launch_element(const RopeArgs& a, dim3 grid, dim3 block, hipStream_t s) {
+  if (fast_index<ADDR>(a)) hipLaunchKernelGGL((rope_element_kernel<T, ADDR, true>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((rope_element_kernel<T, ADDR, false>), grid, block, 0, s, a);
 }
 
 template <typename T, Addressing ADDR>
 void launch_vector(const RopeArgs& a, bool tail, dim3 grid, dim3 block, hipStream_t s) {
-  const bool fast = a.pos_bytes == 4 && (ADDR == kNoCache || a.bs_shift >= 0) && (ADDR != kSlots || a.slot_bytes == 8);
+  const bool fast = fast_index<ADDR>(a);
   const auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, s, a); };
   switch (kvc::g_rope_tune.nt & 3) {
     case 0:
@@ -424,8 +453,10 @@ void launch_vector(const RopeArgs& a, bool tail, dim3 grid, dim3 block, hipStrea
 template <typename T>
 int launch_rope(RopeArgs a, int64_t num_tokens, bool vector, bool tail, unsigned threads, hipStream_t s) {
   if (!vector) {
-    hipLaunchKernelGGL((rope_element_kernel<T>), dim3((unsigned)(num_tokens * a.groups_per_token)), dim3(threads),
-                       0, s, a);
+    const dim3 grid((unsigned)(num_tokens * a.groups_per_token)), block(threads);
+    if (!a.key_cache) launch_element<T, kNoCache>(a, grid, block, s);
+    else if (a.batch_indices) launch_element<T, kPages>(a, grid, block, s);
+    else launch_element<T, kSlots>(a, grid, block, s);
     KVC_HIP(hipGetLastError());
     return KVC_OK;
   }

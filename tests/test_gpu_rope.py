@@ -513,6 +513,62 @@ def test_shapes_at_the_edges_of_the_vector_kernel(gpu, T, Hq, Hkv, D, rd, dtype,
     assert torch.equal(q_odd, q_out) and torch.equal(k_odd, k_out)
 
 
+@pytest.mark.parametrize("T,Hq,Hkv,D,rd,dtype,bs,shift", [
+    (1, 1, 1, 2, 2, torch.bfloat16, 16, 0),          # one pair a head
+    (37, 5, 3, 36, 36, torch.float16, 12, 0),        # half heads that are no whole vectors
+    (70, 4, 2, 20, 12, torch.float32, 16, 0),
+    (29, 3, 1, 7, 6, torch.bfloat16, 16, 0),         # heads of an odd size
+    (40, 4, 2, 64, 64, torch.bfloat16, 16, 1),       # rows that start at any element
+    (40, 4, 2, 80, 32, torch.float16, 12, 1),
+])
+@pytest.mark.parametrize("wide_positions,wide_slots", [(False, True), (True, False)])
+def test_element_path_in_every_form(gpu, T, Hq, Hkv, D, rd, dtype, bs, shift, wide_positions, wide_slots):
+    """Rotation alone, by slot mapping and by page table: the float64 formula (half an ulp), rows and their places in
+    the cache bit for bit; tokens without a slot are rotated, tokens without a position are left alone."""
+    def rows(x):
+        return torch.cat([x.flatten()[:shift], x.flatten()]).to(gpu)[shift:].view(x.shape)
+
+    q, k, v, pos, cs = _case(gpu, T, Hq, Hkv, D, rd, dtype, max_pos=T + bs, seed=T + D)
+    pos = torch.arange(T, dtype=torch.int32)
+    q, k, v = rows(q), rows(k), rows(v)
+    nb = T // bs + 3
+    pages = torch.from_numpy(np.random.default_rng(T).permutation(nb)[:T // bs + 1].astype(np.int32)).to(gpu)
+    p, c = pos.to(gpu), cs.to(gpu)
+    slots = pages.long()[(p // bs).long()] * bs + p.long() % bs
+    owner = torch.zeros(T, dtype=torch.int32, device=gpu)
+    if T > 1:
+        slots[0], owner[0] = -1, -1
+    wide = p.long() if wide_positions else p
+    q_out, k_out = kvc.rotary_pos_emb(q, k, wide, c, D)
+    _check_rotation(q_out.cpu(), q.cpu(), pos, cs, D, dtype, "query")
+    _check_rotation(k_out.cpu(), k.cpu(), pos, cs, D, dtype, "key")
+    want = torch.zeros(nb, 2, bs, Hkv, D, dtype=dtype, device=gpu)
+    some = slots >= 0
+    b, e = slots[some] // bs, slots[some] % bs
+    want[b, 0, e] = k_out[some].view(-1, Hkv, D)
+    want[b, 1, e] = v[some].view(-1, Hkv, D)
+    pool = torch.zeros_like(want)
+    q_got, k_got = kvc.rotary_pos_emb_and_cache(q, k, v, wide, c, D, pool, slots if wide_slots else slots.int())
+    assert torch.equal(pool, want) and torch.equal(q_got, q_out) and torch.equal(k_got, k_out)
+    pool.zero_()
+    indptr = torch.tensor([0, pages.numel()], dtype=torch.int32, device=gpu)
+    last = torch.tensor([(T - 1) % bs + 1], dtype=torch.int32, device=gpu)
+    q_got, k_got = kvc.rotary_pos_emb_and_append_paged(q, k, v, owner, p, c, D, pool, pages, indptr, last)
+    assert torch.equal(pool, want) and torch.equal(q_got, q_out) and torch.equal(k_got, k_out)
+    # in place, the last token without a position: its rows and its slot stay as they are
+    wide = wide.clone()
+    wide[-1] = -1
+    before = q[-1].clone()
+    in_place = rows(q.cpu())
+    rc = _lib.lib().kvc_rotary_pos_emb(in_place.data_ptr(), k.data_ptr(), wide.data_ptr(), wide.element_size(),
+                                       c.data_ptr(), c.shape[0], T, Hq, Hkv, D, rd, Hq * D, Hkv * D,
+                                       in_place.data_ptr(), k.data_ptr(), Hq * D, Hkv * D, rotary._DTYPES[dtype],
+                                       torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    assert torch.equal(in_place[:-1], q_out[:-1]) and torch.equal(in_place[-1], before)
+    assert torch.equal(k[:-1], k_out[:-1])
+
+
 @pytest.mark.parametrize("L,T,Hq,Hkv,D,rd,dtype,bs,form", [
     (2, 1, 32, 8, 64, 64, torch.bfloat16, 16, "one"),
     (65, 7, 5, 3, 96, 96, torch.float16, 16, "one"),        # one layer more than a launch holds

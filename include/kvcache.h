@@ -373,7 +373,8 @@ int kvc_order_pairs_by_host_id(int64_t* gpu_ids, int64_t* host_ids, int64_t n);
  * pinned id bounce buffers, the staging ring of step inputs) and the staging
  * rings of threads that have ended; it waits for their pending reads. Optional:
  * a thread that never calls it keeps a few KiB of pinned memory until the
- * process ends, and its staging ring goes to the next thread that needs one. */
+ * process ends, and its staging ring (256 KiB and up, by the largest step)
+ * goes to the next thread that needs one. */
 int kvc_swap_prepare(const int64_t* gpu_ids, const int64_t* host_ids, int64_t n,
                      int64_t num_gpu_blocks, int64_t num_host_blocks,
                      void* staging, int64_t staging_bytes, void* stream);

@@ -111,9 +111,11 @@ int kvc_write_runs_layers(const void* key, const void* value,
  * calling thread's pinned buffers (at least `bytes`, 16-byte aligned), to be filled by
  * the caller; the next of the two calls below on the same thread launches a kernel that
  * reads it over the link, and the buffer is reused by itself once the kernel has. An
- * acquired buffer that no launch follows is handed out again. A thread that ends leaves
- * its buffers to the next thread that needs some; kvc_thread_release frees the caller's
- * and those. Not under stream capture (KVC_ERR_UNSUPPORTED): a replay would read what the
+ * acquired buffer that no launch follows is handed out again. The ring has four buffers,
+ * each of which grows to the next power of two of what is asked for (64 KiB at least); an
+ * outgrown one is kept, since freeing pinned memory waits for the device, so a thread holds
+ * up to eight times its largest `bytes`, rounded up. A thread that ends leaves its buffers
+ * to the next thread that needs some; kvc_thread_release frees the caller's and those. Not under stream capture (KVC_ERR_UNSUPPORTED): a replay would read what the
  * buffer holds by then. No counterpart in the reference, which uploads six tensors per
  * step (runtime/worker/llm_worker/model_worker.py:399-423).
  *

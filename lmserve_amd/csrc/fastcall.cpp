@@ -501,7 +501,9 @@ bool pack_requests(const Requests& q, int64_t stride, int64_t ids_at, int32_t* d
   return true;
 }
 
-constexpr int64_t kStagingMost = int64_t(1) << 30;  // bytes of one staging buffer; the callers' own paths take more
+// Bytes of a step that go through the staging ring (4 million block ids): its buffers keep the size they have grown
+// to, here 16 MiB each. The callers' own paths take larger ones.
+constexpr int64_t kStagingMost = (int64_t(16) << 20) - 4096;
 
 // A staging buffer, without the interpreter's lock: where the device is far behind this waits for one, and what
 // the device waits for may be another thread's work.

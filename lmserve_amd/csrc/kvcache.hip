@@ -2565,12 +2565,16 @@ int kvc_copy_blocks_host_pairs(void* kv_caches, const int64_t* pairs, int64_t nu
   }
   if (!scratch) return fail(KVC_ERR_STAGING, "%s: this list needs %lld bytes of scratch", fn, (long long)(16 * num_pairs));
   if ((uintptr_t)scratch % 16) return fail(KVC_ERR_INVALID_ARG, "%s: misaligned scratch", fn);
-  void* staged = nullptr;
-  int rc = kvc_staging_acquire(16 * num_pairs, &staged);
-  if (rc != KVC_OK) return rc;
-  memcpy(staged, pairs, 16 * num_pairs);
-  rc = kvc_staging_upload(scratch, 16 * num_pairs, stream);
-  if (rc != KVC_OK) return rc;
+  constexpr int64_t kPiece = 65000;  // pairs staged at a time, so that the ring stays at 1 MiB a buffer
+  for (int64_t done = 0; done < num_pairs; done += kPiece) {
+    const int64_t n = std::min(kPiece, num_pairs - done);
+    void* staged = nullptr;
+    int rc = kvc_staging_acquire(16 * n, &staged);
+    if (rc != KVC_OK) return rc;
+    memcpy(staged, pairs + 2 * done, 16 * n);
+    rc = kvc_staging_upload(scratch + 2 * done, 16 * n, stream);
+    if (rc != KVC_OK) return rc;
+  }
   return run_copy_blocks(fn, kv_caches, scratch, nullptr, num_pairs, num_layers, layer_stride_bytes, block_bytes,
                          num_blocks, stream);
 }

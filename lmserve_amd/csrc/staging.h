@@ -20,22 +20,31 @@ namespace {
 // kernel then reads over the link itself: no copy command, no event (a recorded
 // event costs 3 us of host time here, a launch 3). Each workgroup of the reading
 // kernel sets a word in the buffer's head when it has read its share; a buffer is
-// handed out again once all have. Bounded: kStageSlots buffers of the largest size
-// asked for (rounded up to a power of two). A thread that ends leaves its ring to
-// the next one that needs a ring; kvc_thread_release frees the caller's and those.
+// handed out again once all have. A buffer that is too small is replaced, its
+// reader queued or not, by one of the next power of two; the outgrown one is kept
+// until kvc_thread_release, because freeing pinned memory synchronises the device.
+// So a thread holds kStageSlots times twice the largest size it asked for at most.
+// A thread that ends leaves its ring to the next one that needs a ring;
+// kvc_thread_release frees the caller's and those.
 constexpr int kStageSlots = 4;
 constexpr int kStageMaxWgs = 64;
 constexpr int64_t kStageHead = kStageMaxWgs * (int64_t)sizeof(uint32_t);
 
-struct StageRing {
+struct StageBuffer {
   char* base = nullptr;
-  int64_t slot_bytes = 0;  // head included
+  int64_t bytes = 0;  // head included
+  uint32_t used_seq = 0;
+  int used_wgs = 0;     // workgroups of the last kernel that read it, 0 = none
+  int used_device = 0;  // the device it runs on
+  StageBuffer* next = nullptr;  // of the outgrown ones
+};
+
+struct StageRing {
+  StageBuffer slot[kStageSlots];
+  StageBuffer* outgrown = nullptr;
   int next = 0;
   uint32_t seq = 0;
-  uint32_t used_seq[kStageSlots] = {};
-  int used_wgs[kStageSlots] = {};     // workgroups of the last kernel that read the slot, 0 = none
-  int used_device[kStageSlots] = {};  // the device it runs on
-  int64_t acquired = -1;              // bytes of the slot that is being filled, -1 = none
+  int64_t acquired = -1;  // bytes of the slot that is being filled, -1 = none
   StageRing* idle_next = nullptr;
 };
 
@@ -54,17 +63,17 @@ struct StageHolder {
 };
 thread_local StageHolder g_stage;
 
-// Wait until the last reader of slot i is through. It normally has been for several
+// Wait until the last reader of a buffer is through. It normally has been for several
 // calls; one that is still queued behind long work is waited for by looking at its
 // words now and then, which holds up no other stream, thread or recording. Words that
 // stay unset for a minute belong to a device that is in trouble, or to work that is
 // very long indeed: the wait is then handed to that device, which says which.
-int stage_wait(StageRing& r, int i) {
-  if (!r.used_wgs[i]) return KVC_OK;
-  const uint32_t* flags = reinterpret_cast<const uint32_t*>(r.base + i * r.slot_bytes);
+int stage_wait(StageBuffer& b) {
+  if (!b.used_wgs) return KVC_OK;
+  const uint32_t* flags = reinterpret_cast<const uint32_t*>(b.base);
   const auto read = [&] {
-    for (int w = 0; w < r.used_wgs[i]; ++w)
-      if (__atomic_load_n(flags + w, __ATOMIC_ACQUIRE) != r.used_seq[i]) return false;
+    for (int w = 0; w < b.used_wgs; ++w)
+      if (__atomic_load_n(flags + w, __ATOMIC_ACQUIRE) != b.used_seq) return false;
     return true;
   };
   bool done = false;
@@ -76,28 +85,48 @@ int stage_wait(StageRing& r, int i) {
   if (!done) {
     int dev = 0;
     KVC_HIP(hipGetDevice(&dev));
-    KVC_HIP(hipSetDevice(r.used_device[i]));
+    KVC_HIP(hipSetDevice(b.used_device));
     const hipError_t e = hipDeviceSynchronize();
     KVC_HIP(hipSetDevice(dev));
     KVC_HIP(e);
   }
-  r.used_wgs[i] = 0;
+  b.used_wgs = 0;
   return KVC_OK;
 }
 
-// the buffers of one ring, once nothing reads them
-int stage_free(StageRing& r) {
-  if (!r.base) return KVC_OK;
-  for (int i = 0; i < kStageSlots; ++i) {
-    const int rc = stage_wait(r, i);
-    if (rc != KVC_OK) return rc;
-  }
-  char* base = r.base;
-  r.base = nullptr;
-  r.slot_bytes = 0;
-  r.next = 0;
-  r.acquired = -1;
+// a buffer, once nothing reads it
+int stage_free(StageBuffer& b) {
+  if (!b.base) return KVC_OK;
+  const int rc = stage_wait(b);
+  if (rc != KVC_OK) return rc;
+  char* base = b.base;
+  b.base = nullptr;
+  b.bytes = 0;
   KVC_HIP(hipHostFree(base));
+  return KVC_OK;
+}
+
+// A larger buffer in the place of one that its last reader may still be reading
+int stage_grow(StageRing& r, StageBuffer& b, int64_t need) {
+  int64_t bytes = 64 << 10;
+  while (bytes < need) bytes *= 2;
+  StageBuffer* old = nullptr;
+  if (b.base && !(old = new (std::nothrow) StageBuffer)) return fail(KVC_ERR_HIP, "kvc_staging_acquire: out of host memory");
+  void* base = nullptr;  // coherent: the words are polled while kernels run
+  const hipError_t e = hipHostMalloc(&base, bytes, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent);
+  if (e != hipSuccess) {
+    delete old;
+    KVC_HIP(e);
+  }
+  std::memset(base, 0, kStageHead);
+  if (old) {
+    *old = b;
+    old->next = r.outgrown;
+    r.outgrown = old;
+  }
+  b = StageBuffer{};
+  b.base = (char*)base;
+  b.bytes = bytes;
   return KVC_OK;
 }
 
@@ -118,8 +147,16 @@ int stage_release() {
   while (all) {
     StageRing* r = all;
     all = r->idle_next;
-    const int rc_one = stage_free(*r);
-    if (rc_one != KVC_OK) rc = rc_one;
+    const auto release = [&](StageBuffer& b) {
+      const int rc_one = stage_free(b);
+      if (rc_one != KVC_OK) rc = rc_one;
+    };
+    for (StageBuffer& b : r->slot) release(b);
+    while (StageBuffer* b = r->outgrown) {
+      r->outgrown = b->next;
+      release(*b);
+      delete b;
+    }
     delete r;
   }
   return rc;
@@ -138,21 +175,11 @@ int stage_acquire(int64_t bytes, void** out) {
   }
   StageRing& r = *g_stage.ring;
   r.acquired = -1;
-  if (kStageHead + bytes > r.slot_bytes) {
-    int64_t slot = 64 << 10;
-    while (slot < kStageHead + bytes) slot *= 2;
-    const int rc = stage_free(r);
-    if (rc != KVC_OK) return rc;
-    void* base = nullptr;  // coherent: the words are polled while kernels run
-    KVC_HIP(hipHostMalloc(&base, kStageSlots * slot, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent));
-    r.base = (char*)base;
-    r.slot_bytes = slot;
-    for (int i = 0; i < kStageSlots; ++i) std::memset(r.base + i * slot, 0, kStageHead);
-  }
-  const int rc = stage_wait(r, r.next);
+  StageBuffer& b = r.slot[r.next];
+  const int rc = kStageHead + bytes > b.bytes ? stage_grow(r, b, kStageHead + bytes) : stage_wait(b);
   if (rc != KVC_OK) return rc;
   r.acquired = bytes;
-  *out = r.base + r.next * r.slot_bytes + kStageHead;
+  *out = b.base + kStageHead;
   return KVC_OK;
 }
 
@@ -168,13 +195,13 @@ int stage_hand_over(const char* fn, int64_t bytes, int wgs, void* stream, uint32
   KVC_HIP(hipStreamIsCapturing((hipStream_t)stream, &capturing));
   if (capturing != hipStreamCaptureStatusNone)
     return fail(KVC_ERR_UNSUPPORTED, "%s: the staging buffer of a recorded launch would be overwritten before a replay", fn);
-  const int i = r.next;
-  KVC_HIP(hipGetDevice(&r.used_device[i]));
+  StageBuffer& b = r.slot[r.next];
+  KVC_HIP(hipGetDevice(&b.used_device));
   if (++r.seq == 0) r.seq = 1;
-  r.used_seq[i] = *value = r.seq;
-  r.used_wgs[i] = wgs;
-  *flags = reinterpret_cast<uint32_t*>(r.base + i * r.slot_bytes);
-  r.next = (i + 1) % kStageSlots;
+  b.used_seq = *value = r.seq;
+  b.used_wgs = wgs;
+  *flags = reinterpret_cast<uint32_t*>(b.base);
+  r.next = (r.next + 1) % kStageSlots;
   r.acquired = -1;
   return KVC_OK;
 }
@@ -184,7 +211,7 @@ int stage_launched() {
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
     StageRing& r = *g_stage.ring;
-    r.used_wgs[(r.next + kStageSlots - 1) % kStageSlots] = 0;
+    r.slot[(r.next + kStageSlots - 1) % kStageSlots].used_wgs = 0;
   }
   KVC_HIP(e);
   return KVC_OK;

@@ -205,6 +205,7 @@ def test_stream_kernel_dense_buffer_beyond_the_last_level_cache(gpu):
     (4096, 448, 2),        # one more: staged
     (4096, 300, 8),        # the stream kernel
     (2051, 20, 2),         # 2-byte vectors: staged
+    (8, 65001, 1),         # staged in two pieces
 ])
 def test_pairs_from_a_dict_reach_the_device_with_the_launch(gpu, block_elems, n, L):
     """Lists on either side of what a launch's arguments hold, ids outside the pool skipped, back to back with

@@ -157,6 +157,22 @@ def test_index_from_requests_at_the_edges_of_its_launch(gpu, sizes):
             assert np.array_equal(g.cpu().numpy(), w)
 
 
+def test_a_step_beyond_what_is_staged(gpu):
+    """Block tables of 16 MiB and one request more than that take the unstaged path: the same index."""
+    small = kvc.InferInput(1, [], 3, 5, 8, [9])
+    for ids in ((16 << 20) // 4 - 2000, (16 << 20) // 4):
+        table = list(range(ids))
+        reqs = [small, kvc.InferInput(0, [], 2, 16 * ids - 2, 16 * ids, table)]
+        got = kvc.to_device_one_launch(reqs, 16, gpu)
+        step = kvc.KVWriteStep(1, 64, 16, torch.bfloat16, gpu, max_requests=2, max_tokens=5, max_block_ids=ids + 1)
+        assert step.set_requests(reqs) == [0, 1]
+        step.build_index()
+        want = [9 * 16 + 5, 9 * 16 + 6, 9 * 16 + 7, 16 * ids - 2, 16 * ids - 1]
+        assert got.slot_mapping.tolist() == want and step.slot_mapping.tolist() == want
+        assert torch.equal(got.kv_block_indices, torch.tensor([9] + table, dtype=torch.int32, device=gpu))
+        assert torch.equal(step.kv_indices, got.kv_block_indices)
+
+
 def _check_build(reqs, gpu):
     want = kvc.to_device(kvc.make_kv_index_inputs(reqs, 16), 16, gpu)
     got = kvc.to_device_one_launch(reqs, 16, gpu)

@@ -1,7 +1,7 @@
 """Sanitizer builds of the host-only native code (no GPU) under ThreadSanitizer
 and under AddressSanitizer + UBSan: the row mover's threads, bounded waits, cancel
 and destroy; the disk tier's threaded block I/O, buffered and direct, with aligned
-and unaligned pools. Skipped where g++ or its sanitizer runtimes are absent."""
+and unaligned pools; the staging ring of a step's inputs over a stubbed runtime. Skipped where g++ or its sanitizer runtimes are absent."""
 import os
 import shutil
 import subprocess
@@ -14,7 +14,8 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
 @pytest.mark.parametrize("sanitize", ["thread", "address,undefined"])
 @pytest.mark.parametrize("driver,source,needs_hip", [("row_mover_sanitize.cpp", "host_rows.cpp", True),
-                                                     ("disk_tier_sanitize.cpp", "disk_tier.cpp", False)])
+                                                     ("disk_tier_sanitize.cpp", "disk_tier.cpp", False),
+                                                     ("staging_sanitize.cpp", None, False)])
 def test_host_code_under_sanitizers(tmp_path, sanitize, driver, source, needs_hip):
     gxx = shutil.which("g++")
     if gxx is None or (needs_hip and not os.path.isdir(os.path.join(ROCM, "include", "hip"))):
@@ -23,7 +24,9 @@ def test_host_code_under_sanitizers(tmp_path, sanitize, driver, source, needs_hi
     cmd = [gxx, "-std=c++17", "-O1", "-g", f"-fsanitize={sanitize}", "-D__HIP_PLATFORM_AMD__",
            "-I", os.path.join(ROCM, "include"), "-I", os.path.join(ROOT, "include"),
            "-I", os.path.join(ROOT, "lmserve_amd", "csrc"),
-           os.path.join(ROOT, "tests", "native", driver), os.path.join(ROOT, "lmserve_amd", "csrc", source)]
+           os.path.join(ROOT, "tests", "native", driver)]
+    if source is not None:
+        cmd.append(os.path.join(ROOT, "lmserve_amd", "csrc", source))
     if needs_hip:
         cmd += ["-L", os.path.join(ROCM, "lib"), "-lamdhip64", f"-Wl,-rpath,{os.path.join(ROCM, 'lib')}"]
     cmd += ["-lpthread", "-o", str(exe)]

@@ -115,7 +115,8 @@ int kvc_write_runs_layers(const void* key, const void* value,
  * each of which grows to the next power of two of what is asked for (64 KiB at least); an
  * outgrown one is kept, since freeing pinned memory waits for the device, so a thread holds
  * up to eight times its largest `bytes`, rounded up. A thread that ends leaves its buffers
- * to the next thread that needs some; kvc_thread_release frees the caller's and those. Not under stream capture (KVC_ERR_UNSUPPORTED): a replay would read what the
+ * to the next thread that needs some; kvc_thread_release frees the caller's and those.
+ * KVC_ERR_STAGING where there is no pinned memory for a buffer: nothing has changed. Not under stream capture (KVC_ERR_UNSUPPORTED): a replay would read what the
  * buffer holds by then. No counterpart in the reference, which uploads six tensors per
  * step (runtime/worker/llm_worker/model_worker.py:399-423).
  *

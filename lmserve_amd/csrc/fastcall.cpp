@@ -506,7 +506,8 @@ bool pack_requests(const Requests& q, int64_t stride, int64_t ids_at, int32_t* d
 constexpr int64_t kStagingMost = (int64_t(16) << 20) - 4096;
 
 // A staging buffer, without the interpreter's lock: where the device is far behind this waits for one, and what
-// the device waits for may be another thread's work.
+// the device waits for may be another thread's work. KVC_ERR_STAGING: there is no pinned memory for it, and the
+// callers' own paths need none.
 int acquire_staging(int64_t bytes, void** out) {
   int rc;
   Py_BEGIN_ALLOW_THREADS
@@ -559,7 +560,7 @@ PyObject* fast_build_index(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if ((ids_at + N + 4) * 4 > kStagingMost) return PyLong_FromLong(NOT_FAST);
   void* staged = nullptr;
   int rc = acquire_staging((ids_at + N + 4) * 4, &staged);
-  if (rc < 0) return PyLong_FromLong(rc);
+  if (rc < 0) return PyLong_FromLong(rc == KVC_ERR_STAGING ? NOT_FAST : rc);
   if (!pack_requests(q, B, ids_at, (int32_t*)staged)) return PyLong_FromLong(NOT_FAST);
   // one allocation, every piece 16-byte aligned: slots first (8 bytes an element), then int32 pieces
   const auto up = [](int64_t bytes) { return (bytes + 15) / 16 * 16; };
@@ -699,7 +700,7 @@ PyObject* fast_upload_index(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
                 end = o_seq + up(4 * B);
   void* staged = nullptr;
   int rc = acquire_staging(staged_bytes, &staged);
-  if (rc < 0) return PyLong_FromLong(rc);
+  if (rc < 0) return PyLong_FromLong(rc == KVC_ERR_STAGING ? NOT_FAST : rc);
   for (int i = 0; i < arrays; ++i) memcpy((char*)staged + at[i], a[i].view.buf, (size_t)a[i].view.len);
   const at::Tensor buf = device_bytes(end, (int)device);
   char* p = (char*)buf.data_ptr();
@@ -742,7 +743,7 @@ PyObject* fast_upload_requests(PyObject*, PyObject* const* args, Py_ssize_t narg
   const int64_t bytes = (ids_at + q.ids + 3) / 4 * 16;
   if (bytes > kStagingMost) return PyLong_FromLong(NOT_FAST);
   int rc = acquire_staging(bytes, &staged);
-  if (rc < 0) return PyLong_FromLong(rc);
+  if (rc < 0) return PyLong_FromLong(rc == KVC_ERR_STAGING ? NOT_FAST : rc);
   if (!pack_requests(q, max_requests, ids_at, (int32_t*)staged)) return PyLong_FromLong(NOT_FAST);
   rc = kvc_staging_upload(dst, bytes, stream);
   if (rc < 0) return PyLong_FromLong(rc);
@@ -799,6 +800,7 @@ PyObject* fast_copy_blocks(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     rc = kvc_copy_blocks_host_pairs(pool, pairs.data(), n, scratch, layers, layer_bytes, layer_bytes / blocks, blocks,
                                     stream);
     Py_END_ALLOW_THREADS
+    if (rc == KVC_ERR_STAGING) return PyLong_FromLong(NOT_FAST);
   }
   return PyLong_FromLong(rc);
   END_HANDLE_TH_ERRORS

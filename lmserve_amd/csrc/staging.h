@@ -111,12 +111,15 @@ int stage_grow(StageRing& r, StageBuffer& b, int64_t need) {
   int64_t bytes = 64 << 10;
   while (bytes < need) bytes *= 2;
   StageBuffer* old = nullptr;
-  if (b.base && !(old = new (std::nothrow) StageBuffer)) return fail(KVC_ERR_HIP, "kvc_staging_acquire: out of host memory");
+  if (b.base && !(old = new (std::nothrow) StageBuffer))
+    return fail(KVC_ERR_STAGING, "kvc_staging_acquire: out of host memory");
   void* base = nullptr;  // coherent: the words are polled while kernels run
   const hipError_t e = hipHostMalloc(&base, bytes, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent);
-  if (e != hipSuccess) {
+  if (e != hipSuccess) {  // the caller has a path without staging: no error may stay behind for its next call
     delete old;
-    KVC_HIP(e);
+    (void)hipGetLastError();
+    return fail(KVC_ERR_STAGING, "kvc_staging_acquire: no %lld bytes of pinned memory (%s)", (long long)bytes,
+                hipGetErrorString(e));
   }
   std::memset(base, 0, kStageHead);
   if (old) {
@@ -170,7 +173,7 @@ int stage_acquire(int64_t bytes, void** out) {
       g_stage.ring = g_stage_idle;
       g_stage_idle = g_stage_idle->idle_next;
     } else if (!(g_stage.ring = new (std::nothrow) StageRing)) {
-      return fail(KVC_ERR_HIP, "kvc_staging_acquire: out of host memory");
+      return fail(KVC_ERR_STAGING, "kvc_staging_acquire: out of host memory");
     }
   }
   StageRing& r = *g_stage.ring;

@@ -125,6 +125,26 @@ int main() {
     CHECK(kvc::stage_release() == KVC_OK);
     CHECK(pinned_bytes() == 0);
   }
+  {  // no pinned memory: said as such, no error left behind, and what the ring has stays in use
+    Reader first = launch(100, 2, 'p');
+    for (int k = 0; k < 3; ++k) launch(100, 1, 'q').done();
+    void* p = nullptr;
+    g_out_of_memory = true;
+    g_cleared = 0;
+    CHECK(kvc::stage_acquire(1 << 20, &p) == KVC_ERR_STAGING && p == nullptr && g_cleared == 1);
+    CHECK(holds(first, 100, 'p'));
+    first.done();
+    CHECK(kvc::stage_acquire(200, &p) == KVC_OK && p == first.data());
+    g_out_of_memory = false;
+    launch(1 << 20, 1, 'r').done();
+    CHECK(kvc::stage_release() == KVC_OK);
+    CHECK(pinned_bytes() == 0);
+    g_out_of_memory = true;
+    CHECK(kvc::stage_acquire(100, &p) == KVC_ERR_STAGING);
+    g_out_of_memory = false;
+    launch(100, 1, 's').done();
+    CHECK(kvc::stage_release() == KVC_OK);
+  }
   {  // threads that end: six of them come round to buffers that a reader of an ended thread still has
     std::vector<Reader> queued;
     std::vector<std::thread> devices;

@@ -6,6 +6,9 @@ before their first HIP call (argument validation, pure host arithmetic).
 import ctypes
 import os
 import re
+import shutil
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -555,3 +558,32 @@ def test_queue_sharing_query_without_a_launch():
     assert L.kvc_streams_share_hw_queue(None, None, ctypes.byref(out)) == _lib.KVC_OK and out.value == 1
     assert L.kvc_streams_share_hw_queue(None, None, None) == _lib.KVC_ERR_INVALID_ARG
     assert _lib.streams_share_hw_queue(0, 0) is True
+
+
+def test_calls_without_pinned_memory_take_the_unstaged_path(tmp_path):
+    """The native readers hand a step back (1) where no staging buffer can be had; a stub in front of the library
+    says so, and stands in for the runtime's queries of the current device and stream."""
+    gxx = shutil.which("g++")
+    if gxx is None or _lib.fast() is None:
+        pytest.skip("needs g++ and the call extension")
+    stub = tmp_path / "stub.cpp"
+    stub.write_text("extern \"C\" {\n"
+                    "int hipGetDevice(int* d) { *d = 0; return 0; }\n"
+                    "int hipStreamIsCapturing(void*, int* s) { *s = 0; return 0; }\n"
+                    "int kvc_staging_acquire(long, void** out) { *out = nullptr; return -4; }\n"
+                    "}\n")
+    so = tmp_path / "libstub.so"
+    subprocess.run([gxx, "-shared", "-fPIC", str(stub), "-o", str(so)], check=True)
+    code = ("import ctypes, sys, numpy as np, torch\n"
+            f"ctypes.CDLL({str(so)!r}, mode=ctypes.RTLD_GLOBAL)\n"
+            f"sys.path.insert(0, {REPO!r})\n"
+            "from lmserve_amd import _lib\n"
+            "from lmserve_amd.index_prep import InferInput, make_kv_index_inputs\n"
+            "reqs = [InferInput(0, [], 2, 1, 3, [7])]\n"
+            "h = make_kv_index_inputs(reqs, 16)\n"
+            "f = _lib.fast()\n"
+            "print(f.build_index(reqs, 16, True, 0, 0), f.upload_requests(reqs, 4, 4, 4, 0, 0, 0),\n"
+            "      f.upload_index(h.position_ids, h.cu_seqlens_q, h.kv_block_indices, h.kv_block_indptrs,\n"
+            "                     h.kv_last_block_lens, h.slot_mapping, 16, 0, 0))\n")
+    ran = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+    assert ran.stdout.split() == ["1", "1", "1"], ran.stdout + ran.stderr[-2000:]

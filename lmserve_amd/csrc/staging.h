@@ -193,6 +193,9 @@ int stage_hand_over(const char* fn, int64_t bytes, int wgs, void* stream, uint32
   if (!ring || ring->acquired < bytes)
     return fail(KVC_ERR_STAGING, "%s: %lld bytes wanted of a staging buffer of %lld (kvc_staging_acquire comes first)",
                 fn, (long long)bytes, ring ? (long long)ring->acquired : -1ll);
+  // an error that an earlier call of the application left: stage_launched would take it for the launch's own, and
+  // the buffer for free while the kernel reads it
+  KVC_HIP(hipGetLastError());
   StageRing& r = *ring;
   hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
   KVC_HIP(hipStreamIsCapturing((hipStream_t)stream, &capturing));

@@ -18,6 +18,7 @@ std::mutex g_mutex;
 std::map<void*, size_t> g_pinned;  // live allocations
 std::atomic<int> g_frees{0}, g_device_waits{0}, g_cleared{0};
 std::atomic<bool> g_out_of_memory{false};
+std::atomic<hipError_t> g_last_error{hipSuccess};
 
 size_t pinned_bytes() {
   std::lock_guard<std::mutex> hold(g_mutex);
@@ -45,7 +46,7 @@ hipError_t hipHostFree(void* p) {
 hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }
 hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipDeviceSynchronize() { return ++g_device_waits, hipSuccess; }
-hipError_t hipGetLastError() { return ++g_cleared, hipSuccess; }
+hipError_t hipGetLastError() { return ++g_cleared, g_last_error.exchange(hipSuccess); }
 hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* s) {
   return *s = hipStreamCaptureStatusNone, hipSuccess;
 }
@@ -143,6 +144,18 @@ int main() {
     CHECK(kvc::stage_acquire(100, &p) == KVC_ERR_STAGING);
     g_out_of_memory = false;
     launch(100, 1, 's').done();
+    CHECK(kvc::stage_release() == KVC_OK);
+  }
+  {  // an error from before the launch is reported before it; one of the launch leaves the buffer free
+    void* p = nullptr;
+    uint32_t *flags = nullptr, value = 0;
+    CHECK(kvc::stage_acquire(100, &p) == KVC_OK);
+    g_last_error = hipErrorInvalidValue;
+    CHECK(kvc::stage_hand_over("driver", 100, 1, nullptr, &flags, &value) == KVC_ERR_HIP);
+    CHECK(kvc::stage_hand_over("driver", 100, 1, nullptr, &flags, &value) == KVC_OK);
+    g_last_error = hipErrorInvalidConfiguration;
+    CHECK(kvc::stage_launched() == KVC_ERR_HIP);
+    for (int k = 0; k < 4; ++k) launch(100, 1, 't').done();
     CHECK(kvc::stage_release() == KVC_OK);
   }
   {  // threads that end: six of them come round to buffers that a reader of an ended thread still has

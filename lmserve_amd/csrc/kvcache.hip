@@ -1457,6 +1457,19 @@ void launch_tiles_nt(const TileArgs& a, unsigned grid, hipStream_t s, bool nt) {
 // What a launch copies between: blocks of a pool, or a dense buffer on one side.
 enum class TileSides { kPools, kGather, kScatter };
 
+// Lanes of one launch: HIP takes fewer than 2^32 along a dimension.
+constexpr int64_t kMaxLanes = 0xffffffffll;
+
+// Workgroup of the stream kernel. A gather streams best one vector per lane (6.6 against 6.45 TB/s), a copy and a
+// scatter no worse with two.
+struct StreamShape {
+  int64_t threads, unroll;
+  int64_t chunk() const { return threads * unroll * 16; }
+};
+constexpr StreamShape stream_shape(TileSides sides) {
+  return sides == TileSides::kGather ? StreamShape{64, 1} : StreamShape{256, 2};
+}
+
 // The stream kernel for a launch of `n` tiles per layer. The dense side of a gather or
 // scatter is kept in, or taken from, the 256 MiB last-level cache while it fits (plain
 // accesses): a scatter right behind the gather of the same buffer then moves 7.0
@@ -1472,9 +1485,9 @@ int launch_stream(const TileArgs& t, TileSides sides, int64_t n, hipStream_t s, 
   a.src_layer_stride = t.src_layer_stride; a.src_block_stride = t.src_block_stride;
   a.dst_layer_stride = t.dst_layer_stride; a.dst_block_stride = t.dst_block_stride;
   a.num_src_blocks = t.num_src_blocks; a.num_dst_blocks = t.num_dst_blocks;
-  // a gather streams best one vector per lane (6.6 against 6.45 TB/s), a copy and a scatter no worse with two
   const bool gather = sides == TileSides::kGather;
-  const uint32_t threads = gather ? 64 : 256, unroll = gather ? 1 : 2, chunk = threads * unroll * 16;
+  const StreamShape shape = stream_shape(sides);
+  const uint32_t threads = (uint32_t)shape.threads, unroll = (uint32_t)shape.unroll, chunk = (uint32_t)shape.chunk();
   a.chunks_per_tile = (a.tile_bytes + chunk - 1) / chunk;
   a.total_chunks = (uint32_t)(n * a.num_layers * a.chunks_per_tile);
   a.xcd_run = gather ? 256 : 64;
@@ -1509,8 +1522,8 @@ int launch_tiles_vec(TileArgs a, int unroll, int max_wgs, hipStream_t s, bool nt
     // per workgroup while that stays within half the resident set): 6-8 % faster
     // than 4 vectors per lane from 32 to 128 MiB (a gather: 12-15 % faster than
     // with 1). Larger launches go through the stream kernel; what it does not take
-    // (narrow vectors, tiles below 8 KiB, a capped grid, more than 2^31 chunks, plain copies or another
-    // tile order by request) runs with 2 vectors per lane, or 1 when the scattered
+    // (narrow vectors, tiles below 8 KiB, a capped grid, plain copies or another tile order by request, and
+    // more lanes than a launch has: a gather of 64 GiB, a copy or scatter of 128) runs with 2 vectors per lane, or 1 when the scattered
     // side is the one being read (gather).
     const int64_t resident = resident_workgroups();
     const auto chunks = [&](int u) {
@@ -1523,10 +1536,11 @@ int launch_tiles_vec(TileArgs a, int unroll, int max_wgs, hipStream_t s, bool nt
     if (!unroll && chunks(16) <= resident / 2) unroll = 16;
     if (!unroll) {
       // (a tile below one chunk would leave lanes of every workgroup without work)
-      const int64_t one_chunk = sides == TileSides::kGather ? 1024 : 8192;
-      if (VEC == 16 && max_wgs <= 0 && nt && !g_tune.copy_order && a.tile_bytes >= one_chunk &&
+      const StreamShape shape = stream_shape(sides);
+      const int64_t chunk = shape.chunk();
+      if (VEC == 16 && max_wgs <= 0 && nt && !g_tune.copy_order && a.tile_bytes >= chunk &&
           a.tile_bytes <= (int64_t(1) << 30) &&
-          n * (int64_t)a.num_layers * ((a.tile_bytes + 1023) / 1024) <= 0x7fffffffll)
+          n * (int64_t)a.num_layers * ((a.tile_bytes + chunk - 1) / chunk) <= kMaxLanes / shape.threads)
         return launch_stream(a, sides, n, s, pairs);
       unroll = sides == TileSides::kGather ? 1 : 2;
     }
@@ -1540,7 +1554,7 @@ int launch_tiles_vec(TileArgs a, int unroll, int max_wgs, hipStream_t s, bool nt
   a.layer_slowest = g_tune.copy_order;
   uint64_t grid = a.total_chunks;
   if (max_wgs > 0) grid = std::min<uint64_t>(grid, (uint64_t)max_wgs);
-  grid = std::min<uint64_t>(grid, 0x7fffffffull);
+  grid = std::min<uint64_t>(grid, (uint64_t)(kMaxLanes / kThreads));  // each walks chunks grid-stride
   if (pairs) {  // 16-byte vectors and non-temporal accesses: the caller has looked
     const dim3 g((unsigned)grid), b(kThreads);
     switch (unroll) {

@@ -234,3 +234,35 @@ def test_pairs_from_a_dict_reach_the_device_with_the_launch(gpu, block_elems, n,
     assert np.array_equal(bits_of(dpool), pool) and np.array_equal(bits_of(dlist), pool)
     with pytest.raises((TypeError, ValueError)):
         kvc.copy_blocks(dpool, {0: ["x"]})
+
+
+@pytest.mark.parametrize("block_bytes,n,per_lane,grid", [
+    (1 << 20, 131071, 2, 131071 * 128),                # the largest that the stream kernel takes: 2^32 - 2^15 lanes
+    (1 << 20, 131073, 2, (2**32 - 1) // 256),          # past it: chunks walked grid-stride
+    ((1 << 20) + 8, 70000, 2, (2**32 - 1) // 256),     # 8-byte vectors, never taken by the stream kernel
+])
+def test_copies_of_more_lanes_than_a_launch_has(gpu, block_bytes, n, per_lane, grid):
+    """A list of that many pairs over a small pool: all but the first and the last are outside the pool."""
+    pool = random_pool((1, 8, block_bytes // 2), seed=n)
+    dpool = to_bf16(pool, gpu)
+    pairs = torch.full((n, 2), -1, dtype=torch.int64, device=gpu)
+    pairs[0] = torch.tensor([0, 1])
+    pairs[-1] = torch.tensor([2, 7])
+    kvc.copy_blocks(dpool, pairs.flatten())
+    ran = _lib.last_launch()
+    assert (ran["per_lane"], ran["grid"]) == (per_lane, grid)
+    pool[0, 1], pool[0, 7] = pool[0, 0], pool[0, 2]
+    assert np.array_equal(bits_of(dpool), pool)
+
+
+def test_a_gather_of_more_lanes_than_a_launch_has(gpu):
+    """67 million chunks of 1 KiB, all but the first block's outside the pool: nothing is written for those."""
+    block_bytes, n = 1 << 20, 65537
+    pool = torch.randint(-2**15, 2**15, (1, 2, block_bytes // 2), dtype=torch.int16, device=gpu)
+    dense = torch.zeros(block_bytes // 2, dtype=torch.int16, device=gpu)
+    ids = torch.full((n,), -1, dtype=torch.int64, device=gpu)
+    ids[0] = 1
+    rc = _lib.lib().kvc_gather_blocks(pool.data_ptr(), dense.data_ptr(), ids.data_ptr(), n, 1, block_bytes * 2,
+                                      block_bytes, 2, 0, 1, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0 and _lib.last_launch()["threads"] == 256 and _lib.last_launch()["grid"] == (2**32 - 1) // 256
+    assert torch.equal(dense, pool[0, 1])

@@ -21,13 +21,13 @@ inline int log2_exact(int64_t x) {
 }
 
 // Launch shape of the rotation kernel, set through kvc_set_tuning
-// ("rope_threads": 64/128/256 lanes per workgroup, 0 = by size; "rope_nt":
+// ("rope_threads": 64/128/192/256 lanes per workgroup, 0 = by size; "rope_nt":
 // non-temporal loads, bit 0 the K and V rows, bit 1 the Q rows). Off by default:
-// with both bits a launch whose Q/K/V come from HBM gains 7-9 % (9.25 against
-// 9.94 us per layer at a 2048-token chunk over 28 distinct source sets), but
-// a forward pass hands the kernel rows its projection has just written, and
-// with sources that are still in cache the same launch is 10 % slower (8.77
-// against 7.95 us) and a 256-token decode launch is unchanged.
+// with both bits a launch whose Q/K/V come from HBM gains 1-2 % (9.35 against
+// 9.50 us per layer at a 2048-token chunk over 28 distinct source sets; 3.53
+// against 3.30 at 256 tokens over 32), but a forward pass hands the kernel rows
+// its projection has just written, and with sources that are still in cache the
+// chunk is 36 % slower (8.51 against 6.25 us) and the decode launch unchanged.
 struct RopeTuning {
   int threads = 0;
   int nt = 0;

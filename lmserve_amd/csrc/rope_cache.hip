@@ -434,19 +434,21 @@ void launch_element(const RopeArgs& a, dim3 grid, dim3 block, hipStream_t s) {
   else hipLaunchKernelGGL((rope_element_kernel<T, ADDR, false>), grid, block, 0, s, a);
 }
 
-template <typename T, Addressing ADDR>
+template <typename T, Addressing ADDR, int NTL>
 void launch_vector(const RopeArgs& a, bool tail, dim3 grid, dim3 block, hipStream_t s) {
   const bool fast = fast_index<ADDR>(a);
-  const auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, s, a); };
+  if (fast && !tail) hipLaunchKernelGGL((rope_vector_kernel<T, ADDR, true, false, NTL>), grid, block, 0, s, a);
+  else if (fast) hipLaunchKernelGGL((rope_vector_kernel<T, ADDR, true, true, NTL>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((rope_vector_kernel<T, ADDR, false, true, NTL>), grid, block, 0, s, a);
+}
+
+template <typename T, Addressing ADDR>
+void launch_vector(const RopeArgs& a, bool tail, dim3 grid, dim3 block, hipStream_t s) {
   switch (kvc::g_rope_tune.nt & 3) {
-    case 0:
-      if (fast && !tail) launch(rope_vector_kernel<T, ADDR, true, false, 0>);
-      else if (fast) launch(rope_vector_kernel<T, ADDR, true, true, 0>);
-      else launch(rope_vector_kernel<T, ADDR, false, true, 0>);
-      break;
-    case 1: launch(rope_vector_kernel<T, ADDR, false, true, 1>); break;
-    case 2: launch(rope_vector_kernel<T, ADDR, false, true, 2>); break;
-    default: launch(rope_vector_kernel<T, ADDR, false, true, 3>); break;
+    case 0: launch_vector<T, ADDR, 0>(a, tail, grid, block, s); break;
+    case 1: launch_vector<T, ADDR, 1>(a, tail, grid, block, s); break;
+    case 2: launch_vector<T, ADDR, 2>(a, tail, grid, block, s); break;
+    default: launch_vector<T, ADDR, 3>(a, tail, grid, block, s); break;
   }
 }
 

@@ -52,6 +52,7 @@ KVC_LAUNCH_PIPE = 6
 KVC_LAUNCH_SWAP_MODE = 7
 
 KVC_ABI_VERSION = 6
+FAST_INTERFACE = 2      # names and arguments of the `_kvc_fast` extension's functions
 KVC_NOALLOC_MAX_BLOCKS = 8192
 
 KVC_DTYPE_BF16 = 0
@@ -175,7 +176,10 @@ def lib() -> ctypes.CDLL:
             f"{LIB_PATH} has ABI version {handle.kvc_abi_version()}, this package needs "
             f"{KVC_ABI_VERSION}: rebuild it with `python -m lmserve_amd.build`")
     for name, (restype, argtypes) in SIGNATURES.items():
-        fn = getattr(handle, name)
+        fn = getattr(handle, name, None)
+        if fn is None:    # of the experimental surface, which the ABI version does not cover
+            raise KVCacheLibraryError(
+                f"{LIB_PATH} has no {name}, which this package needs: rebuild it with `python -m lmserve_amd.build`")
         fn.restype = restype
         fn.argtypes = argtypes
     _lib = handle
@@ -187,8 +191,8 @@ _fast = None
 
 def fast():
     """The `_kvc_fast` extension module (METH_FASTCALL wrappers of the per-layer
-    calls), or None when it is not built or `KVC_DISABLE_CALL_EXTENSION` is set in
-    the environment; callers then go through ctypes to the same entry points."""
+    calls), or None when it is not built, is of another interface, or
+    `KVC_DISABLE_CALL_EXTENSION` is set in the environment; callers then go through ctypes to the same entry points."""
     global _fast
     if _fast is None:
         lib()   # the shared library first: the extension binds to the same instance
@@ -197,7 +201,8 @@ def fast():
             return None
         try:
             from . import _kvc_fast
-            _fast = _kvc_fast if _kvc_fast.abi_version == KVC_ABI_VERSION else False
+            same = _kvc_fast.abi_version == KVC_ABI_VERSION and getattr(_kvc_fast, "interface", 1) == FAST_INTERFACE
+            _fast = _kvc_fast if same else False
         except ImportError:
             _fast = False
     return _fast or None

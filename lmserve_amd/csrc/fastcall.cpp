@@ -44,6 +44,7 @@
 namespace {
 
 constexpr long NOT_FAST = 1;
+constexpr long kInterface = 2;  // changes with the names or arguments of the functions below; _lib.py checks it
 
 bool as_ptr(PyObject* o, void** out) {
   if (o == Py_None) {
@@ -851,6 +852,7 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_kvc_fast",
 PyMODINIT_FUNC PyInit__kvc_fast(void) {
   PyObject* m = PyModule_Create(&module);
   if (m && (PyModule_AddIntConstant(m, "abi_version", KVC_ABI_VERSION) < 0 ||
+            PyModule_AddIntConstant(m, "interface", kInterface) < 0 ||
             PyModule_AddIntConstant(m, "NOT_FAST", NOT_FAST) < 0)) {
     Py_DECREF(m);
     return nullptr;

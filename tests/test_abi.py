@@ -400,7 +400,7 @@ def test_call_extension_is_built_and_binds_the_same_library():
         pytest.skip("switched off in the environment")
     mod = _lib.fast()
     assert mod is not None, "lmserve_amd/_kvc_fast.so is missing: run python -m lmserve_amd.build"
-    assert mod.abi_version == _lib.KVC_ABI_VERSION and mod.NOT_FAST == 1
+    assert mod.abi_version == _lib.KVC_ABI_VERSION and mod.NOT_FAST == 1 and mod.interface == _lib.FAST_INTERFACE
     for name in ("write_plan_append", "rotary_plan_run", "append_paged", "reshape_and_cache",
                  "rotary_pos_emb", "rotary_append_paged", "scalar_type_code"):
         assert callable(getattr(mod, name)), name
@@ -587,3 +587,35 @@ def test_calls_without_pinned_memory_take_the_unstaged_path(tmp_path):
             "                     h.kv_last_block_lens, h.slot_mapping, 16, 0, 0))\n")
     ran = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
     assert ran.stdout.split() == ["1", "1", "1"], ran.stdout + ran.stderr[-2000:]
+
+
+def test_an_older_build_is_refused_with_a_message_that_says_so(monkeypatch, tmp_path):
+    """A library of the same ABI version without the experimental entry points, and a call extension of another
+    interface beside the right library; the host's index arrays need neither."""
+    from types import SimpleNamespace
+
+    import lmserve_amd
+    from lmserve_amd.index_prep import InferInput, make_kv_index_inputs
+
+    gxx = shutil.which("g++")
+    if gxx is None:
+        pytest.skip("needs g++")
+    want = make_kv_index_inputs([InferInput(0, [], 2, 1, 3, [7])], 16).slot_mapping.tolist()
+    older = SimpleNamespace(abi_version=_lib.KVC_ABI_VERSION)
+    _lib.lib()
+    with monkeypatch.context() as m:
+        m.setattr(lmserve_amd, "_kvc_fast", older, raising=False)
+        m.setattr(_lib, "_fast", None)
+        m.setattr(_lib, "_fast_entries", {})
+        assert _lib.fast() is None and _lib.fast_entry("host_index") is None
+    src, so = tmp_path / "old.cpp", tmp_path / "libkvcache.so"
+    src.write_text(f'extern "C" int kvc_abi_version() {{ return {_lib.KVC_ABI_VERSION}; }}')
+    subprocess.run([gxx, "-shared", "-fPIC", str(src), "-o", str(so)], check=True)
+    with monkeypatch.context() as m:
+        m.setattr(_lib, "LIB_PATH", str(so))
+        m.setattr(_lib, "_lib", None)
+        m.setattr(_lib, "_fast", None)
+        m.setattr(_lib, "_fast_entries", {})
+        with pytest.raises(_lib.KVCacheLibraryError, match="rebuild it"):
+            _lib.lib()
+        assert make_kv_index_inputs([InferInput(0, [], 2, 1, 3, [7])], 16).slot_mapping.tolist() == want

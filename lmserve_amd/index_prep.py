@@ -146,7 +146,8 @@ def to_device(host: KVIndexInputs, page_size: int, device="cuda",
     from .paged import get_batch_indices_positions, get_seq_lens
 
     fast = _lib.fast_entry("upload_index")
-    if fast is not None and (dev := torch.device(device)).type == "cuda":
+    if fast is not None and (host.slot_mapping is not None or not with_slot_mapping) \
+            and (dev := torch.device(device)).type == "cuda":
         index = torch.cuda.current_device() if dev.index is None else dev.index
         got = fast(host.position_ids, host.cu_seqlens_q, host.kv_block_indices, host.kv_block_indptrs,
                    host.kv_last_block_lens, host.slot_mapping if with_slot_mapping else None, page_size, index,

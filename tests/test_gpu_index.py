@@ -261,6 +261,10 @@ def test_host_arrays_on_the_device_in_every_form(gpu, tokens, page):
             if t is not None:
                 assert t.is_contiguous() and t.device == gpu and np.array_equal(t.cpu().numpy(), want), name
     assert got[1].slot_mapping is None and got[3].slot_mapping is None
+    host.slot_mapping = None
+    assert kvc.to_device(host, page, gpu, False).slot_mapping is None
+    with pytest.raises(TypeError):                        # slots wanted, none there
+        kvc.to_device(host, page, gpu)
 
 
 # (a general path reads what an int subclass stores, by struct.pack: "ids converted" is the host arrays' own)

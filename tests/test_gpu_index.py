@@ -4,6 +4,7 @@ import pytest
 import torch
 
 import lmserve_amd as kvc
+from lmserve_amd import _lib
 from oracle import kvc_oracle as orc
 from tests.helpers import MAPPED_FORMS, mapped_requests
 
@@ -196,45 +197,89 @@ def test_one_launch_index_build_reports_an_allocation_that_fails(gpu):
     _check_build(wl.decode_step(wl.LLAMA_3_8B, num_blocks=256, batch=8, max_context=100, seed=1).inputs, gpu)
 
 
+def _long_work(gpu, x):
+    """About 0.2 s on the current stream; the event behind it."""
+    for _ in range(150):
+        x @ x
+    done = torch.cuda.Event()
+    done.record()
+    return done
+
+
 def test_index_builds_far_ahead_of_the_device_and_from_threads_that_end(gpu):
-    """More builds than staging buffers behind long work: each waits for a buffer without the interpreter's lock and
-    reads its own requests. Threads that end pass their buffers on, readers still queued included."""
+    """More builds than staging buffers behind long work: the fifth waits for a buffer without the interpreter's lock.
+    Of threads that end, the fifth comes round to a buffer whose reader, an ended thread's, is still queued. Every
+    build reads its own requests."""
     import threading
     import time
     import workloads as wl
     steps = [wl.decode_step(wl.LLAMA_3_8B, num_blocks=512, batch=8 + i, max_context=300, seed=i).inputs
              for i in range(12)]
     want = [kvc.to_device(kvc.make_kv_index_inputs(r, 16), 16, gpu) for r in steps]
+    x = torch.ones(4096, 4096, device=gpu)
+    _long_work(gpu, x)
     torch.cuda.synchronize()
-    ticks, stop, got = [0], threading.Event(), []
+    ticks, stop, got, waits = [0], threading.Event(), [], []
 
     def tick():
         while not stop.is_set():
             time.sleep(0.001)
             ticks[0] += 1
 
+    def build(requests):
+        t0 = time.perf_counter()
+        got.append(kvc.to_device_one_launch(requests, 16, gpu))
+        waits.append(time.perf_counter() - t0)
+
     ticker = threading.Thread(target=tick)
     ticker.start()
-    x = torch.ones(4096, 4096, device=gpu)
-    x @ x
+    try:
+        _long_work(gpu, x)
+        for r in steps[:4]:
+            build(r)
+        before = ticks[0]
+        build(steps[4])
+        ticked = ticks[0] - before
+        for r in steps[5:6]:
+            build(r)
+        torch.cuda.synchronize()
+        _long_work(gpu, x)
+        for r in steps[6:]:
+            worker = threading.Thread(target=build, args=(r,))
+            worker.start()
+            worker.join()
+    finally:
+        stop.set()
+        ticker.join()
     torch.cuda.synchronize()
-    before, t0 = ticks[0], time.perf_counter()
-    for _ in range(60):
-        y = x @ x                                            # about 0.1 s of queued work
-    for r in steps[:8]:
-        got.append(kvc.to_device_one_launch(r, 16, gpu))
-    waited, ticked = time.perf_counter() - t0, ticks[0] - before
-    for r in steps[8:]:
-        worker = threading.Thread(target=lambda: got.append(kvc.to_device_one_launch(r, 16, gpu)))
-        y = x @ x
-        worker.start()
-        worker.join()
-    stop.set()
-    ticker.join()
-    torch.cuda.synchronize()
-    assert ticked >= waited / 0.02 - 2
+    assert len(got) == len(steps)
+    assert waits[4] >= 0.05 and ticked >= waits[4] / 0.005, (waits, ticked)
+    assert waits[10] >= 0.05 and max(waits[6:10]) < waits[10], waits
     for g, w in zip(got, want):
         assert torch.equal(g.slot_mapping, w.slot_mapping) and torch.equal(g.kv_block_indices, w.kv_block_indices)
+
+
+def test_staging_grows_while_its_readers_are_queued(gpu):
+    """A step whose tables outgrow the buffers behind long work: the call waits for no buffer and for no device, and
+    the builds queued before it still read what they were given."""
+    def step(ids, start):
+        return [kvc.InferInput(0, [], 2, 16 * ids - 2, 16 * ids, list(range(start, start + ids)))]
+
+    small, large = [step(3000, k) for k in range(8)], [step(20000 << k, 7) for k in range(3)]
+    _lib.check(_lib.lib().kvc_thread_release())
+    for r in small[:4]:                                      # four buffers of 64 KiB
+        kvc.to_device_one_launch(r, 16, gpu)
+    x = torch.ones(4096, 4096, device=gpu)
+    torch.empty(1 << 22, device=gpu)                         # room for the outputs below in the allocator's cache
+    _long_work(gpu, x)
+    torch.cuda.synchronize()
+    done = _long_work(gpu, x)
+    got = [kvc.to_device_one_launch(r, 16, gpu) for r in small[4:] + large]
+    assert not done.query()
+    for g, r in zip(got, small[4:] + large):
+        ids = r[0].block_ids
+        assert torch.equal(g.kv_block_indices, torch.tensor(ids, dtype=torch.int32, device=gpu))
+        assert g.slot_mapping.tolist() == [16 * ids[-1] + 14, 16 * ids[-1] + 15]
 
 
 @pytest.mark.parametrize("tokens,page", [(1, 16), (3, 1), (1023, 16), (4099, 7)])

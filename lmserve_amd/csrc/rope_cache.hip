@@ -32,7 +32,7 @@ using kvc::fail;
 using kvc::log2_exact;
 
 constexpr int kThreads = 256;
-constexpr int kMaxRotaryDim = 512;  // cos + sin of one position in LDS as fp32: 4 KiB
+constexpr int kMaxRotaryDim = 512;  // at most 64 pair-vectors a head (fp32): what the division by pairs_magic relies on
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
@@ -161,8 +161,8 @@ __device__ __forceinline__ int64_t index_of(const void* array, int width, uint32
 // write skips the token. Uniform over the workgroup: scalar loads. FAST: int32
 // positions, int64 slots and a block size that is a power of two, as the index
 // build makes them; the other form handles either width and carries 64-bit
-// divisions (a decode launch of 256 tokens takes 2.65 us with the widths fixed, 2.73
-// with both words loaded side by side, 3.4 with the divisions as well).
+// divisions (a decode launch of 256 tokens, rows in cache, takes 2.65 us with the widths
+// fixed, 2.73 with both words loaded side by side, 3.4 with the divisions as well).
 template <Addressing ADDR, bool FAST>
 __device__ __forceinline__ int64_t slot_offset(const RopeArgs& a, uint32_t t, int64_t pos) {
   if constexpr (ADDR == kNoCache) return -1;
@@ -213,15 +213,15 @@ __device__ __forceinline__ void st16(char* p, u32x4 v) {
 //   - the lane's own four 16-byte pieces of the cos/sin row go straight to
 //     registers; staging the row in LDS as fp32 for all heads puts an LDS write, a
 //     barrier and 32 LDS words per lane on that chain. Two and four heads per lane
-//     share the pieces and lose more in wavefronts in flight (3.3 and 3.9 us where
-//     one head takes 2.8; 8.5 and 8.4 where it takes 7.7);
+//     share the pieces and lose more in wavefronts in flight (a fifth and two fifths
+//     more time at decode sizes, a tenth at 2048 tokens);
 //   - nothing waits for the position before the Q, K and V loads are issued;
-//   - an instantiation holds only the code its launch needs: with every addressing
-//     form, 64-bit divisions and the tails in one kernel a decode launch takes 3.9
-//     instead of 3.4 us.
-// Per launch, 8 launches to a graph, before (LDS, V on lanes of its own) and now:
-// 2 tokens x 40 heads x 64 3.37 -> 2.84 us, 256 x 40 x 128 4.03 -> 3.41, 2048 x 32 x
-// 128 8.87 -> 7.65 (4.9 TB/s), 8192 x 72 x 128 60.1 -> 56.8 (5.9 TB/s).
+//   - an instantiation holds only the code its launch needs: every addressing form,
+//     64-bit divisions and the tails in one kernel cost a decode launch 15 %.
+// Per launch of a recorded step of 28 to 32 layers, first form (LDS, V on lanes of its
+// own) and now, rows from cache and from memory: 256 tokens x 40 heads x 128 3.46 -> 2.69
+// and 4.03 -> 3.30 us, 2048 x 32 x 128 8.04 -> 6.25 and 9.97 -> 9.50 (4.1 TB/s);
+// 8192 x 72 x 128 60.1 -> 58.3 (5.75 TB/s).
 // TAIL: up to two pass-through vectors per lane, from V and from the heads'
 // unrotated lanes; without it at most one, from V.
 // NTL: non-temporal loads, bit 0 for the K and V rows, bit 1 for the Q rows.
@@ -344,10 +344,12 @@ __global__ __launch_bounds__(kThreads) void rope_vector_kernel(RopeArgs a) {
 
 // The same for several layers of one step, blockIdx.z the layer, their pointers in the
 // kernel arguments. A recorded step has every layer's buffers at hand before it begins;
-// as one node per layer it is bound by what a node costs, not by its bytes. A replay with
-// the index build, per layer -> one launch (us): 64 tokens x 32 heads x 128 x 28 layers
-// 66.6 -> 17.8 (the index build alone 17.4), 256 x 48 heads x 32 88.9 -> 27.1, 717 tokens
-// of those 139.5 -> 91.0, 3001 x 10 heads x 80 326 -> 198 (6.2 TB/s).
+// as one node per layer it is bound by what a node costs, not by its bytes. (A model loop
+// has a layer's projections only after the layer before it, and records a launch per
+// layer.) A replay with the index build, every layer's buffers its own, per layer -> one
+// launch (us): 64 tokens x 28 + 4 heads x 128 x 28 layers 66.5 -> 18.1 (the index build
+// alone 17.8), 256 x 32 + 8 heads x 32 109 -> 40, 717 tokens of those 199 -> 104, 3001 x
+// 8 + 1 heads x 80 490 -> 257 (5.15 TB/s).
 constexpr int kLayersPerLaunch = 64;  // 3.5 KiB of the 4 KiB a launch's arguments may take
 struct RopeLayersArgs {
   RopeArgs a;

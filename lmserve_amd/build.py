@@ -90,7 +90,8 @@ def build_fastcall(verbose: bool = False) -> str:
     return FAST_PATH
 
 
-HEADERS = [os.path.join(PKG_DIR, "csrc", "common.h"), os.path.join(PKG_DIR, "csrc", "staging.h"),
+HEADERS = [os.path.join(PKG_DIR, "csrc", "common.h"), os.path.join(PKG_DIR, "csrc", "device.h"),
+           os.path.join(PKG_DIR, "csrc", "staging.h"),
            os.path.join(INCLUDE, "kvcache.h"), os.path.join(INCLUDE, "kvcache_experimental.h")]
 
 

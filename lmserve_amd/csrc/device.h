@@ -1,0 +1,31 @@
+// Device-side helpers shared by the HIP sources of libkvcache.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+namespace kvc {
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// Store policies: the cache bits of the instruction. What a kernel leaves dirty in the L2s of the 8 XCDs is written
+// back when it ends; a store at device scope is written through to the last-level cache, where a reader on any
+// XCD finds it. The non-temporal forms are for rows that nothing reads soon.
+enum StorePolicy : int { kPlain = 0, kNonTemporal = 2, kThrough = 16, kThroughNt = 16 | 2 };
+
+// A run of bytes that one workgroup writes, `base` and `bytes` uniform over it. A store at or past `bytes` is dropped by
+// the hardware's own range check, so a lane past the end needs no branch. Through the compiler's buffer store and not in
+// inline asm: an instruction that overwrites the data of a 16-byte store too soon behind it corrupts the store, and
+// only for stores it knows does the compiler keep the two apart.
+struct OutRow {
+  __amdgpu_buffer_rsrc_t rsrc;
+  __device__ __forceinline__ OutRow(char* base, uint32_t bytes)
+      : rsrc(__builtin_amdgcn_make_buffer_rsrc(base, 0, (int)bytes, 0x00020000)) {}
+  template <StorePolicy POLICY>
+  __device__ __forceinline__ void store(uint32_t offset, u32x4 v) const {
+    __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, offset, 0, POLICY);
+  }
+};
+
+}  // namespace kvc

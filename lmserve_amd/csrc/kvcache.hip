@@ -43,6 +43,7 @@
 #include <vector>
 
 #include "common.h"
+#include "device.h"
 #include "staging.h"
 #include "kvcache.h"
 #include "kvcache_experimental.h"
@@ -183,7 +184,7 @@ thread_local int g_last_swap_mode = -1;  // the mode this thread's most recent s
 
 constexpr int kThreads = 256;
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+using kvc::u32x4;
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 template <int BYTES> struct VecOf;
@@ -463,6 +464,30 @@ struct InlineIds {
   __device__ __forceinline__ int64_t dst(int64_t i) const { return p.id[2 * i + 1]; }
 };
 
+// One chunk of a tile: the lane's UNROLL vectors, STEP bytes apart from byte `at` on. Loads are straight-line (an
+// offset past the tile's end is clamped to the last vector), and a chunk that lies in the tile `whole`, which is uniform over the
+// workgroup, is stored without a look at the lane's offsets: with a branch per lane and vector the compiler waits
+// for all memory operations at each of them.
+template <int UNROLL, int STEP, bool NT, typename V, typename OFF>
+__device__ __forceinline__ void load_chunk(V (&data)[UNROLL], const char* src, OFF at, OFF tile_bytes) {
+#pragma unroll
+  for (int j = 0; j < UNROLL; ++j) {
+    const OFF off = at + j * STEP, last = tile_bytes - (OFF)sizeof(V);
+    data[j] = ld<NT>(reinterpret_cast<const V*>(src + (off < last ? off : last)));
+  }
+}
+template <int UNROLL, int STEP, bool NT, typename V, typename OFF>
+__device__ __forceinline__ void store_chunk(const V (&data)[UNROLL], char* dst, OFF at, OFF tile_bytes, bool whole) {
+  if (whole) {
+#pragma unroll
+    for (int j = 0; j < UNROLL; ++j) st<NT>(reinterpret_cast<V*>(dst + at + j * STEP), data[j]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < UNROLL; ++j)
+      if (at + j * STEP < tile_bytes) st<NT>(reinterpret_cast<V*>(dst + at + j * STEP), data[j]);
+  }
+}
+
 template <int VEC, int UNROLL, bool NT, typename IDS>
 __device__ __forceinline__ void copy_tiles_chunks(const TileArgs& a, const IDS& ids) {
   using V = typename VecOf<VEC>::type;
@@ -500,17 +525,27 @@ __device__ __forceinline__ void copy_tiles_chunks(const TileArgs& a, const IDS& 
     const char* src = a.src_base + layer * a.src_layer_stride + sid * a.src_block_stride;
     char* dst = a.dst_base + layer * a.dst_layer_stride + did * a.dst_block_stride;
     if (src == dst) continue;
-    const int64_t base = chunk * kChunk + (int64_t)threadIdx.x * VEC;
-    V data[UNROLL];
+    if constexpr (UNROLL >= 8) {
+      // Such a launch is resident all at once, and lanes that store as fast as they can leave it a read phase and a
+      // write phase. The branches, and the waits that come with them, keep the lanes apart (us, so and straight:
+      // 16 blocks of 2 MiB 12.5 and 13.7, 24 18.2 and 21.5; 4 blocks, 4 vectors, 5.6 and 5.3).
+      const int64_t base = chunk * kChunk + (int64_t)threadIdx.x * VEC;
+      V data[UNROLL];
 #pragma unroll
-    for (int j = 0; j < UNROLL; ++j) {
-      const int64_t off = base + (int64_t)j * kThreads * VEC;
-      if (off < a.tile_bytes) data[j] = ld<NT>(reinterpret_cast<const V*>(src + off));
-    }
+      for (int j = 0; j < UNROLL; ++j) {
+        const int64_t off = base + (int64_t)j * kThreads * VEC;
+        if (off < a.tile_bytes) data[j] = ld<NT>(reinterpret_cast<const V*>(src + off));
+      }
 #pragma unroll
-    for (int j = 0; j < UNROLL; ++j) {
-      const int64_t off = base + (int64_t)j * kThreads * VEC;
-      if (off < a.tile_bytes) st<NT>(reinterpret_cast<V*>(dst + off), data[j]);
+      for (int j = 0; j < UNROLL; ++j) {
+        const int64_t off = base + (int64_t)j * kThreads * VEC;
+        if (off < a.tile_bytes) st<NT>(reinterpret_cast<V*>(dst + off), data[j]);
+      }
+    } else {
+      const int64_t base = chunk * kChunk, at = base + (int64_t)threadIdx.x * VEC;
+      V data[UNROLL];
+      load_chunk<UNROLL, kThreads * VEC, NT>(data, src, at, a.tile_bytes);
+      store_chunk<UNROLL, kThreads * VEC, NT>(data, dst, at, a.tile_bytes, base + kChunk <= a.tile_bytes);
     }
   }
 }
@@ -529,14 +564,16 @@ __global__ __launch_bounds__(kThreads) void copy_pairs_kernel(TileArgs a, PairLi
 // the addresses in flight costs. Workgroups are dealt round-robin to the 8 XCDs;
 // here each XCD walks a run of `xcd_run` neighbouring chunks (a few hundred KiB)
 // instead of every eighth chunk, and the launch keeps the region in flight small:
-// either one vector per lane in workgroups of 64 lanes, or two in workgroups of 256
-// of which a CU holds 5 instead of 8 (dynamic LDS that nothing uses). TB/s, copy of
-// 1024 blocks x 32 layers of 64 KiB in a pool of 4104 blocks / in one of 16384 / a
-// gather of 256 x 80 / a scatter of them:
-//   two vectors, no runs (what ran before; the gather one)   5.2  4.9  6.3  5.3
-//   two vectors, runs of 64 chunks                           5.45 5.6  -    5.7
-//   two vectors, runs, 5 workgroups per CU                   6.05 6.05 6.45 6.35
-//   one vector, 64 lanes, runs of 64 / of 256 chunks         6.1/6.2 6.2/6.2 6.6/6.7 6.4/6.25
+// either one vector per lane in workgroups of 64 lanes (a gather), or two in workgroups
+// of 256, the second asked for when the first has arrived, of which a CU holds 6
+// instead of 8 (dynamic LDS that nothing uses; a launch that fits the GPU at once goes
+// without). Both loads at once with 5 to a CU, non-temporal stores -> this, stores
+// through the L2 (us): copy of 300 blocks of 2 MiB 208 -> 202, of 2048 1419 -> 1400; gather
+// and scatter of 100 x 2 MiB 124.5 -> 119.5, of 600 829 -> 784, of 256 x 5 MiB 858 -> 830.
+// Up to 128 MiB a copy reads its sources with plain loads: blocks that are copied on write
+// have just been read, and of 200 x 12 layers of 18 KiB that the last-level cache holds a
+// copy takes 14.7 us instead of 18.6, of 20 x 80 of 8 KiB 5.2 instead of 6.2; where it does
+// not it is the same, and from there on non-temporal loads are 1 % faster.
 struct StreamArgs {
   const char* src_base;
   char* dst_base;
@@ -549,8 +586,11 @@ struct StreamArgs {
   int64_t num_src_blocks, num_dst_blocks;
 };
 
-template <int THREADS, int UNROLL, bool NTL, bool NTS, typename SRC, typename DST>
-__device__ __forceinline__ void stream_tile_chunk(const StreamArgs& a, const SRC& src_id, const DST& dst_id) {
+// What the workgroup copies: item, layer and chunk of a tile
+struct StreamPlace {
+  uint32_t i, layer, chunk;
+};
+__device__ __forceinline__ StreamPlace stream_place(const StreamArgs& a) {
   uint32_t w = blockIdx.x;
   const uint32_t span = 8 * a.xcd_run;
   const uint32_t in_span = w % span;
@@ -558,31 +598,32 @@ __device__ __forceinline__ void stream_tile_chunk(const StreamArgs& a, const SRC
   if (w - in_span + span <= a.total_chunks) w = w - in_span + (in_span & 7u) * a.xcd_run + (in_span >> 3);
   const uint32_t tile = w / a.chunks_per_tile;
   const uint32_t chunk = w - tile * a.chunks_per_tile;
-  uint32_t i, layer;
   if (a.layer_slowest) {
-    layer = tile / a.num_items;
-    i = tile - layer * a.num_items;
-  } else {
-    i = tile / a.num_layers;
-    layer = tile - i * a.num_layers;
+    const uint32_t layer = tile / a.num_items;
+    return {tile - layer * a.num_items, layer, chunk};
   }
+  const uint32_t i = tile / a.num_layers;
+  return {i, tile - i * a.num_layers, chunk};
+}
+
+template <int THREADS, int UNROLL, bool NTL, bool NTS, typename SRC, typename DST>
+__device__ __forceinline__ void stream_tile_chunk(const StreamArgs& a, const SRC& src_id, const DST& dst_id) {
+  const auto [i, layer, chunk] = stream_place(a);
   const int64_t sid = src_id(i), did = dst_id(i);
   if (sid < 0 || sid >= a.num_src_blocks || did < 0 || did >= a.num_dst_blocks) return;
   const char* src = a.src_base + layer * a.src_layer_stride + sid * a.src_block_stride;
   char* dst = a.dst_base + layer * a.dst_layer_stride + did * a.dst_block_stride;
   if (src == dst) return;
-  const uint32_t base = chunk * (THREADS * UNROLL * 16) + threadIdx.x * 16;
+  const uint32_t at = chunk * (THREADS * UNROLL * 16) + threadIdx.x * 16;
+  const kvc::OutRow out(dst, a.tile_bytes);
   u32x4 data[UNROLL];
 #pragma unroll
   for (int j = 0; j < UNROLL; ++j) {
-    const uint32_t off = base + j * (THREADS * 16);
-    if (off < a.tile_bytes) data[j] = ld<NTL>(reinterpret_cast<const u32x4*>(src + off));
+    if (j) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    data[j] = ld<NTL>(reinterpret_cast<const u32x4*>(src + min(at + j * (THREADS * 16), a.tile_bytes - 16)));
   }
 #pragma unroll
-  for (int j = 0; j < UNROLL; ++j) {
-    const uint32_t off = base + j * (THREADS * 16);
-    if (off < a.tile_bytes) st<NTS>(reinterpret_cast<u32x4*>(dst + off), data[j]);
-  }
+  for (int j = 0; j < UNROLL; ++j) out.store<NTS ? kvc::kThroughNt : kvc::kPlain>(at + j * (THREADS * 16), data[j]);
 }
 
 template <int THREADS, int UNROLL, bool NTL, bool NTS>
@@ -591,8 +632,9 @@ __global__ __launch_bounds__(THREADS) void stream_tiles_kernel(StreamArgs a) {
       a, [&](uint32_t i) { return a.src_ids ? a.src_ids[(int64_t)i * a.id_stride] : (int64_t)i; },
       [&](uint32_t i) { return a.dst_ids ? a.dst_ids[(int64_t)i * a.id_stride] : (int64_t)i; });
 }
+template <bool NTL>
 __global__ __launch_bounds__(kThreads) void stream_pairs_kernel(StreamArgs a, PairList p) {
-  stream_tile_chunk<kThreads, 2, true, true>(
+  stream_tile_chunk<kThreads, 2, NTL, true>(
       a, [&](uint32_t i) { return (int64_t)p.id[2 * i]; }, [&](uint32_t i) { return (int64_t)p.id[2 * i + 1]; });
 }
 
@@ -1460,8 +1502,7 @@ enum class TileSides { kPools, kGather, kScatter };
 // Lanes of one launch: HIP takes fewer than 2^32 along a dimension.
 constexpr int64_t kMaxLanes = 0xffffffffll;
 
-// Workgroup of the stream kernel. A gather streams best one vector per lane (6.6 against 6.45 TB/s), a copy and a
-// scatter no worse with two.
+// Workgroup of the stream kernel. A gather streams best one vector per lane (6.6 against 6.45 TB/s).
 struct StreamShape {
   int64_t threads, unroll;
   int64_t chunk() const { return threads * unroll * 16; }
@@ -1496,20 +1537,34 @@ int launch_stream(const TileArgs& t, TileSides sides, int64_t n, hipStream_t s, 
   // touches as many far-apart pages (8 KiB x 80 layers: 4000 blocks 5.05 -> 5.2 TB/s, 300 blocks 4.85 -> 5.3;
   // from 32 KiB on it makes no difference, and a dense side wants its own order: gather 6.2 -> 5.1).
   a.layer_slowest = sides == TileSides::kPools && t.tile_bytes < (32 << 10);
-  const bool dense_cached = n * (int64_t)a.num_layers * t.tile_bytes <= (int64_t(256) << 20);
-  const bool plain_load = sides == TileSides::kScatter && dense_cached;
-  const bool plain_store = gather && dense_cached;
+  const int64_t bytes = n * (int64_t)a.num_layers * t.tile_bytes, llc = int64_t(256) << 20;
+  const bool plain_load = (sides == TileSides::kScatter && bytes <= llc) || (sides == TileSides::kPools && bytes <= llc / 2);
+  const bool plain_store = gather && bytes <= llc;
   const dim3 grid(a.total_chunks), block(threads);
-  constexpr unsigned kFivePerCu = 160 * 1024 / 5;
-  if (pairs) hipLaunchKernelGGL(stream_pairs_kernel, grid, block, kFivePerCu, s, a, *pairs);
+  const unsigned six_per_cu = (int64_t)a.total_chunks > resident_workgroups() ? 160 * 1024 / 6 : 0;
+  if (pairs && plain_load) hipLaunchKernelGGL((stream_pairs_kernel<false>), grid, block, six_per_cu, s, a, *pairs);
+  else if (pairs) hipLaunchKernelGGL((stream_pairs_kernel<true>), grid, block, six_per_cu, s, a, *pairs);
   else if (gather && plain_store) hipLaunchKernelGGL((stream_tiles_kernel<64, 1, true, false>), grid, block, 0, s, a);
   else if (gather) hipLaunchKernelGGL((stream_tiles_kernel<64, 1, true, true>), grid, block, 0, s, a);
-  else if (plain_load) hipLaunchKernelGGL((stream_tiles_kernel<256, 2, false, true>), grid, block, kFivePerCu, s, a);
-  else hipLaunchKernelGGL((stream_tiles_kernel<256, 2, true, true>), grid, block, kFivePerCu, s, a);
+  else if (plain_load) hipLaunchKernelGGL((stream_tiles_kernel<256, 2, false, true>), grid, block, six_per_cu, s, a);
+  else hipLaunchKernelGGL((stream_tiles_kernel<256, 2, true, true>), grid, block, six_per_cu, s, a);
   g_last = LastLaunch{KVC_KERNEL_COPY_TILES, 16, (int64_t)unroll, (int64_t)threads, (int64_t)a.total_chunks,
-                      plain_load || plain_store ? 0 : 1};
+                      plain_store || (plain_load && sides == TileSides::kScatter) ? 0 : 1};
   KVC_HIP(hipGetLastError());
   return KVC_OK;
+}
+
+// Vectors per lane of a launch that 3/8 of the resident workgroups hold: the fewest that bring it there, of which a
+// tile fills the lanes of its workgroups to three quarters or needs only one. 0: it takes more than `most`.
+// A quarter, and tiles that fill their workgroups to any part (before -> now, us): 6 blocks x 32 tiles of 64 KiB 7.0 ->
+// 6.1 (8 vectors -> 4), 12 11.2 -> 9.9 (16 -> 8), 20 x 16 of 32 KiB 6.5 -> 5.8, 20 x 12 of 36 KiB 6.8 -> 5.4.
+int small_unroll(int64_t tiles, int64_t tile_bytes, int vec, int most, int64_t resident) {
+  for (int u = 1; u <= most; u *= 2) {
+    const int64_t chunk = (int64_t)kThreads * vec * u, per_tile = (tile_bytes + chunk - 1) / chunk;
+    if (tiles * per_tile <= resident * 3 / 8 && (per_tile == 1 || 4 * tile_bytes >= 3 * per_tile * chunk))
+      return u;
+  }
+  return 0;
 }
 
 template <int VEC>
@@ -1517,8 +1572,8 @@ int launch_tiles_vec(TileArgs a, int unroll, int max_wgs, hipStream_t s, bool nt
                      const PairList* pairs) {
   if (unroll <= 0) {
     // By size, from sweeps of copy_blocks (1 to 4096 pairs x 32 layers x 64 KiB):
-    // a launch that fits a quarter of the resident workgroups runs best as few,
-    // deep workgroups (the smallest depth that gets it there; up to a whole tile
+    // a launch that fits three eighths of the resident workgroups runs best as few,
+    // deep workgroups (small_unroll; up to a whole tile
     // per workgroup while that stays within half the resident set): 6-8 % faster
     // than 4 vectors per lane from 32 to 128 MiB (a gather: 12-15 % faster than
     // with 1). Larger launches go through the stream kernel; what it does not take
@@ -1530,9 +1585,7 @@ int launch_tiles_vec(TileArgs a, int unroll, int max_wgs, hipStream_t s, bool nt
       const int64_t c = (int64_t)kThreads * VEC * u;
       return n * (int64_t)a.num_layers * ((a.tile_bytes + c - 1) / c);
     };
-    unroll = 0;
-    for (int u = 1; u <= 16 && !unroll; u *= 2)
-      if (chunks(u) <= resident / 4) unroll = u;
+    unroll = small_unroll(n * (int64_t)a.num_layers, a.tile_bytes, VEC, 16, resident);
     if (!unroll && chunks(16) <= resident / 2) unroll = 16;
     if (!unroll) {
       // (a tile below one chunk would leave lanes of every workgroup without work)

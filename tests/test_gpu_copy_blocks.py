@@ -147,6 +147,34 @@ def test_every_launch_shape_the_size_rule_picks_matches_the_oracle(gpu, n):
     assert np.array_equal(bits_of(dpool), want)
 
 
+@pytest.mark.parametrize("tile_bytes,n,L,per_lane", [
+    (65536, 6, 32, 4),       # 768 workgroups of 16 KiB: three eighths of the resident ones
+    (65536, 7, 32, 8),       # more
+    (36864, 20, 12, 4),      # the last workgroup of a tile a quarter full: three quarters of all lanes
+    (34816, 20, 12, 16),     # less than that at 4 and at 8 vectors: a tile per workgroup
+    (4112, 30, 8, 2),        # one vector past a chunk
+    (4096, 96, 8, 1),
+])
+def test_depth_of_small_copies(gpu, tile_bytes, n, L, per_lane):
+    """Vectors per lane by launch size and by how far a tile fills its workgroups; copy, gather and scatter against
+    NumPy, at tiles that end inside a workgroup's chunk."""
+    nb = 2 * n + 3
+    pool = random_pool((L, nb, tile_bytes // 2), seed=n)
+    ids = np.random.default_rng(n).permutation(nb)
+    src, dst = ids[:n], ids[n:2 * n]
+    dpool = to_bf16(pool, gpu)
+    kvc.copy_blocks(dpool, {int(a): [int(b)] for a, b in zip(src, dst)})
+    assert _lib.last_launch()["per_lane"] == per_lane
+    pool[:, dst] = pool[:, src]
+    assert np.array_equal(bits_of(dpool), pool)
+    dense = kvc.gather_blocks(dpool, torch.from_numpy(dst.copy()).to(gpu))
+    assert _lib.last_launch()["per_lane"] == per_lane
+    assert np.array_equal(bits_of(dense), pool[:, dst].swapaxes(0, 1))
+    kvc.scatter_blocks(dpool, torch.from_numpy(ids[3:3 + n].copy()).to(gpu), dense)
+    pool[:, ids[3:3 + n]] = pool[:, dst].copy()
+    assert np.array_equal(bits_of(dpool), pool)
+
+
 @pytest.mark.parametrize("tile_bytes,n,L", [
     (8192, 400, 3),        # one chunk per tile
     (8208, 400, 3),        # a second chunk of one vector

@@ -638,6 +638,55 @@ __global__ __launch_bounds__(kThreads) void stream_pairs_kernel(StreamArgs a, Pa
       a, [&](uint32_t i) { return (int64_t)p.id[2 * i]; }, [&](uint32_t i) { return (int64_t)p.id[2 * i + 1]; });
 }
 
+// Copies of blocks that go to several destinations each (a fork of one sequence into
+// several): a chunk is read once and stored to each of up to FAN destinations. Bound as
+// the copies above; a list of pairs reads a source once per copy, whatever the caches
+// hold. Two and three copies of each source, as pairs -> this (us): 6 x 2 of 2 MiB 8.2 ->
+// 6.7, 12 x 3 28 -> 18.5, 64 x 2 93 -> 74, 600 x 3 1205 -> 870 (5.75 TB/s); 33 x 3 x 24
+// layers of 40 KiB 39 -> 26.6, 2000 x 2 x 80 of 8 KiB 775 -> 722. Large launches take one
+// vector per lane, 5 workgroups to a CU (two vectors 950 at 600 x 3, 6 to a CU 920) and
+// plain non-temporal stores (through the L2 872, and 772 at 2000 x 2).
+// The list holds FAN + 1 words an item, its source and its destinations (-1: none), so
+// that one scalar load brings an item's ids: with a table of offsets and a loop over the
+// destinations each id is a dependent load of its own (6 x 2 8.7).
+constexpr int kFanWords = 896;  // 3.5 KiB of the 4 KiB a launch's arguments may take
+struct FanList {
+  int32_t word[kFanWords];
+};
+
+template <int UNROLL, int FAN>
+__device__ __forceinline__ void fan_tile_chunk(const StreamArgs& a, const int32_t* list) {
+  const auto [i, layer, chunk] = stream_place(a);
+  int32_t id[FAN + 1];
+#pragma unroll
+  for (int d = 0; d <= FAN; ++d) id[d] = list[(FAN + 1) * i + d];
+  if (id[0] < 0 || id[0] >= a.num_src_blocks) return;
+  const char* src = a.src_base + layer * a.src_layer_stride + id[0] * a.src_block_stride;
+  char* dst_layer = a.dst_base + layer * a.dst_layer_stride;
+  const uint32_t at = chunk * (kThreads * UNROLL * 16) + threadIdx.x * 16;
+  u32x4 data[UNROLL];
+  load_chunk<UNROLL, kThreads * 16, true>(data, src, at, a.tile_bytes);
+#pragma unroll
+  for (int d = 1; d <= FAN; ++d) {
+    if (id[d] < 0 || id[d] >= a.num_dst_blocks) continue;
+    const kvc::OutRow out(dst_layer + id[d] * a.dst_block_stride, a.tile_bytes);
+#pragma unroll
+    for (int j = 0; j < UNROLL; ++j) {
+      if constexpr (UNROLL >= 8) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // paced, as in copy_tiles_chunks
+      out.store<kvc::kNonTemporal>(at + j * (kThreads * 16), data[j]);
+    }
+  }
+}
+
+template <int UNROLL, int FAN>
+__global__ __launch_bounds__(kThreads) void fan_tiles_kernel(StreamArgs a, const int32_t* list) {
+  fan_tile_chunk<UNROLL, FAN>(a, list);
+}
+template <int UNROLL, int FAN>
+__global__ __launch_bounds__(kThreads) void fan_inline_kernel(StreamArgs a, FanList list) {
+  fan_tile_chunk<UNROLL, FAN>(a, list.word);
+}
+
 // ---------------------------------------------------------------------------
 // write_runs_kernel
 // ---------------------------------------------------------------------------
@@ -1629,6 +1678,53 @@ int launch_tiles_vec(TileArgs a, int unroll, int max_wgs, hipStream_t s, bool nt
   return KVC_OK;
 }
 
+// Copies through the fan kernels: `list` in the launch's own arguments, or in device memory.
+template <int UNROLL>
+void launch_fan(const StreamArgs& a, int fan, const FanList* list, const int32_t* device_list, unsigned lds, hipStream_t s) {
+  const dim3 grid(a.total_chunks), block(kThreads);
+  if (list && fan == 3) hipLaunchKernelGGL((fan_inline_kernel<UNROLL, 3>), grid, block, lds, s, a, *list);
+  else if (list) hipLaunchKernelGGL((fan_inline_kernel<UNROLL, 7>), grid, block, lds, s, a, *list);
+  else if (fan == 3) hipLaunchKernelGGL((fan_tiles_kernel<UNROLL, 3>), grid, block, lds, s, a, device_list);
+  else hipLaunchKernelGGL((fan_tiles_kernel<UNROLL, 7>), grid, block, lds, s, a, device_list);
+}
+
+// Shape of a fan launch: vectors per lane as of a small copy, up to 8, while the workgroups are resident at once;
+// beyond, the large form (24 x 2 x 32 tiles of 64 KiB as 1536 workgroups of 8 vectors 27.0 us, as the large form 29.5;
+// 40 x 2 as 1280 of 16 47.2, as the large form 45). unroll 0: more chunks than a launch has.
+struct FanShape {
+  int unroll;
+  bool large;
+};
+FanShape fan_shape(int64_t items, int64_t layers, int64_t tile_bytes) {
+  const int64_t resident = resident_workgroups(), tiles = items * layers;
+  const auto per_tile = [&](int u) { return (tile_bytes + u * 4096 - 1) / (u * 4096); };
+  if (tiles > kMaxLanes / kThreads / per_tile(1)) return {0, false};
+  int unroll = small_unroll(tiles, tile_bytes, 16, 8, resident);
+  if (!unroll && tiles * per_tile(8) <= resident) unroll = 8;
+  const bool large = !unroll;
+  if (large) unroll = 1;
+  while (unroll > 1 && (int64_t)kThreads * 16 * (unroll / 2) >= tile_bytes) unroll /= 2;
+  return {unroll, large};
+}
+
+int launch_fan_copy(StreamArgs a, FanShape shape, int fan, const FanList* list, const int32_t* device_list, hipStream_t s) {
+  const uint32_t chunk = kThreads * 16 * shape.unroll;
+  a.chunks_per_tile = (a.tile_bytes + chunk - 1) / chunk;
+  a.total_chunks = a.num_items * a.num_layers * a.chunks_per_tile;
+  a.xcd_run = shape.large ? 64 : 1;
+  a.layer_slowest = shape.large && a.tile_bytes < (32 << 10);
+  const unsigned lds = shape.large ? 160 * 1024 / 5 : 0;
+  switch (shape.unroll) {
+    case 1: launch_fan<1>(a, fan, list, device_list, lds, s); break;
+    case 2: launch_fan<2>(a, fan, list, device_list, lds, s); break;
+    case 4: launch_fan<4>(a, fan, list, device_list, lds, s); break;
+    default: launch_fan<8>(a, fan, list, device_list, lds, s); break;
+  }
+  g_last = LastLaunch{KVC_KERNEL_COPY_TILES, 16, shape.unroll, kThreads, (int64_t)a.total_chunks, 1};
+  KVC_HIP(hipGetLastError());
+  return KVC_OK;
+}
+
 constexpr int kNotInline = 1;  // launch_tiles: nothing launched, the kernels that take `pairs` do not take this copy
 
 // vectors per lane: the gather_unroll knob for a gather, else copy_unroll; by size unless set
@@ -2606,12 +2702,102 @@ int kvc_copy_blocks(void* kv_caches, const int64_t* block_maps, int64_t num_pair
                          block_bytes, num_blocks, stream);
 }
 
+// A list in host memory to `to` on the device, in pieces, so that the staging ring stays at 1 MiB a buffer. Whole
+// 16-byte vectors are written.
+static int stage_list(const void* list, int64_t bytes, void* to, void* stream) {
+  constexpr int64_t kPiece = 65000 * 16;
+  for (int64_t done = 0; done < bytes; done += kPiece) {
+    const int64_t n = std::min(kPiece, bytes - done), whole = round_up(n, 16);
+    void* staged = nullptr;
+    int rc = kvc_staging_acquire(whole, &staged);
+    if (rc != KVC_OK) return rc;
+    memcpy(staged, (const char*)list + done, (size_t)n);
+    memset((char*)staged + n, 0, (size_t)(whole - n));
+    rc = kvc_staging_upload((char*)to + done, whole, stream);
+    if (rc != KVC_OK) return rc;
+  }
+  return KVC_OK;
+}
+
+// Pairs of one source that follow each other, as items for the fan kernels. kNotInline where no source has two pairs
+// in a row, or the copy is not for those kernels.
+static int run_fan_copy(char* pool, const int64_t* pairs, int64_t num_pairs, int64_t* scratch, int64_t num_layers,
+                        int64_t layer_stride_bytes, int64_t block_bytes, int64_t num_blocks, hipStream_t s) {
+  bool several = false;
+  for (int64_t i = 1; i < num_pairs && !several; ++i) several = pairs[2 * i] == pairs[2 * i - 2];
+  if (!several || num_blocks > INT32_MAX || num_pairs > (1 << 28) || num_layers > INT32_MAX ||
+      block_bytes > (int64_t(1) << 30) || !g_tune.copy_nt || g_tune.copy_unroll || g_tune.copy_order ||
+      g_tune.copy_max_wgs > 0 ||
+      common_vec({(uint64_t)(uintptr_t)pool, (uint64_t)layer_stride_bytes, (uint64_t)block_bytes}) != 16)
+    return kNotInline;
+  std::vector<int32_t> list;
+  // a pair with an id outside the pool, or onto itself, copies nothing
+  const auto copies = [&](int64_t i) {
+    const int64_t from = pairs[2 * i], to = pairs[2 * i + 1];
+    return from >= 0 && from < num_blocks && to >= 0 && to < num_blocks && from != to;
+  };
+  const auto fill = [&](int fan) {
+    list.clear();
+    int64_t last = -1;
+    int held = fan;
+    for (int64_t i = 0; i < num_pairs; ++i) {
+      if (!copies(i)) continue;
+      if (pairs[2 * i] != last || held == fan) {
+        list.resize(list.size() + fan + 1, -1);
+        list[list.size() - fan - 1] = (int32_t)(last = pairs[2 * i]);
+        held = 0;
+      }
+      list[list.size() - fan + held++] = (int32_t)pairs[2 * i + 1];
+    }
+    return (int64_t)list.size() / (fan + 1);
+  };
+  // Up to 3 destinations an item, or up to 7 where that leaves less than half as many items.
+  int fan = 3;
+  int64_t items;
+  try {
+    items = fill(3);
+    const int64_t with3 = items;
+    if (fill(7) * 2 < with3) fan = 7, items = (int64_t)list.size() / 8;
+    else fill(3);
+  } catch (const std::bad_alloc&) {
+    return kNotInline;
+  }
+  if (items == 0) return KVC_OK;
+  const FanShape shape = fan_shape(items, num_layers, block_bytes);
+  if (!shape.unroll) return kNotInline;
+  StreamArgs a{};
+  a.src_base = pool;
+  a.dst_base = pool;
+  a.tile_bytes = (uint32_t)block_bytes;
+  a.num_layers = (uint32_t)num_layers;
+  a.num_items = (uint32_t)items;
+  a.src_layer_stride = a.dst_layer_stride = layer_stride_bytes;
+  a.src_block_stride = a.dst_block_stride = block_bytes;
+  a.num_src_blocks = a.num_dst_blocks = num_blocks;
+  const int64_t words = (int64_t)list.size();
+  if (words <= kFanWords) {
+    FanList inline_list;
+    std::copy(list.begin(), list.end(), inline_list.word);
+    return launch_fan_copy(a, shape, fan, &inline_list, nullptr, s);
+  }
+  if (!scratch || (uintptr_t)scratch % 16) return kNotInline;  // the caller says what is wrong
+  // at most 16 bytes a pair, which scratch holds: an item of 4 words has a pair, and items of 8 are fewer than half
+  // as many as those of 4
+  const int rc = stage_list(list.data(), words * (int64_t)sizeof(int32_t), scratch, s);
+  return rc != KVC_OK ? rc : launch_fan_copy(a, shape, fan, nullptr, (const int32_t*)scratch, s);
+}
+
 int kvc_copy_blocks_host_pairs(void* kv_caches, const int64_t* pairs, int64_t num_pairs, int64_t* scratch,
                                int64_t num_layers, int64_t layer_stride_bytes, int64_t block_bytes,
                                int64_t num_blocks, void* stream) {
   const char* fn = "kvc_copy_blocks_host_pairs";
   if (num_pairs <= 0 || !pairs)
     return num_pairs == 0 ? KVC_OK : fail(KVC_ERR_INVALID_ARG, "%s: bad pair list", fn);
+  if (kv_caches && num_layers > 0 && block_bytes > 0 && num_blocks >= 0 && layer_stride_bytes >= block_bytes) {
+    const int rc = run_fan_copy((char*)kv_caches, pairs, num_pairs, scratch, num_layers, layer_stride_bytes, block_bytes,
+                                num_blocks, (hipStream_t)stream);
+    if (rc != kNotInline) return rc;
+  }
   if (num_pairs <= kInlinePairs) {
     PairList list;
     int64_t n = 0;
@@ -2632,16 +2818,8 @@ int kvc_copy_blocks_host_pairs(void* kv_caches, const int64_t* pairs, int64_t nu
   }
   if (!scratch) return fail(KVC_ERR_STAGING, "%s: this list needs %lld bytes of scratch", fn, (long long)(16 * num_pairs));
   if ((uintptr_t)scratch % 16) return fail(KVC_ERR_INVALID_ARG, "%s: misaligned scratch", fn);
-  constexpr int64_t kPiece = 65000;  // pairs staged at a time, so that the ring stays at 1 MiB a buffer
-  for (int64_t done = 0; done < num_pairs; done += kPiece) {
-    const int64_t n = std::min(kPiece, num_pairs - done);
-    void* staged = nullptr;
-    int rc = kvc_staging_acquire(16 * n, &staged);
-    if (rc != KVC_OK) return rc;
-    memcpy(staged, pairs + 2 * done, 16 * n);
-    rc = kvc_staging_upload(scratch + 2 * done, 16 * n, stream);
-    if (rc != KVC_OK) return rc;
-  }
+  const int rc = stage_list(pairs, 16 * num_pairs, scratch, stream);
+  if (rc != KVC_OK) return rc;
   return run_copy_blocks(fn, kv_caches, scratch, nullptr, num_pairs, num_layers, layer_stride_bytes, block_bytes,
                          num_blocks, stream);
 }

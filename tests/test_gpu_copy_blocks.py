@@ -264,6 +264,41 @@ def test_pairs_from_a_dict_reach_the_device_with_the_launch(gpu, block_elems, n,
         kvc.copy_blocks(dpool, {0: ["x"]})
 
 
+@pytest.mark.parametrize("tile_bytes,L,fans,per_lane", [
+    (65536, 2, (2, 1, 3), 1),              # items of up to 3 destinations, one short of full
+    (65536, 16, (3, 3, 2, 4, 1, 3), 4),    # a group of 4 is two items
+    (65536, 16, (7, 7, 7, 16, 14), 4),     # up to 7 an item; groups beyond
+    (65552, 30, (3,) * 12, 8),             # one vector past 64 KiB
+    (65552, 60, (3,) * 12, 1),             # 2160 workgroups of 8 vectors: the large form
+    (65536, 32, (2,) * 30, 8),             # 1920 workgroups: two per tile, paced
+    (36864, 12, (3,) * 20, 4),
+    (8192, 30, (3,) * 300, 1),             # longer than a launch's arguments: staged; the large form
+    (8208, 3, (1,) * 400 + (2,) * 30, 4),  # staged, most items of one destination
+])
+def test_copies_of_blocks_with_several_destinations(gpu, tile_bytes, L, fans, per_lane):
+    """One read for several destinations, with ids outside the pool and a pair onto itself among them; then the same
+    as a list of pairs on the device, which reads once per copy."""
+    n = sum(fans)
+    nb = n + len(fans) + 3
+    pool = random_pool((L, nb, tile_bytes // 2), seed=n)
+    ids = np.random.default_rng(n).permutation(nb).tolist()
+    d, at = {}, len(fans)
+    for src, fan in zip(ids, fans):
+        d[src] = ids[at:at + fan]
+        at += fan
+    dpool, dlist = to_bf16(pool, gpu), to_bf16(pool, gpu)
+    for src, dsts in d.items():
+        pool[:, dsts] = pool[:, src:src + 1]
+    d[ids[0]][1:1] = [nb, -1, 2**40]       # outside the pool
+    d[ids[1]] = [ids[1]] + d[ids[1]]       # onto itself
+    kvc.copy_blocks(dpool, d)
+    ran = _lib.last_launch()
+    assert ran["kernel"] == _lib.KVC_KERNEL_COPY_TILES and ran["per_lane"] == per_lane
+    assert np.array_equal(bits_of(dpool), pool)
+    kvc.copy_blocks(dlist, torch.tensor(kvc.flatten_block_maps(d), device=gpu))
+    assert np.array_equal(bits_of(dlist), pool)
+
+
 @pytest.mark.parametrize("block_bytes,n,per_lane,grid", [
     (1 << 20, 131071, 2, 131071 * 128),                # the largest that the stream kernel takes: 2^32 - 2^15 lanes
     (1 << 20, 131073, 2, (2**32 - 1) // 256),          # past it: chunks walked grid-stride

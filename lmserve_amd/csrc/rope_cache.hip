@@ -19,6 +19,7 @@
 #include <new>
 
 #include "common.h"
+#include "device.h"
 #include "kvcache.h"
 #include "kvcache_experimental.h"
 
@@ -30,11 +31,11 @@ namespace {
 
 using kvc::fail;
 using kvc::log2_exact;
+using kvc::OutRow;
+using kvc::u32x4;
 
 constexpr int kThreads = 256;
 constexpr int kMaxRotaryDim = 512;  // at most 64 pair-vectors a head (fp32): what the division by pairs_magic relies on
-
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // ---- storage types ---------------------------------------------------------
 struct BF16 {
@@ -82,6 +83,23 @@ struct Vec {
       oy[i] = T::store2(o[1][0], o[1][1]);
     }
   }
+  // one 16-byte vector of either half, `other` the same lanes of the other half: own cos -+ other sin, the minus by
+  // `flip` in the sign bits of the x half; contracted by hand, as the compiler contracts `rotate`: the same bits
+  static constexpr uint32_t kSign = 0x80008000u;
+  static __device__ __forceinline__ u32x4 rotate_one(u32x4 own, u32x4 other, u32x4 c, u32x4 s, uint32_t flip) {
+    u32x4 out;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float r[2];
+#pragma unroll
+      for (int w = 0; w < 2; ++w) {
+        const auto f = [&](uint32_t v) { return T::load((uint16_t)(w ? v >> 16 : v & 0xffffu)); };
+        r[w] = __builtin_fmaf(f(own[i]), f(c[i]), f(other[i]) * f(s[i] ^ flip));
+      }
+      out[i] = T::store2(r[0], r[1]);
+    }
+    return out;
+  }
   // one element
   typedef uint16_t Word;
   static __device__ __forceinline__ float wide(Word w) { return T::load(w); }
@@ -97,6 +115,15 @@ struct Vec<F32> {
       ox[i] = __float_as_uint(f(x) * f(cx) - f(y) * f(sx));
       oy[i] = __float_as_uint(f(y) * f(cy) + f(x) * f(sy));
     }
+  }
+  static constexpr uint32_t kSign = 0x80000000u;
+  static __device__ __forceinline__ u32x4 rotate_one(u32x4 own, u32x4 other, u32x4 c, u32x4 s, uint32_t flip) {
+    u32x4 out;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      out[i] = __float_as_uint(__builtin_fmaf(__uint_as_float(own[i]), __uint_as_float(c[i]),
+                                              __uint_as_float(other[i]) * __uint_as_float(s[i] ^ flip)));
+    return out;
   }
   typedef uint32_t Word;
   static __device__ __forceinline__ float wide(Word w) { return __uint_as_float(w); }
@@ -130,11 +157,12 @@ struct RopeArgs {
   int64_t cache_block_stride, cache_slot_stride;  // bytes
   int64_t num_cache_blocks;
   uint32_t groups_per_token;  // workgroups per token
-  // vector kernel
+  // vector kernels
   uint32_t lanes_per_token;   // lanes that have work
   uint32_t pairs_per_head;    // pair-vectors of one head
-  uint32_t pairs_magic;       // ceil(2^32 / pairs_per_head): lane / pairs_per_head = mulhi(lane, magic)
-  uint32_t pairs_one;         // all ones where pairs_per_head is 1 (magic is then 0)
+  uint32_t split;             // a lane's head is lane / split: pairs_per_head, or the vectors of a head (rows kernel)
+  uint32_t split_magic;       // ceil(2^32 / split): lane / split = mulhi(lane, magic); 0 where that is not exact
+  uint32_t head_step;         // rows kernel: heads between a lane's two
   uint32_t v_items;           // 16-byte vectors of the token's V row (0 without a cache)
 };
 
@@ -198,16 +226,15 @@ typedef u32x4 __attribute__((aligned(2))) u32x4_at_any_element;
 __device__ __forceinline__ u32x4 ld16_cos_sin(const char* p) {
   return *reinterpret_cast<const u32x4_at_any_element*>(p);
 }
-template <bool NT>
-__device__ __forceinline__ void st16(char* p, u32x4 v) {
-  if constexpr (NT) __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
-  else *reinterpret_cast<u32x4*>(p) = v;
+// lane / split, the magic uniform
+__device__ __forceinline__ uint32_t head_of_lane(const RopeArgs& a, uint32_t lane) {
+  return a.split_magic ? __umulhi(lane, a.split_magic) : lane / a.split;
 }
 
-// 16-byte path. A lane owns ONE pair-vector of one Q or K head and carries
-// pass-through vectors (V, then the lanes beyond rotary_dim) along, so a token is
-// as few wavefronts as its pair-vectors need (a V row of its own lanes costs
-// 8 heads x 128 a sixth wavefront, 4 heads a fifth). blockIdx = (group, token).
+// Whole heads rotated, halves of whole 64-byte pieces. A lane owns ONE pair-vector of one
+// Q or K head and carries a V vector along, so a token is as few wavefronts as its
+// pair-vectors need (a V row of its own lanes costs 8 heads x 128 a sixth wavefront, 4
+// heads a fifth). blockIdx = (group, token).
 // What bounds it: at decode sizes the chain launch -> position -> cos/sin row ->
 // store and the instructions on it; at prefill sizes HBM. Hence
 //   - the lane's own four 16-byte pieces of the cos/sin row go straight to
@@ -216,130 +243,162 @@ __device__ __forceinline__ void st16(char* p, u32x4 v) {
 //     share the pieces and lose more in wavefronts in flight (a fifth and two fifths
 //     more time at decode sizes, a tenth at 2048 tokens);
 //   - nothing waits for the position before the Q, K and V loads are issued;
-//   - an instantiation holds only the code its launch needs: every addressing form,
-//     64-bit divisions and the tails in one kernel cost a decode launch 15 %.
-// Per launch of a recorded step of 28 to 32 layers, first form (LDS, V on lanes of its
-// own) and now, rows from cache and from memory: 256 tokens x 40 heads x 128 3.46 -> 2.69
-// and 4.03 -> 3.30 us, 2048 x 32 x 128 8.04 -> 6.25 and 9.97 -> 9.50 (4.1 TB/s);
-// 8192 x 72 x 128 60.1 -> 58.3 (5.75 TB/s).
-// TAIL: up to two pass-through vectors per lane, from V and from the heads'
-// unrotated lanes; without it at most one, from V.
+//   - an instantiation holds only the code its launch needs: every addressing form
+//     and 64-bit divisions in one kernel cost a decode launch 15 %.
+// query_out is stored at device scope, the cache rows the same and non-temporal. What
+// plain stores leave dirty in the L2s is written back when the launch ends, and a reader,
+// mostly on another XCD, finds it in the last-level cache either way. Launch of a recorded
+// step alone, and with a copy of query_out behind it, plain and non-temporal stores -> these
+// (us): 256 tokens x 40 heads x 128 3.10 -> 2.80 and 5.55 -> 5.20; 1024 of those 5.87 ->
+// 5.38 and 9.57 -> 9.20; 2048 x 32 x 128 8.45 -> 7.74 and 13.72 -> 13.13; 2048 x 72 x 128
+// 17.15 -> 16.61 and 27.44 -> 26.79; 8192 of those 59.4 -> 58.1 (5.8 TB/s) and 124 -> 120.5.
+// Non-temporal query_out is faster still alone and costs its reader more (1024 tokens 5.21
+// and 10.07; 2048 x 72 14.24 and 30.02). Stores at device scope of pieces that are
+// no whole 64 bytes lose (2048 x 15 x 96 in bf16, halves of 96 bytes, 4.68 -> 5.16): such
+// heads, and outputs that start within 64 bytes, go to the rows kernel.
 // NTL: non-temporal loads, bit 0 for the K and V rows, bit 1 for the Q rows.
-// query_out by plain stores, whatever its size: non-temporal ones take a part of this launch into the kernel that
-// reads it, and more than that part. Launch alone, then launch + a copy of query_out, then launch + the maximum of
-// every head (us; plain -> non-temporal): 8 MiB of 32 heads x 128 5.7 -> 5.1, 9.4 -> 9.8, 13.6 -> 13.4; 14 MiB of 28
-// heads 8.3 -> 7.4, 13.5 -> 14.5, 19.6 -> 19.6; 32 MiB of 64 heads 17.8 -> 14.0, 27.2 -> 29.8, 39.8 -> 41.4; 64 MiB
-// 31.5 -> 29.8, 52.2 -> 54.0, 70.6 -> 75.5; 187 MiB 85.0 -> 81.5, 159 -> 164, 203 -> 211; 80 MiB of 32 heads x 80 with
-// 32 lanes rotated 66 -> 79, 100 -> 110, 217 -> 254.
-template <typename T, Addressing ADDR, bool FAST, bool TAIL, int NTL>
-__device__ __forceinline__ void rope_vector_lane(const RopeArgs& a, const RopeLayer p) {
-  using VT = Vec<T>;
+template <typename T, Addressing ADDR, int NTL>
+__device__ __forceinline__ void rope_pairs_lane(const RopeArgs& a, const RopeLayer p) {
   constexpr uint32_t E = T::kBytes;
+  const uint32_t t = blockIdx.y;
+  const uint32_t lane = blockIdx.x * blockDim.x + threadIdx.x;
+  if (lane >= a.lanes_per_token) return;
+  const int64_t pos = reinterpret_cast<const int32_t*>(a.positions)[t];
+
+  const uint32_t half = (a.rotary_dim >> 1) * E;  // bytes
+  const uint32_t h = head_of_lane(a, lane);
+  const uint32_t pv = (lane - h * a.split) * 16;
+  const bool is_k = h >= a.num_heads;
+  const uint32_t head_off = (is_k ? h - a.num_heads : h) * a.head_dim * E + pv;
+  u32x4 x, y;
+  if (NTL == 1 || NTL == 2) {
+    if (is_k) {
+      const char* in = p.key + (int64_t)t * a.k_token_stride + head_off;
+      x = ld16<(NTL & 1) != 0>(in);
+      y = ld16<(NTL & 1) != 0>(in + half);
+    } else {
+      const char* in = p.query + (int64_t)t * a.q_token_stride + head_off;
+      x = ld16<(NTL & 2) != 0>(in);
+      y = ld16<(NTL & 2) != 0>(in + half);
+    }
+  } else {
+    const char* in = (is_k ? p.key + (int64_t)t * a.k_token_stride : p.query + (int64_t)t * a.q_token_stride) + head_off;
+    x = ld16<NTL != 0>(in);
+    y = ld16<NTL != 0>(in + half);
+  }
+  const bool has_v = ADDR != kNoCache && lane < a.v_items;
+  u32x4 v = {};
+  if (has_v) v = ld16<(NTL & 1) != 0>(p.value + (int64_t)t * a.v_token_stride + lane * 16);
+
+  if (pos < 0 || pos >= a.max_position) return;  // no cos/sin row: the token is left alone
+  const char* row = a.cos_sin_cache + pos * (int64_t)(4 * half) + pv;
+  const u32x4 cos_x = ld16_cos_sin(row), cos_y = ld16_cos_sin(row + half), sin_x = ld16_cos_sin(row + 2 * half),
+              sin_y = ld16_cos_sin(row + 3 * half);
+  const int64_t slot = slot_offset<ADDR, true>(a, t, pos);
+
+  u32x4 ox, oy;
+  Vec<T>::rotate(x, y, cos_x, cos_y, sin_x, sin_y, ox, oy);
+  const uint32_t kv_bytes = a.num_kv_heads * a.head_dim * E;
+  if (!is_k) {
+    const OutRow out(p.query_out + (int64_t)t * a.qo_token_stride, a.num_heads * a.head_dim * E);
+    out.store<kvc::kThrough>(head_off, ox);
+    out.store<kvc::kThrough>(head_off + half, oy);
+  } else {
+    if (p.key_out) {
+      const OutRow out(p.key_out + (int64_t)t * a.ko_token_stride, kv_bytes);
+      out.store<kvc::kThrough>(head_off, ox);
+      out.store<kvc::kThrough>(head_off + half, oy);
+    }
+    if (ADDR != kNoCache && slot >= 0) {
+      const OutRow out(p.key_cache + slot, kv_bytes);
+      out.store<kvc::kThroughNt>(head_off, ox);
+      out.store<kvc::kThroughNt>(head_off + half, oy);
+    }
+  }
+  if (has_v && slot >= 0) OutRow(p.value_cache + slot, kv_bytes).store<kvc::kThroughNt>(lane * 16, v);
+}
+
+// Every other shape of aligned rows: heads rotated in part, halves that are no whole
+// 64-byte pieces, more V vectors than pair-vectors, other index types. A lane owns the same
+// 16-byte vector of two heads (Q, then K, then V heads), so the lanes write the rows out in
+// order, whole lines whatever the halves are; its other half's vector is a second load, from the
+// first-level cache. With the pair form, a lane's unrotated vectors carried along, a
+// partial rotation wrote pieces of 32 and 96 bytes. Launch of a recorded step alone, and
+// with a copy of query_out behind it, that form -> this (us): 838 tokens x 40 heads x 80, 32
+// rotated, 4.99 -> 3.99 and 8.00 -> 7.12; 8192 of those 33.7 -> 23.7 and 43.5 -> 35.0; 256 3.49 ->
+// 2.93; 2048 x 15 x 96 in bf16 4.65 -> 4.25 and 7.74 -> 7.28; 2048 x 40 x 128, 64 rotated, 9.6 -> 9.7
+// and 15.3 -> 15.9, 300 of those 3.80 -> 3.13, 8192 38.5 -> 35.9 and 61.2 -> 59.5. One head per lane
+// is 5 to 9 % slower at prefill sizes, three 2 to 7 %; the other half by shuffles is no
+// faster than by the load.
+template <typename T, Addressing ADDR, bool FAST, int NTL>
+__device__ __forceinline__ void rope_rows_lane(const RopeArgs& a, const RopeLayer p) {
+  constexpr uint32_t E = T::kBytes;
+  constexpr int HEADS = 2;
   const uint32_t t = blockIdx.y;
   const uint32_t lane = blockIdx.x * blockDim.x + threadIdx.x;
   if (lane >= a.lanes_per_token) return;
   const int64_t pos = FAST ? (int64_t) reinterpret_cast<const int32_t*>(a.positions)[t] : index_of(a.positions, a.pos_bytes, t);
 
-  const uint32_t half = (a.rotary_dim >> 1) * E;  // bytes
-  const uint32_t h = __umulhi(lane, a.pairs_magic) + (lane & a.pairs_one);
-  const uint32_t pv = (lane - h * a.pairs_per_head) * 16;
-  const uint32_t heads = a.num_heads + a.num_kv_heads;
-  const bool rotates = !TAIL || (a.pairs_per_head != 0 && h < heads);
-  const bool is_k = h >= a.num_heads;
-  const uint32_t head_off = (is_k ? h - a.num_heads : h) * a.head_dim * E + pv;
-  u32x4 x, y;
-  if (rotates) {
-    if (NTL == 1 || NTL == 2) {
-      if (is_k) {
-        const char* in = p.key + (int64_t)t * a.k_token_stride + head_off;
-        x = ld16<(NTL & 1) != 0>(in);
-        y = ld16<(NTL & 1) != 0>(in + half);
-      } else {
-        const char* in = p.query + (int64_t)t * a.q_token_stride + head_off;
-        x = ld16<(NTL & 2) != 0>(in);
-        y = ld16<(NTL & 2) != 0>(in + half);
-      }
-    } else {
-      const char* in = (is_k ? p.key + (int64_t)t * a.k_token_stride : p.query + (int64_t)t * a.q_token_stride) + head_off;
-      x = ld16<NTL != 0>(in);
-      y = ld16<NTL != 0>(in + half);
-    }
-  }
-  // pass-through vectors of this lane: V first, then the tails of the heads
-  constexpr int kExtra = TAIL ? 2 : (ADDR == kNoCache ? 0 : 1);
-  u32x4 ev[kExtra + 1];
-  uint32_t eoff[kExtra + 1];  // byte offset inside the row it comes from == inside the row it goes to
-  int ekind[kExtra + 1];      // 0 none, 1 V, 2 tail of a Q head, 3 tail of a K head
+  const uint32_t h0 = head_of_lane(a, lane), v = lane - h0 * a.split, head_bytes = a.head_dim * E;
+  const uint32_t hq = a.num_heads, hk = hq + a.num_kv_heads, heads = ADDR == kNoCache ? hk : hk + a.num_kv_heads;
+  const bool first = v < a.pairs_per_head, rotates = v < 2 * a.pairs_per_head;
+  const int32_t to_other = !rotates ? 0 : first ? (int32_t)a.pairs_per_head * 16 : -(int32_t)a.pairs_per_head * 16;
+  const char* q_row = p.query + (int64_t)t * a.q_token_stride;
+  const char* k_row = p.key + (int64_t)t * a.k_token_stride;
+  const char* v_row = ADDR == kNoCache ? nullptr : p.value + (int64_t)t * a.v_token_stride;
+  u32x4 own[HEADS], other[HEADS];
+  uint32_t off[HEADS];
 #pragma unroll
-  for (int j = 0; j < kExtra; ++j) {
-    const uint32_t e = lane + j * a.lanes_per_token;
-    ekind[j] = 0;
-    if (ADDR != kNoCache && e < a.v_items) {
-      ekind[j] = 1;
-      eoff[j] = e * 16;
-      ev[j] = ld16<(NTL & 1) != 0>(p.value + (int64_t)t * a.v_token_stride + eoff[j]);
-    } else if (TAIL) {
-      const uint32_t tail_per_head = (a.head_dim - a.rotary_dim) * E / 16;
-      if (e < a.v_items + heads * tail_per_head) {
-        const uint32_t i = e - a.v_items;
-        const uint32_t th = i / tail_per_head;
-        const bool tk = th >= a.num_heads;
-        ekind[j] = tk ? 3 : 2;
-        eoff[j] = ((tk ? th - a.num_heads : th) * a.head_dim + a.rotary_dim) * E + (i - th * tail_per_head) * 16;
-        ev[j] = tk ? ld16<(NTL & 1) != 0>(p.key + (int64_t)t * a.k_token_stride + eoff[j])
-                   : ld16<(NTL & 2) != 0>(p.query + (int64_t)t * a.q_token_stride + eoff[j]);
-      }
+  for (int j = 0; j < HEADS; ++j) {
+    const uint32_t h = min(h0 + j * a.head_step, heads - 1);  // a lane without a second head loads the last and stores none
+    const bool is_q = h < hq, is_v = h >= hk;
+    off[j] = (h - (is_q ? 0 : is_v ? hk : hq)) * head_bytes + v * 16;
+    const char* in = (is_q ? q_row : is_v ? v_row : k_row) + off[j];
+    if ((NTL == 1 || NTL == 2) && is_q != (NTL == 2)) {
+      own[j] = ld16<false>(in);
+      other[j] = ld16<false>(in + to_other);
+    } else {
+      own[j] = ld16<NTL != 0>(in);
+      other[j] = ld16<NTL != 0>(in + to_other);
     }
   }
 
   if (pos < 0 || pos >= a.max_position) return;  // no cos/sin row: the token is left alone
-  u32x4 cos_x, cos_y, sin_x, sin_y;
+  u32x4 c = {}, s = {};
   if (rotates) {
-    const char* row = a.cos_sin_cache + pos * (int64_t)(4 * half) + pv;
-    cos_x = ld16_cos_sin(row);
-    cos_y = ld16_cos_sin(row + half);
-    sin_x = ld16_cos_sin(row + 2 * half);
-    sin_y = ld16_cos_sin(row + 3 * half);
+    const char* row = a.cos_sin_cache + pos * (int64_t)(2 * a.rotary_dim * E) + v * 16;
+    c = ld16_cos_sin(row);
+    s = ld16_cos_sin(row + a.rotary_dim * E);
   }
   const int64_t slot = slot_offset<ADDR, FAST>(a, t, pos);
 
-  if (rotates) {
-    u32x4 ox, oy;
-    VT::rotate(x, y, cos_x, cos_y, sin_x, sin_y, ox, oy);
-    if (!is_k) {  // read again by attention right away
-      char* out = p.query_out + (int64_t)t * a.qo_token_stride + head_off;
-      st16<false>(out, ox);
-      st16<false>(out + half, oy);
-    } else {
-      if (p.key_out) {
-        char* out = p.key_out + (int64_t)t * a.ko_token_stride + head_off;
-        st16<false>(out, ox);
-        st16<false>(out + half, oy);
-      }
-      if (ADDR != kNoCache && slot >= 0) {  // the cache row is not read again by this step
-        char* out = p.key_cache + slot + head_off;
-        st16<true>(out, ox);
-        st16<true>(out + half, oy);
-      }
-    }
-  }
+  const uint32_t flip = first ? Vec<T>::kSign : 0u, kv_bytes = a.num_kv_heads * head_bytes;
 #pragma unroll
-  for (int j = 0; j < kExtra; ++j) {
-    if (ekind[j] == 1) {
-      if (slot >= 0) st16<true>(p.value_cache + slot + eoff[j], ev[j]);
-    } else if (TAIL && ekind[j] == 2) {
-      st16<false>(p.query_out + (int64_t)t * a.qo_token_stride + eoff[j], ev[j]);
-    } else if (TAIL && ekind[j] == 3) {
-      if (p.key_out) st16<false>(p.key_out + (int64_t)t * a.ko_token_stride + eoff[j], ev[j]);
-      if (ADDR != kNoCache && slot >= 0) st16<true>(p.key_cache + slot + eoff[j], ev[j]);
+  for (int j = 0; j < HEADS; ++j) {
+    const uint32_t h = h0 + j * a.head_step;
+    u32x4 out = own[j];
+    if (rotates && h < hk) out = Vec<T>::rotate_one(own[j], other[j], c, s, flip);
+    if (h < hq) {
+      OutRow(p.query_out + (int64_t)t * a.qo_token_stride, hq * head_bytes).store<kvc::kThrough>(off[j], out);
+    } else if (h < hk) {
+      if (p.key_out) OutRow(p.key_out + (int64_t)t * a.ko_token_stride, kv_bytes).store<kvc::kThrough>(off[j], out);
+      if (ADDR != kNoCache && slot >= 0) OutRow(p.key_cache + slot, kv_bytes).store<kvc::kThroughNt>(off[j], out);
+    } else if (h < heads && slot >= 0) {
+      OutRow(p.value_cache + slot, kv_bytes).store<kvc::kThroughNt>(off[j], out);
     }
   }
 }
 
-template <typename T, Addressing ADDR, bool FAST, bool TAIL, int NTL>
-__global__ __launch_bounds__(kThreads) void rope_vector_kernel(RopeArgs a) {
-  rope_vector_lane<T, ADDR, FAST, TAIL, NTL>(
-      a, RopeLayer{a.query, a.key, a.value, a.query_out, a.key_out, a.key_cache, a.value_cache});
+__device__ __forceinline__ RopeLayer only_layer(const RopeArgs& a) {
+  return RopeLayer{a.query, a.key, a.value, a.query_out, a.key_out, a.key_cache, a.value_cache};
+}
+template <typename T, Addressing ADDR, int NTL>
+__global__ __launch_bounds__(kThreads) void rope_pairs_kernel(RopeArgs a) {
+  rope_pairs_lane<T, ADDR, NTL>(a, only_layer(a));
+}
+template <typename T, Addressing ADDR, bool FAST, int NTL>
+__global__ __launch_bounds__(kThreads) void rope_rows_kernel(RopeArgs a) {
+  rope_rows_lane<T, ADDR, FAST, NTL>(a, only_layer(a));
 }
 
 // The same for several layers of one step, blockIdx.z the layer, their pointers in the
@@ -357,9 +416,10 @@ struct RopeLayersArgs {
 };
 static_assert(sizeof(RopeLayersArgs) <= 4096, "kernel arguments");
 
-template <typename T, bool TAIL>
+template <typename T, bool PAIRS>
 __global__ __launch_bounds__(kThreads) void rope_layers_kernel(RopeLayersArgs args) {
-  rope_vector_lane<T, kSlots, true, TAIL, 0>(args.a, args.layer[blockIdx.z]);
+  if constexpr (PAIRS) rope_pairs_lane<T, kSlots, 0>(args.a, args.layer[blockIdx.z]);
+  else rope_rows_lane<T, kSlots, true, 0>(args.a, args.layer[blockIdx.z]);
 }
 
 // Element path: rows that are no whole number of aligned 16-byte vectors. One
@@ -436,27 +496,29 @@ void launch_element(const RopeArgs& a, dim3 grid, dim3 block, hipStream_t s) {
   else hipLaunchKernelGGL((rope_element_kernel<T, ADDR, false>), grid, block, 0, s, a);
 }
 
+// The kernels of rows of aligned 16-byte vectors
+enum VectorForm { kElements, kPairs, kRows };
+
 template <typename T, Addressing ADDR, int NTL>
-void launch_vector(const RopeArgs& a, bool tail, dim3 grid, dim3 block, hipStream_t s) {
-  const bool fast = fast_index<ADDR>(a);
-  if (fast && !tail) hipLaunchKernelGGL((rope_vector_kernel<T, ADDR, true, false, NTL>), grid, block, 0, s, a);
-  else if (fast) hipLaunchKernelGGL((rope_vector_kernel<T, ADDR, true, true, NTL>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((rope_vector_kernel<T, ADDR, false, true, NTL>), grid, block, 0, s, a);
+void launch_vector(const RopeArgs& a, VectorForm form, dim3 grid, dim3 block, hipStream_t s) {
+  if (form == kPairs) hipLaunchKernelGGL((rope_pairs_kernel<T, ADDR, NTL>), grid, block, 0, s, a);
+  else if (fast_index<ADDR>(a)) hipLaunchKernelGGL((rope_rows_kernel<T, ADDR, true, NTL>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((rope_rows_kernel<T, ADDR, false, NTL>), grid, block, 0, s, a);
 }
 
 template <typename T, Addressing ADDR>
-void launch_vector(const RopeArgs& a, bool tail, dim3 grid, dim3 block, hipStream_t s) {
+void launch_vector(const RopeArgs& a, VectorForm form, dim3 grid, dim3 block, hipStream_t s) {
   switch (kvc::g_rope_tune.nt & 3) {
-    case 0: launch_vector<T, ADDR, 0>(a, tail, grid, block, s); break;
-    case 1: launch_vector<T, ADDR, 1>(a, tail, grid, block, s); break;
-    case 2: launch_vector<T, ADDR, 2>(a, tail, grid, block, s); break;
-    default: launch_vector<T, ADDR, 3>(a, tail, grid, block, s); break;
+    case 0: launch_vector<T, ADDR, 0>(a, form, grid, block, s); break;
+    case 1: launch_vector<T, ADDR, 1>(a, form, grid, block, s); break;
+    case 2: launch_vector<T, ADDR, 2>(a, form, grid, block, s); break;
+    default: launch_vector<T, ADDR, 3>(a, form, grid, block, s); break;
   }
 }
 
 template <typename T>
-int launch_rope(RopeArgs a, int64_t num_tokens, bool vector, bool tail, unsigned threads, hipStream_t s) {
-  if (!vector) {
+int launch_rope(RopeArgs a, int64_t num_tokens, VectorForm form, unsigned threads, hipStream_t s) {
+  if (form == kElements) {
     const dim3 grid((unsigned)(num_tokens * a.groups_per_token)), block(threads);
     if (!a.key_cache) launch_element<T, kNoCache>(a, grid, block, s);
     else if (a.batch_indices) launch_element<T, kPages>(a, grid, block, s);
@@ -468,9 +530,9 @@ int launch_rope(RopeArgs a, int64_t num_tokens, bool vector, bool tail, unsigned
   const int64_t slot_step = a.slot_bytes, pos_step = a.pos_bytes;
   for (int64_t t0 = 0; t0 < num_tokens; t0 += kMaxY) {
     const dim3 grid(a.groups_per_token, (unsigned)std::min(kMaxY, num_tokens - t0)), block(threads);
-    if (!a.key_cache) launch_vector<T, kNoCache>(a, tail, grid, block, s);
-    else if (a.batch_indices) launch_vector<T, kPages>(a, tail, grid, block, s);
-    else launch_vector<T, kSlots>(a, tail, grid, block, s);
+    if (!a.key_cache) launch_vector<T, kNoCache>(a, form, grid, block, s);
+    else if (a.batch_indices) launch_vector<T, kPages>(a, form, grid, block, s);
+    else launch_vector<T, kSlots>(a, form, grid, block, s);
     KVC_HIP(hipGetLastError());
     a.query += kMaxY * a.q_token_stride;
     a.key += kMaxY * a.k_token_stride;
@@ -486,7 +548,7 @@ int launch_rope(RopeArgs a, int64_t num_tokens, bool vector, bool tail, unsigned
 
 // Several layers of slot-mapped writes, as many to a launch as the arguments hold
 template <typename T>
-int launch_rope_layers(RopeArgs a, const RopeLayer* layers, int64_t num_layers, int64_t num_tokens, bool tail,
+int launch_rope_layers(RopeArgs a, const RopeLayer* layers, int64_t num_layers, int64_t num_tokens, VectorForm form,
                        unsigned threads, hipStream_t s) {
   RopeLayersArgs args{};
   for (int64_t l0 = 0; l0 < num_layers; l0 += kLayersPerLaunch) {
@@ -494,7 +556,7 @@ int launch_rope_layers(RopeArgs a, const RopeLayer* layers, int64_t num_layers, 
     args.a = a;
     std::copy(layers + l0, layers + l0 + n, args.layer);
     const dim3 grid(a.groups_per_token, (unsigned)num_tokens, (unsigned)n), block(threads);
-    if (tail) hipLaunchKernelGGL((rope_layers_kernel<T, true>), grid, block, 0, s, args);
+    if (form == kPairs) hipLaunchKernelGGL((rope_layers_kernel<T, true>), grid, block, 0, s, args);
     else hipLaunchKernelGGL((rope_layers_kernel<T, false>), grid, block, 0, s, args);
     KVC_HIP(hipGetLastError());
   }
@@ -599,9 +661,8 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
   a.qo_token_stride = g.qo_token_stride * E;
   a.ko_token_stride = g.ko_token_stride * E;
 
-  uint64_t align = (uintptr_t)query | (uintptr_t)key | (uintptr_t)query_out | (uintptr_t)key_out |
-                   (uint64_t)a.q_token_stride | (uint64_t)a.k_token_stride |
-                   (uint64_t)a.qo_token_stride | (uint64_t)a.ko_token_stride;
+  uint64_t in_align = (uintptr_t)query | (uintptr_t)key | (uint64_t)a.q_token_stride | (uint64_t)a.k_token_stride;
+  uint64_t out_align = (uintptr_t)query_out | (uintptr_t)key_out | (uint64_t)a.qo_token_stride | (uint64_t)a.ko_token_stride;
   if (c) {
     if (!value || !c->key_cache || !c->value_cache)
       return fail(KVC_ERR_INVALID_ARG, "%s: null value/cache pointer", fn);
@@ -634,36 +695,48 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
     a.cache_block_stride = c->cache_block_stride * E;
     a.cache_slot_stride = c->cache_slot_stride * E;
     a.num_cache_blocks = c->num_cache_blocks;
-    align |= (uintptr_t)value | (uintptr_t)c->key_cache | (uintptr_t)c->value_cache |
-             (uint64_t)a.v_token_stride | (uint64_t)a.cache_block_stride |
-             (uint64_t)a.cache_slot_stride;
+    in_align |= (uintptr_t)value | (uint64_t)a.v_token_stride;
+    out_align |= (uintptr_t)c->key_cache | (uintptr_t)c->value_cache | (uint64_t)a.cache_block_stride |
+                 (uint64_t)a.cache_slot_stride;
   }
   for (int64_t l = 0; l < num_layers; ++l) {
     const RopeLayer& p = layers[l];
-    align |= (uintptr_t)p.query | (uintptr_t)p.key | (uintptr_t)p.value | (uintptr_t)p.query_out |
-             (uintptr_t)p.key_out | (uintptr_t)p.key_cache | (uintptr_t)p.value_cache;
+    in_align |= (uintptr_t)p.query | (uintptr_t)p.key | (uintptr_t)p.value;
+    out_align |= (uintptr_t)p.query_out | (uintptr_t)p.key_out | (uintptr_t)p.key_cache | (uintptr_t)p.value_cache;
   }
   // 16-byte vectors need aligned rows and halves that hold whole vectors (and offsets inside a row that fit
   // 32 bits); the cos/sin table may start anywhere
   const int ev = 16 / E;
-  const bool vector = (align % 16 == 0) && (g.num_heads + g.num_kv_heads) * g.head_dim * E <= (int64_t(1) << 29) && ((g.rotary_dim / 2) % ev == 0) &&
-                      ((g.head_dim - g.rotary_dim) % ev == 0) && (g.head_dim % ev == 0);
   const int64_t heads = g.num_heads + g.num_kv_heads;
+  const bool vector = (in_align | out_align) % 16 == 0 && heads * g.head_dim * E <= (int64_t(1) << 29) &&
+                      (g.rotary_dim / 2) % ev == 0 && (g.head_dim - g.rotary_dim) % ev == 0 && g.head_dim % ev == 0;
+  VectorForm form = kElements;
   unsigned threads = (unsigned)kvc::g_rope_tune.threads;
   const bool fixed = threads == 64 || threads == 128 || threads == 192 || threads == 256;
-  bool tail = false;
   if (vector) {
-    const int64_t pairs = heads * ((g.rotary_dim / 2) / ev);
-    const int64_t v_items = c ? g.num_kv_heads * g.head_dim / ev : 0;
-    const int64_t extras = heads * ((g.head_dim - g.rotary_dim) / ev) + v_items;
-    const int64_t lanes = std::max(pairs, (extras + 1) / 2);  // at most two pass-through vectors per lane
-    tail = g.rotary_dim < g.head_dim || v_items > pairs;
+    const int64_t half = (g.rotary_dim / 2) * E, v_items = c ? g.num_kv_heads * g.head_dim / ev : 0;
+    const bool fast = !c ? fast_index<kNoCache>(a) : a.batch_indices ? fast_index<kPages>(a) : fast_index<kSlots>(a);
     a.v_items = (uint32_t)v_items;
-    a.lanes_per_token = (uint32_t)lanes;
     a.pairs_per_head = (uint32_t)((g.rotary_dim / 2) / ev);
-    // exact for every lane: lanes * pairs_per_head < 2^32 (lanes < 2^25, at most 64 pair-vectors per head)
-    a.pairs_magic = a.pairs_per_head > 1 ? (uint32_t)(((uint64_t(1) << 32) + a.pairs_per_head - 1) / a.pairs_per_head) : 0;
-    a.pairs_one = a.pairs_per_head == 1 ? ~0u : 0u;
+    // Halves of 64 bytes are whole pieces of half a line each; from 16 MiB of Q and K rows on, whole lines are worth
+    // more than the pair form's fewer lanes (pairs and rows, us: 32 + 8 heads x 64 in bf16, 1024 tokens 3.57 and 3.73,
+    // 4096 10.13 and 10.17, with a reader of query_out 16.08 and 15.84, 6000 13.3 and 13.3, 24.7 and 22.8, 8192 21.7
+    // and 20.0, 31.1 and 29.0)
+    const bool pairs = fast && g.rotary_dim == g.head_dim && v_items <= heads * a.pairs_per_head && half % 64 == 0 &&
+                       out_align % 64 == 0 && !(half == 64 && g.num_tokens * heads * g.head_dim * E >= (int64_t(16) << 20));
+    form = pairs ? kPairs : kRows;
+    if (pairs) {
+      a.split = a.pairs_per_head;
+      a.lanes_per_token = (uint32_t)(heads * a.pairs_per_head);
+    } else {
+      a.split = (uint32_t)(g.head_dim / ev);
+      a.head_step = (uint32_t)((heads + (c ? g.num_kv_heads : 0) + 1) / 2);
+      a.lanes_per_token = a.head_step * a.split;
+    }
+    const int64_t lanes = a.lanes_per_token;
+    // exact for every lane where lanes * split < 2^32 (pairs: lanes < 2^25, at most 64 pair-vectors per head)
+    a.split_magic = a.split > 1 && lanes * a.split < (int64_t(1) << 32)
+                        ? (uint32_t)(((uint64_t(1) << 32) + a.split - 1) / a.split) : 0;
     // The largest workgroup that cuts a token into an ODD number of workgroups. They are dealt round-robin to
     // the 8 XCDs; with an even number every second XCD gets only first halves (with the V vectors), the others
     // only the short last ones: 40 heads x 128 (5 wavefronts), 2048 tokens, as 3 x 128 lanes 9.5 us, as 5 x 64
@@ -689,19 +762,19 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
                 (long long)(g.num_tokens * (int64_t)a.groups_per_token));
   hipStream_t s = (hipStream_t)stream;
   if (layers) {
-    if (!vector || !c->slot_mapping || c->slot_bytes != 8 || pos_bytes != 4 || a.bs_shift < 0 ||
+    if (form == kElements || !c->slot_mapping || c->slot_bytes != 8 || pos_bytes != 4 || a.bs_shift < 0 ||
         (kvc::g_rope_tune.nt & 3) || g.num_tokens > 65535)
       return kLayerByLayer;
     switch (g.dtype) {
-      case KVC_DTYPE_BF16: return launch_rope_layers<BF16>(a, layers, num_layers, g.num_tokens, tail, threads, s);
-      case KVC_DTYPE_F16: return launch_rope_layers<F16>(a, layers, num_layers, g.num_tokens, tail, threads, s);
-      default: return launch_rope_layers<F32>(a, layers, num_layers, g.num_tokens, tail, threads, s);
+      case KVC_DTYPE_BF16: return launch_rope_layers<BF16>(a, layers, num_layers, g.num_tokens, form, threads, s);
+      case KVC_DTYPE_F16: return launch_rope_layers<F16>(a, layers, num_layers, g.num_tokens, form, threads, s);
+      default: return launch_rope_layers<F32>(a, layers, num_layers, g.num_tokens, form, threads, s);
     }
   }
   switch (g.dtype) {
-    case KVC_DTYPE_BF16: return launch_rope<BF16>(a, g.num_tokens, vector, tail, threads, s);
-    case KVC_DTYPE_F16: return launch_rope<F16>(a, g.num_tokens, vector, tail, threads, s);
-    default: return launch_rope<F32>(a, g.num_tokens, vector, tail, threads, s);
+    case KVC_DTYPE_BF16: return launch_rope<BF16>(a, g.num_tokens, form, threads, s);
+    case KVC_DTYPE_F16: return launch_rope<F16>(a, g.num_tokens, form, threads, s);
+    default: return launch_rope<F32>(a, g.num_tokens, form, threads, s);
   }
 }
 

@@ -513,6 +513,40 @@ def test_shapes_at_the_edges_of_the_vector_kernel(gpu, T, Hq, Hkv, D, rd, dtype,
     assert torch.equal(q_odd, q_out) and torch.equal(k_odd, k_out)
 
 
+@pytest.mark.parametrize("T,Hq,Hkv,D,dtype", [
+    (3, 1, 1, 64, torch.float32),          # three heads in all: a lane without a second one
+    (37, 5, 3, 128, torch.bfloat16),
+    (33, 6, 2, 256, torch.float16),        # 32 vectors a head
+    (3276, 32, 8, 64, torch.bfloat16),     # Q and K rows just short of 16 MiB,
+    (3277, 32, 8, 64, torch.bfloat16),     # and past it: 64-byte halves go to the rows kernel
+    (9, 2, 1, 4096, torch.bfloat16),       # heads of 512 vectors, 512 of 4096 lanes rotated
+])
+def test_both_forms_of_the_vector_kernel_give_the_same_bits(gpu, T, Hq, Hkv, D, dtype):
+    """The same call with outputs that start on a 64-byte boundary and 16 bytes past one, with int64 positions and
+    int32 slots, and layer by layer through a plan."""
+    bs, rd = 16, min(D, 512)
+    q, k, v, pos, cs = (t.to(gpu) for t in _case(gpu, T, Hq, Hkv, D, rd, dtype, seed=T + D))
+    nb = T // bs + 3
+    slots = torch.from_numpy(np.random.default_rng(T).permutation(nb * bs)[:T]).to(gpu)
+    slots[T // 2] = -1
+    pool = torch.zeros(nb, 2, bs, Hkv, D, dtype=dtype, device=gpu)
+    q_out, k_out = kvc.rotary_pos_emb_and_cache(q, k, v, pos, cs, D, pool, slots)
+    some = slice(0, T, max(1, T // 300))
+    for got, x, name in ((q_out, q, "query"), (k_out, k, "key")):
+        _check_rotation(got[some].cpu(), x[some].cpu(), pos[some].cpu(), cs.cpu(), D, dtype, name)
+    other = torch.zeros_like(pool)
+    q2, k2 = kvc.rotary_pos_emb_and_cache(q, k, v, pos.long(), cs, D, other, slots.int())
+    assert torch.equal(other, pool) and torch.equal(q2, q_out) and torch.equal(k2, k_out)
+    index = torch.zeros(T, dtype=torch.int32, device=gpu)
+    plan = kvc.PagedRotaryWritePlan(index, pos, index[:1], torch.tensor([0, 1], dtype=torch.int32, device=gpu), index[:1],
+                                    cs, Hq, Hkv, D, bs, slots=slots)
+    for shift in (0, 16 // q.element_size()):
+        shifted = torch.zeros(shift + q.numel(), dtype=dtype, device=gpu)[shift:].view(q.shape)
+        cache = torch.zeros(shift + pool.numel(), dtype=dtype, device=gpu)[shift:].view(pool.shape)
+        plan.run(q, k, v, cache, query_out=shifted)
+        assert torch.equal(cache, pool) and torch.equal(shifted, q_out)
+
+
 @pytest.mark.parametrize("T,Hq,Hkv,D,rd,dtype,bs,shift", [
     (1, 1, 1, 2, 2, torch.bfloat16, 16, 0),          # one pair a head
     (37, 5, 3, 36, 36, torch.float16, 12, 0),        # half heads that are no whole vectors

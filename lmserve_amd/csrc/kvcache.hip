@@ -205,6 +205,18 @@ __device__ __forceinline__ void st(V* p, V v) {
   else *p = v;
 }
 
+// One vector of a cache row; `through`: at device scope (kvc::st_through_nt), 16-byte vectors only.
+template <bool NT, typename V>
+__device__ __forceinline__ void st_row(char* p, V v, bool through) {
+  if constexpr (NT && sizeof(V) == 16) {
+    if (through) {
+      kvc::st_through_nt(p, v);
+      return;
+    }
+  }
+  st<NT>(reinterpret_cast<V*>(p), v);
+}
+
 // ---------------------------------------------------------------------------
 // write_rows_kernel
 // ---------------------------------------------------------------------------
@@ -233,6 +245,7 @@ struct WriteArgs {
   int pipe;                  // 1 = a lane waits for each of its loads before issuing the next one,
                              // so that the lanes of a launch that is resident all at once drift
                              // apart and reads overlap writes
+  int through;               // 1 = the rows are stored at device scope
   int64_t key_token_stride, value_token_stride;
   int64_t key_layer_stride, value_layer_stride;
   int64_t block_size;
@@ -244,6 +257,46 @@ struct WriteArgs {
   uint32_t tokens_per_wg;     // blockDim.x / vecs_per_row
   uint32_t num_token_groups;  // ceil(num_tokens / tokens_per_wg)
 };
+
+// Block and entry of token t's slot; false where the write skips the token. The page-table form is three steps of loads,
+// those of a step side by side and an index that is out of range read as 0 (the host launches nothing without
+// requests or pages): with a branch per check it was five, one load each. One layer, rows of 2 KiB (us): 256 tokens 2.80
+// -> 2.65, 838 3.65 -> 3.48, 2048 4.81 -> 4.56; 3000 of 256 bytes 3.1 -> 2.85.
+template <bool PAGED>
+__device__ __forceinline__ bool find_slot(const WriteArgs& a, uint32_t t, int64_t& blk, int64_t& off) {
+  bool ok;
+  int64_t page_index = 0;
+  if constexpr (PAGED) {
+    const int64_t b = a.batch_indices[t], p = a.positions[t];
+    ok = b >= 0 && b < a.batch_size && p >= 0;
+    const int64_t bc = ok ? b : 0, begin = a.kv_indptr[bc], end = a.kv_indptr[bc + 1];
+    int64_t pg;
+    if (a.bs_shift >= 0) {
+      pg = p >> a.bs_shift;
+      off = p & (a.block_size - 1);
+    } else {
+      pg = p / a.block_size;
+      off = p - pg * a.block_size;
+    }
+    // the page must lie inside this request's own table (and inside the array)
+    page_index = begin + pg;
+    ok = ok && page_index >= 0 && page_index < end && page_index < a.num_kv_indices;
+    blk = a.kv_indices[ok ? page_index : 0];
+  } else {
+    const int64_t s = (a.slot_bytes == 8)
+                          ? reinterpret_cast<const int64_t*>(a.slot_mapping)[t]
+                          : (int64_t) reinterpret_cast<const int32_t*>(a.slot_mapping)[t];
+    ok = s >= 0;
+    if (a.bs_shift >= 0) {
+      blk = s >> a.bs_shift;
+      off = s & (a.block_size - 1);
+    } else {
+      blk = s / a.block_size;
+      off = s - blk * a.block_size;
+    }
+  }
+  return ok && blk >= 0 && blk < a.num_cache_blocks;
+}
 
 // One workgroup = one token x a run of VPT*blockDim.x vectors out of the
 // token's 2*L rows (K and V of every layer). The token, hence its slot and
@@ -296,36 +349,7 @@ __global__ __launch_bounds__(kThreads) void write_rows_kernel(WriteArgs a) {
   }
 
   int64_t blk, off;
-  if constexpr (PAGED) {
-    const int64_t b = a.batch_indices[t];
-    const int64_t p = a.positions[t];
-    if (b < 0 || b >= a.batch_size || p < 0) return;
-    int64_t pg;
-    if (a.bs_shift >= 0) {
-      pg = p >> a.bs_shift;
-      off = p & (a.block_size - 1);
-    } else {
-      pg = p / a.block_size;
-      off = p - pg * a.block_size;
-    }
-    // the page must lie inside this request's own table (and inside the array)
-    const int64_t it = (int64_t)a.kv_indptr[b] + pg;
-    if (it < 0 || it >= (int64_t)a.kv_indptr[b + 1] || it >= a.num_kv_indices) return;
-    blk = a.kv_indices[it];
-  } else {
-    const int64_t s = (a.slot_bytes == 8)
-                          ? reinterpret_cast<const int64_t*>(a.slot_mapping)[t]
-                          : (int64_t) reinterpret_cast<const int32_t*>(a.slot_mapping)[t];
-    if (s < 0) return;
-    if (a.bs_shift >= 0) {
-      blk = s >> a.bs_shift;
-      off = s & (a.block_size - 1);
-    } else {
-      blk = s / a.block_size;
-      off = s - blk * a.block_size;
-    }
-  }
-  if (blk < 0 || blk >= a.num_cache_blocks) return;
+  if (!find_slot<PAGED>(a, t, blk, off)) return;
   const int64_t slot_off = blk * a.cache_block_stride + off * a.cache_slot_stride;
   char* kc_row = a.key_cache + slot_off;
   char* vc_row = a.value_cache + slot_off;
@@ -336,7 +360,7 @@ __global__ __launch_bounds__(kThreads) void write_rows_kernel(WriteArgs a) {
       uint32_t r, vec;
       split(item, r, vec);
       char* dst = ((r & 1u) ? vc_row : kc_row) + (int64_t)(r >> 1) * a.cache_layer_stride + (int64_t)vec * VEC;
-      st<NT>(reinterpret_cast<V*>(dst), data[j]);
+      st_row<NT>(dst, data[j], a.through != 0);
     }
   }
 }
@@ -383,35 +407,7 @@ __global__ __launch_bounds__(1024) void write_planes_kernel(WriteArgs a) {
     if (VPT > 1 && a.pipe == 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
   int64_t blk, off;
-  if constexpr (PAGED) {
-    const int64_t b = a.batch_indices[t];
-    const int64_t p = a.positions[t];
-    if (b < 0 || b >= a.batch_size || p < 0) return;
-    int64_t pgi;
-    if (a.bs_shift >= 0) {
-      pgi = p >> a.bs_shift;
-      off = p & (a.block_size - 1);
-    } else {
-      pgi = p / a.block_size;
-      off = p - pgi * a.block_size;
-    }
-    const int64_t it = (int64_t)a.kv_indptr[b] + pgi;
-    if (it < 0 || it >= (int64_t)a.kv_indptr[b + 1] || it >= a.num_kv_indices) return;
-    blk = a.kv_indices[it];
-  } else {
-    const int64_t s = (a.slot_bytes == 8)
-                          ? reinterpret_cast<const int64_t*>(a.slot_mapping)[t]
-                          : (int64_t) reinterpret_cast<const int32_t*>(a.slot_mapping)[t];
-    if (s < 0) return;
-    if (a.bs_shift >= 0) {
-      blk = s >> a.bs_shift;
-      off = s & (a.block_size - 1);
-    } else {
-      blk = s / a.block_size;
-      off = s - blk * a.block_size;
-    }
-  }
-  if (blk < 0 || blk >= a.num_cache_blocks) return;
+  if (!find_slot<PAGED>(a, t, blk, off)) return;
   const int64_t slot_off = blk * a.cache_block_stride + off * a.cache_slot_stride + vec_off;
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
@@ -419,7 +415,7 @@ __global__ __launch_bounds__(1024) void write_planes_kernel(WriteArgs a) {
     if (plane < a.num_planes) {
       char* dst = ((plane & 1u) ? a.value_cache : a.key_cache) + slot_off +
                   (int64_t)(plane >> 1) * a.cache_layer_stride;
-      st<NT>(reinterpret_cast<V*>(dst), data[j]);
+      st_row<NT>(dst, data[j], a.through != 0);
     }
   }
 }
@@ -1242,6 +1238,7 @@ int run_write(const char* fn, const void* key, const void* value, void* kc, void
       return fail(KVC_ERR_INVALID_ARG, "%s: null index array", fn);
     if (batch_size < 0 || num_kv_indices < 0)
       return fail(KVC_ERR_INVALID_ARG, "%s: negative batch_size/num_kv_indices", fn);
+    if (batch_size == 0 || num_kv_indices == 0) return KVC_OK;  // every token is skipped; find_slot counts on both
   } else {
     if (!slot_mapping) return fail(KVC_ERR_INVALID_ARG, "%s: null slot_mapping", fn);
     if (slot_bytes != 4 && slot_bytes != 8)
@@ -1281,6 +1278,11 @@ int run_write(const char* fn, const void* key, const void* value, void* kc, void
   if (items64 > 0x7fffffffll)
     return fail(KVC_ERR_UNSUPPORTED, "%s: %lld vectors per token exceed 2^31", fn, (long long)items64);
   a.items_per_token = (uint32_t)items64;
+  // Small launches store the rows at device scope, so that nothing is left to write back when they end; larger ones
+  // lose by it (one layer, rows of 2 KiB, us, non-temporal and through: 256 tokens by slot 2.55 and 2.36, by page
+  // table 2.65 and 2.57; 838 3.25 and 3.42, 3.48 and 3.23; 2048 4.5 and 5.2, 4.56 and 4.98; 256-byte rows, 3000 tokens
+  // 2.65 and 2.46)
+  a.through = g.num_tokens * items64 * vec <= (int64_t(2) << 20) << (paged ? 1 : 0);
 
   // The plane kernel (lanes over consecutive tokens of one (layer, K|V) plane)
   // takes rows of a power-of-two number of 16-byte vectors up to 4 KiB. The rule

@@ -196,13 +196,17 @@ __device__ __forceinline__ int64_t slot_offset(const RopeArgs& a, uint32_t t, in
   if constexpr (ADDR == kNoCache) return -1;
   int64_t blk = -1, off = 0;
   if constexpr (ADDR == kPages) {
+    // an index that is out of range is read as 0 (the host has looked that there are requests and pages): a branch
+    // per check makes each load wait for the one before
     const int64_t b = a.batch_indices[t];
-    if (b >= 0 && b < a.batch_size) {
-      const int64_t pg = FAST ? (pos >> a.bs_shift) : pos / a.block_size;
-      off = pos - (FAST ? pg << a.bs_shift : pg * a.block_size);
-      const int64_t it = (int64_t)a.kv_indptr[b] + pg;
-      if (it >= 0 && it < (int64_t)a.kv_indptr[b + 1] && it < a.num_kv_indices) blk = a.kv_indices[it];
-    }
+    const bool known = b >= 0 && b < a.batch_size;
+    const int64_t bc = known ? b : 0, begin = a.kv_indptr[bc], end = a.kv_indptr[bc + 1];
+    const int64_t pg = FAST ? (pos >> a.bs_shift) : pos / a.block_size;
+    off = pos - (FAST ? pg << a.bs_shift : pg * a.block_size);
+    const int64_t it = begin + pg;
+    const bool ok = known && it >= 0 && it < end && it < a.num_kv_indices;
+    const int64_t page = a.kv_indices[ok ? it : 0];
+    if (ok) blk = page;
   } else {
     const int64_t s = FAST ? reinterpret_cast<const int64_t*>(a.slot_mapping)[t] : index_of(a.slot_mapping, a.slot_bytes, t);
     if (s >= 0) {
@@ -698,6 +702,10 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
     in_align |= (uintptr_t)value | (uint64_t)a.v_token_stride;
     out_align |= (uintptr_t)c->key_cache | (uintptr_t)c->value_cache | (uint64_t)a.cache_block_stride |
                  (uint64_t)a.cache_slot_stride;
+    if (c->batch_indices && (c->batch_size == 0 || c->num_kv_indices == 0)) {  // the write skips every token
+      a.key_cache = nullptr;
+      c = nullptr;
+    }
   }
   for (int64_t l = 0; l < num_layers; ++l) {
     const RopeLayer& p = layers[l];

@@ -642,3 +642,55 @@ def test_corners_of_the_launch_rule(gpu, case, paged):
     assert _lib.lib().kvc_tuning_modified() == 0
     assert (ran["kernel"], ran["per_lane"], ran["threads"], ran["pipe"]) == (want_paged if paged else want_slot)
     assert np.array_equal(bits_of(dpool), want)
+
+
+@pytest.mark.parametrize("T", [512, 513, 1024, 1025])   # 2 MiB of written rows by slot, 4 by page table, and one token more
+@pytest.mark.parametrize("bad", [False, True])
+def test_rows_on_either_side_of_the_store_policy(gpu, T, bad):
+    """By page table and by slot, the whole pool against the oracle; with an index that is out of range at each step of
+    the page table's chain, those tokens are left out."""
+    H, D, bs = 8, 128, 16
+    nb = T // bs + 4
+    rng = np.random.default_rng(T)
+    key, value, pool = bf16_bits((T, H, D), 1), bf16_bits((T, H, D), 2), sentinel_pool((nb, 2, bs, H, D), 3)
+    split = T // 3                                       # two requests; one more page between their tables
+    pages = rng.permutation(nb)[:T // bs + 3].astype(np.int32)
+    first = (split + bs - 1) // bs
+    indptr = np.asarray([0, first, pages.size], dtype=np.int32)
+    owner = (np.arange(T) >= split).astype(np.int32)
+    pos = np.where(owner == 0, np.arange(T), np.arange(T) - split).astype(np.int32)
+    good = np.ones(T, dtype=bool)
+    if bad:
+        owner[[3, 9]] = -1, 2
+        pos[[20, 31, T - 1]] = -1, first * bs, 1 << 30   # before the table, in the next request's, past the array
+        good[[3, 9, 20, 31, T - 1]] = False
+        pages[0], pages[first] = nb, -1                  # pages outside the pool
+        good &= ~((owner == 0) & (pos < bs)) & ~((owner == 1) & (pos < bs))
+    want = pool.copy()
+    orc.append_paged_kv_cache_np(key[good], value[good], owner[good], pos[good], want, pages, indptr)
+    dev = lambda a: torch.from_numpy(a).to(gpu)
+    cache = to_bf16(pool, gpu)
+    last = torch.ones(2, dtype=torch.int32, device=gpu)
+    kvc.append_paged_kv_cache(to_bf16(key, gpu), to_bf16(value, gpu), dev(owner), dev(pos), cache, dev(pages), dev(indptr), last)
+    assert np.array_equal(bits_of(cache), want)
+    slots = np.full(T, -1, dtype=np.int64)
+    slots[good] = pages[indptr[owner[good]] + pos[good] // bs].astype(np.int64) * bs + pos[good] % bs
+    cache = to_bf16(pool, gpu)
+    kvc.reshape_and_cache(to_bf16(key, gpu), to_bf16(value, gpu), cache, dev(slots))
+    assert np.array_equal(bits_of(cache), want)
+
+
+def test_page_table_without_requests_writes_nothing(gpu):
+    H, D, bs, nb, T = 2, 64, 16, 4, 5
+    pool = sentinel_pool((nb, 2, bs, H, D), 3)
+    cache = to_bf16(pool, gpu)
+    rows = to_bf16(bf16_bits((T, H, D), 1), gpu)
+    i32 = lambda *v: torch.tensor(v, dtype=torch.int32, device=gpu)
+    index = torch.zeros(T, dtype=torch.int32, device=gpu)
+    cs = kvc.make_cos_sin_cache(D, 32, 10000.0, dtype=torch.bfloat16, device="cuda")
+    alone = kvc.rotary_pos_emb(rows.view(T, -1), rows.view(T, -1), index, cs, D)
+    kvc.append_paged_kv_cache(rows, rows, index, index, cache, i32(1), i32(0), i32())
+    got = kvc.rotary_pos_emb_and_append_paged(rows.view(T, -1), rows.view(T, -1), rows.view(T, -1), index, index, cs, D,
+                                              cache, i32(1), i32(0), i32())
+    assert torch.equal(got[0], alone[0]) and torch.equal(got[1], alone[1])
+    assert np.array_equal(bits_of(cache), pool)

@@ -99,18 +99,14 @@ struct Tuning {
   int write_pipe = -1;                   // 1 = a lane waits for each load before issuing its next,
                                          // 0 = loads back to back, -1 = by rule
   int write_planes_vpt = 0; // planes per lane in that kernel (1, 2, 4, 8), 0 = by size
-  int direct_max_wgs = 96;  // grid cap of the direct swap kernel: one direction of PCIe saturates
-                            // with 48-64 workgroups (more cost a 16 MiB one-layer launch 2-4 %),
-                            // both directions at once want 96 or more each (91-92 against 87 GB/s
-                            // in sum); the rest of the GPU stays free for the model
+  int direct_max_wgs = 96;  // grid cap of the direct swap kernel (GPU->Host in 16-byte vectors takes 16 at
+                            // most: kToHostWgs)
   int direct_max_wgs_in = 16;  // the same cap for Host->GPU (0 = direct_max_wgs). Reads over PCIe hold back
                                // the kernels of other streams in proportion to what is in flight: 16
                                // workgroups keep the link rate (57.1 against 57.3 GB/s) and let a forward
                                // pass that waits for each fetched layer through after 22.8 ms instead of
                                // 31.5 (13.8 alone, fetch alone 19.5); 8-12 are through after 22.1-22.3 but
-                               // lose the rate on large calls (36-52 GB/s). The price: beside a direct
-                               // swap-out the fetch gets less of the link (54 against 91 GB/s in sum).
-                               // Stores over PCIe hold others back whatever the cap (4 workgroups: +110 %)
+                               // lose the rate on large calls (36-52 GB/s)
   int runs_unroll = 0;       // write_runs: 16-byte vectors per lane (1, 2, 4), 0 = by size
   int runs_order = 1;        // write_runs: 1 = all runs of a plane are neighbours in the grid, 0 = all planes of a run
   int runs_nt = 1;           // write_runs: non-temporal loads and stores
@@ -484,7 +480,7 @@ __device__ __forceinline__ void store_chunk(const V (&data)[UNROLL], char* dst, 
   }
 }
 
-template <int VEC, int UNROLL, bool NT, typename IDS>
+template <int VEC, int UNROLL, bool NT, bool THROUGH, typename IDS>
 __device__ __forceinline__ void copy_tiles_chunks(const TileArgs& a, const IDS& ids) {
   using V = typename VecOf<VEC>::type;
   constexpr int64_t kChunk = (int64_t)kThreads * UNROLL * VEC;
@@ -541,18 +537,34 @@ __device__ __forceinline__ void copy_tiles_chunks(const TileArgs& a, const IDS& 
       const int64_t base = chunk * kChunk, at = base + (int64_t)threadIdx.x * VEC;
       V data[UNROLL];
       load_chunk<UNROLL, kThreads * VEC, NT>(data, src, at, a.tile_bytes);
-      store_chunk<UNROLL, kThreads * VEC, NT>(data, dst, at, a.tile_bytes, base + kChunk <= a.tile_bytes);
+      if constexpr (THROUGH) {
+        const kvc::OutRow out(dst, (uint32_t)a.tile_bytes);
+#pragma unroll
+        for (int j = 0; j < UNROLL; ++j) out.store<kvc::kThroughNt>((uint32_t)at + j * kThreads * VEC, data[j]);
+      } else {
+        store_chunk<UNROLL, kThreads * VEC, NT>(data, dst, at, a.tile_bytes, base + kChunk <= a.tile_bytes);
+      }
     }
   }
 }
 
 template <int VEC, int UNROLL, bool NT>
 __global__ __launch_bounds__(kThreads) void copy_tiles_kernel(TileArgs a) {
-  copy_tiles_chunks<VEC, UNROLL, NT>(a, ListIds{a});
+  copy_tiles_chunks<VEC, UNROLL, NT, false>(a, ListIds{a});
 }
 template <int UNROLL>
 __global__ __launch_bounds__(kThreads) void copy_pairs_kernel(TileArgs a, PairList p) {
-  copy_tiles_chunks<16, UNROLL, true>(a, InlineIds{p});
+  copy_tiles_chunks<16, UNROLL, true, false>(a, InlineIds{p});
+}
+// Pool -> mapped host pool. Plain and non-temporal stores to host memory gather dirty in the L2s, and their
+// write-back over the link holds up whatever else the XCD wants from its L2; stored through, 16 workgroups keep the
+// link full and the rest of the GPU goes on. 96 workgroups of non-temporal stores -> this, 192 MiB of scattered blocks:
+// 54.6 -> 56.2 GB/s, 83 instead of 60 in sum beside a direct swap-in, one layer of 96 blocks 130 -> 118 us; a bf16
+// product of 4096^3 beside it 226 -> 154 us (106-116 alone), one of 3000 rows 191 -> 100 (87 alone, 98 beside the
+// copy engines); a forward pass of 13.4 ms with 1 GiB leaving layer by layer beside it 32.0 -> 21.1 ms. 32 and 96 workgroups stored through: 3000 rows 157 and 189, both directions 68 and 63 GB/s.
+constexpr int kToHostWgs = 16;
+__global__ __launch_bounds__(kThreads) void copy_to_host_kernel(TileArgs a) {
+  copy_tiles_chunks<16, 2, true, true>(a, ListIds{a});
 }
 
 // Large copies: one chunk of one tile per workgroup, 16-byte vectors, the order of
@@ -1547,8 +1559,9 @@ void launch_tiles_nt(const TileArgs& a, unsigned grid, hipStream_t s, bool nt) {
   else hipLaunchKernelGGL((copy_tiles_kernel<VEC, UNROLL, false>), dim3(grid), dim3(kThreads), 0, s, a);
 }
 
-// What a launch copies between: blocks of a pool, or a dense buffer on one side.
-enum class TileSides { kPools, kGather, kScatter };
+// What a launch copies between: blocks of a pool, or a dense buffer on one side; kToHost: blocks of the mapped host pool
+// are written.
+enum class TileSides { kPools, kGather, kScatter, kToHost };
 
 // Lanes of one launch: HIP takes fewer than 2^32 along a dimension.
 constexpr int64_t kMaxLanes = 0xffffffffll;
@@ -1621,7 +1634,12 @@ int small_unroll(int64_t tiles, int64_t tile_bytes, int vec, int most, int64_t r
 template <int VEC>
 int launch_tiles_vec(TileArgs a, int unroll, int max_wgs, hipStream_t s, bool nt, int64_t n, TileSides sides,
                      const PairList* pairs) {
-  if (unroll <= 0) {
+  const bool to_host = VEC == 16 && sides == TileSides::kToHost && unroll <= 0 && nt && a.tile_bytes > kThreads * 16 &&
+                       a.tile_bytes <= (int64_t(1) << 30);
+  if (to_host) {
+    unroll = 2;
+    max_wgs = max_wgs > 0 ? std::min(max_wgs, kToHostWgs) : kToHostWgs;
+  } else if (unroll <= 0) {
     // By size, from sweeps of copy_blocks (1 to 4096 pairs x 32 layers x 64 KiB):
     // a launch that fits three eighths of the resident workgroups runs best as few,
     // deep workgroups (small_unroll; up to a whole tile
@@ -1668,6 +1686,8 @@ int launch_tiles_vec(TileArgs a, int unroll, int max_wgs, hipStream_t s, bool nt
       case 8: hipLaunchKernelGGL((copy_pairs_kernel<8>), g, b, 0, s, a, *pairs); break;
       default: hipLaunchKernelGGL((copy_pairs_kernel<16>), g, b, 0, s, a, *pairs); break;
     }
+  } else if (to_host && unroll == 2) {
+    hipLaunchKernelGGL(copy_to_host_kernel, dim3((unsigned)grid), dim3(kThreads), 0, s, a);
   } else switch (unroll) {
     case 1: launch_tiles_nt<VEC, 1>(a, (unsigned)grid, s, nt); break;
     case 2: launch_tiles_nt<VEC, 2>(a, (unsigned)grid, s, nt); break;
@@ -2083,7 +2103,7 @@ int run_swap(const char* fn, bool out, char* pool, char* host_pool, const int64_
   if (mode == KVC_SWAP_DIRECT && prepared) {
     // nothing but the launch: no events, no upload
     const TileArgs t = direct_swap_tiles(out, pool, host_pool, d_gpu_ids, d_host_ids, g);
-    return launch_tiles(t, g.n, direct_wgs(out), ks);
+    return launch_tiles(t, g.n, direct_wgs(out), ks, out ? TileSides::kToHost : TileSides::kPools);
   }
   rc = swap_ctx_prepare();
   if (rc != KVC_OK) return rc;
@@ -2099,7 +2119,7 @@ int run_swap(const char* fn, bool out, char* pool, char* host_pool, const int64_
   if (mode == KVC_SWAP_DIRECT) {
     // pool <-> mapped host pool in a single kernel
     const TileArgs t = direct_swap_tiles(out, pool, host_pool, d_gpu_ids, d_host_ids, g);
-    return launch_tiles(t, g.n, direct_wgs(out), ks);
+    return launch_tiles(t, g.n, direct_wgs(out), ks, out ? TileSides::kToHost : TileSides::kPools);
   }
 
   TileArgs t{};
@@ -3039,7 +3059,7 @@ int kvc_swap_noalloc(int to_host, void* pool, void* host_pool, const int64_t* gp
   const SwapGeom g{n, num_layers, layer_stride_bytes, block_bytes, num_gpu_blocks, num_host_blocks,
                    layer_begin, layer_end};
   const TileArgs t = direct_swap_tiles(to_host != 0, (char*)pool, (char*)host_pool, ids, ids + n, g);
-  return launch_tiles(t, n, direct_wgs(to_host != 0), s);
+  return launch_tiles(t, n, direct_wgs(to_host != 0), s, to_host ? TileSides::kToHost : TileSides::kPools);
 }
 
 void* kvc_host_alloc_pinned(size_t bytes) {

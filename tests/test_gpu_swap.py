@@ -94,6 +94,30 @@ def test_direct_swap_under_every_grid_cap(gpu, cap_out, cap_in):
         w.close()
 
 
+@pytest.mark.parametrize("block_shape,n,per_lane,grid", [
+    ((2, 16, 8, 128), 29, 2, 16),      # 64 KiB tiles: as many workgroups as the link needs
+    ((2, 16, 1, 128), 2, 2, 6),        # 8 KiB tiles, three layers: a workgroup each
+    ((2, 16, 3, 44), 29, 2, 16),       # 8448 bytes: a tile ends inside its second chunk
+    ((2, 16, 1, 64), 29, 1, 87),       # one chunk of 4 KiB: the general form
+    ((2, 16, 1, 65), 29, None, None),  # rows of 2-byte vectors
+])
+def test_direct_swap_out_stored_through(gpu, block_shape, n, per_lane, grid):
+    L, nb, nhb = 3, 48, 40
+    pool, dpool, w = _worker(gpu, L, nb, block_shape, nhb, "direct", 0, seed=33)
+    try:
+        rng = np.random.default_rng(34)
+        src, dst = rng.permutation(nb)[:n].astype(np.int64), rng.permutation(nhb)[:n].astype(np.int64)
+        want = w.host_kv_caches.copy()
+        orc.c_save_blocks_to_host(pool.reshape(L, nb, -1), want, src, dst)
+        w.copy_kv_sync(_mappings(src, dst), kvc.Device.GPU, kvc.Device.Host)
+        ran = _lib.last_launch()
+        if per_lane:
+            assert (ran["per_lane"], ran["grid"]) == (per_lane, grid)
+        assert np.array_equal(w.host_kv_caches, want)
+    finally:
+        w.close()
+
+
 @pytest.mark.parametrize("mode", MODES)
 def test_swap_layer_ranges_compose_to_the_full_swap(gpu, mode):
     """One call per layer range (the reference's layer-pipelined protocol) equals

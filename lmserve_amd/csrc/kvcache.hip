@@ -1155,10 +1155,10 @@ struct WriteLaunch {
 template <int VEC, int VPT, bool PAGED>
 void launch_write_nt(const WriteArgs& a, const WriteLaunch& l, hipStream_t s) {
   const dim3 grid(l.grid), block(l.threads);
-  if (l.nt && l.ntl) hipLaunchKernelGGL((write_rows_kernel<VEC, VPT, PAGED, true, true>), grid, block, 0, s, a);
-  else if (l.nt) hipLaunchKernelGGL((write_rows_kernel<VEC, VPT, PAGED, true, false>), grid, block, 0, s, a);
-  else if (l.ntl) hipLaunchKernelGGL((write_rows_kernel<VEC, VPT, PAGED, false, true>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((write_rows_kernel<VEC, VPT, PAGED, false, false>), grid, block, 0, s, a);
+  if (l.nt && l.ntl) kvc::launch((write_rows_kernel<VEC, VPT, PAGED, true, true>), grid, block, 0, s, a);
+  else if (l.nt) kvc::launch((write_rows_kernel<VEC, VPT, PAGED, true, false>), grid, block, 0, s, a);
+  else if (l.ntl) kvc::launch((write_rows_kernel<VEC, VPT, PAGED, false, true>), grid, block, 0, s, a);
+  else kvc::launch((write_rows_kernel<VEC, VPT, PAGED, false, false>), grid, block, 0, s, a);
 }
 
 template <int VEC, bool PAGED>
@@ -1185,10 +1185,10 @@ void launch_write(const WriteArgs& a, int vec, const WriteLaunch& l, hipStream_t
 template <int VPT, bool PAGED>
 void launch_planes_nt(const WriteArgs& a, const WriteLaunch& l, hipStream_t s) {
   const dim3 grid(l.grid), block(l.threads);
-  if (l.nt && l.ntl) hipLaunchKernelGGL((write_planes_kernel<VPT, PAGED, true, true>), grid, block, 0, s, a);
-  else if (l.nt) hipLaunchKernelGGL((write_planes_kernel<VPT, PAGED, true, false>), grid, block, 0, s, a);
-  else if (l.ntl) hipLaunchKernelGGL((write_planes_kernel<VPT, PAGED, false, true>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((write_planes_kernel<VPT, PAGED, false, false>), grid, block, 0, s, a);
+  if (l.nt && l.ntl) kvc::launch((write_planes_kernel<VPT, PAGED, true, true>), grid, block, 0, s, a);
+  else if (l.nt) kvc::launch((write_planes_kernel<VPT, PAGED, true, false>), grid, block, 0, s, a);
+  else if (l.ntl) kvc::launch((write_planes_kernel<VPT, PAGED, false, true>), grid, block, 0, s, a);
+  else kvc::launch((write_planes_kernel<VPT, PAGED, false, false>), grid, block, 0, s, a);
 }
 
 template <bool PAGED>
@@ -1466,8 +1466,8 @@ int run_write(const char* fn, const void* key, const void* value, void* kc, void
 // --------------------------- run write launch -------------------------------
 template <int VEC, int UNROLL>
 void launch_runs_nt(const RunArgs& a, unsigned grid, hipStream_t s, bool nt) {
-  if (nt) hipLaunchKernelGGL((write_runs_kernel<VEC, UNROLL, true>), dim3(grid), dim3(kThreads), 0, s, a);
-  else hipLaunchKernelGGL((write_runs_kernel<VEC, UNROLL, false>), dim3(grid), dim3(kThreads), 0, s, a);
+  if (nt) kvc::launch((write_runs_kernel<VEC, UNROLL, true>), dim3(grid), dim3(kThreads), 0, s, a);
+  else kvc::launch((write_runs_kernel<VEC, UNROLL, false>), dim3(grid), dim3(kThreads), 0, s, a);
 }
 
 template <int VEC>
@@ -1555,8 +1555,8 @@ int run_write_runs(const char* fn, const void* key, const void* value, void* kc,
 // --------------------------- tile copy launch -------------------------------
 template <int VEC, int UNROLL>
 void launch_tiles_nt(const TileArgs& a, unsigned grid, hipStream_t s, bool nt) {
-  if (nt) hipLaunchKernelGGL((copy_tiles_kernel<VEC, UNROLL, true>), dim3(grid), dim3(kThreads), 0, s, a);
-  else hipLaunchKernelGGL((copy_tiles_kernel<VEC, UNROLL, false>), dim3(grid), dim3(kThreads), 0, s, a);
+  if (nt) kvc::launch((copy_tiles_kernel<VEC, UNROLL, true>), dim3(grid), dim3(kThreads), 0, s, a);
+  else kvc::launch((copy_tiles_kernel<VEC, UNROLL, false>), dim3(grid), dim3(kThreads), 0, s, a);
 }
 
 // What a launch copies between: blocks of a pool, or a dense buffer on one side; kToHost: blocks of the mapped host pool
@@ -1606,12 +1606,12 @@ int launch_stream(const TileArgs& t, TileSides sides, int64_t n, hipStream_t s, 
   const bool plain_store = gather && bytes <= llc;
   const dim3 grid(a.total_chunks), block(threads);
   const unsigned six_per_cu = (int64_t)a.total_chunks > resident_workgroups() ? 160 * 1024 / 6 : 0;
-  if (pairs && plain_load) hipLaunchKernelGGL((stream_pairs_kernel<false>), grid, block, six_per_cu, s, a, *pairs);
-  else if (pairs) hipLaunchKernelGGL((stream_pairs_kernel<true>), grid, block, six_per_cu, s, a, *pairs);
-  else if (gather && plain_store) hipLaunchKernelGGL((stream_tiles_kernel<64, 1, true, false>), grid, block, 0, s, a);
-  else if (gather) hipLaunchKernelGGL((stream_tiles_kernel<64, 1, true, true>), grid, block, 0, s, a);
-  else if (plain_load) hipLaunchKernelGGL((stream_tiles_kernel<256, 2, false, true>), grid, block, six_per_cu, s, a);
-  else hipLaunchKernelGGL((stream_tiles_kernel<256, 2, true, true>), grid, block, six_per_cu, s, a);
+  if (pairs && plain_load) kvc::launch((stream_pairs_kernel<false>), grid, block, six_per_cu, s, a, *pairs);
+  else if (pairs) kvc::launch((stream_pairs_kernel<true>), grid, block, six_per_cu, s, a, *pairs);
+  else if (gather && plain_store) kvc::launch((stream_tiles_kernel<64, 1, true, false>), grid, block, 0, s, a);
+  else if (gather) kvc::launch((stream_tiles_kernel<64, 1, true, true>), grid, block, 0, s, a);
+  else if (plain_load) kvc::launch((stream_tiles_kernel<256, 2, false, true>), grid, block, six_per_cu, s, a);
+  else kvc::launch((stream_tiles_kernel<256, 2, true, true>), grid, block, six_per_cu, s, a);
   g_last = LastLaunch{KVC_KERNEL_COPY_TILES, 16, (int64_t)unroll, (int64_t)threads, (int64_t)a.total_chunks,
                       plain_store || (plain_load && sides == TileSides::kScatter) ? 0 : 1};
   KVC_HIP(hipGetLastError());
@@ -1680,14 +1680,14 @@ int launch_tiles_vec(TileArgs a, int unroll, int max_wgs, hipStream_t s, bool nt
   if (pairs) {  // 16-byte vectors and non-temporal accesses: the caller has looked
     const dim3 g((unsigned)grid), b(kThreads);
     switch (unroll) {
-      case 1: hipLaunchKernelGGL((copy_pairs_kernel<1>), g, b, 0, s, a, *pairs); break;
-      case 2: hipLaunchKernelGGL((copy_pairs_kernel<2>), g, b, 0, s, a, *pairs); break;
-      case 4: hipLaunchKernelGGL((copy_pairs_kernel<4>), g, b, 0, s, a, *pairs); break;
-      case 8: hipLaunchKernelGGL((copy_pairs_kernel<8>), g, b, 0, s, a, *pairs); break;
-      default: hipLaunchKernelGGL((copy_pairs_kernel<16>), g, b, 0, s, a, *pairs); break;
+      case 1: kvc::launch((copy_pairs_kernel<1>), g, b, 0, s, a, *pairs); break;
+      case 2: kvc::launch((copy_pairs_kernel<2>), g, b, 0, s, a, *pairs); break;
+      case 4: kvc::launch((copy_pairs_kernel<4>), g, b, 0, s, a, *pairs); break;
+      case 8: kvc::launch((copy_pairs_kernel<8>), g, b, 0, s, a, *pairs); break;
+      default: kvc::launch((copy_pairs_kernel<16>), g, b, 0, s, a, *pairs); break;
     }
   } else if (to_host && unroll == 2) {
-    hipLaunchKernelGGL(copy_to_host_kernel, dim3((unsigned)grid), dim3(kThreads), 0, s, a);
+    kvc::launch(copy_to_host_kernel, dim3((unsigned)grid), dim3(kThreads), 0, s, a);
   } else switch (unroll) {
     case 1: launch_tiles_nt<VEC, 1>(a, (unsigned)grid, s, nt); break;
     case 2: launch_tiles_nt<VEC, 2>(a, (unsigned)grid, s, nt); break;
@@ -1704,10 +1704,10 @@ int launch_tiles_vec(TileArgs a, int unroll, int max_wgs, hipStream_t s, bool nt
 template <int UNROLL>
 void launch_fan(const StreamArgs& a, int fan, const FanList* list, const int32_t* device_list, unsigned lds, hipStream_t s) {
   const dim3 grid(a.total_chunks), block(kThreads);
-  if (list && fan == 3) hipLaunchKernelGGL((fan_inline_kernel<UNROLL, 3>), grid, block, lds, s, a, *list);
-  else if (list) hipLaunchKernelGGL((fan_inline_kernel<UNROLL, 7>), grid, block, lds, s, a, *list);
-  else if (fan == 3) hipLaunchKernelGGL((fan_tiles_kernel<UNROLL, 3>), grid, block, lds, s, a, device_list);
-  else hipLaunchKernelGGL((fan_tiles_kernel<UNROLL, 7>), grid, block, lds, s, a, device_list);
+  if (list && fan == 3) kvc::launch((fan_inline_kernel<UNROLL, 3>), grid, block, lds, s, a, *list);
+  else if (list) kvc::launch((fan_inline_kernel<UNROLL, 7>), grid, block, lds, s, a, *list);
+  else if (fan == 3) kvc::launch((fan_tiles_kernel<UNROLL, 3>), grid, block, lds, s, a, device_list);
+  else kvc::launch((fan_tiles_kernel<UNROLL, 7>), grid, block, lds, s, a, device_list);
 }
 
 // Shape of a fan launch: vectors per lane as of a small copy, up to 8, while the workgroups are resident at once;
@@ -2199,7 +2199,7 @@ unsigned index_grid(int64_t batch_size, int64_t nnz, int64_t upload_ids) {
 
 // shared driver of the two index-build entry points
 int launch_build_index(const IndexArgs& a, void* stream, unsigned grid) {
-  hipLaunchKernelGGL(build_write_index_kernel, dim3(grid), dim3(kPrepThreads), 0, (hipStream_t)stream, a);
+  kvc::launch(build_write_index_kernel, dim3(grid), dim3(kPrepThreads), 0, (hipStream_t)stream, a);
   if (a.read_flags) return stage_launched();
   KVC_HIP(hipGetLastError());
   return KVC_OK;
@@ -2261,7 +2261,7 @@ int launch_resolve_slots(const char* fn, const int32_t* batch_indices, const int
   if (!slots) return fail(KVC_ERR_INVALID_ARG, "%s: null slot array", fn);
   if (nnz > (int64_t(1) << 40)) return fail(KVC_ERR_UNSUPPORTED, "%s: %lld tokens", fn, (long long)nnz);
   const unsigned grid = (unsigned)((nnz + kThreads - 1) / kThreads);
-  hipLaunchKernelGGL(resolve_slots_kernel, dim3(grid), dim3(kThreads), 0, stream, batch_indices,
+  kvc::launch(resolve_slots_kernel, dim3(grid), dim3(kThreads), 0, stream, batch_indices,
                      positions, kv_indices, kv_indptr, batch_size, num_kv_indices, page_size, nnz, slots);
   KVC_HIP(hipGetLastError());
   return KVC_OK;
@@ -2483,7 +2483,7 @@ int kvc_get_seq_lens(const int32_t* kv_indptr, const int32_t* kv_last_page_len, 
   if (!kv_indptr || !kv_last_page_len || !seq_lens)
     return fail(KVC_ERR_INVALID_ARG, "kvc_get_seq_lens: null pointer");
   const unsigned grid = (unsigned)((batch_size + kThreads - 1) / kThreads);
-  hipLaunchKernelGGL(seq_lens_kernel, dim3(grid), dim3(kThreads), 0, (hipStream_t)stream, kv_indptr,
+  kvc::launch(seq_lens_kernel, dim3(grid), dim3(kThreads), 0, (hipStream_t)stream, kv_indptr,
                      kv_last_page_len, batch_size, (int32_t)page_size, seq_lens);
   KVC_HIP(hipGetLastError());
   return KVC_OK;
@@ -2498,7 +2498,7 @@ int kvc_get_batch_indices_positions(const int32_t* append_indptr, const int32_t*
   if (batch_size == 0 || nnz == 0) return KVC_OK;
   if (!append_indptr || !seq_lens || !batch_indices || !positions)
     return fail(KVC_ERR_INVALID_ARG, "kvc_get_batch_indices_positions: null pointer");
-  hipLaunchKernelGGL(batch_indices_positions_kernel, dim3((unsigned)batch_size), dim3(kThreads), 0,
+  kvc::launch(batch_indices_positions_kernel, dim3((unsigned)batch_size), dim3(kThreads), 0,
                      (hipStream_t)stream, append_indptr, seq_lens, nnz, batch_indices, positions);
   KVC_HIP(hipGetLastError());
   return KVC_OK;
@@ -2562,7 +2562,7 @@ int kvc_staging_upload(void* dst, int64_t bytes, void* stream) {
   const int rc = stage_hand_over(fn, bytes, grid, stream, &flags, &value);
   if (rc != KVC_OK) return rc;
   const char* src = reinterpret_cast<const char*>(flags) + kStageHead;
-  hipLaunchKernelGGL(upload_kernel, dim3(grid), dim3(kThreads), 0, (hipStream_t)stream,
+  kvc::launch(upload_kernel, dim3(grid), dim3(kThreads), 0, (hipStream_t)stream,
                      reinterpret_cast<const int4*>(src), (int4*)dst, words4, flags, value);
   return stage_launched();
 }
@@ -2605,8 +2605,8 @@ int kvc_streams_share_hw_queue(void* stream_x, void* stream_y, int* shared) {
       return fail(KVC_ERR_INVALID_ARG, "%s: a stream is being captured", fn);
   }
   // first use of a stream creates or attaches its hardware queue: keep that out of the timing
-  hipLaunchKernelGGL(touch_queue_kernel, dim3(1), dim3(64), 0, x);
-  hipLaunchKernelGGL(touch_queue_kernel, dim3(1), dim3(64), 0, y);
+  kvc::launch(touch_queue_kernel, dim3(1), dim3(64), 0, x);
+  kvc::launch(touch_queue_kernel, dim3(1), dim3(64), 0, y);
   KVC_HIP(hipGetLastError());
   KVC_HIP(hipStreamSynchronize(x));
   KVC_HIP(hipStreamSynchronize(y));
@@ -2624,10 +2624,10 @@ int kvc_streams_share_hw_queue(void* stream_x, void* stream_y, int* shared) {
   int blocked_rounds = 0;
   constexpr int kRounds = 3;
   for (int round = 0; round < kRounds && rc == KVC_OK; ++round) {
-    hipLaunchKernelGGL(hold_queue_kernel, dim3(1), dim3(64), 0, x, (uint64_t)20000, (uint32_t)4000);
+    kvc::launch(hold_queue_kernel, dim3(1), dim3(64), 0, x, (uint64_t)20000, (uint32_t)4000);
     hipError_t e = hipEventRecord(ex, x);
     if (e == hipSuccess) {
-      hipLaunchKernelGGL(touch_queue_kernel, dim3(1), dim3(64), 0, y);
+      kvc::launch(touch_queue_kernel, dim3(1), dim3(64), 0, y);
       e = hipEventRecord(ey, y);
     }
     bool blocked = false;
@@ -2672,7 +2672,7 @@ int kvc_slot_runs(const void* slot_mapping, int slot_bytes, int64_t num_tokens, 
   if (max_runs < num_tokens)
     return fail(KVC_ERR_INVALID_ARG, "kvc_slot_runs: max_runs=%lld cannot hold the %lld runs that many "
                 "tokens may form", (long long)max_runs, (long long)num_tokens);
-  hipLaunchKernelGGL(slot_runs_kernel, dim3(1), dim3(kPrepThreads), 0, (hipStream_t)stream,
+  kvc::launch(slot_runs_kernel, dim3(1), dim3(kPrepThreads), 0, (hipStream_t)stream,
                      slot_mapping, slot_bytes, num_tokens, block_size, runs, num_runs, max_runs);
   KVC_HIP(hipGetLastError());
   return KVC_OK;
@@ -3052,7 +3052,7 @@ int kvc_swap_noalloc(int to_host, void* pool, void* host_pool, const int64_t* gp
       packet.gpu[i] = (int32_t)gpu_ids[first + i];
       packet.host[i] = (int32_t)host_ids[first + i];
     }
-    hipLaunchKernelGGL(stage_ids_kernel, dim3(1), dim3((count + 63) / 64 * 64), 0, s, packet, ids, first,
+    kvc::launch(stage_ids_kernel, dim3(1), dim3((count + 63) / 64 * 64), 0, s, packet, ids, first,
                        count, n);
     KVC_HIP(hipGetLastError());
   }

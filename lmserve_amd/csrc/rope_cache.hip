@@ -496,8 +496,8 @@ bool fast_index(const RopeArgs& a) {
 
 template <typename T, Addressing ADDR>
 void launch_element(const RopeArgs& a, dim3 grid, dim3 block, hipStream_t s) {
-  if (fast_index<ADDR>(a)) hipLaunchKernelGGL((rope_element_kernel<T, ADDR, true>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((rope_element_kernel<T, ADDR, false>), grid, block, 0, s, a);
+  if (fast_index<ADDR>(a)) kvc::launch((rope_element_kernel<T, ADDR, true>), grid, block, 0, s, a);
+  else kvc::launch((rope_element_kernel<T, ADDR, false>), grid, block, 0, s, a);
 }
 
 // The kernels of rows of aligned 16-byte vectors
@@ -505,9 +505,9 @@ enum VectorForm { kElements, kPairs, kRows };
 
 template <typename T, Addressing ADDR, int NTL>
 void launch_vector(const RopeArgs& a, VectorForm form, dim3 grid, dim3 block, hipStream_t s) {
-  if (form == kPairs) hipLaunchKernelGGL((rope_pairs_kernel<T, ADDR, NTL>), grid, block, 0, s, a);
-  else if (fast_index<ADDR>(a)) hipLaunchKernelGGL((rope_rows_kernel<T, ADDR, true, NTL>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((rope_rows_kernel<T, ADDR, false, NTL>), grid, block, 0, s, a);
+  if (form == kPairs) kvc::launch((rope_pairs_kernel<T, ADDR, NTL>), grid, block, 0, s, a);
+  else if (fast_index<ADDR>(a)) kvc::launch((rope_rows_kernel<T, ADDR, true, NTL>), grid, block, 0, s, a);
+  else kvc::launch((rope_rows_kernel<T, ADDR, false, NTL>), grid, block, 0, s, a);
 }
 
 template <typename T, Addressing ADDR>
@@ -560,8 +560,8 @@ int launch_rope_layers(RopeArgs a, const RopeLayer* layers, int64_t num_layers, 
     args.a = a;
     std::copy(layers + l0, layers + l0 + n, args.layer);
     const dim3 grid(a.groups_per_token, (unsigned)num_tokens, (unsigned)n), block(threads);
-    if (form == kPairs) hipLaunchKernelGGL((rope_layers_kernel<T, true>), grid, block, 0, s, args);
-    else hipLaunchKernelGGL((rope_layers_kernel<T, false>), grid, block, 0, s, args);
+    if (form == kPairs) kvc::launch((rope_layers_kernel<T, true>), grid, block, 0, s, args);
+    else kvc::launch((rope_layers_kernel<T, false>), grid, block, 0, s, args);
     KVC_HIP(hipGetLastError());
   }
   return KVC_OK;

@@ -843,12 +843,17 @@ __global__ void batch_indices_positions_kernel(const int32_t* append_indptr,
 // link overlap).
 // Bound: latency. Every workgroup scans the (at most 1024) requests for itself and
 // takes its share of the tokens and of the tables; one workgroup for all of them
-// walked 8192 tokens in 8 rounds of dependent loads (12.7 us; 6.3 at 2048).
+// walked 8192 tokens in 8 rounds of dependent loads (12.7 us; 6.3 at 2048). Tables of up
+// to 4096 ids each workgroup reads whole, ahead of the scans: with a read over the link for
+// each token's block behind them, a chunk of 2048 tokens took 8.1 us and one of 8192 9.2, now
+// 5.2 and 6.4; decode steps of 2, 16 and 64 requests 5.0 -> 4.8, 5.5 -> 5.3, 5.7 -> 5.4, of 256
+// with 24000 ids 10.4 -> 10.0 (the last words read up front, no wavefront sums of empty wavefronts).
 constexpr int kPrepThreads = 1024;
 
 // Inclusive scan of three values over the workgroup's 1024 lanes: shuffles inside
 // each wavefront, then the 16 wavefront totals through LDS (two barriers).
-__device__ __forceinline__ void scan3(int32_t& q, int32_t& n, int32_t& r, int32_t (*wave_sums)[3]) {
+// `waves`: the wavefronts that can hold a value other than 0.
+__device__ __forceinline__ void scan3(int32_t& q, int32_t& n, int32_t& r, int32_t (*wave_sums)[3], int waves) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) {
@@ -866,7 +871,7 @@ __device__ __forceinline__ void scan3(int32_t& q, int32_t& n, int32_t& r, int32_
     wave_sums[wave][2] = r;
   }
   __syncthreads();
-  for (int w = 0; w < wave; ++w) {
+  for (int w = 0; w < min(wave, waves); ++w) {
     q += wave_sums[w][0];
     n += wave_sums[w][1];
     r += wave_sums[w][2];
@@ -902,15 +907,22 @@ __global__ __launch_bounds__(kPrepThreads) void build_write_index_kernel(IndexAr
   // prefix sums of a batch that fits one chunk stay in LDS for the per-token part
   __shared__ int32_t lds_cu[kPrepThreads + 1], lds_indptr[kPrepThreads + 1], lds_runptr[kPrepThreads + 1];
   __shared__ int32_t lds_ctx[kPrepThreads];
+  // block tables that one workgroup reads whole on the way to the device
+  __shared__ __align__(16) int32_t lds_ids[4 * kPrepThreads];
   const int tid = threadIdx.x;
   const bool first_wg = blockIdx.x == 0;
   const int32_t page_size = a.page_size;
   const int64_t lane0 = (int64_t)blockIdx.x * kPrepThreads + tid, lanes = (int64_t)gridDim.x * kPrepThreads;
-  // the lane's first 16 bytes of the block tables
+  // The lane's first 16 bytes of the block tables, and of their last words. Tables of up to 4096 ids every workgroup reads
+  // whole, into LDS: a token's block then needs no read over the link behind the scans.
   const int64_t words4 = a.ids_out ? a.num_kv_indices / 4 : 0;
-  const bool has_ids = lane0 < words4;
+  const bool ids_in_lds = a.ids_out && a.num_kv_indices <= 4 * kPrepThreads;
+  const int64_t lane_ids = ids_in_lds ? tid : lane0;
+  const bool has_ids = lane_ids < words4, has_last = a.ids_out && 4 * words4 + lane_ids < a.num_kv_indices;
   int4 ids = make_int4(0, 0, 0, 0);
-  if (has_ids) ids = reinterpret_cast<const int4*>(a.kv_indices)[lane0];
+  int32_t last_id = 0;
+  if (has_ids) ids = reinterpret_cast<const int4*>(a.kv_indices)[lane_ids];
+  if (has_last) last_id = a.kv_indices[4 * words4 + lane_ids];
   // a batch beyond one chunk keeps its prefix sums in the outputs and is launched as one workgroup
   const bool in_lds = a.batch_size <= kPrepThreads;
   if (tid == 0) {
@@ -935,7 +947,7 @@ __global__ __launch_bounds__(kPrepThreads) void build_write_index_kernel(IndexAr
     const int32_t ctx = b < a.batch_size ? a.context_lens[b] : 0;
     // runs of the request: the blocks its new positions [ctx - q, ctx) touch
     int32_t nr = (q > 0 && ctx >= q) ? (ctx - 1) / page_size - (ctx - q) / page_size + 1 : 0;
-    scan3(q, n, nr, wave_sums);
+    scan3(q, n, nr, wave_sums, (min(a.batch_size - base, kPrepThreads) + 63) >> 6);
     q += carry[0];
     n += carry[1];
     nr += carry[2];
@@ -952,6 +964,10 @@ __global__ __launch_bounds__(kPrepThreads) void build_write_index_kernel(IndexAr
         lds_runptr[b + 1] = nr;
         lds_ctx[b] = ctx;
       }
+    }
+    if (ids_in_lds && base == 0) {
+      if (has_ids) reinterpret_cast<int4*>(lds_ids)[tid] = ids;
+      if (has_last) lds_ids[4 * words4 + tid] = last_id;
     }
     __syncthreads();  // everyone has read the carry
     if (tid == kPrepThreads - 1) {
@@ -995,7 +1011,7 @@ __global__ __launch_bounds__(kPrepThreads) void build_write_index_kernel(IndexAr
     const int64_t it = (int64_t)indptr[b] + pos / page_size;
     const int64_t table_end = indptr[b + 1] < a.num_kv_indices ? indptr[b + 1] : a.num_kv_indices;
     const bool in_table = pos >= 0 && it >= 0 && it < table_end;
-    const int32_t block = in_table ? a.kv_indices[it] : -1;
+    const int32_t block = !in_table ? -1 : ids_in_lds ? lds_ids[it] : a.kv_indices[it];
     if (a.slot_mapping) a.slot_mapping[out] = in_table ? (int64_t)block * page_size + pos % page_size : -1;
     if (a.runs && pos >= 0 && ctx >= n_new && (j == 0 || pos % page_size == 0)) {
       const int32_t first_pos = ctx - n_new;
@@ -1008,12 +1024,11 @@ __global__ __launch_bounds__(kPrepThreads) void build_write_index_kernel(IndexAr
       }
     }
   }
-  if (a.ids_out) {
-    if (has_ids) reinterpret_cast<int4*>(a.ids_out)[lane0] = ids;
-    for (int64_t i = lane0 + lanes; i < words4; i += lanes)
+  if (a.ids_out && (first_wg || !ids_in_lds)) {
+    if (has_ids) reinterpret_cast<int4*>(a.ids_out)[lane_ids] = ids;
+    if (has_last) a.ids_out[4 * words4 + lane_ids] = last_id;
+    for (int64_t i = lane_ids + lanes; i < words4; i += lanes)
       reinterpret_cast<int4*>(a.ids_out)[i] = reinterpret_cast<const int4*>(a.kv_indices)[i];
-    const int64_t i = 4 * words4 + lane0;  // the last words
-    if (i < a.num_kv_indices) a.ids_out[i] = a.kv_indices[i];
   }
   if (a.read_flags) tell_host(a.read_flags, a.flag_value);
 }

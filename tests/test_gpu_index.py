@@ -182,6 +182,16 @@ def _check_build(reqs, gpu):
         assert torch.equal(getattr(got, name), getattr(want, name)), name
 
 
+@pytest.mark.parametrize("ids", [1, 3, 4095, 4096, 4097, 4099])
+@pytest.mark.parametrize("tokens", [1, 1500])
+def test_tables_that_one_workgroup_reads_whole_and_longer_ones(gpu, ids, tokens):
+    """On either side of 4096 block ids, with one workgroup of tokens and with two."""
+    table = np.random.default_rng(ids + tokens).integers(0, 1 << 20, ids).tolist()
+    cut = ids - ids // 3
+    _check_build([kvc.InferInput(i, [], n, 16 * len(t) - n, 16 * len(t), t)
+                  for i, t in enumerate((table[:cut], table[cut:])) if t for n in (min(tokens, 16 * len(t)),)], gpu)
+
+
 def test_one_launch_index_build_reports_an_allocation_that_fails(gpu):
     """As an exception of the interpreter; the next call works."""
     huge = [kvc.InferInput(seq_id=0, input_ids=[], input_len=1 << 29, filled_token_len=0, context_len=1 << 29,

@@ -334,7 +334,7 @@ int kvc_swap_in(void* pool, const void* host_pool,
  * calls), a layer range of num_layers_in_range layers and a staging buffer of
  * staging_bytes. The direct kernel holds the PCIe rate whatever the ids are, but
  * holds back the kernels of other streams while it runs (a forward pass beside a
- * direct write-through of 1 GiB took 2.3 times as long on MI355X); a caller that
+ * direct write-through of 1 GiB took 1.6 times as long on MI355X); a caller that
  * runs a model on the same GPU should give AUTO a staging buffer of
  * kvc_swap_staging_bytes(..., KVC_SWAP_STAGED, ...) and host blocks that form
  * runs, or move the rows through a dense pinned buffer (kvcache_experimental.h).

@@ -1,6 +1,6 @@
 // libkvcache: paged KV-cache data movement for MI355X (gfx950, CDNA4).
 //
-// Five kernels carry the whole path; all are HBM-bound byte movers, so the
+// These kernels carry the whole path; all are HBM-bound byte movers, so the
 // design is about coalescing and bytes in flight, not arithmetic:
 //
 //   write_rows_kernel   a workgroup owns ONE token and a run of 16-byte vectors
@@ -19,13 +19,16 @@
 //                       contiguous on both sides). A workgroup owns a chunk of
 //                       256 lanes x UNROLL x 16 bytes, issues all its loads
 //                       before its first store, and walks chunks grid-stride.
-//                       Small launches, narrow vectors, and the direct swap
-//                       (pool <-> mapped host pool).
+//                       Small launches, narrow vectors, and the direct swap-in
+//                       (mapped host pool -> pool).
+//   copy_to_host_kernel the direct swap-out: few workgroups, stores through the L2.
 //   stream_tiles_kernel the same for large launches: copy_blocks (pool -> pool)
 //                       and the swap gather/scatter (pool <-> staging ring in
 //                       host layout), chunks ordered per XCD.
-//   index kernels       seq_lens and (batch_indices, positions) for the paged
-//                       write; a few KiB of int32.
+//   fan_tiles_kernel    copy_blocks where a block has several destinations: it is
+//                       read once and stored to each.
+//   index kernels       a step's whole index in one launch, and its parts; a few
+//                       KiB of int32.
 //
 // The C ABI is declared in include/kvcache.h.
 

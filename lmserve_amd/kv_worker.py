@@ -277,8 +277,8 @@ class KVWorker:
       move at a ninth of the link rate. "direct": one kernel addresses the
       mapped host pool, no staging traffic, one launch per call and the link
       rate whatever the ids are; but while that kernel runs, kernels of other
-      streams are held back (a stream of short GEMMs stands still beside a
-      direct swap-out, measured on MI355X). "auto" (default): per call, staged
+      streams are held back (a forward pass beside a direct swap-out of
+      1 GiB takes 1.6 times as long on MI355X). "auto" (default): per call, staged
       when the call's extents are 1 MiB or more in the mean, else direct. The
       mappings of a call are sorted by host block id first (their order does not
       matter to the result), so a call's host blocks form the longest runs they

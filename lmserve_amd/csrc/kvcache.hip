@@ -564,7 +564,8 @@ __global__ __launch_bounds__(kThreads) void copy_pairs_kernel(TileArgs a, PairLi
 // link full and the rest of the GPU goes on. 96 workgroups of non-temporal stores -> this, 192 MiB of scattered blocks:
 // 54.6 -> 56.2 GB/s, 83 instead of 60 in sum beside a direct swap-in, one layer of 96 blocks 130 -> 118 us; a bf16
 // product of 4096^3 beside it 226 -> 154 us (106-116 alone), one of 3000 rows 191 -> 100 (87 alone, 98 beside the
-// copy engines); a forward pass of 13.4 ms with 1 GiB leaving layer by layer beside it 32.0 -> 21.1 ms. 32 and 96 workgroups stored through: 3000 rows 157 and 189, both directions 68 and 63 GB/s.
+// copy engines); a forward pass of 13.4 ms with 1 GiB leaving layer by layer beside it 32.0 -> 21.1 ms.
+// 32 and 96 workgroups stored through: 3000 rows 157 and 189, both directions 68 and 63 GB/s.
 constexpr int kToHostWgs = 16;
 __global__ __launch_bounds__(kThreads) void copy_to_host_kernel(TileArgs a) {
   copy_tiles_chunks<16, 2, true, true>(a, ListIds{a});
@@ -1660,13 +1661,13 @@ int launch_tiles_vec(TileArgs a, int unroll, int max_wgs, hipStream_t s, bool nt
   } else if (unroll <= 0) {
     // By size, from sweeps of copy_blocks (1 to 4096 pairs x 32 layers x 64 KiB):
     // a launch that fits three eighths of the resident workgroups runs best as few,
-    // deep workgroups (small_unroll; up to a whole tile
-    // per workgroup while that stays within half the resident set): 6-8 % faster
+    // deep workgroups (small_unroll; up to a whole tile per workgroup while that
+    // stays within half the resident set): 6-8 % faster
     // than 4 vectors per lane from 32 to 128 MiB (a gather: 12-15 % faster than
     // with 1). Larger launches go through the stream kernel; what it does not take
     // (narrow vectors, tiles below 8 KiB, a capped grid, plain copies or another tile order by request, and
-    // more lanes than a launch has: a gather of 64 GiB, a copy or scatter of 128) runs with 2 vectors per lane, or 1 when the scattered
-    // side is the one being read (gather).
+    // more lanes than a launch has: a gather of 64 GiB, a copy or scatter of 128) runs with 2 vectors per lane, or 1 when
+    // the scattered side is the one being read (gather).
     const int64_t resident = resident_workgroups();
     const auto chunks = [&](int u) {
       const int64_t c = (int64_t)kThreads * VEC * u;

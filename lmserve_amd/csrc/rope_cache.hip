@@ -65,7 +65,8 @@ struct F32 {
   static constexpr int kBytes = 4;
 };
 
-// one 16-byte pair-vector in fp32 with one rounding: ox = x cos - y sin, oy = y cos + x sin
+// one 16-byte pair-vector in fp32 with one rounding: ox = x cos - y sin, oy = y cos + x sin; contracted by hand, the
+// own half's product in the fma: the same bits in every kernel
 template <typename T>
 struct Vec {
   static __device__ __forceinline__ void rotate(u32x4 x, u32x4 y, u32x4 cx, u32x4 cy, u32x4 sx, u32x4 sy,
@@ -76,15 +77,15 @@ struct Vec {
 #pragma unroll
       for (int w = 0; w < 2; ++w) {
         const auto f = [&](u32x4 v) { return T::load((uint16_t)(w ? v[i] >> 16 : v[i] & 0xffffu)); };
-        o[0][w] = f(x) * f(cx) - f(y) * f(sx);
-        o[1][w] = f(y) * f(cy) + f(x) * f(sy);
+        o[0][w] = __builtin_fmaf(f(x), f(cx), -(f(y) * f(sx)));
+        o[1][w] = __builtin_fmaf(f(y), f(cy), f(x) * f(sy));
       }
       ox[i] = T::store2(o[0][0], o[0][1]);
       oy[i] = T::store2(o[1][0], o[1][1]);
     }
   }
   // one 16-byte vector of either half, `other` the same lanes of the other half: own cos -+ other sin, the minus by
-  // `flip` in the sign bits of the x half; contracted by hand, as the compiler contracts `rotate`: the same bits
+  // `flip` in the sign bits of the x half; contracted as `rotate` is
   static constexpr uint32_t kSign = 0x80008000u;
   static __device__ __forceinline__ u32x4 rotate_one(u32x4 own, u32x4 other, u32x4 c, u32x4 s, uint32_t flip) {
     u32x4 out;
@@ -112,8 +113,8 @@ struct Vec<F32> {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const auto f = [&](u32x4 v) { return __uint_as_float(v[i]); };
-      ox[i] = __float_as_uint(f(x) * f(cx) - f(y) * f(sx));
-      oy[i] = __float_as_uint(f(y) * f(cy) + f(x) * f(sy));
+      ox[i] = __float_as_uint(__builtin_fmaf(f(x), f(cx), -(f(y) * f(sx))));
+      oy[i] = __float_as_uint(__builtin_fmaf(f(y), f(cy), f(x) * f(sy)));
     }
   }
   static constexpr uint32_t kSign = 0x80000000u;
@@ -322,7 +323,7 @@ __device__ __forceinline__ void rope_pairs_lane(const RopeArgs& a, const RopeLay
   if (has_v && slot >= 0) OutRow(p.value_cache + slot, kv_bytes).store<kvc::kThroughNt>(lane * 16, v);
 }
 
-// Every other shape of aligned rows: heads rotated in part, halves that are no whole
+// Every other shape of aligned rows, written elsewhere than where they are read: heads rotated in part, halves that are no whole
 // 64-byte pieces, more V vectors than pair-vectors, other index types. A lane owns the same
 // 16-byte vector of two heads (Q, then K, then V heads), so the lanes write the rows out in
 // order, whole lines whatever the halves are; its other half's vector is a second load, from the
@@ -393,7 +394,106 @@ __device__ __forceinline__ void rope_rows_lane(const RopeArgs& a, const RopeLaye
   }
 }
 
-__device__ __forceinline__ RopeLayer only_layer(const RopeArgs& a) {
+// An output in its input's own rows: the pair form for every shape, since a lane of the rows kernel reads a vector
+// that another lane overwrites. A lane owns both halves of a pair and carries vectors that pass through along: one of
+// V, with TAIL up to two of V and of the heads' unrotated lanes. Bound as the pair form; plain stores, as its pieces
+// are of any size. TAIL costs a launch without tails a tenth. us a launch of a recorded step, in place here and
+// elsewhere by the rows kernel: 838 tokens x 40 heads x 80 in fp16, 32 rotated, 5.4 and 4.4, 8192 of those 30.1 and
+// 21.8; 2048 x 15 x 96 in bf16 4.9 and 4.5, 256 of those 3.25 and 3.3.
+template <typename T, Addressing ADDR, bool FAST, bool TAIL>
+__device__ __forceinline__ void rope_owner_lane(const RopeArgs& a, const RopeLayer p) {
+  constexpr uint32_t E = T::kBytes;
+  const uint32_t t = blockIdx.y;
+  const uint32_t lane = blockIdx.x * blockDim.x + threadIdx.x;
+  if (lane >= a.lanes_per_token) return;
+  const int64_t pos = FAST ? (int64_t) reinterpret_cast<const int32_t*>(a.positions)[t] : index_of(a.positions, a.pos_bytes, t);
+
+  const uint32_t half = (a.rotary_dim >> 1) * E;  // bytes
+  const uint32_t h = head_of_lane(a, lane);
+  const uint32_t pv = (lane - h * a.split) * 16;
+  const uint32_t heads = a.num_heads + a.num_kv_heads;
+  const bool rotates = !TAIL || h < heads, is_k = h >= a.num_heads;
+  const uint32_t head_off = (is_k ? h - a.num_heads : h) * a.head_dim * E + pv;
+  const char* q_row = p.query + (int64_t)t * a.q_token_stride;
+  const char* k_row = p.key + (int64_t)t * a.k_token_stride;
+  u32x4 x = {}, y = {};
+  if (rotates) {
+    const char* in = (is_k ? k_row : q_row) + head_off;
+    x = ld16<false>(in);
+    y = ld16<false>(in + half);
+  }
+  enum Kind { kNone, kV, kTailQ, kTailK };
+  constexpr int kCarried = TAIL ? 2 : 1;
+  u32x4 carried[kCarried] = {};
+  uint32_t carried_off[kCarried] = {};  // in the row it comes from and in the row it goes to
+  Kind kind[kCarried];
+#pragma unroll
+  for (int j = 0; j < kCarried; ++j) {
+    const uint32_t e = lane + j * a.lanes_per_token;
+    kind[j] = kNone;
+    if (ADDR != kNoCache && e < a.v_items) {
+      kind[j] = kV;
+      carried_off[j] = e * 16;
+      carried[j] = ld16<false>(p.value + (int64_t)t * a.v_token_stride + carried_off[j]);
+    } else if constexpr (TAIL) {
+      const uint32_t tail_per_head = (a.head_dim - a.rotary_dim) * E / 16;
+      if (e < a.v_items + heads * tail_per_head) {
+        const uint32_t i = e - a.v_items, th = i / tail_per_head;
+        const bool tk = th >= a.num_heads;
+        kind[j] = tk ? kTailK : kTailQ;
+        carried_off[j] = ((tk ? th - a.num_heads : th) * a.head_dim + a.rotary_dim) * E + (i - th * tail_per_head) * 16;
+        carried[j] = ld16<false>((tk ? k_row : q_row) + carried_off[j]);
+      }
+    }
+  }
+
+  if (pos < 0 || pos >= a.max_position) return;  // no cos/sin row: the token is left alone
+  u32x4 cos_x = {}, cos_y = {}, sin_x = {}, sin_y = {};
+  if (rotates) {
+    const char* row = a.cos_sin_cache + pos * (int64_t)(4 * half) + pv;
+    cos_x = ld16_cos_sin(row);
+    cos_y = ld16_cos_sin(row + half);
+    sin_x = ld16_cos_sin(row + 2 * half);
+    sin_y = ld16_cos_sin(row + 3 * half);
+  }
+  const int64_t slot = slot_offset<ADDR, FAST>(a, t, pos);
+
+  const auto put = [](char* out, u32x4 v) { *reinterpret_cast<u32x4*>(out) = v; };
+  const auto put_cache = [](char* out, u32x4 v) { __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(out)); };
+  if (rotates) {
+    u32x4 ox, oy;
+    Vec<T>::rotate(x, y, cos_x, cos_y, sin_x, sin_y, ox, oy);
+    if (!is_k) {
+      char* out = p.query_out + (int64_t)t * a.qo_token_stride + head_off;
+      put(out, ox);
+      put(out + half, oy);
+    } else {
+      if (p.key_out) {
+        char* out = p.key_out + (int64_t)t * a.ko_token_stride + head_off;
+        put(out, ox);
+        put(out + half, oy);
+      }
+      if (ADDR != kNoCache && slot >= 0) {
+        char* out = p.key_cache + slot + head_off;
+        put_cache(out, ox);
+        put_cache(out + half, oy);
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < kCarried; ++j) {
+    if (kind[j] == kV) {
+      if (slot >= 0) put_cache(p.value_cache + slot + carried_off[j], carried[j]);
+    } else if (TAIL && kind[j] == kTailQ) {
+      put(p.query_out + (int64_t)t * a.qo_token_stride + carried_off[j], carried[j]);
+    } else if (TAIL && kind[j] == kTailK) {
+      if (p.key_out) put(p.key_out + (int64_t)t * a.ko_token_stride + carried_off[j], carried[j]);
+      if (ADDR != kNoCache && slot >= 0) put_cache(p.key_cache + slot + carried_off[j], carried[j]);
+    }
+  }
+}
+
+__host__ __device__ __forceinline__ RopeLayer only_layer(const RopeArgs& a) {
   return RopeLayer{a.query, a.key, a.value, a.query_out, a.key_out, a.key_cache, a.value_cache};
 }
 template <typename T, Addressing ADDR, int NTL>
@@ -403,6 +503,10 @@ __global__ __launch_bounds__(kThreads) void rope_pairs_kernel(RopeArgs a) {
 template <typename T, Addressing ADDR, bool FAST, int NTL>
 __global__ __launch_bounds__(kThreads) void rope_rows_kernel(RopeArgs a) {
   rope_rows_lane<T, ADDR, FAST, NTL>(a, only_layer(a));
+}
+template <typename T, Addressing ADDR, bool FAST, bool TAIL>
+__global__ __launch_bounds__(kThreads) void rope_owner_kernel(RopeArgs a) {
+  rope_owner_lane<T, ADDR, FAST, TAIL>(a, only_layer(a));
 }
 
 // The same for several layers of one step, blockIdx.z the layer, their pointers in the
@@ -420,10 +524,15 @@ struct RopeLayersArgs {
 };
 static_assert(sizeof(RopeLayersArgs) <= 4096, "kernel arguments");
 
-template <typename T, bool PAIRS>
+// The kernels of rows of aligned 16-byte vectors, and the one of all other rows
+enum VectorForm { kElements, kPairs, kRows, kOwner, kOwnerTail };
+
+template <typename T, VectorForm FORM>
 __global__ __launch_bounds__(kThreads) void rope_layers_kernel(RopeLayersArgs args) {
-  if constexpr (PAIRS) rope_pairs_lane<T, kSlots, 0>(args.a, args.layer[blockIdx.z]);
-  else rope_rows_lane<T, kSlots, true, 0>(args.a, args.layer[blockIdx.z]);
+  const RopeLayer p = args.layer[blockIdx.z];
+  if constexpr (FORM == kPairs) rope_pairs_lane<T, kSlots, 0>(args.a, p);
+  else if constexpr (FORM == kRows) rope_rows_lane<T, kSlots, true, 0>(args.a, p);
+  else rope_owner_lane<T, kSlots, true, FORM == kOwnerTail>(args.a, p);
 }
 
 // Element path: rows that are no whole number of aligned 16-byte vectors. One
@@ -500,9 +609,6 @@ void launch_element(const RopeArgs& a, dim3 grid, dim3 block, hipStream_t s) {
   else kvc::launch((rope_element_kernel<T, ADDR, false>), grid, block, 0, s, a);
 }
 
-// The kernels of rows of aligned 16-byte vectors
-enum VectorForm { kElements, kPairs, kRows };
-
 template <typename T, Addressing ADDR, int NTL>
 void launch_vector(const RopeArgs& a, VectorForm form, dim3 grid, dim3 block, hipStream_t s) {
   if (form == kPairs) kvc::launch((rope_pairs_kernel<T, ADDR, NTL>), grid, block, 0, s, a);
@@ -512,6 +618,12 @@ void launch_vector(const RopeArgs& a, VectorForm form, dim3 grid, dim3 block, hi
 
 template <typename T, Addressing ADDR>
 void launch_vector(const RopeArgs& a, VectorForm form, dim3 grid, dim3 block, hipStream_t s) {
+  if (form == kOwner || form == kOwnerTail) {
+    if (!fast_index<ADDR>(a)) kvc::launch((rope_owner_kernel<T, ADDR, false, true>), grid, block, 0, s, a);
+    else if (form == kOwner) kvc::launch((rope_owner_kernel<T, ADDR, true, false>), grid, block, 0, s, a);
+    else kvc::launch((rope_owner_kernel<T, ADDR, true, true>), grid, block, 0, s, a);
+    return;
+  }
   switch (kvc::g_rope_tune.nt & 3) {
     case 0: launch_vector<T, ADDR, 0>(a, form, grid, block, s); break;
     case 1: launch_vector<T, ADDR, 1>(a, form, grid, block, s); break;
@@ -560,8 +672,10 @@ int launch_rope_layers(RopeArgs a, const RopeLayer* layers, int64_t num_layers, 
     args.a = a;
     std::copy(layers + l0, layers + l0 + n, args.layer);
     const dim3 grid(a.groups_per_token, (unsigned)num_tokens, (unsigned)n), block(threads);
-    if (form == kPairs) kvc::launch((rope_layers_kernel<T, true>), grid, block, 0, s, args);
-    else kvc::launch((rope_layers_kernel<T, false>), grid, block, 0, s, args);
+    if (form == kPairs) kvc::launch((rope_layers_kernel<T, kPairs>), grid, block, 0, s, args);
+    else if (form == kRows) kvc::launch((rope_layers_kernel<T, kRows>), grid, block, 0, s, args);
+    else if (form == kOwner) kvc::launch((rope_layers_kernel<T, kOwner>), grid, block, 0, s, args);
+    else kvc::launch((rope_layers_kernel<T, kOwnerTail>), grid, block, 0, s, args);
     KVC_HIP(hipGetLastError());
   }
   return KVC_OK;
@@ -608,6 +722,25 @@ bool layers_depend(const RopeLayer* layers, int64_t n, const LayerExtents& e) {
     }
   }
   return false;
+}
+
+// Does a row that a layer writes meet a Q or K row that it reads? (V passes through, vector by vector.) Bytes.
+bool writes_its_input(const RopeLayer& p, const RopeGeom& g, const CacheGeom* c, int64_t E) {
+  typedef __int128 Wide;  // a cache may be said to have any number of blocks
+  const auto rows = [&](int64_t stride, int64_t row) { return ((Wide)(g.num_tokens - 1) * stride + row) * E; };
+  const auto meet = [](const char* x, Wide x_bytes, const char* y, Wide y_bytes) {
+    const Wide bx = (uintptr_t)x, by = (uintptr_t)y;
+    return x && bx < by + y_bytes && by < bx + x_bytes;
+  };
+  const int64_t q_row = g.num_heads * g.head_dim, k_row = g.num_kv_heads * g.head_dim;
+  const auto meets_input = [&](const char* out, Wide bytes) {
+    return meet(out, bytes, p.query, rows(g.q_token_stride, q_row)) || meet(out, bytes, p.key, rows(g.k_token_stride, k_row));
+  };
+  return meets_input(p.query_out, rows(g.qo_token_stride, q_row)) ||
+         meets_input(p.key_out, rows(g.ko_token_stride, k_row)) ||
+         (c && c->num_cache_blocks > 0 &&
+          meets_input(p.key_cache, ((Wide)(c->num_cache_blocks - 1) * c->cache_block_stride +
+                                    (Wide)(c->block_size - 1) * c->cache_slot_stride + k_row) * E));
 }
 
 constexpr int kLayerByLayer = 1;  // run_rope: nothing launched, the layers' buffers do not suit one launch
@@ -707,8 +840,10 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
       c = nullptr;
     }
   }
+  bool in_place = writes_its_input(only_layer(a), g, c, E);
   for (int64_t l = 0; l < num_layers; ++l) {
     const RopeLayer& p = layers[l];
+    in_place = in_place || writes_its_input(p, g, c, E);
     in_align |= (uintptr_t)p.query | (uintptr_t)p.key | (uintptr_t)p.value;
     out_align |= (uintptr_t)p.query_out | (uintptr_t)p.key_out | (uintptr_t)p.key_cache | (uintptr_t)p.value_cache;
   }
@@ -732,10 +867,15 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
     // and 20.0, 31.1 and 29.0)
     const bool pairs = fast && g.rotary_dim == g.head_dim && v_items <= heads * a.pairs_per_head && half % 64 == 0 &&
                        out_align % 64 == 0 && !(half == 64 && g.num_tokens * heads * g.head_dim * E >= (int64_t(16) << 20));
-    form = pairs ? kPairs : kRows;
+    // In place the pair form stays, which reads no vector that another lane writes, and the owner form stands in for rows
+    const int64_t extras = v_items + heads * ((g.head_dim - g.rotary_dim) / ev), pair_lanes = heads * a.pairs_per_head;
+    form = pairs ? kPairs : !in_place || !g.rotary_dim ? kRows : extras > v_items || v_items > pair_lanes ? kOwnerTail : kOwner;
     if (pairs) {
       a.split = a.pairs_per_head;
-      a.lanes_per_token = (uint32_t)(heads * a.pairs_per_head);
+      a.lanes_per_token = (uint32_t)pair_lanes;
+    } else if (form != kRows) {
+      a.split = a.pairs_per_head;
+      a.lanes_per_token = (uint32_t)(form == kOwner ? pair_lanes : std::max(pair_lanes, (extras + 1) / 2));
     } else {
       a.split = (uint32_t)(g.head_dim / ev);
       a.head_step = (uint32_t)((heads + (c ? g.num_kv_heads : 0) + 1) / 2);

@@ -603,6 +603,48 @@ def test_element_path_in_every_form(gpu, T, Hq, Hkv, D, rd, dtype, bs, shift, wi
     assert torch.equal(k[:-1], k_out[:-1])
 
 
+# Heads whose two halves do not share a wavefront, or not a workgroup, where every 16-byte vector has a lane of its own
+@pytest.mark.parametrize("T,Hq,Hkv,D,rd,dtype", [
+    (3000, 32, 8, 96, 96, torch.bfloat16),
+    (3000, 32, 8, 80, 32, torch.float16),      # a rotated pair on either side of lane 192
+    (2000, 12, 3, 192, 192, torch.bfloat16),
+    (1500, 28, 4, 112, 112, torch.float16),
+    (600, 4, 2, 512, 512, torch.float32),      # halves of a wavefront each
+    (3300, 32, 8, 64, 64, torch.bfloat16),     # more than 16 MiB of rows with 64-byte halves
+    (700, 2, 6, 72, 16, torch.float32),        # most lanes pass through
+    (300, 2, 6, 64, 64, torch.bfloat16),       # more V vectors than pair-vectors
+])
+def test_rotation_in_its_own_rows_gives_the_bits_of_one_elsewhere(gpu, T, Hq, Hkv, D, rd, dtype):
+    bs, L = 16, 2
+    q, k, v, pos, cs = (t.to(gpu) for t in _case(gpu, T, Hq, Hkv, D, rd, dtype, max_pos=T + 9, seed=T + D))
+    nb = T // bs + 3
+    slots = torch.from_numpy(np.random.default_rng(T).permutation(nb * bs)[:T]).to(gpu)
+    pos[T // 3], slots[T // 2] = -1, -1
+    pool = torch.zeros(nb, 2, bs, Hkv, D, dtype=dtype, device=gpu)
+    index = torch.zeros(T, dtype=torch.int32, device=gpu)
+    plan = kvc.PagedRotaryWritePlan(index, pos, index[:1], torch.tensor([0, 1], dtype=torch.int32, device=gpu), index[:1],
+                                    cs, Hq, Hkv, D, bs, slots=slots)
+    q_out, k_out = q.clone(), k.clone()         # the token without a position keeps its rows
+    plan.run(q, k, v, pool, query_out=q_out, key_out=k_out)
+    some = [t for t in range(0, T, max(1, T // 300)) if t != T // 3]
+    for got, x, name in ((q_out, q, "query"), (k_out, k, "key")):
+        _check_rotation(got[some].cpu(), x[some].cpu(), pos[some].cpu(), cs.cpu(), D, dtype, name)
+
+    q_in, k_in, cache = q.clone(), k.clone(), torch.zeros_like(pool)
+    plan.run(q_in, k_in, v, cache, query_out=q_in, key_out=k_in)
+    assert torch.equal(q_in, q_out) and torch.equal(k_in, k_out) and torch.equal(cache, pool)
+    for wide in (pos, pos.long()):
+        q_in, k_in = q.clone(), k.clone()
+        _lib.check(_lib.lib().kvc_rotary_pos_emb(
+            q_in.data_ptr(), k_in.data_ptr(), wide.data_ptr(), wide.element_size(), cs.data_ptr(), T + 9, T, Hq, Hkv, D, rd,
+            Hq * D, Hkv * D, q_in.data_ptr(), k_in.data_ptr(), Hq * D, Hkv * D, rotary._DTYPES[dtype],
+            torch.cuda.current_stream().cuda_stream))
+        assert torch.equal(q_in, q_out) and torch.equal(k_in, k_out)
+    queries, caches = [q.clone() for _ in range(L)], torch.zeros(L, *pool.shape, dtype=dtype, device=gpu)
+    assert plan.run_layers(queries, [k] * L, [v] * L, list(caches), queries)
+    assert all(torch.equal(o, q_out) for o in queries) and all(torch.equal(c, pool) for c in caches)
+
+
 @pytest.mark.parametrize("L,T,Hq,Hkv,D,rd,dtype,bs,form", [
     (2, 1, 32, 8, 64, 64, torch.bfloat16, 16, "one"),
     (65, 7, 5, 3, 96, 96, torch.float16, 16, "one"),        # one layer more than a launch holds

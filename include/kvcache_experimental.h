@@ -191,6 +191,13 @@ int kvc_copy_blocks_host_pairs(void* kv_caches, const int64_t* pairs, int64_t nu
 int kvc_streams_share_hw_queue(void* stream_x, void* stream_y, int* shared);
 
 /*
+ * A new stream on the current device, of default priority, that does not wait for the
+ * null stream. Unlike a stream of a framework's pool it is held by the caller alone, so
+ * that no one else records it or queues work on it. It lives as long as the process.
+ */
+int kvc_stream_create(void** stream);
+
+/*
  * Host side of a one-layer swap to or from scattered host blocks, on host threads.
  * Serves
  *   _save_layer_kv_blocks_to_host     (runtime/worker/llm_worker/kv_worker.py:213-227)

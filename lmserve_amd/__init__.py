@@ -9,6 +9,7 @@
     disk_tier   DiskTier (host <-> block file, native positional I/O)
     kv_pool     pool sizing, layer-sync handle and model-side hooks, hand-over to a second process
     kv_service  the KV worker as a process of its own (pool mapped from an IPC handle)
+    streams     the streams of the KV worker and of a recording, held by no one else
     step_graph  KVWriteStep: fixed-capacity index buffers and plans, so that a step's index build
                 and per-layer writes can be recorded once into a hipGraph and replayed for later steps
 

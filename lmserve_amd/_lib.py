@@ -111,6 +111,7 @@ SIGNATURES = {
     "kvc_build_write_index_staged": (c_int, [_I64, _I64, _I64, _I64, _P, _P, _P, _P, _P, _P, _P, _P]),
     "kvc_slot_runs": (c_int, [_P, c_int, _I64, _I64, _P, _P, _I64, _P]),
     "kvc_streams_share_hw_queue": (c_int, [_P, _P, _P]),
+    "kvc_stream_create": (c_int, [ctypes.POINTER(_P)]),
     "kvc_write_runs_layers": (c_int, [_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64,
                                       _I64, _I64, _I64, _I64, _I64, _I64, c_int, _P]),
     "kvc_write_plan_set_slots": (c_int, [_P, _P]),
@@ -256,6 +257,13 @@ def get_tuning(key: str) -> int:
 
 def reset_tuning() -> None:
     check(lib().kvc_reset_tuning())
+
+
+def stream_create() -> int:
+    """Raw handle of a new stream on the current device; it lives as long as the process."""
+    out = c_void_p()
+    check(lib().kvc_stream_create(ctypes.byref(out)))
+    return out.value
 
 
 def streams_share_hw_queue(stream_x: int, stream_y: int) -> bool:

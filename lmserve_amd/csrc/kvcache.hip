@@ -2677,6 +2677,13 @@ int kvc_streams_share_hw_queue(void* stream_x, void* stream_y, int* shared) {
   return KVC_OK;
 }
 
+int kvc_stream_create(void** stream) {
+  if (!stream) return fail(KVC_ERR_INVALID_ARG, "kvc_stream_create: null result pointer");
+  *stream = nullptr;
+  KVC_HIP(hipStreamCreateWithFlags(reinterpret_cast<hipStream_t*>(stream), hipStreamNonBlocking));
+  return KVC_OK;
+}
+
 int kvc_slot_runs(const void* slot_mapping, int slot_bytes, int64_t num_tokens, int64_t block_size,
                   int32_t* runs, int32_t* num_runs, int64_t max_runs, void* stream) {
   if (num_tokens < 0 || block_size <= 0 || max_runs < 0 || num_tokens > 0x7fffffffll)

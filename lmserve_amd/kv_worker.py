@@ -47,7 +47,7 @@ from typing import Callable, Iterable, List, Optional, Sequence, Tuple
 import numpy as np
 import torch
 
-from . import _lib
+from . import _lib, streams
 from .disk_tier import DiskTier
 
 
@@ -319,7 +319,7 @@ class KVWorker:
       found them is `streams_have_own_queues`; if not it warns once: with the
       runtime's default of 4 hardware queues a process that already runs many
       streams may have none left, `GPU_MAX_HW_QUEUES=8` helps.
-    own_queues: False takes the two streams as torch hands them out, as the
+    own_queues: False takes the two streams as they come, as the
       reference does, without looking at their queues (for measurements).
     validate: check on the host that no block is the destination of two pairs of
       one GPU<->Host call (`ValueError`). The reference copies the pairs one
@@ -407,13 +407,22 @@ class KVWorker:
         with torch.cuda.device(self.device):
             if model_streams is None:
                 model_streams = [torch.cuda.current_stream(self.device)]
+            drawn = []
+
+            def draw():
+                drawn.append(streams.take(self.device))
+                return drawn[-1]
             if own_queues:
                 (self.dtoh_stream, self.htod_stream), self.streams_have_own_queues = pick_streams_apart(
-                    2, list(model_streams), torch.cuda.Stream,
+                    2, list(model_streams), draw,
                     lambda a, b: _lib.streams_share_hw_queue(a.cuda_stream, b.cuda_stream))
             else:
-                self.dtoh_stream, self.htod_stream = torch.cuda.Stream(), torch.cuda.Stream()
+                self.dtoh_stream, self.htod_stream = draw(), draw()
                 self.streams_have_own_queues = True    # not looked at: nothing to warn about
+            mine = (self.dtoh_stream, self.htod_stream)
+            streams.give_back(s for s in drawn if s not in mine)
+            self._give_streams_back = weakref.finalize(self, streams.give_back, mine)
+            self._give_streams_back.atexit = False
         self._staging = {}   # (direction, stream handle) -> [workspace, weak reference to its PreparedSwap]
         self.kv_worker_handle = kv_worker_handle
         if not self.streams_have_own_queues:
@@ -817,6 +826,7 @@ class KVWorker:
                 self._bounce[direction] = None
         self._host_pool.close()
         self._staging = {}
+        self._give_streams_back()
         # let go of the pool now: the direction table holds bound methods, so the
         # worker is part of a reference cycle and would otherwise keep tens of GiB
         # of HBM alive until the cycle collector runs

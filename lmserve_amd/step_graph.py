@@ -30,7 +30,7 @@ from typing import Optional, Sequence
 import numpy as np
 import torch
 
-from . import _lib
+from . import _lib, streams
 from .index_prep import InferInput
 from .paged import BlockRuns, PagedKVWritePlan, build_write_index, max_block_runs
 from .rotary import PagedRotaryWritePlan
@@ -198,8 +198,9 @@ class KVWriteStep:
                 else:
                     self.rotate_and_append(queries[l], k, v, c,
                                            query_out=query_outs[l] if query_outs is not None else None)
-        with torch.cuda.device(self.device):
-            side = torch.cuda.Stream()
+        # a stream that no other thread holds: what one queues on the stream that is recorded would be recorded with
+        # it, and a query of its event there breaks the recording
+        with torch.cuda.device(self.device), streams.recording_stream(self.device) as side:
             side.wait_stream(torch.cuda.current_stream())
             with torch.cuda.stream(side):
                 body()
@@ -208,6 +209,6 @@ class KVWriteStep:
             graph = torch.cuda.CUDAGraph()
             # thread-local capture: a KV worker's threads (row mover, notifier) may
             # query events and enqueue copies on their own streams meanwhile
-            with torch.cuda.graph(graph, capture_error_mode="thread_local"):
+            with torch.cuda.graph(graph, stream=side, capture_error_mode="thread_local"):
                 body()
         return graph

@@ -560,6 +560,10 @@ def test_queue_sharing_query_without_a_launch():
     assert _lib.streams_share_hw_queue(0, 0) is True
 
 
+def test_a_stream_needs_somewhere_to_go():
+    assert _lib.lib().kvc_stream_create(None) == _lib.KVC_ERR_INVALID_ARG
+
+
 def test_calls_without_pinned_memory_take_the_unstaged_path(tmp_path):
     """The native readers hand a step back (1) where no staging buffer can be had; a stub in front of the library
     says so, and stands in for the runtime's queries of the current device and stream."""

@@ -307,3 +307,34 @@ def test_a_step_is_recorded_while_another_thread_works_on_its_own_stream(gpu):
                                     [b for r in rs for b in r.block_ids], index[1])
     assert np.array_equal(bits_of(dpool), want)
     _check_index(step, rs, index, padded)
+
+
+def test_recordings_and_workers_have_streams_that_torchs_pool_does_not_hand_out(gpu):
+    """`torch.cuda.Stream()` comes round after 32 streams; none of them may be one that a step is recorded on or a KV
+    worker copies on. Streams come back when a recording or a worker is done with them, unless the recording failed."""
+    from lmserve_amd import streams
+
+    pool = {torch.cuda.Stream().cuda_stream for _ in range(64)}
+    step = KVWriteStep(2, 8, 4, torch.bfloat16, gpu, max_requests=2, max_tokens=2, max_block_ids=4)
+    step.set_arrays([1], [3], [1], [2])
+    kv = torch.zeros(2, 2, 8, dtype=torch.bfloat16, device=gpu)
+    cache = torch.zeros(4, 2, 4, 2, 8, dtype=torch.bfloat16, device=gpu)
+    seen = []
+    step.append = lambda *a: (seen.append(torch.cuda.current_stream().cuda_stream), KVWriteStep.append(step, *a))
+    for _ in range(3):
+        step.capture([kv], [kv], [cache]).replay()
+    workers = [kvc.KVWorker(cache.unsqueeze(0), 2, own_queues=own) for own in (True, False)]
+    held = [s.cuda_stream for w in workers for s in (w.dtoh_stream, w.htod_stream)]
+    assert len(set(held)) == 4 and not pool & set(seen + held)
+    for w in workers:
+        w.close()
+    free = {s.cuda_stream for s in streams._free[gpu.index]}
+    assert free >= set(seen + held)
+    for _ in range(3):
+        kvc.KVWorker(cache.unsqueeze(0), 2, own_queues=False).close()
+    assert {s.cuda_stream for s in streams._free[gpu.index]} == free
+    with pytest.raises(RuntimeError):
+        with streams.recording_stream(gpu) as failed:
+            raise RuntimeError
+    assert failed.cuda_stream not in {s.cuda_stream for s in streams._free[gpu.index]}
+    torch.cuda.synchronize()

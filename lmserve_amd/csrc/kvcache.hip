@@ -1269,7 +1269,6 @@ int run_write(const char* fn, const void* key, const void* value, void* kc, void
       return fail(KVC_ERR_INVALID_ARG, "%s: null index array", fn);
     if (batch_size < 0 || num_kv_indices < 0)
       return fail(KVC_ERR_INVALID_ARG, "%s: negative batch_size/num_kv_indices", fn);
-    if (batch_size == 0 || num_kv_indices == 0) return KVC_OK;  // every token is skipped; find_slot counts on both
   } else {
     if (!slot_mapping) return fail(KVC_ERR_INVALID_ARG, "%s: null slot_mapping", fn);
     if (slot_bytes != 4 && slot_bytes != 8)
@@ -1309,6 +1308,7 @@ int run_write(const char* fn, const void* key, const void* value, void* kc, void
   if (items64 > 0x7fffffffll)
     return fail(KVC_ERR_UNSUPPORTED, "%s: %lld vectors per token exceed 2^31", fn, (long long)items64);
   a.items_per_token = (uint32_t)items64;
+  if (paged && (batch_size == 0 || num_kv_indices == 0)) return KVC_OK;  // every token is skipped; find_slot counts on both
   // Small launches store the rows at device scope, so that nothing is left to write back when they end; larger ones
   // lose by it (one layer, rows of 2 KiB, us, non-temporal and through: 256 tokens by slot 2.55 and 2.36, by page
   // table 2.65 and 2.57; 838 3.25 and 3.42, 3.48 and 3.23; 2048 4.5 and 5.2, 4.56 and 4.98; 256-byte rows, 3000 tokens

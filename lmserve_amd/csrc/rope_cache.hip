@@ -835,10 +835,6 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
     in_align |= (uintptr_t)value | (uint64_t)a.v_token_stride;
     out_align |= (uintptr_t)c->key_cache | (uintptr_t)c->value_cache | (uint64_t)a.cache_block_stride |
                  (uint64_t)a.cache_slot_stride;
-    if (c->batch_indices && (c->batch_size == 0 || c->num_kv_indices == 0)) {  // the write skips every token
-      a.key_cache = nullptr;
-      c = nullptr;
-    }
   }
   bool in_place = writes_its_input(only_layer(a), g, c, E);
   for (int64_t l = 0; l < num_layers; ++l) {
@@ -908,6 +904,10 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
   if (g.num_tokens * (int64_t)a.groups_per_token > 0x7fffffffll)
     return fail(KVC_ERR_UNSUPPORTED, "%s: launch of %lld workgroups is too large", fn,
                 (long long)(g.num_tokens * (int64_t)a.groups_per_token));
+  if (c && c->batch_indices && (c->batch_size == 0 || c->num_kv_indices == 0)) {  // the write skips every token
+    a.key_cache = nullptr;
+    a.v_items = 0;
+  }
   hipStream_t s = (hipStream_t)stream;
   if (layers) {
     if (form == kElements || !c->slot_mapping || c->slot_bytes != 8 || pos_bytes != 4 || a.bs_shift < 0 ||

@@ -560,6 +560,21 @@ def test_queue_sharing_query_without_a_launch():
     assert _lib.streams_share_hw_queue(0, 0) is True
 
 
+def test_what_is_refused_is_refused_without_requests_too():
+    """Sizes beyond the limits are named whether or not the page table has anything to write; nothing is launched on
+    these addresses."""
+    L, at = _lib.lib(), 1 << 30
+    for batch, ids in ((0, 0), (0, 4), (4, 0), (4, 4)):
+        rc = L.kvc_append_paged_kv_cache_layers(at, at, at, at, at, at, at, at, 1, batch, ids, 8192, 128, 16, 8192 * 128,
+                                                8192 * 128, 32 * 8192 * 128, 4, 32767, 0, 0, 0, 2, None)
+        assert rc == _lib.KVC_ERR_UNSUPPORTED and b"2^31" in L.kvc_last_error_string()
+        q, k, v, q_out, k_out, pool = (i << 44 for i in range(1, 7))      # further apart than the rows reach
+        rc = L.kvc_rotary_pos_emb_and_append_paged(q, k, v, at, at, at, 9, 2**31 - 1, 16, 16, 112, 112, 1792, 1792, 1792,
+                                                   q_out, k_out, 1792, 1792, pool, at, at, batch, ids, 16, 32 * 1792, 4,
+                                                   _lib.KVC_DTYPE_BF16, None)
+        assert rc == _lib.KVC_ERR_UNSUPPORTED and b"too large" in L.kvc_last_error_string()
+
+
 def test_a_stream_needs_somewhere_to_go():
     assert _lib.lib().kvc_stream_create(None) == _lib.KVC_ERR_INVALID_ARG
 

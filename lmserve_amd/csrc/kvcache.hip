@@ -582,10 +582,11 @@ __global__ __launch_bounds__(kThreads) void copy_to_host_kernel(TileArgs a) {
 // without). Both loads at once with 5 to a CU, non-temporal stores -> this, stores
 // through the L2 (us): copy of 300 blocks of 2 MiB 208 -> 202, of 2048 1419 -> 1400; gather
 // and scatter of 100 x 2 MiB 124.5 -> 119.5, of 600 829 -> 784, of 256 x 5 MiB 858 -> 830.
-// Up to 128 MiB a copy reads its sources with plain loads: blocks that are copied on write
-// have just been read, and of 200 x 12 layers of 18 KiB that the last-level cache holds a
-// copy takes 14.7 us instead of 18.6, of 20 x 80 of 8 KiB 5.2 instead of 6.2; where it does
-// not it is the same, and from there on non-temporal loads are 1 % faster.
+// Loads are non-temporal throughout. Plain loads of a copy's sources find a little more of
+// them in the last-level cache (12 layers of 18 KiB, 200 blocks just read: 4 % less), but
+// where it is full of other kernels' dirty lines they push those out: 200 x 80 of 8 KiB
+// 50 -> 75 us, 60 x 32 of 64 KiB 53 -> 71. A scatter's dense side, just written, is the
+// exception.
 struct StreamArgs {
   const char* src_base;
   char* dst_base;
@@ -644,9 +645,8 @@ __global__ __launch_bounds__(THREADS) void stream_tiles_kernel(StreamArgs a) {
       a, [&](uint32_t i) { return a.src_ids ? a.src_ids[(int64_t)i * a.id_stride] : (int64_t)i; },
       [&](uint32_t i) { return a.dst_ids ? a.dst_ids[(int64_t)i * a.id_stride] : (int64_t)i; });
 }
-template <bool NTL>
 __global__ __launch_bounds__(kThreads) void stream_pairs_kernel(StreamArgs a, PairList p) {
-  stream_tile_chunk<kThreads, 2, NTL, true>(
+  stream_tile_chunk<kThreads, 2, true, true>(
       a, [&](uint32_t i) { return (int64_t)p.id[2 * i]; }, [&](uint32_t i) { return (int64_t)p.id[2 * i + 1]; });
 }
 
@@ -1620,19 +1620,18 @@ int launch_stream(const TileArgs& t, TileSides sides, int64_t n, hipStream_t s, 
   // touches as many far-apart pages (8 KiB x 80 layers: 4000 blocks 5.05 -> 5.2 TB/s, 300 blocks 4.85 -> 5.3;
   // from 32 KiB on it makes no difference, and a dense side wants its own order: gather 6.2 -> 5.1).
   a.layer_slowest = sides == TileSides::kPools && t.tile_bytes < (32 << 10);
-  const int64_t bytes = n * (int64_t)a.num_layers * t.tile_bytes, llc = int64_t(256) << 20;
-  const bool plain_load = (sides == TileSides::kScatter && bytes <= llc) || (sides == TileSides::kPools && bytes <= llc / 2);
-  const bool plain_store = gather && bytes <= llc;
+  const bool dense_cached = n * (int64_t)a.num_layers * t.tile_bytes <= (int64_t(256) << 20);
+  const bool plain_load = sides == TileSides::kScatter && dense_cached;
+  const bool plain_store = gather && dense_cached;
   const dim3 grid(a.total_chunks), block(threads);
   const unsigned six_per_cu = (int64_t)a.total_chunks > resident_workgroups() ? 160 * 1024 / 6 : 0;
-  if (pairs && plain_load) kvc::launch((stream_pairs_kernel<false>), grid, block, six_per_cu, s, a, *pairs);
-  else if (pairs) kvc::launch((stream_pairs_kernel<true>), grid, block, six_per_cu, s, a, *pairs);
+  if (pairs) kvc::launch(stream_pairs_kernel, grid, block, six_per_cu, s, a, *pairs);
   else if (gather && plain_store) kvc::launch((stream_tiles_kernel<64, 1, true, false>), grid, block, 0, s, a);
   else if (gather) kvc::launch((stream_tiles_kernel<64, 1, true, true>), grid, block, 0, s, a);
   else if (plain_load) kvc::launch((stream_tiles_kernel<256, 2, false, true>), grid, block, six_per_cu, s, a);
   else kvc::launch((stream_tiles_kernel<256, 2, true, true>), grid, block, six_per_cu, s, a);
   g_last = LastLaunch{KVC_KERNEL_COPY_TILES, 16, (int64_t)unroll, (int64_t)threads, (int64_t)a.total_chunks,
-                      plain_store || (plain_load && sides == TileSides::kScatter) ? 0 : 1};
+                      plain_load || plain_store ? 0 : 1};
   KVC_HIP(hipGetLastError());
   return KVC_OK;
 }

@@ -158,12 +158,12 @@ int kvc_rotary_plan_run_layers(const kvc_rotary_plan* plan, int64_t num_layers, 
 
 /*
  * kvc_copy_blocks on a pair list in host memory, [src, dst] * num_pairs, read before the
- * call returns; nothing waits for the device. Pairs of one source that follow each other
- * are read once for up to 3 destinations (7 where sources have many). Up to 448 pairs, or
- * 224 sources with their destinations, travel in the launch's own arguments (16-byte
- * aligned blocks); any other list is staged as above into `scratch` (16 * num_pairs bytes
- * of device memory, 16-byte aligned, in use until the copy has run). With a NULL scratch
- * such a list is refused with KVC_ERR_STAGING, nothing launched.
+ * call returns; nothing waits for the device. Up to 448 pairs travel in the launch's own
+ * arguments (16-byte aligned blocks); any other list is staged as above into `scratch`
+ * (16 * num_pairs bytes of device memory, 16-byte aligned, in use until the copy has run).
+ * With a NULL scratch such a list is refused with KVC_ERR_STAGING, nothing launched. Where
+ * enough pairs follow another of the same source, that source is read once for up to 3 of
+ * its destinations (7 where sources have many).
  */
 int kvc_copy_blocks_host_pairs(void* kv_caches, const int64_t* pairs, int64_t num_pairs, int64_t* scratch,
                                int64_t num_layers, int64_t layer_stride_bytes, int64_t block_bytes,

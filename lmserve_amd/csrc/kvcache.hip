@@ -2766,52 +2766,67 @@ static int stage_list(const void* list, int64_t bytes, void* to, void* stream) {
   return KVC_OK;
 }
 
-// Pairs of one source that follow each other, as items for the fan kernels. kNotInline where no source has two pairs
-// in a row, or the copy is not for those kernels.
+// Pairs of one source that follow each other, as items for the fan kernels. kNotInline where the copy is not for those
+// kernels: too few of its pairs share a source, or the pairs travel with the launch and the items would not.
 static int run_fan_copy(char* pool, const int64_t* pairs, int64_t num_pairs, int64_t* scratch, int64_t num_layers,
                         int64_t layer_stride_bytes, int64_t block_bytes, int64_t num_blocks, hipStream_t s) {
-  bool several = false;
-  for (int64_t i = 1; i < num_pairs && !several; ++i) several = pairs[2 * i] == pairs[2 * i - 2];
-  if (!several || num_blocks > INT32_MAX || num_pairs > (1 << 28) || num_layers > INT32_MAX ||
-      block_bytes > (int64_t(1) << 30) || !g_tune.copy_nt || g_tune.copy_unroll || g_tune.copy_order ||
-      g_tune.copy_max_wgs > 0 ||
+  const bool inline_pairs = num_pairs <= kInlinePairs;
+  if (!inline_pairs && (!scratch || (uintptr_t)scratch % 16)) return kNotInline;  // the caller says what is wrong
+  if (num_blocks > INT32_MAX || num_pairs > (1 << 28) || num_layers > INT32_MAX || block_bytes > (int64_t(1) << 30) ||
+      !g_tune.copy_nt || g_tune.copy_unroll || g_tune.copy_order || g_tune.copy_max_wgs > 0 ||
       common_vec({(uint64_t)(uintptr_t)pool, (uint64_t)layer_stride_bytes, (uint64_t)block_bytes}) != 16)
     return kNotInline;
-  std::vector<int32_t> list;
   // a pair with an id outside the pool, or onto itself, copies nothing
   const auto copies = [&](int64_t i) {
     const int64_t from = pairs[2 * i], to = pairs[2 * i + 1];
     return from >= 0 && from < num_blocks && to >= 0 && to < num_blocks && from != to;
   };
-  const auto fill = [&](int fan) {
-    list.clear();
-    int64_t last = -1;
-    int held = fan;
-    for (int64_t i = 0; i < num_pairs; ++i) {
-      if (!copies(i)) continue;
-      if (pairs[2 * i] != last || held == fan) {
-        list.resize(list.size() + fan + 1, -1);
-        list[list.size() - fan - 1] = (int32_t)(last = pairs[2 * i]);
-        held = 0;
-      }
-      list[list.size() - fan + held++] = (int32_t)pairs[2 * i + 1];
-    }
-    return (int64_t)list.size() / (fan + 1);
-  };
+  int64_t live = 0, items3 = 0, items7 = 0, last = -1;
+  int held = 0;  // destinations of `last` so far, over the least common multiple of the two fans
+  for (int64_t i = 0; i < num_pairs; ++i) {
+    if (!copies(i)) continue;
+    ++live;
+    if (pairs[2 * i] != last) last = pairs[2 * i], held = 0;
+    items3 += held % 3 == 0;
+    items7 += held % 7 == 0;
+    held = held == 20 ? 0 : held + 1;
+  }
+  if (items3 == live) return kNotInline;
   // Up to 3 destinations an item, or up to 7 where that leaves less than half as many items.
-  int fan = 3;
-  int64_t items;
+  const int fan = items7 * 2 < items3 ? 7 : 3;
+  const int64_t items = fan == 7 ? items7 : items3, words = items * (fan + 1);
+  if (words > kFanWords && inline_pairs) return kNotInline;
+  // What few doubled sources save does not make up for the pairs' better form (a list of pairs and items, us; half,
+  // a quarter and 1 % of the pairs are of sources with two): beyond one resident set 600 pairs x 32 of 64 KiB 418 and
+  // 415, 418 and 460, 418 and 504, 200 x 4 of 128 KiB 38 and 41, 38 and 45, 39 and 49; within it 24 x 32 of 64 KiB 21.3 and 19.9, 21.4 and 21.1,
+  // 21.6 and 21.8; 20 x 80 of 8 KiB 9.2 and 9.0, 9.4 and 9.4, 9.3 and 9.6.
+  const FanShape shape = fan_shape(items, num_layers, block_bytes);
+  if (!shape.unroll || (shape.large ? items * 10 > live * 7 : items * 16 > live * 15)) return kNotInline;
+  if (!inline_pairs) {  // a list that is staged is refused while the stream is recorded, also where its items are few
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) {
+      (void)hipGetLastError();
+      return kNotInline;
+    }
+  }
+  std::vector<int32_t> list;
   try {
-    items = fill(3);
-    const int64_t with3 = items;
-    if (fill(7) * 2 < with3) fan = 7, items = (int64_t)list.size() / 8;
-    else fill(3);
+    list.assign((size_t)words, -1);
   } catch (const std::bad_alloc&) {
     return kNotInline;
   }
-  if (items == 0) return KVC_OK;
-  const FanShape shape = fan_shape(items, num_layers, block_bytes);
-  if (!shape.unroll) return kNotInline;
+  int32_t* word = list.data() - (fan + 1);
+  last = -1;
+  held = fan;
+  for (int64_t i = 0; i < num_pairs; ++i) {
+    if (!copies(i)) continue;
+    if (pairs[2 * i] != last || held == fan) {
+      word += fan + 1;
+      word[0] = (int32_t)(last = pairs[2 * i]);
+      held = 0;
+    }
+    word[++held] = (int32_t)pairs[2 * i + 1];
+  }
   StreamArgs a{};
   a.src_base = pool;
   a.dst_base = pool;
@@ -2821,13 +2836,11 @@ static int run_fan_copy(char* pool, const int64_t* pairs, int64_t num_pairs, int
   a.src_layer_stride = a.dst_layer_stride = layer_stride_bytes;
   a.src_block_stride = a.dst_block_stride = block_bytes;
   a.num_src_blocks = a.num_dst_blocks = num_blocks;
-  const int64_t words = (int64_t)list.size();
   if (words <= kFanWords) {
     FanList inline_list;
     std::copy(list.begin(), list.end(), inline_list.word);
     return launch_fan_copy(a, shape, fan, &inline_list, nullptr, s);
   }
-  if (!scratch || (uintptr_t)scratch % 16) return kNotInline;  // the caller says what is wrong
   // at most 16 bytes a pair, which scratch holds: an item of 4 words has a pair, and items of 8 are fewer than half
   // as many as those of 4
   const int rc = stage_list(list.data(), words * (int64_t)sizeof(int32_t), scratch, s);

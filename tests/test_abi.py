@@ -575,6 +575,15 @@ def test_what_is_refused_is_refused_without_requests_too():
         assert rc == _lib.KVC_ERR_UNSUPPORTED and b"too large" in L.kvc_last_error_string()
 
 
+def test_a_list_beyond_the_launchs_arguments_needs_scratch():
+    """Also where its pairs share few sources; nothing is launched."""
+    L, at = _lib.lib(), 1 << 30
+    pairs = np.stack([np.repeat(np.arange(100), 5), np.arange(100, 600)], axis=1).astype(np.int64)
+    for scratch, want in ((None, _lib.KVC_ERR_STAGING), (at + 8, _lib.KVC_ERR_INVALID_ARG)):
+        rc = L.kvc_copy_blocks_host_pairs(at, pairs.ctypes.data, 500, scratch, 2, 600 * 4096, 4096, 600, None)
+        assert rc == want
+
+
 def test_a_stream_needs_somewhere_to_go():
     assert _lib.lib().kvc_stream_create(None) == _lib.KVC_ERR_INVALID_ARG
 

@@ -299,6 +299,66 @@ def test_copies_of_blocks_with_several_destinations(gpu, tile_bytes, L, fans, pe
     assert np.array_equal(bits_of(dlist), pool)
 
 
+@pytest.mark.parametrize("tile_bytes,L,fans,per_lane", [
+    (8192, 30, (1,) * 540 + (2,) * 30, 2),       # beyond one resident set: one pair in ten is not worth the fan form,
+    (8192, 30, (1,) * 250 + (2,) * 175, 2),      # nor more than half; at 7 items for 10 pairs
+    (8192, 30, (1,) * 240 + (2,) * 180, 1),      # it is
+    (65536, 50, (1,) * 14 + (2,), 8),            # within it 15 items for 16 pairs are enough,
+    (65536, 50, (1,) * 15 + (2,), 16),           # 16 for 17 not
+    (65536, 2, (1,) * 200 + (2,) * 60, 16),      # pairs that travel with the launch, and more items than would
+])
+def test_the_fan_form_is_taken_where_enough_pairs_share_a_source(gpu, tile_bytes, L, fans, per_lane):
+    n = sum(fans)
+    nb = n + len(fans) + 1
+    pool = random_pool((L, nb, tile_bytes // 2), seed=n)
+    dpool = to_bf16(pool, gpu)
+    ids = np.random.default_rng(n).permutation(nb).tolist()
+    d, at = {}, len(fans)
+    for i, src in zip(np.random.default_rng(1).permutation(len(fans)), ids):
+        d[src] = ids[at:at + fans[i]]
+        at += fans[i]
+    for src, dsts in d.items():
+        pool[:, dsts] = pool[:, src:src + 1]
+    kvc.copy_blocks(dpool, d)
+    assert _lib.last_launch()["per_lane"] == per_lane
+    assert np.array_equal(bits_of(dpool), pool)
+
+
+def test_pairs_that_travel_with_the_launch_are_recorded_with_or_without_scratch(gpu):
+    """300 pairs of which two share a source, and scratch at hand: nothing of the list may be left to a staging buffer
+    that a replay would read again."""
+    n, L, elems = 300, 2, 4096
+    nb = 2 * n
+    pool = random_pool((L, nb, elems), seed=5)
+    dpool = to_bf16(pool, gpu)
+    ids = np.random.default_rng(5).permutation(nb)
+    pairs = np.stack([ids[:n], ids[n:]], axis=1).astype(np.int64)
+    pairs[8, 0] = pairs[7, 0]
+    scratch = torch.zeros(2 * n, dtype=torch.int64, device=gpu)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        _lib.check(_lib.lib().kvc_copy_blocks_host_pairs(
+            dpool.data_ptr(), pairs.ctypes.data, n, scratch.data_ptr(), L, nb * elems * 2, elems * 2, nb,
+            torch.cuda.current_stream().cuda_stream))
+    kept, at = pairs.copy(), dpool.clone()
+    pairs[:] = 0
+    for rep in range(3):
+        scratch.fill_(rep)
+        dpool.copy_(at)
+        graph.replay()
+        torch.cuda.synchronize()
+        want = pool.copy()
+        want[:, kept[:, 1]] = want[:, kept[:, 0]]
+        assert np.array_equal(bits_of(dpool), want)
+    with torch.cuda.graph(torch.cuda.CUDAGraph()):     # a longer list is refused there, also where its items are few
+        long = np.stack([np.repeat(ids[:100], 5), np.resize(ids[100:], 500)], axis=1).astype(np.int64)
+        rc = _lib.lib().kvc_copy_blocks_host_pairs(
+            dpool.data_ptr(), long.ctypes.data, 500, torch.zeros(1000, dtype=torch.int64, device=gpu).data_ptr(), L,
+            nb * elems * 2, elems * 2, nb, torch.cuda.current_stream().cuda_stream)
+        assert rc == _lib.KVC_ERR_UNSUPPORTED
+        torch.zeros(4, device=gpu).add_(1)
+
+
 @pytest.mark.parametrize("block_bytes,n,per_lane,grid", [
     (1 << 20, 131071, 2, 131071 * 128),                # the largest that the stream kernel takes: 2^32 - 2^15 lanes
     (1 << 20, 131073, 2, (2**32 - 1) // 256),          # past it: chunks walked grid-stride

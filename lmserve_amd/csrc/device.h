@@ -11,7 +11,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // Store policies: the cache bits of the instruction. What a kernel leaves dirty in the L2s of the 8 XCDs is written
 // back when it ends; a store at device scope is written through to the last-level cache, where a reader on any
-// XCD finds it. The non-temporal forms are for rows that nothing reads soon.
+// XCD finds it. The non-temporal forms are for more rows than the caches would hold for their next reader.
 enum StorePolicy : int { kPlain = 0, kNonTemporal = 2, kThrough = 16, kThroughNt = 16 | 2 };
 
 // A run of bytes that one workgroup writes, `base` and `bytes` uniform over it. A store at or past `bytes` is dropped by
@@ -28,10 +28,10 @@ struct OutRow {
   }
 };
 
-// The same for addresses that differ from lane to lane by more than an offset: 16 bytes, kThroughNt. The two wait
+// The same for addresses that differ from lane to lane by more than an offset: 16 bytes, kThrough. The two wait
 // states behind the store keep a later instruction off its data registers.
-__device__ __forceinline__ void st_through_nt(char* p, u32x4 v) {
-  asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
+__device__ __forceinline__ void st_through(char* p, u32x4 v) {
+  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
 }
 
 // A kernel launch whose arguments go straight to the runtime. The launch by <<<>>> and its macro first store the

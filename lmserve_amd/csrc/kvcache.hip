@@ -204,12 +204,12 @@ __device__ __forceinline__ void st(V* p, V v) {
   else *p = v;
 }
 
-// One vector of a cache row; `through`: at device scope (kvc::st_through_nt), 16-byte vectors only.
+// One vector of a cache row; `through`: at device scope (kvc::st_through), 16-byte vectors only.
 template <bool NT, typename V>
 __device__ __forceinline__ void st_row(char* p, V v, bool through) {
   if constexpr (NT && sizeof(V) == 16) {
     if (through) {
-      kvc::st_through_nt(p, v);
+      kvc::st_through(p, v);
       return;
     }
   }
@@ -1312,7 +1312,9 @@ int run_write(const char* fn, const void* key, const void* value, void* kc, void
   // Small launches store the rows at device scope, so that nothing is left to write back when they end; larger ones
   // lose by it (one layer, rows of 2 KiB, us, non-temporal and through: 256 tokens by slot 2.55 and 2.36, by page
   // table 2.65 and 2.57; 838 3.25 and 3.42, 3.48 and 3.23; 2048 4.5 and 5.2, 4.56 and 4.98; 256-byte rows, 3000 tokens
-  // 2.65 and 2.46)
+  // 2.65 and 2.46). Not non-temporal: the same alone, and a reader of the rows finds them sooner (launch with a gather
+  // of its rows behind it, plain non-temporal, through and non-temporal, through: 1 token of 256 bytes 3.5, 4.0, 3.8; 8
+  // tokens 11.3, 11.7, 9.4; 512 of 2 KiB 5.6, 5.7, 5.3)
   a.through = g.num_tokens * items64 * vec <= (int64_t(2) << 20) << (paged ? 1 : 0);
 
   // The plane kernel (lanes over consecutive tokens of one (layer, K|V) plane)

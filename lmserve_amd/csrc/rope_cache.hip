@@ -165,6 +165,7 @@ struct RopeArgs {
   uint32_t split_magic;       // ceil(2^32 / split): lane / split = mulhi(lane, magic); 0 where that is not exact
   uint32_t head_step;         // rows kernel: heads between a lane's two
   uint32_t v_items;           // 16-byte vectors of the token's V row (0 without a cache)
+  uint32_t cache_nt;          // pair form: cache rows by non-temporal stores
 };
 
 // One layer's buffers, as RopeArgs names them
@@ -250,17 +251,22 @@ __device__ __forceinline__ uint32_t head_of_lane(const RopeArgs& a, uint32_t lan
 //   - nothing waits for the position before the Q, K and V loads are issued;
 //   - an instantiation holds only the code its launch needs: every addressing form
 //     and 64-bit divisions in one kernel cost a decode launch 15 %.
-// query_out is stored at device scope, the cache rows the same and non-temporal. What
-// plain stores leave dirty in the L2s is written back when the launch ends, and a reader,
-// mostly on another XCD, finds it in the last-level cache either way. Launch of a recorded
-// step alone, and with a copy of query_out behind it, plain and non-temporal stores -> these
-// (us): 256 tokens x 40 heads x 128 3.10 -> 2.80 and 5.55 -> 5.20; 1024 of those 5.87 ->
-// 5.38 and 9.57 -> 9.20; 2048 x 32 x 128 8.45 -> 7.74 and 13.72 -> 13.13; 2048 x 72 x 128
-// 17.15 -> 16.61 and 27.44 -> 26.79; 8192 of those 59.4 -> 58.1 (5.8 TB/s) and 124 -> 120.5.
-// Non-temporal query_out is faster still alone and costs its reader more (1024 tokens 5.21
-// and 10.07; 2048 x 72 14.24 and 30.02). Stores at device scope of pieces that are
-// no whole 64 bytes lose (2048 x 15 x 96 in bf16, halves of 96 bytes, 4.68 -> 5.16): such
-// heads, and outputs that start within 64 bytes, go to the rows kernel.
+// query_out is stored at device scope, the cache rows the same, and non-temporal beyond
+// 3 MiB of them. What plain stores leave dirty in the L2s is written back when the launch
+// ends, and a reader, mostly on another XCD, finds it in the last-level cache either way.
+// Launch of a recorded step alone, and with a copy of query_out behind it, plain and
+// non-temporal stores -> these (us): 256 tokens x 40 heads x 128 3.10 -> 2.80 and 5.55 ->
+// 5.20; 1024 of those 5.87 -> 5.38 and 9.57 -> 9.20; 2048 x 32 x 128 8.45 -> 7.74 and 13.72
+// -> 13.13; 2048 x 72 x 128 17.15 -> 16.61 and 27.44 -> 26.79; 8192 of those 59.4 -> 58.1
+// (5.8 TB/s) and 124 -> 120.5. Non-temporal query_out is faster still alone and costs its
+// reader more (1024 tokens 5.21 and 10.07; 2048 x 72 14.24 and 30.02). So do few cache rows,
+// non-temporal -> not, alone and with a gather of the rows behind the launch, in pools that no
+// cache holds: 1 token of 28 + 4 heads x 128 2.17 -> 2.19 and 4.46 -> 4.17, 512 2.78 -> 2.77
+// and 5.69 -> 5.40, 1024 (2 MiB) 4.79 -> 4.53 and 7.64 -> 6.95; 2048 (4 MiB) 7.24 -> 7.19 and
+// 10.6 -> 10.8, of 32 + 8 x 64 5.55 -> 5.80 and 8.84 -> 8.78; 4096 of 32 + 32 x 128 34.7 -> 39.5
+// alone. Stores at device scope of pieces that are no whole 64 bytes lose (2048 x 15 x 96 in
+// bf16, halves of 96 bytes, 4.68 -> 5.16): such heads, and outputs that start within 64 bytes,
+// go to the rows kernel.
 // NTL: non-temporal loads, bit 0 for the K and V rows, bit 1 for the Q rows.
 template <typename T, Addressing ADDR, int NTL>
 __device__ __forceinline__ void rope_pairs_lane(const RopeArgs& a, const RopeLayer p) {
@@ -316,11 +322,20 @@ __device__ __forceinline__ void rope_pairs_lane(const RopeArgs& a, const RopeLay
     }
     if (ADDR != kNoCache && slot >= 0) {
       const OutRow out(p.key_cache + slot, kv_bytes);
-      out.store<kvc::kThroughNt>(head_off, ox);
-      out.store<kvc::kThroughNt>(head_off + half, oy);
+      if (a.cache_nt) {
+        out.store<kvc::kThroughNt>(head_off, ox);
+        out.store<kvc::kThroughNt>(head_off + half, oy);
+      } else {
+        out.store<kvc::kThrough>(head_off, ox);
+        out.store<kvc::kThrough>(head_off + half, oy);
+      }
     }
   }
-  if (has_v && slot >= 0) OutRow(p.value_cache + slot, kv_bytes).store<kvc::kThroughNt>(lane * 16, v);
+  if (has_v && slot >= 0) {
+    const OutRow out(p.value_cache + slot, kv_bytes);
+    if (a.cache_nt) out.store<kvc::kThroughNt>(lane * 16, v);
+    else out.store<kvc::kThrough>(lane * 16, v);
+  }
 }
 
 // Every other shape of aligned rows, written elsewhere than where they are read: heads rotated in part, halves that are no whole
@@ -856,6 +871,7 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
     const int64_t half = (g.rotary_dim / 2) * E, v_items = c ? g.num_kv_heads * g.head_dim / ev : 0;
     const bool fast = !c ? fast_index<kNoCache>(a) : a.batch_indices ? fast_index<kPages>(a) : fast_index<kSlots>(a);
     a.v_items = (uint32_t)v_items;
+    a.cache_nt = g.num_tokens * v_items * 32 > (int64_t(3) << 20);
     a.pairs_per_head = (uint32_t)((g.rotary_dim / 2) / ev);
     // Halves of 64 bytes are whole pieces of half a line each; from 16 MiB of Q and K rows on, whole lines are worth
     // more than the pair form's fewer lanes (pairs and rows, us: 32 + 8 heads x 64 in bf16, 1024 tokens 3.57 and 3.73,

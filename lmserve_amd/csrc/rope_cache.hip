@@ -232,7 +232,11 @@ typedef u32x4 __attribute__((aligned(2))) u32x4_at_any_element;
 __device__ __forceinline__ u32x4 ld16_cos_sin(const char* p) {
   return *reinterpret_cast<const u32x4_at_any_element*>(p);
 }
-// lane / split, the magic uniform
+// lane / split, the magic uniform. Where split is pairs_per_head the magic is 0 for 1 alone, and the kernels do without
+// the division.
+__device__ __forceinline__ uint32_t head_of_pair(const RopeArgs& a, uint32_t lane) {
+  return a.split_magic ? __umulhi(lane, a.split_magic) : lane;
+}
 __device__ __forceinline__ uint32_t head_of_lane(const RopeArgs& a, uint32_t lane) {
   return a.split_magic ? __umulhi(lane, a.split_magic) : lane / a.split;
 }
@@ -277,7 +281,7 @@ __device__ __forceinline__ void rope_pairs_lane(const RopeArgs& a, const RopeLay
   const int64_t pos = reinterpret_cast<const int32_t*>(a.positions)[t];
 
   const uint32_t half = (a.rotary_dim >> 1) * E;  // bytes
-  const uint32_t h = head_of_lane(a, lane);
+  const uint32_t h = head_of_pair(a, lane);
   const uint32_t pv = (lane - h * a.split) * 16;
   const bool is_k = h >= a.num_heads;
   const uint32_t head_off = (is_k ? h - a.num_heads : h) * a.head_dim * E + pv;
@@ -338,9 +342,9 @@ __device__ __forceinline__ void rope_pairs_lane(const RopeArgs& a, const RopeLay
   }
 }
 
-// Every other shape of aligned rows, written elsewhere than where they are read: heads rotated in part, halves that are no whole
-// 64-byte pieces, more V vectors than pair-vectors, other index types. A lane owns the same
-// 16-byte vector of two heads (Q, then K, then V heads), so the lanes write the rows out in
+// Every other shape of aligned rows that are written elsewhere than where they are read:
+// heads rotated in part, halves that are no whole 64-byte pieces, more V vectors than
+// pair-vectors, other index types. A lane owns the same 16-byte vector of two heads (Q, then K, then V heads), so the lanes write the rows out in
 // order, whole lines whatever the halves are; its other half's vector is a second load, from the
 // first-level cache. With the pair form, a lane's unrotated vectors carried along, a
 // partial rotation wrote pieces of 32 and 96 bytes. Launch of a recorded step alone, and
@@ -409,8 +413,8 @@ __device__ __forceinline__ void rope_rows_lane(const RopeArgs& a, const RopeLaye
   }
 }
 
-// An output in its input's own rows: the pair form for every shape, since a lane of the rows kernel reads a vector
-// that another lane overwrites. A lane owns both halves of a pair and carries vectors that pass through along: one of
+// Small launches of whole heads, and an output in its input's own rows: the pair form for every shape, since a lane of
+// the rows kernel reads a vector that another lane overwrites. A lane owns both halves of a pair and carries vectors that pass through along: one of
 // V, with TAIL up to two of V and of the heads' unrotated lanes. Bound as the pair form; plain stores, as its pieces
 // are of any size. TAIL costs a launch without tails a tenth. us a launch of a recorded step, in place here and
 // elsewhere by the rows kernel: 838 tokens x 40 heads x 80 in fp16, 32 rotated, 5.4 and 4.4, 8192 of those 30.1 and
@@ -424,7 +428,7 @@ __device__ __forceinline__ void rope_owner_lane(const RopeArgs& a, const RopeLay
   const int64_t pos = FAST ? (int64_t) reinterpret_cast<const int32_t*>(a.positions)[t] : index_of(a.positions, a.pos_bytes, t);
 
   const uint32_t half = (a.rotary_dim >> 1) * E;  // bytes
-  const uint32_t h = head_of_lane(a, lane);
+  const uint32_t h = head_of_pair(a, lane);
   const uint32_t pv = (lane - h * a.split) * 16;
   const uint32_t heads = a.num_heads + a.num_kv_heads;
   const bool rotates = !TAIL || h < heads, is_k = h >= a.num_heads;
@@ -873,25 +877,41 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
     a.v_items = (uint32_t)v_items;
     a.cache_nt = g.num_tokens * v_items * 32 > (int64_t(3) << 20);
     a.pairs_per_head = (uint32_t)((g.rotary_dim / 2) / ev);
+    const int64_t pair_lanes = heads * a.pairs_per_head, extras = v_items + heads * ((g.head_dim - g.rotary_dim) / ev);
+    const int64_t bytes = g.num_tokens * heads * g.head_dim * E * std::max<int64_t>(num_layers, 1);  // Q and K rows
+    // Whole heads, as the pair and the owner form without tails take them
+    const bool whole = fast && g.rotary_dim == g.head_dim && v_items <= pair_lanes;
+    const bool lines = half % 64 == 0 && out_align % 64 == 0;
+    // Small launches are latency, and the owner form has the shortest chain (launches of a recorded step of 32 layers
+    // alone, then with a gather of the new cache rows behind each, us; owner and pairs: 16 tokens x 28 + 4 heads x 128
+    // 2.23 and 2.28, 3.83 and 4.14; 64 of those (512 KiB) 2.29 and 2.31, 3.89 and 4.17; 192 2.46 and 2.42, 4.45 and 4.33;
+    // with wider cache rows the pair form's reader makes up for it: 16 x 32 + 8 x 128 2.19 and 2.22, 4.15 and 4.10.
+    // Owner and rows: 64 tokens x 28 + 4 x 96 2.26 and 2.51, 3.88 and 4.42; 192 x 32 + 8 x 96 (1.4 MiB) 2.50 and 2.67,
+    // 4.84 and 5.28; 400 x 32 + 8 x 80 (2.4 MiB) 2.90 and 2.84; in fp32, 400 lanes a token, 64 of those 2.67 and 2.39)
+    const bool small = lines ? bytes <= (512 << 10) && g.num_kv_heads * g.head_dim * E < 1536
+                             : bytes <= (2 << 20) && pair_lanes <= 320;
+    // Large ones whose token is one workgroup as pairs and three, of which the last is mostly idle, as rows (32 + 8 heads
+    // x 96 in bf16, owner and rows, us: 838 tokens, 6 MiB, 4.6 and 4.5, 1600 6.8 and 6.9, 2048 7.5 and 8.2, 5000 15.3 and
+    // 16.9, 8192 27.3 and 27.3)
+    const int64_t row_lanes = (heads + (c ? g.num_kv_heads : 0) + 1) / 2 * (g.head_dim / ev);
+    const bool one_group = !lines && bytes >= (8 << 20) && pair_lanes <= kThreads && row_lanes > kThreads;
     // Halves of 64 bytes are whole pieces of half a line each; from 16 MiB of Q and K rows on, whole lines are worth
     // more than the pair form's fewer lanes (pairs and rows, us: 32 + 8 heads x 64 in bf16, 1024 tokens 3.57 and 3.73,
     // 4096 10.13 and 10.17, with a reader of query_out 16.08 and 15.84, 6000 13.3 and 13.3, 24.7 and 22.8, 8192 21.7
     // and 20.0, 31.1 and 29.0)
-    const bool pairs = fast && g.rotary_dim == g.head_dim && v_items <= heads * a.pairs_per_head && half % 64 == 0 &&
-                       out_align % 64 == 0 && !(half == 64 && g.num_tokens * heads * g.head_dim * E >= (int64_t(16) << 20));
+    const bool pairs = lines && !(half == 64 && g.num_tokens * heads * g.head_dim * E >= (int64_t(16) << 20));
     // In place the pair form stays, which reads no vector that another lane writes, and the owner form stands in for rows
-    const int64_t extras = v_items + heads * ((g.head_dim - g.rotary_dim) / ev), pair_lanes = heads * a.pairs_per_head;
-    form = pairs ? kPairs : !in_place || !g.rotary_dim ? kRows : extras > v_items || v_items > pair_lanes ? kOwnerTail : kOwner;
-    if (pairs) {
+    if (whole && (small || one_group)) form = kOwner;
+    else if (whole && pairs) form = kPairs;
+    else if (!in_place || !g.rotary_dim) form = kRows;
+    else form = extras > v_items || v_items > pair_lanes ? kOwnerTail : kOwner;
+    if (form != kRows) {
       a.split = a.pairs_per_head;
-      a.lanes_per_token = (uint32_t)pair_lanes;
-    } else if (form != kRows) {
-      a.split = a.pairs_per_head;
-      a.lanes_per_token = (uint32_t)(form == kOwner ? pair_lanes : std::max(pair_lanes, (extras + 1) / 2));
+      a.lanes_per_token = (uint32_t)(form == kOwnerTail ? std::max(pair_lanes, (extras + 1) / 2) : pair_lanes);
     } else {
       a.split = (uint32_t)(g.head_dim / ev);
       a.head_step = (uint32_t)((heads + (c ? g.num_kv_heads : 0) + 1) / 2);
-      a.lanes_per_token = a.head_step * a.split;
+      a.lanes_per_token = (uint32_t)row_lanes;
     }
     const int64_t lanes = a.lanes_per_token;
     // exact for every lane where lanes * split < 2^32 (pairs: lanes < 2^25, at most 64 pair-vectors per head)

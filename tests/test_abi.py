@@ -568,8 +568,9 @@ def test_what_is_refused_is_refused_without_requests_too():
         rc = L.kvc_append_paged_kv_cache_layers(at, at, at, at, at, at, at, at, 1, batch, ids, 8192, 128, 16, 8192 * 128,
                                                 8192 * 128, 32 * 8192 * 128, 4, 32767, 0, 0, 0, 2, None)
         assert rc == _lib.KVC_ERR_UNSUPPORTED and b"2^31" in L.kvc_last_error_string()
-        q, k, v, q_out, k_out, pool = (i << 44 for i in range(1, 7))      # further apart than the rows reach
-        rc = L.kvc_rotary_pos_emb_and_append_paged(q, k, v, at, at, at, 9, 2**31 - 1, 16, 16, 112, 112, 1792, 1792, 1792,
+        # buffers further apart than the rows reach; 336 lanes a token, 224 without its V row
+        q, k, v, q_out, k_out, pool = (i << 44 for i in range(1, 7))
+        rc = L.kvc_rotary_pos_emb_and_append_paged(q, k, v, at, at, at, 9, 2**31 - 1, 16, 16, 112, 96, 1792, 1792, 1792,
                                                    q_out, k_out, 1792, 1792, pool, at, at, batch, ids, 16, 32 * 1792, 4,
                                                    _lib.KVC_DTYPE_BF16, None)
         assert rc == _lib.KVC_ERR_UNSUPPORTED and b"too large" in L.kvc_last_error_string()

@@ -603,6 +603,34 @@ def test_element_path_in_every_form(gpu, T, Hq, Hkv, D, rd, dtype, bs, shift, wi
     assert torch.equal(k[:-1], k_out[:-1])
 
 
+@pytest.mark.parametrize("T,Hq,Hkv,D,dtype", [
+    (64, 28, 4, 128, torch.bfloat16),     # 512 KiB of Q and K rows, halves of whole 64 bytes
+    (273, 32, 8, 96, torch.float16),      # just under 2 MiB, other halves
+    (1092, 32, 8, 96, torch.bfloat16),    # just under 8 MiB: three workgroups a token, from there on one
+    (300, 12, 3, 80, torch.float32),
+])
+def test_one_token_more_takes_another_form_and_gives_the_same_bits(gpu, T, Hq, Hkv, D, dtype):
+    bs = 16
+    q, k, v, pos, cs = (t.to(gpu) for t in _case(gpu, T + 1, Hq, Hkv, D, D, dtype, seed=T + D))
+    nb = T // bs + 3
+    slots = torch.from_numpy(np.random.default_rng(T).permutation(nb * bs)[:T + 1]).to(gpu)
+    slots[T // 2] = -1
+    got = []
+    for n in (T, T + 1):
+        pool = torch.zeros(nb, 2, bs, Hkv, D, dtype=dtype, device=gpu)
+        q_out, k_out = kvc.rotary_pos_emb_and_cache(q[:n], k[:n], v[:n], pos[:n], cs, D, pool, slots[:n])
+        want = torch.zeros_like(pool)
+        b, e, keep = slots[:n] // bs, slots[:n] % bs, slots[:n] >= 0
+        want[b[keep], 0, e[keep]] = k_out[keep].view(-1, Hkv, D)
+        want[b[keep], 1, e[keep]] = v[:n][keep].view(-1, Hkv, D)
+        assert torch.equal(pool, want)
+        got.append((q_out[:T], k_out[:T]))
+    assert all(torch.equal(x, y) for x, y in zip(*got))
+    some = slice(0, T, max(1, T // 300))
+    for out, x, name in ((got[0][0], q, "query"), (got[0][1], k, "key")):
+        _check_rotation(out[some].cpu(), x[:T][some].cpu(), pos[:T][some].cpu(), cs.cpu(), D, dtype, name)
+
+
 # Heads whose two halves do not share a wavefront, or not a workgroup, where every 16-byte vector has a lane of its own
 @pytest.mark.parametrize("T,Hq,Hkv,D,rd,dtype", [
     (3000, 32, 8, 96, 96, torch.bfloat16),

@@ -66,7 +66,8 @@ def test_swap_out_then_in_matches_oracle(gpu, mode, chunk):
 def test_direct_swap_under_every_grid_cap(gpu, cap_out, cap_in):
     """The direct kernel walks its chunks grid-stride under a cap per direction
     (`direct_max_wgs`, `direct_max_wgs_in`; 0 = the other's): one workgroup, a
-    few, the defaults and more workgroups than chunks all move the same bytes."""
+    few, the defaults and more workgroups than chunks all move the same bytes.
+    GPU->Host takes 16 workgroups at most."""
     s = wl.LLAMA_3_8B
     L, nb, nhb, n = 3, 48, 40, 29
     block_shape = (2, s.block_size, s.num_kv_heads, s.head_dim)
@@ -83,6 +84,7 @@ def test_direct_swap_under_every_grid_cap(gpu, cap_out, cap_in):
         orc.c_save_blocks_to_host(gpu_np, host_np, old, host_ids)
         w.copy_kv_sync(_mappings(old, host_ids), kvc.Device.GPU, kvc.Device.Host)
         assert _lib.last_swap_mode() == _lib.KVC_SWAP_DIRECT
+        assert _lib.last_launch()["grid"] == min(cap_out, 16)
         assert np.array_equal(w.host_kv_caches, host_np)
         orc.c_load_blocks_from_host(gpu_np, host_np, host_ids[:19], new)
         w.copy_kv_sync(_mappings(host_ids[:19], new), kvc.Device.Host, kvc.Device.GPU)

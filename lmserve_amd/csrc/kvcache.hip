@@ -2774,8 +2774,11 @@ static int run_fan_copy(char* pool, const int64_t* pairs, int64_t num_pairs, int
                         int64_t layer_stride_bytes, int64_t block_bytes, int64_t num_blocks, hipStream_t s) {
   const bool inline_pairs = num_pairs <= kInlinePairs;
   if (!inline_pairs && (!scratch || (uintptr_t)scratch % 16)) return kNotInline;  // the caller says what is wrong
-  if (num_blocks > INT32_MAX || num_pairs > (1 << 28) || num_layers > INT32_MAX || block_bytes > (int64_t(1) << 30) ||
-      !g_tune.copy_nt || g_tune.copy_unroll || g_tune.copy_order || g_tune.copy_max_wgs > 0 ||
+  bool several = false;
+  for (int64_t i = 1; i < num_pairs && !several; ++i) several = pairs[2 * i] == pairs[2 * i - 2];
+  if (!several || num_blocks > INT32_MAX || num_pairs > (1 << 28) || num_layers > INT32_MAX ||
+      block_bytes > (int64_t(1) << 30) || !g_tune.copy_nt || g_tune.copy_unroll || g_tune.copy_order ||
+      g_tune.copy_max_wgs > 0 ||
       common_vec({(uint64_t)(uintptr_t)pool, (uint64_t)layer_stride_bytes, (uint64_t)block_bytes}) != 16)
     return kNotInline;
   // a pair with an id outside the pool, or onto itself, copies nothing
@@ -2793,15 +2796,15 @@ static int run_fan_copy(char* pool, const int64_t* pairs, int64_t num_pairs, int
     items7 += held % 7 == 0;
     held = held == 20 ? 0 : held + 1;
   }
-  if (items3 == live) return kNotInline;
+  if (items3 == live) return kNotInline;  // none among them that copies
   // Up to 3 destinations an item, or up to 7 where that leaves less than half as many items.
   const int fan = items7 * 2 < items3 ? 7 : 3;
   const int64_t items = fan == 7 ? items7 : items3, words = items * (fan + 1);
   if (words > kFanWords && inline_pairs) return kNotInline;
-  // What few doubled sources save does not make up for the pairs' better form (a list of pairs and items, us; half,
-  // a quarter and 1 % of the pairs are of sources with two): beyond one resident set 600 pairs x 32 of 64 KiB 418 and
-  // 415, 418 and 460, 418 and 504, 200 x 4 of 128 KiB 38 and 41, 38 and 45, 39 and 49; within it 24 x 32 of 64 KiB 21.3 and 19.9, 21.4 and 21.1,
-  // 21.6 and 21.8; 20 x 80 of 8 KiB 9.2 and 9.0, 9.4 and 9.4, 9.3 and 9.6.
+  // What few doubled sources save does not make up for the pairs' better form (pairs and items, us; half, a quarter
+  // and 1 % of the pairs are of sources with two): beyond one resident set 600 pairs x 32 of 64 KiB 418 and 415, 418
+  // and 460, 418 and 504, 200 x 4 of 128 KiB 38 and 41, 38 and 45, 39 and 49; within it 24 x 32 of 64 KiB 21.3 and
+  // 19.9, 21.4 and 21.1, 21.6 and 21.8; 20 x 80 of 8 KiB 9.2 and 9.0, 9.4 and 9.4, 9.3 and 9.6.
   const FanShape shape = fan_shape(items, num_layers, block_bytes);
   if (!shape.unroll || (shape.large ? items * 10 > live * 7 : items * 16 > live * 15)) return kNotInline;
   if (!inline_pairs) {  // a list that is staged is refused while the stream is recorded, also where its items are few

@@ -324,6 +324,17 @@ def test_the_fan_form_is_taken_where_enough_pairs_share_a_source(gpu, tile_bytes
     assert np.array_equal(bits_of(dpool), pool)
 
 
+@pytest.mark.parametrize("n", [6, 600])     # in the launch's arguments, and staged
+def test_a_list_of_which_nothing_copies(gpu, n):
+    pool = random_pool((2, 8, 4096), seed=n)
+    dpool = to_bf16(pool, gpu)
+    pairs = np.stack([np.full(n, 3), np.resize([3, 8, -1], n)], axis=1).astype(np.int64)
+    scratch = torch.zeros(2 * n, dtype=torch.int64, device=gpu)
+    _lib.check(_lib.lib().kvc_copy_blocks_host_pairs(dpool.data_ptr(), pairs.ctypes.data, n, scratch.data_ptr(), 2, 8 * 8192,
+                                                     8192, 8, torch.cuda.current_stream().cuda_stream))
+    assert np.array_equal(bits_of(dpool), pool)
+
+
 def test_pairs_that_travel_with_the_launch_are_recorded_with_or_without_scratch(gpu):
     """300 pairs of which two share a source, and scratch at hand: nothing of the list may be left to a staging buffer
     that a replay would read again."""

@@ -22,12 +22,10 @@ inline int log2_exact(int64_t x) {
 
 // Launch shape of the rotation kernel, set through kvc_set_tuning
 // ("rope_threads": 64/128/192/256 lanes per workgroup, 0 = by size; "rope_nt":
-// non-temporal loads, bit 0 the K and V rows, bit 1 the Q rows). Off by default:
-// with both bits a launch whose Q/K/V come from HBM gains 1-2 % (9.35 against
-// 9.50 us per layer at a 2048-token chunk over 28 distinct source sets; 3.53
-// against 3.30 at 256 tokens over 32), but a forward pass hands the kernel rows
-// its projection has just written, and with sources that are still in cache the
-// chunk is 36 % slower (8.51 against 6.25 us) and the decode launch unchanged.
+// non-temporal loads, bit 0 the K and V rows, bit 1 the Q rows, 0 = by size: both
+// for whole heads from 40 MiB of rows on). A forward pass hands the kernel rows its projection has
+// just written; while these are still in cache, non-temporal loads make a 2048-token
+// chunk 36 % slower (8.51 against 6.25 us) and leave a decode launch unchanged.
 struct RopeTuning {
   int threads = 0;
   int nt = 0;

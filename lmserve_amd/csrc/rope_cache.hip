@@ -271,7 +271,7 @@ __device__ __forceinline__ uint32_t head_of_lane(const RopeArgs& a, uint32_t lan
 // alone. Stores at device scope of pieces that are no whole 64 bytes lose (2048 x 15 x 96 in
 // bf16, halves of 96 bytes, 4.68 -> 5.16): such heads, and outputs that start within 64 bytes,
 // go to the rows kernel.
-// NTL: non-temporal loads, bit 0 for the K and V rows, bit 1 for the Q rows.
+// NTL: non-temporal loads, bit 0 for the K and V rows, bit 1 for the Q rows; by size, see run_rope.
 template <typename T, Addressing ADDR, int NTL>
 __device__ __forceinline__ void rope_pairs_lane(const RopeArgs& a, const RopeLayer p) {
   constexpr uint32_t E = T::kBytes;
@@ -546,10 +546,10 @@ static_assert(sizeof(RopeLayersArgs) <= 4096, "kernel arguments");
 // The kernels of rows of aligned 16-byte vectors, and the one of all other rows
 enum VectorForm { kElements, kPairs, kRows, kOwner, kOwnerTail };
 
-template <typename T, VectorForm FORM>
+template <typename T, VectorForm FORM, int NTL = 0>
 __global__ __launch_bounds__(kThreads) void rope_layers_kernel(RopeLayersArgs args) {
   const RopeLayer p = args.layer[blockIdx.z];
-  if constexpr (FORM == kPairs) rope_pairs_lane<T, kSlots, 0>(args.a, p);
+  if constexpr (FORM == kPairs) rope_pairs_lane<T, kSlots, NTL>(args.a, p);
   else if constexpr (FORM == kRows) rope_rows_lane<T, kSlots, true, 0>(args.a, p);
   else rope_owner_lane<T, kSlots, true, FORM == kOwnerTail>(args.a, p);
 }
@@ -636,14 +636,14 @@ void launch_vector(const RopeArgs& a, VectorForm form, dim3 grid, dim3 block, hi
 }
 
 template <typename T, Addressing ADDR>
-void launch_vector(const RopeArgs& a, VectorForm form, dim3 grid, dim3 block, hipStream_t s) {
+void launch_vector(const RopeArgs& a, VectorForm form, int ntl, dim3 grid, dim3 block, hipStream_t s) {
   if (form == kOwner || form == kOwnerTail) {
     if (!fast_index<ADDR>(a)) kvc::launch((rope_owner_kernel<T, ADDR, false, true>), grid, block, 0, s, a);
     else if (form == kOwner) kvc::launch((rope_owner_kernel<T, ADDR, true, false>), grid, block, 0, s, a);
     else kvc::launch((rope_owner_kernel<T, ADDR, true, true>), grid, block, 0, s, a);
     return;
   }
-  switch (kvc::g_rope_tune.nt & 3) {
+  switch (ntl) {
     case 0: launch_vector<T, ADDR, 0>(a, form, grid, block, s); break;
     case 1: launch_vector<T, ADDR, 1>(a, form, grid, block, s); break;
     case 2: launch_vector<T, ADDR, 2>(a, form, grid, block, s); break;
@@ -652,7 +652,7 @@ void launch_vector(const RopeArgs& a, VectorForm form, dim3 grid, dim3 block, hi
 }
 
 template <typename T>
-int launch_rope(RopeArgs a, int64_t num_tokens, VectorForm form, unsigned threads, hipStream_t s) {
+int launch_rope(RopeArgs a, int64_t num_tokens, VectorForm form, int ntl, unsigned threads, hipStream_t s) {
   if (form == kElements) {
     const dim3 grid((unsigned)(num_tokens * a.groups_per_token)), block(threads);
     if (!a.key_cache) launch_element<T, kNoCache>(a, grid, block, s);
@@ -665,9 +665,9 @@ int launch_rope(RopeArgs a, int64_t num_tokens, VectorForm form, unsigned thread
   const int64_t slot_step = a.slot_bytes, pos_step = a.pos_bytes;
   for (int64_t t0 = 0; t0 < num_tokens; t0 += kMaxY) {
     const dim3 grid(a.groups_per_token, (unsigned)std::min(kMaxY, num_tokens - t0)), block(threads);
-    if (!a.key_cache) launch_vector<T, kNoCache>(a, form, grid, block, s);
-    else if (a.batch_indices) launch_vector<T, kPages>(a, form, grid, block, s);
-    else launch_vector<T, kSlots>(a, form, grid, block, s);
+    if (!a.key_cache) launch_vector<T, kNoCache>(a, form, ntl, grid, block, s);
+    else if (a.batch_indices) launch_vector<T, kPages>(a, form, ntl, grid, block, s);
+    else launch_vector<T, kSlots>(a, form, ntl, grid, block, s);
     KVC_HIP(hipGetLastError());
     a.query += kMaxY * a.q_token_stride;
     a.key += kMaxY * a.k_token_stride;
@@ -684,14 +684,15 @@ int launch_rope(RopeArgs a, int64_t num_tokens, VectorForm form, unsigned thread
 // Several layers of slot-mapped writes, as many to a launch as the arguments hold
 template <typename T>
 int launch_rope_layers(RopeArgs a, const RopeLayer* layers, int64_t num_layers, int64_t num_tokens, VectorForm form,
-                       unsigned threads, hipStream_t s) {
+                       bool nt, unsigned threads, hipStream_t s) {
   RopeLayersArgs args{};
   for (int64_t l0 = 0; l0 < num_layers; l0 += kLayersPerLaunch) {
     const int64_t n = std::min<int64_t>(kLayersPerLaunch, num_layers - l0);
     args.a = a;
     std::copy(layers + l0, layers + l0 + n, args.layer);
     const dim3 grid(a.groups_per_token, (unsigned)num_tokens, (unsigned)n), block(threads);
-    if (form == kPairs) kvc::launch((rope_layers_kernel<T, kPairs>), grid, block, 0, s, args);
+    if (form == kPairs && nt) kvc::launch((rope_layers_kernel<T, kPairs, 3>), grid, block, 0, s, args);
+    else if (form == kPairs) kvc::launch((rope_layers_kernel<T, kPairs>), grid, block, 0, s, args);
     else if (form == kRows) kvc::launch((rope_layers_kernel<T, kRows>), grid, block, 0, s, args);
     else if (form == kOwner) kvc::launch((rope_layers_kernel<T, kOwner>), grid, block, 0, s, args);
     else kvc::launch((rope_layers_kernel<T, kOwnerTail>), grid, block, 0, s, args);
@@ -868,6 +869,7 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
   const int64_t heads = g.num_heads + g.num_kv_heads;
   const bool vector = (in_align | out_align) % 16 == 0 && heads * g.head_dim * E <= (int64_t(1) << 29) &&
                       (g.rotary_dim / 2) % ev == 0 && (g.head_dim - g.rotary_dim) % ev == 0 && g.head_dim % ev == 0;
+  int ntl = kvc::g_rope_tune.nt & 3;
   VectorForm form = kElements;
   unsigned threads = (unsigned)kvc::g_rope_tune.threads;
   const bool fixed = threads == 64 || threads == 128 || threads == 192 || threads == 256;
@@ -905,6 +907,19 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
     else if (whole && pairs) form = kPairs;
     else if (!in_place || !g.rotary_dim) form = kRows;
     else form = extras > v_items || v_items > pair_lanes ? kOwnerTail : kOwner;
+    // From 40 MiB of Q, K and V rows on the pair form's loads are non-temporal. Plain ones allocate in caches that no longer
+    // hold the rows anyway, and push out the dirty lines of whatever ran before, the projection that wrote these rows
+    // first of all. Smaller rows are still in the last-level cache, from where plain loads are faster. Plain and
+    // non-temporal, us a launch: four sets of rows in turn; the rows just written; those and query_out read behind it:
+    // 8192 tokens x 64 + 8 heads x 128 59.5 and 56.1; 114.9 and 105.9; 163.5 and 147.1
+    // 5500 x 32 + 8 (64 MiB)           26.3 and 25.1; 48.4 and 44.0; 61.7 and 58.4
+    // 3500 of those (41 MiB)           17.9 and 16.0; 30.1 and 28.9; 40.7 and 39.1
+    // 3000 (35 MiB)                    13.7 and 14.3; 25.2 and 24.8; 35.8 and 33.9
+    // 2048 (24 MiB)                    9.3 and 10.9; 18.1 and 18.0; 24.6 and 24.1
+    // Steps of the rows form lose by it (8192 tokens x 24 layers, 32 + 8 heads x 80, 32 rotated, 570 and 587 us; 16 layers
+    // of 32 + 8 x 64 323 and 330), and so does a rotation without the cache (5000 x 32 + 8 x 128, 954 and 961).
+    if (!ntl && form == kPairs && c && g.num_tokens * (heads + g.num_kv_heads) * g.head_dim * E >= (int64_t(40) << 20))
+      ntl = 3;
     if (form != kRows) {
       a.split = a.pairs_per_head;
       a.lanes_per_token = (uint32_t)(form == kOwnerTail ? std::max(pair_lanes, (extras + 1) / 2) : pair_lanes);
@@ -950,15 +965,15 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
         (kvc::g_rope_tune.nt & 3) || g.num_tokens > 65535)
       return kLayerByLayer;
     switch (g.dtype) {
-      case KVC_DTYPE_BF16: return launch_rope_layers<BF16>(a, layers, num_layers, g.num_tokens, form, threads, s);
-      case KVC_DTYPE_F16: return launch_rope_layers<F16>(a, layers, num_layers, g.num_tokens, form, threads, s);
-      default: return launch_rope_layers<F32>(a, layers, num_layers, g.num_tokens, form, threads, s);
+      case KVC_DTYPE_BF16: return launch_rope_layers<BF16>(a, layers, num_layers, g.num_tokens, form, ntl != 0, threads, s);
+      case KVC_DTYPE_F16: return launch_rope_layers<F16>(a, layers, num_layers, g.num_tokens, form, ntl != 0, threads, s);
+      default: return launch_rope_layers<F32>(a, layers, num_layers, g.num_tokens, form, ntl != 0, threads, s);
     }
   }
   switch (g.dtype) {
-    case KVC_DTYPE_BF16: return launch_rope<BF16>(a, g.num_tokens, form, threads, s);
-    case KVC_DTYPE_F16: return launch_rope<F16>(a, g.num_tokens, form, threads, s);
-    default: return launch_rope<F32>(a, g.num_tokens, form, threads, s);
+    case KVC_DTYPE_BF16: return launch_rope<BF16>(a, g.num_tokens, form, ntl, threads, s);
+    case KVC_DTYPE_F16: return launch_rope<F16>(a, g.num_tokens, form, ntl, threads, s);
+    default: return launch_rope<F32>(a, g.num_tokens, form, ntl, threads, s);
   }
 }
 

@@ -732,3 +732,38 @@ def test_layers_of_a_plan_in_one_launch_equal_layer_by_layer(gpu, L, T, Hq, Hkv,
     assert all(torch.equal(a, b) for a, b in zip([pool] + outs, want))
     with pytest.raises(ValueError):
         plan.run_layers(q, k[1:], v, caches, outs)
+
+
+@pytest.mark.parametrize("T,Hq,Hkv,D,rd,dtype", [
+    (3413, 32, 8, 128, 128, torch.bfloat16), (3414, 32, 8, 128, 128, torch.bfloat16),     # either side of 40 MiB
+    (5470, 32, 8, 80, 32, torch.float16), (5826, 12, 3, 98, 98, torch.float32),           # rows form; elements
+])
+def test_loads_of_many_rows_give_the_bits_of_the_same_rows_in_parts(gpu, T, Hq, Hkv, D, rd, dtype):
+    """From 40 MiB of rows on the loads are of another kind: a call, and two layers in one launch, against calls
+    on a third of the tokens each, which stay below."""
+    bs, L = 16, 2
+    g = torch.Generator(device=gpu).manual_seed(T)
+    qkv = torch.randn(L, T, (Hq + 2 * Hkv) * D, dtype=dtype, device=gpu, generator=g)
+    q, k, v = qkv.split([Hq * D, Hkv * D, Hkv * D], dim=2)
+    pos = torch.randint(0, 4096, (T,), dtype=torch.int32, device=gpu, generator=g)
+    cs = rotary.make_cos_sin_cache(rd, 4096, 500000.0, dtype=dtype, device=gpu)
+    nb = T // bs + 2
+    slots = torch.randperm(nb * bs, device=gpu, generator=g)[:T].contiguous()
+    none = torch.zeros(T, dtype=torch.int32, device=gpu)
+    want_q, want_pool = torch.zeros(L, T, Hq * D, dtype=dtype, device=gpu), \
+        torch.zeros(L, nb, 2, bs, Hkv, D, dtype=dtype, device=gpu)
+    for l in range(L):
+        for at in range(0, T, T // 3 + 1):
+            part = slice(at, min(T, at + T // 3 + 1))
+            want_q[l, part], _ = kvc.rotary_pos_emb_and_cache(q[l, part], k[l, part], v[l, part], pos[part], cs, D,
+                                                              want_pool[l], slots[part], return_key=False)
+    plan = kvc.PagedRotaryWritePlan(none, pos, none[:1], torch.tensor([0, 1], dtype=torch.int32, device=gpu),
+                                    none[:1], cs, Hq, Hkv, D, bs, slots=slots)
+    for one_launch in (False, True):
+        got_q, got_pool = torch.zeros_like(want_q), torch.zeros_like(want_pool)
+        if one_launch:
+            plan.run_layers(list(q), list(k), list(v), list(got_pool), list(got_q))
+        else:
+            for l in range(L):
+                plan.run(q[l], k[l], v[l], got_pool[l], query_out=got_q[l])
+        assert torch.equal(got_q, want_q) and torch.equal(got_pool, want_pool)

@@ -158,6 +158,7 @@ struct RopeArgs {
   int64_t cache_block_stride, cache_slot_stride;  // bytes
   int64_t num_cache_blocks;
   uint32_t groups_per_token;  // workgroups per token
+  uint32_t threads;           // lanes of a workgroup
   // vector kernels
   uint32_t lanes_per_token;   // lanes that have work
   uint32_t pairs_per_head;    // pair-vectors of one head
@@ -166,6 +167,34 @@ struct RopeArgs {
   uint32_t head_step;         // rows kernel: heads between a lane's two
   uint32_t v_items;           // 16-byte vectors of the token's V row (0 without a cache)
   uint32_t cache_nt;          // pair form: cache rows by non-temporal stores
+};
+
+// The same in 128 bytes, for the kernels that take the index build's types and rows of aligned vectors; byte strides
+// and counts that do not fit send a call to the general form. A launch's arguments are written to memory beyond the
+// host link, and what that costs the host has a step at 128 bytes: launches back to back, us each, of 16 to 128
+// bytes 2.9 to 3.1, of 136 to 352 3.3 to 3.8, of 528 (RopeArgs, and the 256 bytes of launch geometry that a kernel
+// takes along once it reads blockDim) 3.9. Per-layer launches at decode sizes are bound by that: with RopeArgs and with
+// these, us a launch and us a step, 16 layers of 2 tokens x 32 + 8 heads x 64 4.5 and 4.0, 95 and 88; 28 of 64 x 28 + 4 x
+// 128 4.5 and 3.8, 149 and 130; 32 of 256 x 32 + 8 4.4 and 3.6, 163 and 140; 32 of 838 4.4 and 3.6, 182 and 160.
+struct RopeLean {
+  const char *query, *key, *value;
+  char *query_out, *key_out, *key_cache, *value_cache;
+  const void* positions;
+  const char* cos_sin_cache;
+  const void* slot_mapping;
+  uint32_t q_token_stride, k_token_stride, v_token_stride, qo_token_stride, ko_token_stride;  // bytes
+  uint32_t max_position;
+  uint32_t cache_block_stride, cache_slot_stride;  // bytes
+  uint32_t num_cache_blocks;
+  uint32_t split_magic;
+  uint16_t num_heads, num_kv_heads;
+  uint8_t pairs_per_head, vecs_per_head, bs_shift;
+  uint8_t shape;  // cache_nt, then the workgroup's wavefronts
+};
+static_assert(sizeof(RopeLean) == 128, "where a launch's arguments begin to cost more");
+struct RopeLeanPages : RopeLean {
+  const int32_t *batch_indices, *kv_indices, *kv_indptr;
+  uint32_t batch_size, num_kv_indices;
 };
 
 // One layer's buffers, as RopeArgs names them
@@ -177,6 +206,53 @@ struct RopeLayer {
 // How a token finds its cache slot: not at all (plain rotation), through a slot
 // mapping, or through the page table.
 enum Addressing : int { kNoCache, kSlots, kPages };
+
+// The kernels of rows of aligned 16-byte vectors, and the one of all other rows
+enum VectorForm { kElements, kPairs, kRows, kOwner, kOwnerTail };
+
+template <Addressing ADDR> struct LeanOf { using type = RopeLean; };
+template <> struct LeanOf<kPages> { using type = RopeLeanPages; };
+
+// Lanes of a token that have work
+template <typename I>
+__host__ __device__ __forceinline__ I lanes_of(VectorForm form, I heads, I kv_heads, I pairs, I vecs, bool cache) {
+  if (form == kRows) return (heads + (cache ? 2 * kv_heads : kv_heads) + 1) / 2 * vecs;
+  const I pair_lanes = (heads + kv_heads) * pairs;
+  if (form != kOwnerTail) return pair_lanes;
+  const I extras = (cache ? kv_heads * vecs : 0) + (heads + kv_heads) * (vecs - 2 * pairs);
+  return pair_lanes > (extras + 1) / 2 ? pair_lanes : (extras + 1) / 2;
+}
+
+// What a kernel of this form reads of RopeArgs, the rest left alone
+template <typename T, Addressing ADDR, VectorForm FORM>
+__device__ __forceinline__ RopeArgs from_lean(const typename LeanOf<ADDR>::type& l) {
+  RopeArgs a;
+  a.query = l.query; a.key = l.key; a.value = l.value;
+  a.query_out = l.query_out; a.key_out = l.key_out; a.key_cache = l.key_cache; a.value_cache = l.value_cache;
+  a.positions = l.positions; a.cos_sin_cache = l.cos_sin_cache; a.max_position = l.max_position;
+  a.num_heads = l.num_heads; a.num_kv_heads = l.num_kv_heads;
+  a.head_dim = l.vecs_per_head * (16u / T::kBytes);
+  a.rotary_dim = l.pairs_per_head * (32u / T::kBytes);
+  a.q_token_stride = l.q_token_stride; a.k_token_stride = l.k_token_stride; a.v_token_stride = l.v_token_stride;
+  a.qo_token_stride = l.qo_token_stride; a.ko_token_stride = l.ko_token_stride;
+  a.slot_mapping = l.slot_mapping;
+  if constexpr (ADDR == kPages) {
+    a.batch_indices = l.batch_indices; a.kv_indices = l.kv_indices; a.kv_indptr = l.kv_indptr;
+    a.batch_size = l.batch_size; a.num_kv_indices = l.num_kv_indices;
+  }
+  a.bs_shift = l.bs_shift;
+  a.cache_block_stride = l.cache_block_stride; a.cache_slot_stride = l.cache_slot_stride;
+  a.num_cache_blocks = l.num_cache_blocks;
+  a.threads = (uint32_t)(l.shape >> 1) * 64;
+  a.lanes_per_token = lanes_of<uint32_t>(FORM, l.num_heads, l.num_kv_heads, l.pairs_per_head, l.vecs_per_head, ADDR != kNoCache);
+  a.pairs_per_head = l.pairs_per_head;
+  a.split = FORM == kRows ? l.vecs_per_head : l.pairs_per_head;
+  a.split_magic = l.split_magic;
+  a.head_step = ((uint32_t)l.num_heads + (ADDR != kNoCache ? 2 : 1) * (uint32_t)l.num_kv_heads + 1) / 2;
+  a.v_items = ADDR == kNoCache ? 0 : (uint32_t)l.num_kv_heads * l.vecs_per_head;
+  a.cache_nt = l.shape & 1;
+  return a;
+}
 
 // Entry t of an int32 or int64 array (width in bytes). Two loads side by side and no
 // branch: a branch on the width makes the scalar unit wait for the value inside it.
@@ -276,7 +352,7 @@ template <typename T, Addressing ADDR, int NTL>
 __device__ __forceinline__ void rope_pairs_lane(const RopeArgs& a, const RopeLayer p) {
   constexpr uint32_t E = T::kBytes;
   const uint32_t t = blockIdx.y;
-  const uint32_t lane = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t lane = blockIdx.x * a.threads + threadIdx.x;
   if (lane >= a.lanes_per_token) return;
   const int64_t pos = reinterpret_cast<const int32_t*>(a.positions)[t];
 
@@ -359,7 +435,7 @@ __device__ __forceinline__ void rope_rows_lane(const RopeArgs& a, const RopeLaye
   constexpr uint32_t E = T::kBytes;
   constexpr int HEADS = 2;
   const uint32_t t = blockIdx.y;
-  const uint32_t lane = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t lane = blockIdx.x * a.threads + threadIdx.x;
   if (lane >= a.lanes_per_token) return;
   const int64_t pos = FAST ? (int64_t) reinterpret_cast<const int32_t*>(a.positions)[t] : index_of(a.positions, a.pos_bytes, t);
 
@@ -423,7 +499,7 @@ template <typename T, Addressing ADDR, bool FAST, bool TAIL>
 __device__ __forceinline__ void rope_owner_lane(const RopeArgs& a, const RopeLayer p) {
   constexpr uint32_t E = T::kBytes;
   const uint32_t t = blockIdx.y;
-  const uint32_t lane = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t lane = blockIdx.x * a.threads + threadIdx.x;
   if (lane >= a.lanes_per_token) return;
   const int64_t pos = FAST ? (int64_t) reinterpret_cast<const int32_t*>(a.positions)[t] : index_of(a.positions, a.pos_bytes, t);
 
@@ -516,16 +592,28 @@ __host__ __device__ __forceinline__ RopeLayer only_layer(const RopeArgs& a) {
   return RopeLayer{a.query, a.key, a.value, a.query_out, a.key_out, a.key_cache, a.value_cache};
 }
 template <typename T, Addressing ADDR, int NTL>
-__global__ __launch_bounds__(kThreads) void rope_pairs_kernel(RopeArgs a) {
+__global__ __launch_bounds__(kThreads) void rope_pairs_kernel(typename LeanOf<ADDR>::type l) {
+  const RopeArgs a = from_lean<T, ADDR, kPairs>(l);
   rope_pairs_lane<T, ADDR, NTL>(a, only_layer(a));
 }
-template <typename T, Addressing ADDR, bool FAST, int NTL>
-__global__ __launch_bounds__(kThreads) void rope_rows_kernel(RopeArgs a) {
-  rope_rows_lane<T, ADDR, FAST, NTL>(a, only_layer(a));
+template <typename T, Addressing ADDR, int NTL>
+__global__ __launch_bounds__(kThreads) void rope_rows_kernel(typename LeanOf<ADDR>::type l) {
+  const RopeArgs a = from_lean<T, ADDR, kRows>(l);
+  rope_rows_lane<T, ADDR, true, NTL>(a, only_layer(a));
 }
-template <typename T, Addressing ADDR, bool FAST, bool TAIL>
-__global__ __launch_bounds__(kThreads) void rope_owner_kernel(RopeArgs a) {
-  rope_owner_lane<T, ADDR, FAST, TAIL>(a, only_layer(a));
+template <typename T, Addressing ADDR, bool TAIL>
+__global__ __launch_bounds__(kThreads) void rope_owner_kernel(typename LeanOf<ADDR>::type l) {
+  const RopeArgs a = from_lean<T, ADDR, TAIL ? kOwnerTail : kOwner>(l);
+  rope_owner_lane<T, ADDR, true, TAIL>(a, only_layer(a));
+}
+// Other index types, block sizes, and sizes that RopeLean does not hold
+template <typename T, Addressing ADDR, int NTL>
+__global__ __launch_bounds__(kThreads) void rope_rows_general_kernel(RopeArgs a) {
+  rope_rows_lane<T, ADDR, false, NTL>(a, only_layer(a));
+}
+template <typename T, Addressing ADDR>
+__global__ __launch_bounds__(kThreads) void rope_owner_general_kernel(RopeArgs a) {
+  rope_owner_lane<T, ADDR, false, true>(a, only_layer(a));
 }
 
 // The same for several layers of one step, blockIdx.z the layer, their pointers in the
@@ -538,20 +626,18 @@ __global__ __launch_bounds__(kThreads) void rope_owner_kernel(RopeArgs a) {
 // 8 + 1 heads x 80 490 -> 257 (5.15 TB/s).
 constexpr int kLayersPerLaunch = 64;  // 3.5 KiB of the 4 KiB a launch's arguments may take
 struct RopeLayersArgs {
-  RopeArgs a;
+  RopeLean l;
   RopeLayer layer[kLayersPerLaunch];
 };
 static_assert(sizeof(RopeLayersArgs) <= 4096, "kernel arguments");
 
-// The kernels of rows of aligned 16-byte vectors, and the one of all other rows
-enum VectorForm { kElements, kPairs, kRows, kOwner, kOwnerTail };
-
 template <typename T, VectorForm FORM, int NTL = 0>
 __global__ __launch_bounds__(kThreads) void rope_layers_kernel(RopeLayersArgs args) {
   const RopeLayer p = args.layer[blockIdx.z];
-  if constexpr (FORM == kPairs) rope_pairs_lane<T, kSlots, NTL>(args.a, p);
-  else if constexpr (FORM == kRows) rope_rows_lane<T, kSlots, true, 0>(args.a, p);
-  else rope_owner_lane<T, kSlots, true, FORM == kOwnerTail>(args.a, p);
+  const RopeArgs a = from_lean<T, kSlots, FORM>(args.l);
+  if constexpr (FORM == kPairs) rope_pairs_lane<T, kSlots, NTL>(a, p);
+  else if constexpr (FORM == kRows) rope_rows_lane<T, kSlots, true, 0>(a, p);
+  else rope_owner_lane<T, kSlots, true, FORM == kOwnerTail>(a, p);
 }
 
 // Element path: rows that are no whole number of aligned 16-byte vectors. One
@@ -570,7 +656,7 @@ __global__ __launch_bounds__(kThreads) void rope_element_kernel(RopeArgs a) {
   using VT = Vec<T>;
   constexpr int E = T::kBytes;
   const uint32_t t = blockIdx.x / a.groups_per_token;
-  const uint32_t item = (blockIdx.x - t * a.groups_per_token) * blockDim.x + threadIdx.x;
+  const uint32_t item = (blockIdx.x - t * a.groups_per_token) * a.threads + threadIdx.x;
   const int64_t pos = FAST ? (int64_t) reinterpret_cast<const int32_t*>(a.positions)[t] : index_of(a.positions, a.pos_bytes, t);
   const uint32_t rd = a.rotary_dim, half = rd >> 1, D = a.head_dim;
   const uint32_t heads = a.num_heads + a.num_kv_heads;
@@ -628,26 +714,63 @@ void launch_element(const RopeArgs& a, dim3 grid, dim3 block, hipStream_t s) {
   else kvc::launch((rope_element_kernel<T, ADDR, false>), grid, block, 0, s, a);
 }
 
+// Does a call's geometry fit the lean arguments?
+bool lean_fits(const RopeArgs& a, int64_t E) {
+  const auto u32 = [](int64_t v) { return v >= 0 && v <= (int64_t)UINT32_MAX; };
+  const bool strides = u32(a.q_token_stride) && u32(a.k_token_stride) && u32(a.v_token_stride) && u32(a.qo_token_stride) &&
+                       u32(a.ko_token_stride) && a.head_dim * E / 16 <= UINT8_MAX;
+  const bool cache = !a.key_cache || (u32(a.cache_block_stride) && u32(a.cache_slot_stride) && u32(a.num_cache_blocks));
+  return strides && cache && a.num_heads <= UINT16_MAX && a.num_kv_heads <= UINT16_MAX;
+}
+
+// Counts that 32-bit indices are compared with: beyond every such index they are all the same
+uint32_t beyond_int32(int64_t n) { return (uint32_t)std::min<int64_t>(n, int64_t(1) << 31); }
+
+template <Addressing ADDR>
+typename LeanOf<ADDR>::type lean_of(const RopeArgs& a, int64_t E) {
+  typename LeanOf<ADDR>::type l{};
+  l.query = a.query; l.key = a.key; l.value = a.value;
+  l.query_out = a.query_out; l.key_out = a.key_out; l.key_cache = a.key_cache; l.value_cache = a.value_cache;
+  l.positions = a.positions; l.cos_sin_cache = a.cos_sin_cache; l.slot_mapping = a.slot_mapping;
+  l.q_token_stride = (uint32_t)a.q_token_stride; l.k_token_stride = (uint32_t)a.k_token_stride;
+  l.v_token_stride = (uint32_t)a.v_token_stride;
+  l.qo_token_stride = (uint32_t)a.qo_token_stride; l.ko_token_stride = (uint32_t)a.ko_token_stride;
+  l.max_position = beyond_int32(a.max_position);
+  l.cache_block_stride = (uint32_t)a.cache_block_stride; l.cache_slot_stride = (uint32_t)a.cache_slot_stride;
+  l.num_cache_blocks = (uint32_t)a.num_cache_blocks;
+  l.split_magic = a.split_magic;
+  l.num_heads = (uint16_t)a.num_heads; l.num_kv_heads = (uint16_t)a.num_kv_heads;
+  l.pairs_per_head = (uint8_t)a.pairs_per_head; l.vecs_per_head = (uint8_t)(a.head_dim * E / 16);
+  l.bs_shift = (uint8_t)std::max(a.bs_shift, 0);
+  l.shape = (uint8_t)(a.threads / 64 * 2 + (a.cache_nt ? 1 : 0));
+  if constexpr (ADDR == kPages) {
+    l.batch_indices = a.batch_indices; l.kv_indices = a.kv_indices; l.kv_indptr = a.kv_indptr;
+    l.batch_size = beyond_int32(a.batch_size); l.num_kv_indices = beyond_int32(a.num_kv_indices);
+  }
+  return l;
+}
+
 template <typename T, Addressing ADDR, int NTL>
-void launch_vector(const RopeArgs& a, VectorForm form, dim3 grid, dim3 block, hipStream_t s) {
-  if (form == kPairs) kvc::launch((rope_pairs_kernel<T, ADDR, NTL>), grid, block, 0, s, a);
-  else if (fast_index<ADDR>(a)) kvc::launch((rope_rows_kernel<T, ADDR, true, NTL>), grid, block, 0, s, a);
-  else kvc::launch((rope_rows_kernel<T, ADDR, false, NTL>), grid, block, 0, s, a);
+void launch_vector(const RopeArgs& a, VectorForm form, bool lean, dim3 grid, dim3 block, hipStream_t s) {
+  if (form == kPairs) kvc::launch((rope_pairs_kernel<T, ADDR, NTL>), grid, block, 0, s, lean_of<ADDR>(a, T::kBytes));
+  else if (lean) kvc::launch((rope_rows_kernel<T, ADDR, NTL>), grid, block, 0, s, lean_of<ADDR>(a, T::kBytes));
+  else kvc::launch((rope_rows_general_kernel<T, ADDR, NTL>), grid, block, 0, s, a);
 }
 
 template <typename T, Addressing ADDR>
 void launch_vector(const RopeArgs& a, VectorForm form, int ntl, dim3 grid, dim3 block, hipStream_t s) {
+  const bool lean = fast_index<ADDR>(a) && lean_fits(a, T::kBytes);
   if (form == kOwner || form == kOwnerTail) {
-    if (!fast_index<ADDR>(a)) kvc::launch((rope_owner_kernel<T, ADDR, false, true>), grid, block, 0, s, a);
-    else if (form == kOwner) kvc::launch((rope_owner_kernel<T, ADDR, true, false>), grid, block, 0, s, a);
-    else kvc::launch((rope_owner_kernel<T, ADDR, true, true>), grid, block, 0, s, a);
+    if (!lean) kvc::launch((rope_owner_general_kernel<T, ADDR>), grid, block, 0, s, a);
+    else if (form == kOwner) kvc::launch((rope_owner_kernel<T, ADDR, false>), grid, block, 0, s, lean_of<ADDR>(a, T::kBytes));
+    else kvc::launch((rope_owner_kernel<T, ADDR, true>), grid, block, 0, s, lean_of<ADDR>(a, T::kBytes));
     return;
   }
   switch (ntl) {
-    case 0: launch_vector<T, ADDR, 0>(a, form, grid, block, s); break;
-    case 1: launch_vector<T, ADDR, 1>(a, form, grid, block, s); break;
-    case 2: launch_vector<T, ADDR, 2>(a, form, grid, block, s); break;
-    default: launch_vector<T, ADDR, 3>(a, form, grid, block, s); break;
+    case 0: launch_vector<T, ADDR, 0>(a, form, lean, grid, block, s); break;
+    case 1: launch_vector<T, ADDR, 1>(a, form, lean, grid, block, s); break;
+    case 2: launch_vector<T, ADDR, 2>(a, form, lean, grid, block, s); break;
+    default: launch_vector<T, ADDR, 3>(a, form, lean, grid, block, s); break;
   }
 }
 
@@ -688,7 +811,7 @@ int launch_rope_layers(RopeArgs a, const RopeLayer* layers, int64_t num_layers, 
   RopeLayersArgs args{};
   for (int64_t l0 = 0; l0 < num_layers; l0 += kLayersPerLaunch) {
     const int64_t n = std::min<int64_t>(kLayersPerLaunch, num_layers - l0);
-    args.a = a;
+    args.l = lean_of<kSlots>(a, T::kBytes);
     std::copy(layers + l0, layers + l0 + n, args.layer);
     const dim3 grid(a.groups_per_token, (unsigned)num_tokens, (unsigned)n), block(threads);
     if (form == kPairs && nt) kvc::launch((rope_layers_kernel<T, kPairs, 3>), grid, block, 0, s, args);
@@ -875,7 +998,7 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
   const bool fixed = threads == 64 || threads == 128 || threads == 192 || threads == 256;
   if (vector) {
     const int64_t half = (g.rotary_dim / 2) * E, v_items = c ? g.num_kv_heads * g.head_dim / ev : 0;
-    const bool fast = !c ? fast_index<kNoCache>(a) : a.batch_indices ? fast_index<kPages>(a) : fast_index<kSlots>(a);
+    const bool fast = lean_fits(a, E) && (!c ? fast_index<kNoCache>(a) : a.batch_indices ? fast_index<kPages>(a) : fast_index<kSlots>(a));
     a.v_items = (uint32_t)v_items;
     a.cache_nt = g.num_tokens * v_items * 32 > (int64_t(3) << 20);
     a.pairs_per_head = (uint32_t)((g.rotary_dim / 2) / ev);
@@ -895,7 +1018,7 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
     // Large ones whose token is one workgroup as pairs and three, of which the last is mostly idle, as rows (32 + 8 heads
     // x 96 in bf16, owner and rows, us: 838 tokens, 6 MiB, 4.6 and 4.5, 1600 6.8 and 6.9, 2048 7.5 and 8.2, 5000 15.3 and
     // 16.9, 8192 27.3 and 27.3)
-    const int64_t row_lanes = (heads + (c ? g.num_kv_heads : 0) + 1) / 2 * (g.head_dim / ev);
+    const int64_t row_lanes = lanes_of<int64_t>(kRows, g.num_heads, g.num_kv_heads, a.pairs_per_head, g.head_dim / ev, c);
     const bool one_group = !lines && bytes >= (8 << 20) && pair_lanes <= kThreads && row_lanes > kThreads;
     // Halves of 64 bytes are whole pieces of half a line each; from 16 MiB of Q and K rows on, whole lines are worth
     // more than the pair form's fewer lanes (pairs and rows, us: 32 + 8 heads x 64 in bf16, 1024 tokens 3.57 and 3.73,
@@ -922,7 +1045,7 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
       ntl = 3;
     if (form != kRows) {
       a.split = a.pairs_per_head;
-      a.lanes_per_token = (uint32_t)(form == kOwnerTail ? std::max(pair_lanes, (extras + 1) / 2) : pair_lanes);
+      a.lanes_per_token = (uint32_t)lanes_of<int64_t>(form, g.num_heads, g.num_kv_heads, a.pairs_per_head, g.head_dim / ev, c);
     } else {
       a.split = (uint32_t)(g.head_dim / ev);
       a.head_step = (uint32_t)((heads + (c ? g.num_kv_heads : 0) + 1) / 2);
@@ -959,9 +1082,10 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
     a.key_cache = nullptr;
     a.v_items = 0;
   }
+  a.threads = threads;
   hipStream_t s = (hipStream_t)stream;
   if (layers) {
-    if (form == kElements || !c->slot_mapping || c->slot_bytes != 8 || pos_bytes != 4 || a.bs_shift < 0 ||
+    if (form == kElements || !c->slot_mapping || !lean_fits(a, E) || c->slot_bytes != 8 || pos_bytes != 4 || a.bs_shift < 0 ||
         (kvc::g_rope_tune.nt & 3) || g.num_tokens > 65535)
       return kLayerByLayer;
     switch (g.dtype) {

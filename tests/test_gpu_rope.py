@@ -767,3 +767,36 @@ def test_loads_of_many_rows_give_the_bits_of_the_same_rows_in_parts(gpu, T, Hq, 
             for l in range(L):
                 plan.run(q[l], k[l], v[l], got_pool[l], query_out=got_q[l])
         assert torch.equal(got_q, want_q) and torch.equal(got_pool, want_pool)
+
+
+@pytest.mark.parametrize("what", ["query", "value", "pages", "head"])
+@pytest.mark.parametrize("D,rd", [(128, 128), (80, 32)])
+def test_sizes_beyond_the_short_launch_arguments(gpu, what, D, rd):
+    """Token and page strides of 4 GiB and more, and heads of more than 255 vectors, against the same call on
+    dense rows, or with the heads' rotated part alone."""
+    T, Hq, Hkv, bs, dtype = 3, 4, 2, 16, torch.bfloat16
+    if what == "head":
+        D += 16 * 128
+    q, k, v, pos, cs = (t.to(gpu) for t in _case(gpu, T, Hq, Hkv, D, rd, dtype))
+    slots = torch.tensor([18, 3, 30], dtype=torch.int64, device=gpu)
+    none = torch.zeros(T, dtype=torch.int32, device=gpu)
+    plan = kvc.PagedRotaryWritePlan(none, pos, none[:1], torch.tensor([0, 1], dtype=torch.int32, device=gpu),
+                                    none[:1], cs, Hq, Hkv, D, bs, slots=slots)
+    pool = torch.zeros(2, 2, bs, Hkv, D, dtype=dtype, device=gpu)
+    want = torch.empty_like(q)
+    plan.run(q, k, v, pool, query_out=want)
+    _check_rotation(want.cpu(), q.cpu(), pos.cpu(), cs.cpu(), D, dtype, "query")
+    if what == "head":
+        return
+    far = torch.empty(((2 << 30) + 4096) * (1 if what == "pages" else 2) + (1 << 20), dtype=dtype, device=gpu)
+    got, got_pool = torch.empty_like(q), torch.zeros_like(pool)
+    if what == "pages":
+        got_pool = far.as_strided(pool.shape, ((2 << 30) + 4096, *pool.stride()[1:]))
+        got_pool.zero_()
+    else:
+        t = q if what == "query" else v
+        strided = far.as_strided(t.shape, ((2 << 30) + 4096, 1))
+        strided.copy_(t)
+        q, v = (strided, v) if what == "query" else (q, strided)
+    plan.run(q, k, v, got_pool, query_out=got)
+    assert torch.equal(got, want) and torch.equal(got_pool, pool)

@@ -253,9 +253,55 @@ struct WriteArgs {
   int64_t num_cache_blocks;
   // plane kernel only
   uint32_t num_planes;        // 2 * num_layers; plane = (layer, K|V)
-  uint32_t tokens_per_wg;     // blockDim.x / vecs_per_row
+  uint32_t tokens_per_wg;     // threads / vecs_per_row
   uint32_t num_token_groups;  // ceil(num_tokens / tokens_per_wg)
+  uint32_t threads;           // lanes of a workgroup
 };
+
+// What a launch of one layer needs of it, in less than the 128 bytes at which a launch begins to cost the host more: a
+// write per layer at decode sizes is bound by that. WriteArgs, with the 256 bytes of launch geometry that reading blockDim
+// adds, and this, us a launch and us a step, by slot and by page table alike (medians of 16 runs, the host in its slower
+// state; in its faster one both take 2.45): 32 layers of 256 tokens x 8 heads x 128 3.3 to 3.9 and 3.2 to 3.4, 125 to 148
+// and 126 to 131; 24 of 838 x 8 x 80 3.4 to 3.9 and 3.3 to 3.5; 16 of 2 x 8 x 64 3.2 to 3.9 and 3.3 to 3.6.
+struct WriteLean {
+  const char *key, *value;
+  char *key_cache, *value_cache;
+  const void* slot_mapping;
+  const int32_t *positions, *kv_indices, *kv_indptr;
+  uint32_t batch_size, num_kv_indices;
+  uint32_t key_token_stride, value_token_stride, cache_block_stride, cache_slot_stride;  // bytes
+  uint32_t num_cache_blocks, num_tokens, vecs_per_row;
+  uint32_t num_groups;  // of workgroups: a token's, or of tokens (plane kernel)
+  uint16_t threads;
+  uint8_t bs_shift;
+  uint8_t flags;        // WriteLeanFlag
+};
+enum WriteLeanFlag : uint8_t { kLeanThrough = 1, kLeanPipe = 2, kLeanGroupsFastest = 4, kLeanWideSlots = 8 };
+static_assert(sizeof(WriteLean) <= 128, "where a launch's arguments begin to cost more");
+
+__device__ __forceinline__ WriteArgs unfold(const WriteArgs& a) { return a; }
+__device__ __forceinline__ WriteArgs unfold(const WriteLean& l) {
+  WriteArgs a;
+  a.key = l.key; a.value = l.value; a.key_cache = l.key_cache; a.value_cache = l.value_cache;
+  a.slot_mapping = l.slot_mapping; a.slot_bytes = (l.flags & kLeanWideSlots) ? 8 : 4;
+  a.batch_indices = (const int32_t*)l.slot_mapping; a.positions = l.positions;
+  a.kv_indices = l.kv_indices; a.kv_indptr = l.kv_indptr;
+  a.batch_size = l.batch_size; a.num_kv_indices = l.num_kv_indices;
+  a.num_tokens = l.num_tokens; a.vecs_per_row = l.vecs_per_row;
+  a.vpr_shift = (l.vecs_per_row & (l.vecs_per_row - 1)) ? -1 : __builtin_ctz(l.vecs_per_row);
+  a.items_per_token = 2 * l.vecs_per_row;
+  a.num_groups = a.num_token_groups = l.num_groups;
+  a.groups_fastest = l.flags & kLeanGroupsFastest; a.pipe = (l.flags & kLeanPipe) != 0; a.through = l.flags & kLeanThrough;
+  a.key_token_stride = l.key_token_stride; a.value_token_stride = l.value_token_stride;
+  a.key_layer_stride = a.value_layer_stride = a.cache_layer_stride = 0;
+  a.block_size = 1ll << l.bs_shift; a.bs_shift = l.bs_shift;
+  a.cache_block_stride = l.cache_block_stride; a.cache_slot_stride = l.cache_slot_stride;
+  a.num_cache_blocks = l.num_cache_blocks;
+  a.num_planes = 2;
+  a.threads = l.threads;
+  a.tokens_per_wg = a.threads >> a.vpr_shift;  // plane kernel: rows of a power of two of vectors
+  return a;
+}
 
 // Block and entry of token t's slot; false where the write skips the token. The page-table form is three steps of loads,
 // those of a step side by side and an index that is out of range read as 0 (the host launches nothing without
@@ -297,7 +343,7 @@ __device__ __forceinline__ bool find_slot(const WriteArgs& a, uint32_t t, int64_
   return ok && blk >= 0 && blk < a.num_cache_blocks;
 }
 
-// One workgroup = one token x a run of VPT*blockDim.x vectors out of the
+// One workgroup = one token x a run of VPT*threads vectors out of the
 // token's 2*L rows (K and V of every layer). The token, hence its slot and
 // every base address, is uniform across the workgroup.
 // Order of work: the source addresses need only the token, so every lane first
@@ -305,8 +351,9 @@ __device__ __forceinline__ bool find_slot(const WriteArgs& a, uint32_t t, int64_
 // batch_indices -> kv_indptr -> kv_indices) is resolved on the scalar unit
 // while those loads are in flight; the stores follow. A token whose slot is
 // invalid simply returns with its loads unused.
-template <int VEC, int VPT, bool PAGED, bool NT, bool NTL>
-__global__ __launch_bounds__(kThreads) void write_rows_kernel(WriteArgs a) {
+template <int VEC, int VPT, bool PAGED, bool NT, bool NTL, typename ARGS>
+__global__ __launch_bounds__(kThreads) void write_rows_kernel(ARGS args) {
+  const WriteArgs a = unfold(args);
   using V = typename VecOf<VEC>::type;
   // blockIdx.x = group * num_tokens + token by default: neighbouring workgroups
   // read neighbouring token rows of the same layers
@@ -320,7 +367,7 @@ __global__ __launch_bounds__(kThreads) void write_rows_kernel(WriteArgs a) {
   }
   const char* key_row = a.key + (int64_t)t * a.key_token_stride;
   const char* value_row = a.value + (int64_t)t * a.value_token_stride;
-  const uint32_t first = group * (VPT * blockDim.x) + threadIdx.x;
+  const uint32_t first = group * (VPT * a.threads) + threadIdx.x;
   // item -> (row r = 2*layer + K|V, vector inside the row)
   const auto split = [&](uint32_t item, uint32_t& r, uint32_t& vec) {
     if (a.vpr_shift >= 0) {
@@ -339,7 +386,7 @@ __global__ __launch_bounds__(kThreads) void write_rows_kernel(WriteArgs a) {
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
     uint32_t r, vec;
-    split(min(first + j * blockDim.x, last_item), r, vec);
+    split(min(first + j * a.threads, last_item), r, vec);
     const int64_t layer = r >> 1;
     const char* src = ((r & 1u) ? value_row + layer * a.value_layer_stride
                                 : key_row + layer * a.key_layer_stride) + (int64_t)vec * VEC;
@@ -354,7 +401,7 @@ __global__ __launch_bounds__(kThreads) void write_rows_kernel(WriteArgs a) {
   char* vc_row = a.value_cache + slot_off;
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
-    const uint32_t item = first + j * blockDim.x;
+    const uint32_t item = first + j * a.threads;
     if (item <= last_item) {
       uint32_t r, vec;
       split(item, r, vec);
@@ -365,7 +412,7 @@ __global__ __launch_bounds__(kThreads) void write_rows_kernel(WriteArgs a) {
 }
 
 // The lanes of a workgroup run over consecutive TOKENS of one (layer, K|V)
-// plane: the source side is one contiguous run of blockDim.x * 16 bytes, the
+// plane: the source side is one contiguous run of threads * 16 bytes, the
 // cache side one row per token. Each lane looks up its own token's slot (lanes
 // of one row read the same index words) and reuses it for its VPT planes, whose
 // loads are issued before the lookup. Two regimes use it:
@@ -378,8 +425,9 @@ __global__ __launch_bounds__(kThreads) void write_rows_kernel(WriteArgs a) {
 //     several loads in flight per lane.
 // 16-byte vectors and a power-of-two number of them per row (up to 256) only;
 // blockIdx.x = plane_group * num_token_groups + token_group.
-template <int VPT, bool PAGED, bool NT, bool NTL>
-__global__ __launch_bounds__(1024) void write_planes_kernel(WriteArgs a) {
+template <int VPT, bool PAGED, bool NT, bool NTL, typename ARGS>
+__global__ __launch_bounds__(1024) void write_planes_kernel(ARGS args) {
+  const WriteArgs a = unfold(args);
   using V = u32x4;
   const uint32_t pg = blockIdx.x / a.num_token_groups;
   const uint32_t tg = blockIdx.x - pg * a.num_token_groups;
@@ -784,11 +832,12 @@ __global__ __launch_bounds__(kThreads) void write_runs_kernel(RunArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// index kernels
+// index kernels (their launch geometry is constants and arguments: a kernel that reads blockDim or gridDim takes
+// 256 bytes of arguments along, which cost the host 0.3 to 0.6 us a launch)
 // ---------------------------------------------------------------------------
 __global__ void seq_lens_kernel(const int32_t* kv_indptr, const int32_t* last_page_len,
                                 int64_t batch_size, int32_t page_size, int32_t* seq_lens) {
-  const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t b = (int64_t)blockIdx.x * kThreads + threadIdx.x;
   if (b >= batch_size) return;
   int32_t pages = kv_indptr[b + 1] - kv_indptr[b] - 1;
   if (pages < 0) pages = 0;
@@ -801,7 +850,7 @@ __global__ void resolve_slots_kernel(const int32_t* batch_indices, const int32_t
                                      const int32_t* kv_indices, const int32_t* kv_indptr,
                                      int64_t batch_size, int64_t num_kv_indices, int64_t page_size,
                                      int64_t nnz, int64_t* slots) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t t = (int64_t)blockIdx.x * kThreads + threadIdx.x;
   if (t >= nnz) return;
   int64_t slot = -1;
   const int64_t b = batch_indices[t];
@@ -824,7 +873,7 @@ __global__ void batch_indices_positions_kernel(const int32_t* append_indptr,
   const int32_t begin = append_indptr[b];
   const int32_t end = append_indptr[b + 1];
   const int32_t first_pos = seq_lens[b] - (end - begin);
-  for (int32_t j = begin + (int32_t)threadIdx.x; j < end; j += blockDim.x) {
+  for (int32_t j = begin + (int32_t)threadIdx.x; j < end; j += kThreads) {
     if (j < 0 || j >= nnz) continue;
     batch_indices[j] = b;
     positions[j] = first_pos + (j - begin);
@@ -893,6 +942,7 @@ struct IndexArgs {
   int32_t* ids_out;      // copy of kv_indices on the device, or null
   uint32_t* read_flags;  // one word per workgroup in host memory, or null:
   uint32_t flag_value;   // set to this once the workgroup has read its inputs
+  uint32_t grid;         // workgroups
 };
 
 // One word per workgroup tells the host that the workgroup is done with a staging
@@ -916,7 +966,7 @@ __global__ __launch_bounds__(kPrepThreads) void build_write_index_kernel(IndexAr
   const int tid = threadIdx.x;
   const bool first_wg = blockIdx.x == 0;
   const int32_t page_size = a.page_size;
-  const int64_t lane0 = (int64_t)blockIdx.x * kPrepThreads + tid, lanes = (int64_t)gridDim.x * kPrepThreads;
+  const int64_t lane0 = (int64_t)blockIdx.x * kPrepThreads + tid, lanes = (int64_t)a.grid * kPrepThreads;
   // The lane's first 16 bytes of the block tables, and of their last words. Tables of up to 4096 ids every workgroup reads
   // whole, into LDS: a token's block then needs no read over the link behind the scans.
   const int64_t words4 = a.ids_out ? a.num_kv_indices / 4 : 0;
@@ -1039,8 +1089,8 @@ __global__ __launch_bounds__(kPrepThreads) void build_write_index_kernel(IndexAr
 
 // Staging buffer (pinned host memory) -> device buffer, 16 bytes a lane.
 __global__ __launch_bounds__(kThreads) void upload_kernel(const int4* src, int4* dst, int64_t words4,
-                                                          uint32_t* read_flags, uint32_t flag_value) {
-  for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < words4; i += (int64_t)gridDim.x * kThreads)
+                                                          uint32_t* read_flags, uint32_t flag_value, uint32_t grid) {
+  for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < words4; i += (int64_t)grid * kThreads)
     dst[i] = src[i];
   tell_host(read_flags, flag_value);
 }
@@ -1171,13 +1221,40 @@ struct WriteLaunch {
   bool ntl;  // non-temporal loads
 };
 
+// The lean arguments of a launch of one layer, if they hold it. Page-table counts are compared with 32-bit indices:
+// beyond every such index they are all the same.
+bool lean_of(const WriteArgs& a, bool paged, uint32_t num_groups, WriteLean* l) {
+  const auto u32 = [](int64_t v) { return v >= 0 && v <= (int64_t)UINT32_MAX; };
+  if (a.items_per_token != 2 * a.vecs_per_row || a.bs_shift < 0 || !u32(a.key_token_stride) || !u32(a.value_token_stride) ||
+      !u32(a.cache_block_stride) || !u32(a.cache_slot_stride) || !u32(a.num_cache_blocks))
+    return false;
+  const auto beyond_int32 = [](int64_t n) { return (uint32_t)std::min<int64_t>(n, int64_t(1) << 31); };
+  const uint8_t flags = (a.through ? kLeanThrough : 0) | (a.pipe ? kLeanPipe : 0) |
+                        (a.groups_fastest ? kLeanGroupsFastest : 0) | (a.slot_bytes == 8 ? kLeanWideSlots : 0);
+  *l = WriteLean{a.key, a.value, a.key_cache, a.value_cache, paged ? a.batch_indices : a.slot_mapping, a.positions,
+                 a.kv_indices, a.kv_indptr, beyond_int32(a.batch_size), beyond_int32(a.num_kv_indices),
+                 (uint32_t)a.key_token_stride, (uint32_t)a.value_token_stride, (uint32_t)a.cache_block_stride,
+                 (uint32_t)a.cache_slot_stride, (uint32_t)a.num_cache_blocks, a.num_tokens, a.vecs_per_row, num_groups,
+                 (uint16_t)a.threads, (uint8_t)a.bs_shift, flags};
+  return true;
+}
+
 template <int VEC, int VPT, bool PAGED>
-void launch_write_nt(const WriteArgs& a, const WriteLaunch& l, hipStream_t s) {
+void launch_write_nt(WriteArgs a, const WriteLaunch& l, hipStream_t s) {
   const dim3 grid(l.grid), block(l.threads);
-  if (l.nt && l.ntl) kvc::launch((write_rows_kernel<VEC, VPT, PAGED, true, true>), grid, block, 0, s, a);
-  else if (l.nt) kvc::launch((write_rows_kernel<VEC, VPT, PAGED, true, false>), grid, block, 0, s, a);
-  else if (l.ntl) kvc::launch((write_rows_kernel<VEC, VPT, PAGED, false, true>), grid, block, 0, s, a);
-  else kvc::launch((write_rows_kernel<VEC, VPT, PAGED, false, false>), grid, block, 0, s, a);
+  a.threads = l.threads;
+  if constexpr (VEC == 16 && VPT == 1) {
+    WriteLean lean;
+    if (l.nt && lean_of(a, PAGED, a.num_groups, &lean)) {
+      if (l.ntl) kvc::launch((write_rows_kernel<VEC, VPT, PAGED, true, true, WriteLean>), grid, block, 0, s, lean);
+      else kvc::launch((write_rows_kernel<VEC, VPT, PAGED, true, false, WriteLean>), grid, block, 0, s, lean);
+      return;
+    }
+  }
+  if (l.nt && l.ntl) kvc::launch((write_rows_kernel<VEC, VPT, PAGED, true, true, WriteArgs>), grid, block, 0, s, a);
+  else if (l.nt) kvc::launch((write_rows_kernel<VEC, VPT, PAGED, true, false, WriteArgs>), grid, block, 0, s, a);
+  else if (l.ntl) kvc::launch((write_rows_kernel<VEC, VPT, PAGED, false, true, WriteArgs>), grid, block, 0, s, a);
+  else kvc::launch((write_rows_kernel<VEC, VPT, PAGED, false, false, WriteArgs>), grid, block, 0, s, a);
 }
 
 template <int VEC, bool PAGED>
@@ -1202,12 +1279,21 @@ void launch_write(const WriteArgs& a, int vec, const WriteLaunch& l, hipStream_t
 }
 
 template <int VPT, bool PAGED>
-void launch_planes_nt(const WriteArgs& a, const WriteLaunch& l, hipStream_t s) {
+void launch_planes_nt(WriteArgs a, const WriteLaunch& l, hipStream_t s) {
   const dim3 grid(l.grid), block(l.threads);
-  if (l.nt && l.ntl) kvc::launch((write_planes_kernel<VPT, PAGED, true, true>), grid, block, 0, s, a);
-  else if (l.nt) kvc::launch((write_planes_kernel<VPT, PAGED, true, false>), grid, block, 0, s, a);
-  else if (l.ntl) kvc::launch((write_planes_kernel<VPT, PAGED, false, true>), grid, block, 0, s, a);
-  else kvc::launch((write_planes_kernel<VPT, PAGED, false, false>), grid, block, 0, s, a);
+  a.threads = l.threads;
+  if constexpr (VPT <= 2) {  // a layer has two planes
+    WriteLean lean;
+    if (l.nt && lean_of(a, PAGED, a.num_token_groups, &lean)) {
+      if (l.ntl) kvc::launch((write_planes_kernel<VPT, PAGED, true, true, WriteLean>), grid, block, 0, s, lean);
+      else kvc::launch((write_planes_kernel<VPT, PAGED, true, false, WriteLean>), grid, block, 0, s, lean);
+      return;
+    }
+  }
+  if (l.nt && l.ntl) kvc::launch((write_planes_kernel<VPT, PAGED, true, true, WriteArgs>), grid, block, 0, s, a);
+  else if (l.nt) kvc::launch((write_planes_kernel<VPT, PAGED, true, false, WriteArgs>), grid, block, 0, s, a);
+  else if (l.ntl) kvc::launch((write_planes_kernel<VPT, PAGED, false, true, WriteArgs>), grid, block, 0, s, a);
+  else kvc::launch((write_planes_kernel<VPT, PAGED, false, false, WriteArgs>), grid, block, 0, s, a);
 }
 
 template <bool PAGED>
@@ -2218,7 +2304,8 @@ unsigned index_grid(int64_t batch_size, int64_t nnz, int64_t upload_ids) {
 }
 
 // shared driver of the two index-build entry points
-int launch_build_index(const IndexArgs& a, void* stream, unsigned grid) {
+int launch_build_index(IndexArgs a, void* stream, unsigned grid) {
+  a.grid = grid;
   kvc::launch(build_write_index_kernel, dim3(grid), dim3(kPrepThreads), 0, (hipStream_t)stream, a);
   if (a.read_flags) return stage_launched();
   KVC_HIP(hipGetLastError());
@@ -2583,7 +2670,7 @@ int kvc_staging_upload(void* dst, int64_t bytes, void* stream) {
   if (rc != KVC_OK) return rc;
   const char* src = reinterpret_cast<const char*>(flags) + kStageHead;
   kvc::launch(upload_kernel, dim3(grid), dim3(kThreads), 0, (hipStream_t)stream,
-                     reinterpret_cast<const int4*>(src), (int4*)dst, words4, flags, value);
+                     reinterpret_cast<const int4*>(src), (int4*)dst, words4, flags, value, (uint32_t)grid);
   return stage_launched();
 }
 

@@ -694,3 +694,39 @@ def test_page_table_without_requests_writes_nothing(gpu):
                                               cache, i32(1), i32(0), i32())
     assert torch.equal(got[0], alone[0]) and torch.equal(got[1], alone[1])
     assert np.array_equal(bits_of(cache), pool)
+
+
+@pytest.mark.parametrize("by", ["slots", "pages"])
+@pytest.mark.parametrize("planes", [0, 2])
+@pytest.mark.parametrize("what", ["key", "pages"])
+def test_strides_beyond_the_short_launch_arguments(gpu, what, planes, by):
+    """Token and page strides of 4 GiB and more, through both kernels, against the same write on dense rows."""
+    T, H, D, bs = 2, 2, 128, 16
+    g = torch.Generator(device=gpu).manual_seed(3)
+    k, v = (torch.randn(T, H, D, device=gpu, generator=g).to(torch.bfloat16) for _ in range(2))
+    pool = torch.zeros(2, 2, bs, H, D, dtype=torch.bfloat16, device=gpu)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=gpu)
+    slots = torch.tensor([bs + 3, 7], device=gpu)
+    _lib.set_tuning("write_planes", planes)
+
+    def write(k, v, cache):
+        if by == "slots":
+            kvc.reshape_and_cache(k, v, cache, slots)
+        else:
+            kvc.append_paged_kv_cache(k, v, i32([0, 1]), i32([3, 7]), cache, i32([1, 0]), i32([0, 1, 2]), i32([4, 8]))
+
+    write(k, v, pool)
+    want = torch.zeros_like(pool)
+    want[1, 0, 3], want[1, 1, 3], want[0, 0, 7], want[0, 1, 7] = k[0], v[0], k[1], v[1]
+    assert torch.equal(pool, want)
+    far = torch.empty((2 << 30) + (1 << 20), dtype=torch.bfloat16, device=gpu)
+    cache = torch.zeros_like(pool)
+    if what == "key":
+        strided = far.as_strided(k.shape, ((2 << 30) + 4096, D, 1))
+        strided.copy_(k)
+        k = strided
+    else:
+        cache = far.as_strided(pool.shape, ((2 << 30) + 4096, *pool.stride()[1:]))
+        cache.zero_()
+    write(k, v, cache)
+    assert torch.equal(cache, want)

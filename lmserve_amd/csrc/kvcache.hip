@@ -622,14 +622,18 @@ __global__ __launch_bounds__(kThreads) void copy_to_host_kernel(TileArgs a) {
 // Large copies: one chunk of one tile per workgroup, 16-byte vectors, the order of
 // the chunks chosen per XCD. Bound: HBM, and of that the part that the spread of
 // the addresses in flight costs. Workgroups are dealt round-robin to the 8 XCDs;
-// here each XCD walks a run of `xcd_run` neighbouring chunks (a few hundred KiB)
+// here each XCD walks a run of `xcd_run` neighbouring chunks (256 KiB to 2 MiB)
 // instead of every eighth chunk, and the launch keeps the region in flight small:
 // either one vector per lane in workgroups of 64 lanes (a gather), or two in workgroups
-// of 256, the second asked for when the first has arrived, of which a CU holds 6
-// instead of 8 (dynamic LDS that nothing uses; a launch that fits the GPU at once goes
-// without). Both loads at once with 5 to a CU, non-temporal stores -> this, stores
-// through the L2 (us): copy of 300 blocks of 2 MiB 208 -> 202, of 2048 1419 -> 1400; gather
-// and scatter of 100 x 2 MiB 124.5 -> 119.5, of 600 829 -> 784, of 256 x 5 MiB 858 -> 830.
+// of 256, of which a CU holds 5 instead of 8 (dynamic LDS that nothing uses; a launch
+// that fits the GPU at once goes without). Copies walk a layer at a time (launch_stream).
+// Stores are non-temporal and go through the L2. Runs of 512 KiB with 6 to a CU, the second
+// load when the first has arrived, blocks in order, then this (us; sources and destinations
+// in turn over 700 MiB and more): copies of 80 blocks x 32 layers of 64 KiB 58.7 and 55.5, of
+// 400 276 and 266, of 400 x 80 728 and 694, of 100 x 28 of 32 KiB 38.2 and 34.4, of 400 x 16
+// 83.8 and 72, of 150 x 24 of 40 KiB 56.7 and 51.9, of 1000 x 80 of 8 KiB 217 and 214; scatter
+// of 256 x 80 of 64 KiB 431 and 415, of 2000 x 12 of 18 KiB 165 and 160. Single wavefronts with one vector
+// a lane copy 1 to 3 % faster still.
 // Loads are non-temporal throughout. Plain loads of a copy's sources find a little more of
 // them in the last-level cache (12 layers of 18 KiB, 200 blocks just read: 4 % less), but
 // where it is full of other kernels' dirty lines they push those out: 200 x 80 of 8 KiB
@@ -679,10 +683,8 @@ __device__ __forceinline__ void stream_tile_chunk(const StreamArgs& a, const SRC
   const kvc::OutRow out(dst, a.tile_bytes);
   u32x4 data[UNROLL];
 #pragma unroll
-  for (int j = 0; j < UNROLL; ++j) {
-    if (j) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  for (int j = 0; j < UNROLL; ++j)
     data[j] = ld<NTL>(reinterpret_cast<const u32x4*>(src + min(at + j * (THREADS * 16), a.tile_bytes - 16)));
-  }
 #pragma unroll
   for (int j = 0; j < UNROLL; ++j) out.store<NTS ? kvc::kThroughNt : kvc::kPlain>(at + j * (THREADS * 16), data[j]);
 }
@@ -704,8 +706,12 @@ __global__ __launch_bounds__(kThreads) void stream_pairs_kernel(StreamArgs a, Pa
 // hold. Two and three copies of each source, as pairs -> this (us): 6 x 2 of 2 MiB 8.2 ->
 // 6.7, 12 x 3 28 -> 18.5, 64 x 2 93 -> 74, 600 x 3 1205 -> 870 (5.75 TB/s); 33 x 3 x 24
 // layers of 40 KiB 39 -> 26.6, 2000 x 2 x 80 of 8 KiB 775 -> 722. Large launches take one
-// vector per lane, 5 workgroups to a CU (two vectors 950 at 600 x 3, 6 to a CU 920) and
-// plain non-temporal stores (through the L2 872, and 772 at 2000 x 2).
+// vector per lane (two 950 at 600 x 3) and walk a layer at a time. With more than two destinations an item
+// in workgroups of 256 lanes, 5 to a CU (6 to a CU 920), and plain non-temporal stores; with fewer
+// in single wavefronts that store through the L2. Blocks in order, 256 lanes and plain stores
+// throughout, then this, us: 64 x 2 x 32 of 64 KiB 73.3 and 64.7, 30 x 2 x 80 85.7 and 74.6, 200 x
+// 2 x 28 of 32 KiB 106 and 93, 1500 x 2 x 12 of 18 KiB 199 and 190, 2000 x 2 x 80 of 8 KiB 726 and 715; 600 x 3 x 32 of 64
+// KiB 871 and 850, 60 x 3 x 24 of 40 KiB 47.9 and 43.2.
 // The list holds FAN + 1 words an item, its source and its destinations (-1: none), so
 // that one scalar load brings an item's ids: with a table of offsets and a loop over the
 // destinations each id is a dependent load of its own (6 x 2 8.7).
@@ -714,7 +720,7 @@ struct FanList {
   int32_t word[kFanWords];
 };
 
-template <int UNROLL, int FAN>
+template <int THREADS, int UNROLL, int FAN>
 __device__ __forceinline__ void fan_tile_chunk(const StreamArgs& a, const int32_t* list) {
   const auto [i, layer, chunk] = stream_place(a);
   int32_t id[FAN + 1];
@@ -723,9 +729,9 @@ __device__ __forceinline__ void fan_tile_chunk(const StreamArgs& a, const int32_
   if (id[0] < 0 || id[0] >= a.num_src_blocks) return;
   const char* src = a.src_base + layer * a.src_layer_stride + id[0] * a.src_block_stride;
   char* dst_layer = a.dst_base + layer * a.dst_layer_stride;
-  const uint32_t at = chunk * (kThreads * UNROLL * 16) + threadIdx.x * 16;
+  const uint32_t at = chunk * (THREADS * UNROLL * 16) + threadIdx.x * 16;
   u32x4 data[UNROLL];
-  load_chunk<UNROLL, kThreads * 16, true>(data, src, at, a.tile_bytes);
+  load_chunk<UNROLL, THREADS * 16, true>(data, src, at, a.tile_bytes);
 #pragma unroll
   for (int d = 1; d <= FAN; ++d) {
     if (id[d] < 0 || id[d] >= a.num_dst_blocks) continue;
@@ -733,18 +739,18 @@ __device__ __forceinline__ void fan_tile_chunk(const StreamArgs& a, const int32_
 #pragma unroll
     for (int j = 0; j < UNROLL; ++j) {
       if constexpr (UNROLL >= 8) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // paced, as in copy_tiles_chunks
-      out.store<kvc::kNonTemporal>(at + j * (kThreads * 16), data[j]);
+      out.store<THREADS == 64 ? kvc::kThroughNt : kvc::kNonTemporal>(at + j * (THREADS * 16), data[j]);
     }
   }
 }
 
-template <int UNROLL, int FAN>
-__global__ __launch_bounds__(kThreads) void fan_tiles_kernel(StreamArgs a, const int32_t* list) {
-  fan_tile_chunk<UNROLL, FAN>(a, list);
+template <int THREADS, int UNROLL, int FAN>
+__global__ __launch_bounds__(THREADS) void fan_tiles_kernel(StreamArgs a, const int32_t* list) {
+  fan_tile_chunk<THREADS, UNROLL, FAN>(a, list);
 }
-template <int UNROLL, int FAN>
-__global__ __launch_bounds__(kThreads) void fan_inline_kernel(StreamArgs a, FanList list) {
-  fan_tile_chunk<UNROLL, FAN>(a, list.word);
+template <int THREADS, int UNROLL, int FAN>
+__global__ __launch_bounds__(THREADS) void fan_inline_kernel(StreamArgs a, FanList list) {
+  fan_tile_chunk<THREADS, UNROLL, FAN>(a, list.word);
 }
 
 // ---------------------------------------------------------------------------
@@ -1702,22 +1708,24 @@ int launch_stream(const TileArgs& t, TileSides sides, int64_t n, hipStream_t s, 
   const uint32_t threads = (uint32_t)shape.threads, unroll = (uint32_t)shape.unroll, chunk = (uint32_t)shape.chunk();
   a.chunks_per_tile = (a.tile_bytes + chunk - 1) / chunk;
   a.total_chunks = (uint32_t)(n * a.num_layers * a.chunks_per_tile);
-  a.xcd_run = gather ? 256 : 64;
   a.num_items = (uint32_t)n;
-  // Copies of small tiles walk a layer at a time: with the layers of a block as neighbours a run of 64 chunks
-  // touches as many far-apart pages (8 KiB x 80 layers: 4000 blocks 5.05 -> 5.2 TB/s, 300 blocks 4.85 -> 5.3;
-  // from 32 KiB on it makes no difference, and a dense side wants its own order: gather 6.2 -> 5.1).
-  a.layer_slowest = sides == TileSides::kPools && t.tile_bytes < (32 << 10);
+  // Copies walk a layer at a time: with the layers of a block as neighbours a run touches as many far-apart pages, and
+  // what is in flight as many layers (blocks in order and layers in order, us: 400 x 16 layers of 32 KiB 82 and 72, 600 x
+  // 24 of 40 KiB 213 and 202, 64 x 32 of 64 KiB 45.8 and 43.3). Where much of a layer is copied, that alone keeps
+  // neighbours together (1024 x 32 of 64 KiB, 64 MiB a layer, 686 both ways, 2048 1370 and 1385). A dense side wants
+  // its own order (gather 6.2 -> 5.1 TB/s).
+  a.layer_slowest = sides == TileSides::kPools && (t.tile_bytes < (64 << 10) || n * t.tile_bytes < (int64_t(64) << 20));
+  a.xcd_run = a.layer_slowest ? 32 : 256;
   const bool dense_cached = n * (int64_t)a.num_layers * t.tile_bytes <= (int64_t(256) << 20);
   const bool plain_load = sides == TileSides::kScatter && dense_cached;
   const bool plain_store = gather && dense_cached;
   const dim3 grid(a.total_chunks), block(threads);
-  const unsigned six_per_cu = (int64_t)a.total_chunks > resident_workgroups() ? 160 * 1024 / 6 : 0;
-  if (pairs) kvc::launch(stream_pairs_kernel, grid, block, six_per_cu, s, a, *pairs);
+  const unsigned five_per_cu = (int64_t)a.total_chunks > resident_workgroups() ? 160 * 1024 / 5 : 0;
+  if (pairs) kvc::launch(stream_pairs_kernel, grid, block, five_per_cu, s, a, *pairs);
   else if (gather && plain_store) kvc::launch((stream_tiles_kernel<64, 1, true, false>), grid, block, 0, s, a);
   else if (gather) kvc::launch((stream_tiles_kernel<64, 1, true, true>), grid, block, 0, s, a);
-  else if (plain_load) kvc::launch((stream_tiles_kernel<256, 2, false, true>), grid, block, six_per_cu, s, a);
-  else kvc::launch((stream_tiles_kernel<256, 2, true, true>), grid, block, six_per_cu, s, a);
+  else if (plain_load) kvc::launch((stream_tiles_kernel<256, 2, false, true>), grid, block, five_per_cu, s, a);
+  else kvc::launch((stream_tiles_kernel<256, 2, true, true>), grid, block, five_per_cu, s, a);
   g_last = LastLaunch{KVC_KERNEL_COPY_TILES, 16, (int64_t)unroll, (int64_t)threads, (int64_t)a.total_chunks,
                       plain_load || plain_store ? 0 : 1};
   KVC_HIP(hipGetLastError());
@@ -1807,13 +1815,13 @@ int launch_tiles_vec(TileArgs a, int unroll, int max_wgs, hipStream_t s, bool nt
 }
 
 // Copies through the fan kernels: `list` in the launch's own arguments, or in device memory.
-template <int UNROLL>
+template <int THREADS, int UNROLL>
 void launch_fan(const StreamArgs& a, int fan, const FanList* list, const int32_t* device_list, unsigned lds, hipStream_t s) {
-  const dim3 grid(a.total_chunks), block(kThreads);
-  if (list && fan == 3) kvc::launch((fan_inline_kernel<UNROLL, 3>), grid, block, lds, s, a, *list);
-  else if (list) kvc::launch((fan_inline_kernel<UNROLL, 7>), grid, block, lds, s, a, *list);
-  else if (fan == 3) kvc::launch((fan_tiles_kernel<UNROLL, 3>), grid, block, lds, s, a, device_list);
-  else kvc::launch((fan_tiles_kernel<UNROLL, 7>), grid, block, lds, s, a, device_list);
+  const dim3 grid(a.total_chunks), block(THREADS);
+  if (list && fan == 3) kvc::launch((fan_inline_kernel<THREADS, UNROLL, 3>), grid, block, lds, s, a, *list);
+  else if (list) kvc::launch((fan_inline_kernel<THREADS, UNROLL, 7>), grid, block, lds, s, a, *list);
+  else if (fan == 3) kvc::launch((fan_tiles_kernel<THREADS, UNROLL, 3>), grid, block, lds, s, a, device_list);
+  else kvc::launch((fan_tiles_kernel<THREADS, UNROLL, 7>), grid, block, lds, s, a, device_list);
 }
 
 // Shape of a fan launch: vectors per lane as of a small copy, up to 8, while the workgroups are resident at once;
@@ -1835,20 +1843,24 @@ FanShape fan_shape(int64_t items, int64_t layers, int64_t tile_bytes) {
   return {unroll, large};
 }
 
-int launch_fan_copy(StreamArgs a, FanShape shape, int fan, const FanList* list, const int32_t* device_list, hipStream_t s) {
-  const uint32_t chunk = kThreads * 16 * shape.unroll;
+// `pairs`: destinations of all items together
+int launch_fan_copy(StreamArgs a, FanShape shape, int fan, int64_t pairs, const FanList* list, const int32_t* device_list,
+                    hipStream_t s) {
+  const bool wavefronts = shape.large && pairs <= 2 * (int64_t)a.num_items;
+  const uint32_t threads = wavefronts ? 64 : kThreads, chunk = threads * 16 * shape.unroll;
   a.chunks_per_tile = (a.tile_bytes + chunk - 1) / chunk;
   a.total_chunks = a.num_items * a.num_layers * a.chunks_per_tile;
   a.xcd_run = shape.large ? 64 : 1;
-  a.layer_slowest = shape.large && a.tile_bytes < (32 << 10);
-  const unsigned lds = shape.large ? 160 * 1024 / 5 : 0;
-  switch (shape.unroll) {
-    case 1: launch_fan<1>(a, fan, list, device_list, lds, s); break;
-    case 2: launch_fan<2>(a, fan, list, device_list, lds, s); break;
-    case 4: launch_fan<4>(a, fan, list, device_list, lds, s); break;
-    default: launch_fan<8>(a, fan, list, device_list, lds, s); break;
+  a.layer_slowest = shape.large;
+  const unsigned lds = shape.large && !wavefronts ? 160 * 1024 / 5 : 0;
+  if (wavefronts) launch_fan<64, 1>(a, fan, list, device_list, lds, s);
+  else switch (shape.unroll) {
+    case 1: launch_fan<kThreads, 1>(a, fan, list, device_list, lds, s); break;
+    case 2: launch_fan<kThreads, 2>(a, fan, list, device_list, lds, s); break;
+    case 4: launch_fan<kThreads, 4>(a, fan, list, device_list, lds, s); break;
+    default: launch_fan<kThreads, 8>(a, fan, list, device_list, lds, s); break;
   }
-  g_last = LastLaunch{KVC_KERNEL_COPY_TILES, 16, shape.unroll, kThreads, (int64_t)a.total_chunks, 1};
+  g_last = LastLaunch{KVC_KERNEL_COPY_TILES, 16, shape.unroll, (int64_t)threads, (int64_t)a.total_chunks, 1};
   KVC_HIP(hipGetLastError());
   return KVC_OK;
 }
@@ -2931,12 +2943,12 @@ static int run_fan_copy(char* pool, const int64_t* pairs, int64_t num_pairs, int
   if (words <= kFanWords) {
     FanList inline_list;
     std::copy(list.begin(), list.end(), inline_list.word);
-    return launch_fan_copy(a, shape, fan, &inline_list, nullptr, s);
+    return launch_fan_copy(a, shape, fan, live, &inline_list, nullptr, s);
   }
   // at most 16 bytes a pair, which scratch holds: an item of 4 words has a pair, and items of 8 are fewer than half
   // as many as those of 4
   const int rc = stage_list(list.data(), words * (int64_t)sizeof(int32_t), scratch, s);
-  return rc != KVC_OK ? rc : launch_fan_copy(a, shape, fan, nullptr, (const int32_t*)scratch, s);
+  return rc != KVC_OK ? rc : launch_fan_copy(a, shape, fan, live, nullptr, (const int32_t*)scratch, s);
 }
 
 int kvc_copy_blocks_host_pairs(void* kv_caches, const int64_t* pairs, int64_t num_pairs, int64_t* scratch,

@@ -400,3 +400,42 @@ def test_a_gather_of_more_lanes_than_a_launch_has(gpu):
                                       block_bytes, 2, 0, 1, torch.cuda.current_stream().cuda_stream)
     assert rc == 0 and _lib.last_launch()["threads"] == 256 and _lib.last_launch()["grid"] == (2**32 - 1) // 256
     assert torch.equal(dense, pool[0, 1])
+
+
+@pytest.mark.parametrize("tile_bytes,L,fans,threads", [
+    (65552, 60, (2,) * 20, 64),            # one vector past 64 KiB: a wavefront with one lane of work
+    (8208, 30, (2,) * 150, 64),
+    (8208, 30, (2, 1) * 200, 64),          # staged
+    (8208, 30, (3, 1) * 110, 64),          # two an item on average
+    (8208, 30, (3, 2) * 80, 256),          # more
+])
+def test_large_copies_with_two_destinations_a_block(gpu, tile_bytes, L, fans, threads):
+    """Up to two destinations an item go out in single wavefronts: against NumPy at tiles that end inside a chunk."""
+    n = sum(fans)
+    nb = n + len(fans) + 1
+    pool = random_pool((L, nb, tile_bytes // 2), seed=n)
+    dpool = to_bf16(pool, gpu)
+    ids = np.random.default_rng(n).permutation(nb).tolist()
+    d, at = {}, len(fans)
+    for src, fan in zip(ids, fans):
+        d[src] = ids[at:at + fan]
+        at += fan
+    for src, dsts in d.items():
+        pool[:, dsts] = pool[:, src:src + 1]
+    kvc.copy_blocks(dpool, d)
+    ran = _lib.last_launch()
+    assert (ran["per_lane"], ran["threads"]) == (1, threads)
+    assert np.array_equal(bits_of(dpool), pool)
+
+
+@pytest.mark.parametrize("tile_bytes,n", [(65536, 1023), (65536, 1024), (65552, 1024)])
+def test_order_of_large_copies(gpu, tile_bytes, n):
+    """Tiles of 64 KiB and more: below 64 MiB a layer the launch walks layers, from there on blocks."""
+    L = 2
+    g = torch.Generator(device=gpu).manual_seed(n)
+    pool = torch.randint(-2**31, 2**31 - 1, (L, 2 * n + 3, tile_bytes // 4), dtype=torch.int32, device=gpu, generator=g)
+    ids = torch.randperm(2 * n + 3, device=gpu, generator=g)
+    want = pool.clone()
+    want[:, ids[n:2 * n]] = pool[:, ids[:n]]
+    kvc.copy_blocks(pool, torch.stack([ids[:n], ids[n:2 * n]], 1).flatten().contiguous())
+    assert torch.equal(pool, want)

@@ -28,10 +28,13 @@ struct OutRow {
   }
 };
 
-// The same for addresses that differ from lane to lane by more than an offset: 16 bytes, kThrough. The two wait
+// The same for addresses that differ from lane to lane by more than an offset: 16 bytes, kThrough and kThroughNt. The two wait
 // states behind the store keep a later instruction off its data registers.
 __device__ __forceinline__ void st_through(char* p, u32x4 v) {
   asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
+}
+__device__ __forceinline__ void st_through_nt(char* p, u32x4 v) {
+  asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
 }
 
 // A kernel launch whose arguments go straight to the runtime. The launch by <<<>>> and its macro first store the

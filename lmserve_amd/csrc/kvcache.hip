@@ -87,7 +87,7 @@ struct Tuning {
   int copy_order = 0;       // copy_tiles: 1 = walk all blocks of a layer before the next layer
   int write_vpt = 0;        // vectors per lane in write_rows, 0 = by size
   int write_nt = 3;         // write kernels: bit 0 non-temporal stores, bit 1 non-temporal loads (rows of
-                            // 1 KiB or more only: narrower rows measured 4 % slower with them). Loads:
+                            // 1 KiB or more, and narrower ones from 96 MiB on: see run_write). Loads:
                             // -3 % at the 64 MiB decode step, -2 to -3 % at 224-256 MiB, -10 to -15 %
                             // for one layer per launch when the K/V rows come from HBM, neutral when
                             // they are still in cache (one source set, or a producer kernel in front)
@@ -204,12 +204,16 @@ __device__ __forceinline__ void st(V* p, V v) {
   else *p = v;
 }
 
-// One vector of a cache row; `through`: at device scope (kvc::st_through), 16-byte vectors only.
+// One vector of a cache row; `through`: at device scope (kvc::st_through), 2 = non-temporal as well; 16-byte vectors only.
 template <bool NT, typename V>
-__device__ __forceinline__ void st_row(char* p, V v, bool through) {
+__device__ __forceinline__ void st_row(char* p, V v, int through) {
   if constexpr (NT && sizeof(V) == 16) {
-    if (through) {
+    if (through == 1) {
       kvc::st_through(p, v);
+      return;
+    }
+    if (through == 2) {
+      kvc::st_through_nt(p, v);
       return;
     }
   }
@@ -244,7 +248,7 @@ struct WriteArgs {
   int pipe;                  // 1 = a lane waits for each of its loads before issuing the next one,
                              // so that the lanes of a launch that is resident all at once drift
                              // apart and reads overlap writes
-  int through;               // 1 = the rows are stored at device scope
+  int through;               // 1 = the rows are stored at device scope, 2 = and non-temporal
   int64_t key_token_stride, value_token_stride;
   int64_t key_layer_stride, value_layer_stride;
   int64_t block_size;
@@ -276,7 +280,7 @@ struct WriteLean {
   uint8_t bs_shift;
   uint8_t flags;        // WriteLeanFlag
 };
-enum WriteLeanFlag : uint8_t { kLeanThrough = 1, kLeanPipe = 2, kLeanGroupsFastest = 4, kLeanWideSlots = 8 };
+enum WriteLeanFlag : uint8_t { kLeanThrough = 3, kLeanPipe = 4, kLeanGroupsFastest = 8, kLeanWideSlots = 16 };
 static_assert(sizeof(WriteLean) <= 128, "where a launch's arguments begin to cost more");
 
 __device__ __forceinline__ WriteArgs unfold(const WriteArgs& a) { return a; }
@@ -406,7 +410,7 @@ __global__ __launch_bounds__(kThreads) void write_rows_kernel(ARGS args) {
       uint32_t r, vec;
       split(item, r, vec);
       char* dst = ((r & 1u) ? vc_row : kc_row) + (int64_t)(r >> 1) * a.cache_layer_stride + (int64_t)vec * VEC;
-      st_row<NT>(dst, data[j], a.through != 0);
+      st_row<NT>(dst, data[j], a.through);
     }
   }
 }
@@ -462,7 +466,7 @@ __global__ __launch_bounds__(1024) void write_planes_kernel(ARGS args) {
     if (plane < a.num_planes) {
       char* dst = ((plane & 1u) ? a.value_cache : a.key_cache) + slot_off +
                   (int64_t)(plane >> 1) * a.cache_layer_stride;
-      st_row<NT>(dst, data[j], a.through != 0);
+      st_row<NT>(dst, data[j], a.through);
     }
   }
 }
@@ -1235,8 +1239,8 @@ bool lean_of(const WriteArgs& a, bool paged, uint32_t num_groups, WriteLean* l) 
       !u32(a.cache_block_stride) || !u32(a.cache_slot_stride) || !u32(a.num_cache_blocks))
     return false;
   const auto beyond_int32 = [](int64_t n) { return (uint32_t)std::min<int64_t>(n, int64_t(1) << 31); };
-  const uint8_t flags = (a.through ? kLeanThrough : 0) | (a.pipe ? kLeanPipe : 0) |
-                        (a.groups_fastest ? kLeanGroupsFastest : 0) | (a.slot_bytes == 8 ? kLeanWideSlots : 0);
+  const uint8_t flags = (uint8_t)(a.through | (a.pipe ? kLeanPipe : 0) |
+                        (a.groups_fastest ? kLeanGroupsFastest : 0) | (a.slot_bytes == 8 ? kLeanWideSlots : 0));
   *l = WriteLean{a.key, a.value, a.key_cache, a.value_cache, paged ? a.batch_indices : a.slot_mapping, a.positions,
                  a.kv_indices, a.kv_indptr, beyond_int32(a.batch_size), beyond_int32(a.num_kv_indices),
                  (uint32_t)a.key_token_stride, (uint32_t)a.value_token_stride, (uint32_t)a.cache_block_stride,
@@ -1487,7 +1491,14 @@ int run_write(const char* fn, const void* key, const void* value, void* kc, void
     a.tokens_per_wg = l.threads / a.vecs_per_row;
     a.num_planes = (uint32_t)num_planes;
     l.nt = (g_tune.write_nt & 1) != 0;
-    l.ntl = (g_tune.write_nt & 2) != 0 && !narrow;
+    // Many narrow rows: stores go through the L2 as well, from 24 MiB of K and V rows on, and from 96 MiB on, which the
+    // last-level cache does not hold beside what is written, the loads are non-temporal (before, the stores, both; us,
+    // three sets of rows in turn, 80 layers of 256 bytes by slot: 1700 tokens 23.3, 22.5, 28.5; 2600 (102 MiB) 41.0, 39.6,
+    // 39.4; 8000 115.2, 110.1, 109.8; by page table 700 tokens 12.5, 12.4, 11.8; 2300 35.4, 34.8, 38.0; 3001 49.6, 48.9,
+    // 49.1; 8000 121.5, 118.5, 116.3, and with a kernel in front that writes the rows 239, 236, 208)
+    const int64_t rows_bytes = g.num_tokens * num_planes * g.row_elems * E;
+    if (narrow && !a.through && rows_bytes >= (int64_t(24) << 20)) a.through = 2;
+    l.ntl = (g_tune.write_nt & 2) != 0 && (!narrow || rows_bytes >= (int64_t(96) << 20));
     const int64_t plane_groups = (a.num_planes + l.vpt - 1) / l.vpt;
     const int64_t max_groups = std::max<int64_t>(1, 0x7fffffffll / plane_groups);
     const int64_t max_tokens = max_groups * a.tokens_per_wg;

@@ -730,3 +730,29 @@ def test_strides_beyond_the_short_launch_arguments(gpu, what, planes, by):
         cache.zero_()
     write(k, v, cache)
     assert torch.equal(cache, want)
+
+
+@pytest.mark.parametrize("T,L", [(1026, 48), (4098, 48), (1024, 49)])   # 24 and 96 MiB of K and V rows, and more
+@pytest.mark.parametrize("by", ["slots", "pages"])
+def test_many_narrow_rows(gpu, T, L, by):
+    """Rows of 256 bytes of all layers in one launch, either side of where its stores and loads change."""
+    H, D, bs = 1, 128, 16
+    for tokens in (T - 3, T):
+        g = torch.Generator(device=gpu).manual_seed(tokens)
+        k, v = (torch.randint(-2**15, 2**15, (L, tokens, H, D), dtype=torch.int16, device=gpu, generator=g)
+                .view(torch.bfloat16) for _ in range(2))
+        nb = tokens // bs + 3
+        table = torch.randperm(nb, device=gpu, generator=g)
+        pos = torch.arange(tokens, device=gpu) + 5
+        slots = table[pos // bs] * bs + pos % bs
+        pool = torch.zeros(L, nb, 2, bs, H, D, dtype=torch.bfloat16, device=gpu)
+        if by == "slots":
+            kvc.reshape_and_cache_layers(k, v, pool, slots)
+        else:
+            i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=gpu)
+            kvc.append_paged_kv_cache_layers(k, v, torch.zeros(tokens, dtype=torch.int32, device=gpu), pos.int(), pool,
+                                             table.int(), i32([0, nb]), i32([bs]))
+        want = torch.zeros_like(pool)
+        want[:, slots // bs, 0, slots % bs] = k
+        want[:, slots // bs, 1, slots % bs] = v
+        assert torch.equal(pool.view(torch.int16), want.view(torch.int16))

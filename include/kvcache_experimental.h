@@ -123,6 +123,10 @@ int kvc_write_runs_layers(const void* key, const void* value,
  * step (runtime/worker/llm_worker/model_worker.py:399-423).
  *
  * kvc_staging_upload copies the first `bytes` (whole 16-byte vectors) to dst.
+ * kvc_staging_upload_index does the same with a buffer that holds the index arrays of a
+ * step, int32 at these byte offsets: append_indptr and kv_indptr (batch_size + 1 words each)
+ * and kv_last_page_len (batch_size); batch_indices and positions receive what
+ * kvc_get_seq_lens and kvc_get_batch_indices_positions make of them.
  * kvc_build_write_index_staged is kvc_build_write_index on a buffer that holds, as
  * int32, input_lens | context_lens | num_blocks (batch_size each, then padded to a
  * multiple of four words) | the concatenated block tables; kv_indices, 16-byte aligned,
@@ -130,6 +134,10 @@ int kvc_write_runs_layers(const void* key, const void* value,
  */
 int kvc_staging_acquire(int64_t bytes, void** out);
 int kvc_staging_upload(void* dst, int64_t bytes, void* stream);
+int kvc_staging_upload_index(void* dst, int64_t bytes, int64_t append_indptr_at,
+                             int64_t kv_indptr_at, int64_t kv_last_page_len_at,
+                             int64_t batch_size, int64_t page_size, int64_t nnz,
+                             int32_t* batch_indices, int32_t* positions, void* stream);
 int kvc_build_write_index_staged(int64_t batch_size, int64_t num_kv_indices, int64_t page_size,
                                  int64_t nnz, int32_t* cu_seqlens_q, int32_t* kv_indptr,
                                  int32_t* kv_last_page_len, int32_t* kv_indices,

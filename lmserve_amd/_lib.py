@@ -108,6 +108,7 @@ SIGNATURES = {
     "kvc_copy_blocks_host_pairs": (c_int, [_P, _P, _I64, _P, _I64, _I64, _I64, _I64, _P]),
     "kvc_staging_acquire": (c_int, [_I64, ctypes.POINTER(_P)]),
     "kvc_staging_upload": (c_int, [_P, _I64, _P]),
+    "kvc_staging_upload_index": (c_int, [_P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _P, _P, _P]),
     "kvc_build_write_index_staged": (c_int, [_I64, _I64, _I64, _I64, _P, _P, _P, _P, _P, _P, _P, _P]),
     "kvc_slot_runs": (c_int, [_P, c_int, _I64, _I64, _P, _P, _I64, _P]),
     "kvc_streams_share_hw_queue": (c_int, [_P, _P, _P]),

@@ -671,9 +671,8 @@ struct HostArray {
 
 /* upload_index(position_ids, cu_seqlens_q, kv_indices, kv_indptr, kv_last_page_len, slots | None, page_size, device,
  * stream) -> 1, a negative kvc_status, or (position_ids, cu_seqlens_q, kv_indices, kv_indptr, kv_last_page_len,
- * batch_indices, positions, slots | None) on the device, in one allocation: the arrays go through a staging buffer,
- * where a copy of each from pageable memory would wait for all work queued before it; kvc_get_seq_lens and
- * kvc_get_batch_indices_positions follow. */
+ * batch_indices, positions, slots | None) on the device, in one allocation and one launch: the arrays go through a
+ * staging buffer, where a copy of each from pageable memory would wait for all work queued before it. */
 PyObject* fast_upload_index(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS  // an allocation that fails is a Python exception
   int64_t page_size, device;
@@ -697,21 +696,15 @@ PyObject* fast_upload_index(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
   for (int i = 0; i < arrays; ++i) at[i + 1] = at[i] + up(a[i].view.len);
   // more is better off with the copy engine, and would leave the ring that large
   if (at[arrays] > kUploadMost) return PyLong_FromLong(NOT_FAST);
-  const int64_t staged_bytes = at[arrays], o_bi = staged_bytes, o_pos = o_bi + up(4 * T), o_seq = o_pos + up(4 * T),
-                end = o_seq + up(4 * B);
+  const int64_t staged_bytes = at[arrays], o_bi = staged_bytes, o_pos = o_bi + up(4 * T), end = o_pos + up(4 * T);
   void* staged = nullptr;
   int rc = acquire_staging(staged_bytes, &staged);
   if (rc < 0) return PyLong_FromLong(rc == KVC_ERR_STAGING ? NOT_FAST : rc);
   for (int i = 0; i < arrays; ++i) memcpy((char*)staged + at[i], a[i].view.buf, (size_t)a[i].view.len);
   const at::Tensor buf = device_bytes(end, (int)device);
   char* p = (char*)buf.data_ptr();
-  rc = kvc_staging_upload(p, staged_bytes, stream);
-  if (rc == KVC_OK)
-    rc = kvc_get_seq_lens((const int32_t*)(p + at[3]), (const int32_t*)(p + at[4]), B, page_size, (int32_t*)(p + o_seq),
-                          stream);
-  if (rc == KVC_OK)
-    rc = kvc_get_batch_indices_positions((const int32_t*)(p + at[1]), (const int32_t*)(p + o_seq), B, T,
-                                         (int32_t*)(p + o_bi), (int32_t*)(p + o_pos), stream);
+  rc = kvc_staging_upload_index(p, staged_bytes, at[1], at[3], at[4], B, page_size, T, (int32_t*)(p + o_bi),
+                                (int32_t*)(p + o_pos), stream);
   if (rc < 0) return PyLong_FromLong(rc);
   PyObject* slots;
   if (arrays == 6) slots = piece(buf, at::kLong, a[5].size(), at[5]);

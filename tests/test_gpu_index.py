@@ -335,3 +335,36 @@ def test_requests_are_read_as_they_read_themselves(gpu, form):
     assert step.set_requests(reqs) == [0, 1]
     step.build_index()
     assert step.slot_mapping.tolist() == [107 * 16 + 1, 107 * 16 + 2, 103 * 16, -1]
+
+
+@pytest.mark.parametrize("sizes", [
+    [1], [0, 5, 0], [1] * 15 + [300], [1] * 17, [2] * 1030, [4099, 1, 64, 65, 0, 63],
+    [1] * 16500,        # more than a lane of every workgroup has
+])
+def test_host_arrays_uploaded_in_one_launch(gpu, sizes):
+    """batch_indices and positions that the upload derives, against the host's own, requests without new tokens among
+    them."""
+    rng = np.random.default_rng(len(sizes))
+    reqs = []
+    for i, n in enumerate(sizes):
+        filled = int(rng.integers(0 if n else 1, 40))
+        reqs.append(kvc.InferInput(seq_id=i, input_ids=[0] * n, input_len=n, filled_token_len=filled, context_len=filled + n,
+                                   block_ids=rng.integers(0, 1000, (filled + n + 15) // 16).tolist()))
+    host = kvc.make_kv_index_inputs(reqs, 16)
+    got = kvc.to_device(host, 16, gpu)
+    want = np.repeat(np.arange(len(sizes)), np.diff(host.cu_seqlens_q))
+    assert np.array_equal(got.batch_indices.cpu().numpy(), want)
+    assert np.array_equal(got.positions.cpu().numpy(), host.position_ids)
+    for name in ("position_ids", "cu_seqlens_q", "kv_block_indices", "kv_block_indptrs", "kv_last_block_lens", "slot_mapping"):
+        assert np.array_equal(getattr(got, name).cpu().numpy(), getattr(host, name)), name
+
+
+def test_upload_of_index_arrays_refuses_what_lies_outside(gpu):
+    lib = _lib.lib()
+    dst = torch.zeros(64, dtype=torch.int32, device=gpu)
+    out = torch.zeros(8, dtype=torch.int32, device=gpu)
+    for bytes_, cu, ptr, last, batch in ((64, 0, 16, 52, 4), (64, -4, 16, 32, 2), (64, 2, 16, 32, 2), (60, 0, 16, 32, 2),
+                                         (64, 0, 60, 32, 2), (64, 0, 16, 32, 0), (64, 0, 16, 32, 2**40)):
+        rc = lib.kvc_staging_upload_index(dst.data_ptr(), bytes_, cu, ptr, last, batch, 16, 4, out.data_ptr(),
+                                          out.data_ptr(), torch.cuda.current_stream().cuda_stream)
+        assert rc == _lib.KVC_ERR_INVALID_ARG

@@ -205,15 +205,15 @@ __device__ __forceinline__ void st(V* p, V v) {
 }
 
 // One vector of a cache row; `through`: at device scope (kvc::st_through), 2 = non-temporal as well; 16-byte vectors only.
-template <bool NT, typename V>
+template <bool NT, bool THROUGH_NT, typename V>
 __device__ __forceinline__ void st_row(char* p, V v, int through) {
   if constexpr (NT && sizeof(V) == 16) {
-    if (through == 1) {
-      kvc::st_through(p, v);
+    if (THROUGH_NT && through == 2) {
+      kvc::st_through_nt(p, v);
       return;
     }
-    if (through == 2) {
-      kvc::st_through_nt(p, v);
+    if (through) {
+      kvc::st_through(p, v);
       return;
     }
   }
@@ -258,7 +258,6 @@ struct WriteArgs {
   // plane kernel only
   uint32_t num_planes;        // 2 * num_layers; plane = (layer, K|V)
   uint32_t tokens_per_wg;     // threads / vecs_per_row
-  uint32_t num_token_groups;  // ceil(num_tokens / tokens_per_wg)
   uint32_t threads;           // lanes of a workgroup
 };
 
@@ -275,7 +274,7 @@ struct WriteLean {
   uint32_t batch_size, num_kv_indices;
   uint32_t key_token_stride, value_token_stride, cache_block_stride, cache_slot_stride;  // bytes
   uint32_t num_cache_blocks, num_tokens, vecs_per_row;
-  uint32_t num_groups;  // of workgroups: a token's, or of tokens (plane kernel)
+  uint32_t num_groups;  // workgroups per token
   uint16_t threads;
   uint8_t bs_shift;
   uint8_t flags;        // WriteLeanFlag
@@ -283,7 +282,7 @@ struct WriteLean {
 enum WriteLeanFlag : uint8_t { kLeanThrough = 3, kLeanPipe = 4, kLeanGroupsFastest = 8, kLeanWideSlots = 16 };
 static_assert(sizeof(WriteLean) <= 128, "where a launch's arguments begin to cost more");
 
-__device__ __forceinline__ WriteArgs unfold(const WriteArgs& a) { return a; }
+__device__ __forceinline__ const WriteArgs& unfold(const WriteArgs& a) { return a; }
 __device__ __forceinline__ WriteArgs unfold(const WriteLean& l) {
   WriteArgs a;
   a.key = l.key; a.value = l.value; a.key_cache = l.key_cache; a.value_cache = l.value_cache;
@@ -294,7 +293,7 @@ __device__ __forceinline__ WriteArgs unfold(const WriteLean& l) {
   a.num_tokens = l.num_tokens; a.vecs_per_row = l.vecs_per_row;
   a.vpr_shift = (l.vecs_per_row & (l.vecs_per_row - 1)) ? -1 : __builtin_ctz(l.vecs_per_row);
   a.items_per_token = 2 * l.vecs_per_row;
-  a.num_groups = a.num_token_groups = l.num_groups;
+  a.num_groups = l.num_groups;
   a.groups_fastest = l.flags & kLeanGroupsFastest; a.pipe = (l.flags & kLeanPipe) != 0; a.through = l.flags & kLeanThrough;
   a.key_token_stride = l.key_token_stride; a.value_token_stride = l.value_token_stride;
   a.key_layer_stride = a.value_layer_stride = a.cache_layer_stride = 0;
@@ -357,7 +356,7 @@ __device__ __forceinline__ bool find_slot(const WriteArgs& a, uint32_t t, int64_
 // invalid simply returns with its loads unused.
 template <int VEC, int VPT, bool PAGED, bool NT, bool NTL, typename ARGS>
 __global__ __launch_bounds__(kThreads) void write_rows_kernel(ARGS args) {
-  const WriteArgs a = unfold(args);
+  const WriteArgs& a = unfold(args);
   using V = typename VecOf<VEC>::type;
   // blockIdx.x = group * num_tokens + token by default: neighbouring workgroups
   // read neighbouring token rows of the same layers
@@ -410,7 +409,7 @@ __global__ __launch_bounds__(kThreads) void write_rows_kernel(ARGS args) {
       uint32_t r, vec;
       split(item, r, vec);
       char* dst = ((r & 1u) ? vc_row : kc_row) + (int64_t)(r >> 1) * a.cache_layer_stride + (int64_t)vec * VEC;
-      st_row<NT>(dst, data[j], a.through);
+      st_row<NT, false>(dst, data[j], a.through);
     }
   }
 }
@@ -428,13 +427,12 @@ __global__ __launch_bounds__(kThreads) void write_rows_kernel(ARGS args) {
 //     lanes (a decode step of every layer at once): no second round of workgroups,
 //     several loads in flight per lane.
 // 16-byte vectors and a power-of-two number of them per row (up to 256) only;
-// blockIdx.x = plane_group * num_token_groups + token_group.
+// blockIdx = (token group, plane group).
 template <int VPT, bool PAGED, bool NT, bool NTL, typename ARGS>
 __global__ __launch_bounds__(1024) void write_planes_kernel(ARGS args) {
-  const WriteArgs a = unfold(args);
+  const WriteArgs& a = unfold(args);
   using V = u32x4;
-  const uint32_t pg = blockIdx.x / a.num_token_groups;
-  const uint32_t tg = blockIdx.x - pg * a.num_token_groups;
+  const uint32_t tg = blockIdx.x, pg = blockIdx.y;
   const uint32_t t = tg * a.tokens_per_wg + (threadIdx.x >> a.vpr_shift);
   if (t >= a.num_tokens) return;
   const int64_t vec_off = (int64_t)(threadIdx.x & (a.vecs_per_row - 1u)) * 16;
@@ -466,7 +464,7 @@ __global__ __launch_bounds__(1024) void write_planes_kernel(ARGS args) {
     if (plane < a.num_planes) {
       char* dst = ((plane & 1u) ? a.value_cache : a.key_cache) + slot_off +
                   (int64_t)(plane >> 1) * a.cache_layer_stride;
-      st_row<NT>(dst, data[j], a.through);
+      st_row<NT, VPT <= 2>(dst, data[j], a.through);
     }
   }
 }
@@ -1275,7 +1273,8 @@ int resident_workgroups() {
 }
 
 struct WriteLaunch {
-  unsigned grid;     // workgroups
+  unsigned grid;     // workgroups; plane kernel: of one plane group
+  unsigned grid_y;   // plane groups
   unsigned threads;  // lanes per workgroup
   int vpt;
   bool nt;   // non-temporal stores
@@ -1341,11 +1340,11 @@ void launch_write(const WriteArgs& a, int vec, const WriteLaunch& l, hipStream_t
 
 template <int VPT, bool PAGED>
 void launch_planes_nt(WriteArgs a, const WriteLaunch& l, hipStream_t s) {
-  const dim3 grid(l.grid), block(l.threads);
+  const dim3 grid(l.grid, l.grid_y), block(l.threads);
   a.threads = l.threads;
   if constexpr (VPT <= 2) {  // a layer has two planes
     WriteLean lean;
-    if (l.nt && lean_of(a, PAGED, a.num_token_groups, &lean)) {
+    if (l.nt && lean_of(a, PAGED, 0, &lean)) {
       if (l.ntl) kvc::launch((write_planes_kernel<VPT, PAGED, true, true, WriteLean>), grid, block, 0, s, lean);
       else kvc::launch((write_planes_kernel<VPT, PAGED, true, false, WriteLean>), grid, block, 0, s, lean);
       return;
@@ -1496,7 +1495,7 @@ int run_write(const char* fn, const void* key, const void* value, void* kc, void
   //     would walk a cold index chain for 4 KiB of work (one layer of a long
   //     prefill chunk: 15.5 against 17.9 us at 64 MiB).
   const int64_t resident_lanes = (int64_t)resident_workgroups() * kThreads;
-  const bool plane_rows = vec == 16 && a.vpr_shift >= 0 &&
+  const bool plane_rows = vec == 16 && a.vpr_shift >= 0 && g.num_layers <= 32767 &&  // plane groups: blockIdx.y
                           (int64_t)a.vecs_per_row <= std::min(g_tune.write_planes_max_vpr, 256);
   const int64_t num_planes = 2 * g.num_layers;
   const auto plane_lanes = [&](int v) {  // lanes of the launch at v planes per lane, 256-lane workgroups
@@ -1542,22 +1541,22 @@ int run_write(const char* fn, const void* key, const void* value, void* kc, void
     a.tokens_per_wg = l.threads / a.vecs_per_row;
     a.num_planes = (uint32_t)num_planes;
     l.nt = (g_tune.write_nt & 1) != 0;
-    // Many narrow rows: stores go through the L2 as well, from 24 MiB of K and V rows on, and from 96 MiB on, which the
+    // Many narrow rows: stores go through the L2 as well, from 24 MiB of K and V rows on (at one or two planes per lane), and from 96 MiB on, which the
     // last-level cache does not hold beside what is written, the loads are non-temporal (before, the stores, both; us,
     // three sets of rows in turn, 80 layers of 256 bytes by slot: 1700 tokens 23.3, 22.5, 28.5; 2600 (102 MiB) 41.0, 39.6,
     // 39.4; 8000 115.2, 110.1, 109.8; by page table 700 tokens 12.5, 12.4, 11.8; 2300 35.4, 34.8, 38.0; 3001 49.6, 48.9,
     // 49.1; 8000 121.5, 118.5, 116.3, and with a kernel in front that writes the rows 239, 236, 208)
     const int64_t rows_bytes = g.num_tokens * num_planes * g.row_elems * E;
-    if (narrow && !a.through && rows_bytes >= (int64_t(24) << 20)) a.through = 2;
+    if (narrow && l.vpt <= 2 && !a.through && rows_bytes >= (int64_t(24) << 20)) a.through = 2;
     l.ntl = (g_tune.write_nt & 2) != 0 && (!narrow || rows_bytes >= (int64_t(96) << 20));
     const int64_t plane_groups = (a.num_planes + l.vpt - 1) / l.vpt;
+    l.grid_y = (unsigned)plane_groups;
     const int64_t max_groups = std::max<int64_t>(1, 0x7fffffffll / plane_groups);
     const int64_t max_tokens = max_groups * a.tokens_per_wg;
     for (int64_t t0 = 0; t0 < g.num_tokens; t0 += max_tokens) {
       const int64_t n_tok = std::min(max_tokens, g.num_tokens - t0);
       a.num_tokens = (uint32_t)n_tok;
-      a.num_token_groups = (uint32_t)((n_tok + a.tokens_per_wg - 1) / a.tokens_per_wg);
-      l.grid = (unsigned)(a.num_token_groups * plane_groups);
+      l.grid = (unsigned)((n_tok + a.tokens_per_wg - 1) / a.tokens_per_wg);
       a.key = (const char*)key + t0 * a.key_token_stride;
       a.value = (const char*)value + t0 * a.value_token_stride;
       if (paged) {
@@ -1570,7 +1569,7 @@ int run_write(const char* fn, const void* key, const void* value, void* kc, void
       }
       KVC_HIP(hipGetLastError());
     }
-    g_last = LastLaunch{KVC_KERNEL_WRITE_PLANES, 16, l.vpt, l.threads, l.grid, (l.nt ? 1 : 0) | (l.ntl ? 2 : 0), a.pipe};
+    g_last = LastLaunch{KVC_KERNEL_WRITE_PLANES, 16, l.vpt, l.threads, (int64_t)l.grid * l.grid_y, (l.nt ? 1 : 0) | (l.ntl ? 2 : 0), a.pipe};
     return KVC_OK;
   }
 

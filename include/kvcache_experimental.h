@@ -146,7 +146,7 @@ int kvc_build_write_index_staged(int64_t batch_size, int64_t num_kv_indices, int
 
 /*
  * kvc_rotary_plan_run for several layers whose buffers are all at hand, in one launch
- * (one for every 64 layers) where that cannot change the result: the plan has slots, rows
+ * (one for every 82 layers) where that cannot change the result: the plan has slots, rows
  * and caches are 16-byte aligned, and nothing that one layer writes is read or written by
  * another. Otherwise one launch per layer, in order. The layers share their strides and
  * number of pages; key_out may be NULL. *one_launch (may be NULL): 1 where the first

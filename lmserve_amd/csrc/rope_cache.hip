@@ -624,16 +624,23 @@ __global__ __launch_bounds__(kThreads) void rope_owner_general_kernel(RopeArgs a
 // launch (us): 64 tokens x 28 + 4 heads x 128 x 28 layers 66.5 -> 18.1 (the index build
 // alone 17.8), 256 x 32 + 8 heads x 32 109 -> 40, 717 tokens of those 199 -> 104, 3001 x
 // 8 + 1 heads x 80 490 -> 257 (5.15 TB/s).
-constexpr int kLayersPerLaunch = 64;  // 3.5 KiB of the 4 KiB a launch's arguments may take
+// A layer's value planes lie as far behind its key planes as every other layer's, so that 4 KiB, what a launch's
+// arguments may take, name 82 layers.
+constexpr int kLayersPerLaunch = 82;
 struct RopeLayersArgs {
   RopeLean l;
-  RopeLayer layer[kLayersPerLaunch];
+  int64_t key_to_value;  // bytes
+  struct {
+    const char *query, *key, *value;
+    char *query_out, *key_out, *key_cache;
+  } layer[kLayersPerLaunch];
 };
 static_assert(sizeof(RopeLayersArgs) <= 4096, "kernel arguments");
 
 template <typename T, VectorForm FORM, int NTL = 0>
 __global__ __launch_bounds__(kThreads) void rope_layers_kernel(RopeLayersArgs args) {
-  const RopeLayer p = args.layer[blockIdx.z];
+  const auto& y = args.layer[blockIdx.z];
+  const RopeLayer p{y.query, y.key, y.value, y.query_out, y.key_out, y.key_cache, y.key_cache + args.key_to_value};
   const RopeArgs a = from_lean<T, kSlots, FORM>(args.l);
   if constexpr (FORM == kPairs) rope_pairs_lane<T, kSlots, NTL>(a, p);
   else if constexpr (FORM == kRows) rope_rows_lane<T, kSlots, true, 0>(a, p);
@@ -812,7 +819,11 @@ int launch_rope_layers(RopeArgs a, const RopeLayer* layers, int64_t num_layers, 
   for (int64_t l0 = 0; l0 < num_layers; l0 += kLayersPerLaunch) {
     const int64_t n = std::min<int64_t>(kLayersPerLaunch, num_layers - l0);
     args.l = lean_of<kSlots>(a, T::kBytes);
-    std::copy(layers + l0, layers + l0 + n, args.layer);
+    args.key_to_value = a.value_cache - a.key_cache;
+    for (int64_t l = 0; l < n; ++l) {
+      const RopeLayer& p = layers[l0 + l];
+      args.layer[l] = {p.query, p.key, p.value, p.query_out, p.key_out, p.key_cache};
+    }
     const dim3 grid(a.groups_per_token, (unsigned)num_tokens, (unsigned)n), block(threads);
     if (form == kPairs && nt) kvc::launch((rope_layers_kernel<T, kPairs, 3>), grid, block, 0, s, args);
     else if (form == kPairs) kvc::launch((rope_layers_kernel<T, kPairs>), grid, block, 0, s, args);

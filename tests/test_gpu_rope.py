@@ -800,3 +800,21 @@ def test_sizes_beyond_the_short_launch_arguments(gpu, what, D, rd):
         q, v = (strided, v) if what == "query" else (q, strided)
     plan.run(q, k, v, got_pool, query_out=got)
     assert torch.equal(got, want) and torch.equal(got_pool, pool)
+
+
+@pytest.mark.parametrize("L", [82, 83])     # as many layers as a launch's arguments name, and one more
+def test_as_many_layers_as_one_launch_names(gpu, L):
+    T, Hq, Hkv, D, bs = 3, 4, 2, 64, 16
+    q, k, v, pos, cs = (t.to(gpu) for t in _case(gpu, T, Hq, Hkv, D, D, torch.bfloat16, seed=L))
+    slots = torch.tensor([17, 2, 30], device=gpu)
+    none = torch.zeros(T, dtype=torch.int32, device=gpu)
+    plan = kvc.PagedRotaryWritePlan(none, pos, none[:1], torch.tensor([0, 1], dtype=torch.int32, device=gpu),
+                                    none[:1], cs, Hq, Hkv, D, bs, slots=slots)
+    qs, ks, vs = ([t * (l + 1) for l in range(L)] for t in (q, k, v))
+    want_q, want_pool = torch.zeros(L, T, Hq * D, dtype=q.dtype, device=gpu), \
+        torch.zeros(L, 2, 2, bs, Hkv, D, dtype=q.dtype, device=gpu)
+    for l in range(L):
+        plan.run(qs[l], ks[l], vs[l], want_pool[l], query_out=want_q[l])
+    got_q, got_pool = torch.zeros_like(want_q), torch.zeros_like(want_pool)
+    assert plan.run_layers(qs, ks, vs, list(got_pool), list(got_q))
+    assert torch.equal(got_q, want_q) and torch.equal(got_pool, want_pool)

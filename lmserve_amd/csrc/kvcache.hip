@@ -87,7 +87,7 @@ struct Tuning {
   int copy_order = 0;       // copy_tiles: 1 = walk all blocks of a layer before the next layer
   int write_vpt = 0;        // vectors per lane in write_rows, 0 = by size
   int write_nt = 3;         // write kernels: bit 0 non-temporal stores, bit 1 non-temporal loads (rows of
-                            // 1 KiB or more, and narrower ones from 96 MiB on: see run_write). Loads:
+                            // 1 KiB or more, and narrower ones from 128 MiB on: see run_write). Loads:
                             // -3 % at the 64 MiB decode step, -2 to -3 % at 224-256 MiB, -10 to -15 %
                             // for one layer per launch when the K/V rows come from HBM, neutral when
                             // they are still in cache (one source set, or a producer kernel in front)
@@ -1541,14 +1541,14 @@ int run_write(const char* fn, const void* key, const void* value, void* kc, void
     a.tokens_per_wg = l.threads / a.vecs_per_row;
     a.num_planes = (uint32_t)num_planes;
     l.nt = (g_tune.write_nt & 1) != 0;
-    // Many narrow rows: stores go through the L2 as well, from 24 MiB of K and V rows on (at one or two planes per lane), and from 96 MiB on, which the
+    // Many narrow rows: stores go through the L2 as well, from 24 MiB of K and V rows on (at one or two planes per lane), and from 128 MiB on, which the
     // last-level cache does not hold beside what is written, the loads are non-temporal (before, the stores, both; us,
     // three sets of rows in turn, 80 layers of 256 bytes by slot: 1700 tokens 23.3, 22.5, 28.5; 2600 (102 MiB) 41.0, 39.6,
-    // 39.4; 8000 115.2, 110.1, 109.8; by page table 700 tokens 12.5, 12.4, 11.8; 2300 35.4, 34.8, 38.0; 3001 49.6, 48.9,
+    // 39.4 and, one set that is still in cache, 3001 (117 MiB) 41.3, 40.0, 48.0; 8000 115.2, 110.1, 109.8; by page table 700 tokens 12.5, 12.4, 11.8; 2300 35.4, 34.8, 38.0; 3001 49.6, 48.9,
     // 49.1; 8000 121.5, 118.5, 116.3, and with a kernel in front that writes the rows 239, 236, 208)
     const int64_t rows_bytes = g.num_tokens * num_planes * g.row_elems * E;
     if (narrow && l.vpt <= 2 && !a.through && rows_bytes >= (int64_t(24) << 20)) a.through = 2;
-    l.ntl = (g_tune.write_nt & 2) != 0 && (!narrow || rows_bytes >= (int64_t(96) << 20));
+    l.ntl = (g_tune.write_nt & 2) != 0 && (!narrow || rows_bytes >= (int64_t(128) << 20));
     const int64_t plane_groups = (a.num_planes + l.vpt - 1) / l.vpt;
     l.grid_y = (unsigned)plane_groups;
     const int64_t max_groups = std::max<int64_t>(1, 0x7fffffffll / plane_groups);

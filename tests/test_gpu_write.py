@@ -732,7 +732,7 @@ def test_strides_beyond_the_short_launch_arguments(gpu, what, planes, by):
     assert torch.equal(cache, want)
 
 
-@pytest.mark.parametrize("T,L", [(1026, 48), (4098, 48), (1024, 49)])   # 24 and 96 MiB of K and V rows, and more
+@pytest.mark.parametrize("T,L", [(1026, 48), (5462, 48), (1024, 49)])   # 24 and 128 MiB of K and V rows, and more
 @pytest.mark.parametrize("by", ["slots", "pages"])
 def test_many_narrow_rows(gpu, T, L, by):
     """Rows of 256 bytes of all layers in one launch, either side of where its stores and loads change."""

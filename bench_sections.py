@@ -923,7 +923,7 @@ def bench_decode_step_graph(torch, kvc, wl, s8, pool, L, num_blocks, dev, steps=
 def bench_load_policy(torch, kvc, wl, dev):
     """A/B of plain against non-temporal loads of the source rows, per layer, in one
     process: the per-layer write (`write_nt` 1 against 3) and the fused rotation
-    (`rope_nt` 0 against 3), with the layers of a replayed step cycling through
+    (`rope_nt` 4 against 3), with the layers of a replayed step cycling through
     `sets` distinct source sets (1 = rows still in cache, as after the projection
     of a forward pass; one set per layer = rows from HBM or the last-level cache).
     Two rounds, interleaved; microseconds per layer from a hipGraph replay."""
@@ -958,7 +958,7 @@ def bench_load_policy(torch, kvc, wl, dev):
                               query_out=qo)
 
             for fn, knob, values, what in ((write, "write_nt", (1, 3), "PagedKVWritePlan.append"),
-                                           (rotate, "rope_nt", (0, 3), "PagedRotaryWritePlan.run")):
+                                           (rotate, "rope_nt", (4, 3), "PagedRotaryWritePlan.run")):
                 us = {val: [] for val in values}
                 for _ in range(2):
                     for val in values:

@@ -42,7 +42,8 @@ extern "C" {
  *   "auto_min_extent_bytes"           KVC_SWAP_AUTO: mean bytes per PCIe copy from which a call is staged
  *   "rope_threads"                    lanes per workgroup in the rotation kernel (0 = default, 64, 128, 192, 256)
  *   "rope_nt"                         non-temporal loads in that kernel: bit 0 the K and V rows, bit 1 the Q rows,
- *                                     0 = by size (plain where a rotation in place takes a form of its own)
+ *                                     4 = plain loads, 0 = by size (plain where a rotation in place takes a form of
+ *                                     its own)
  *   "disk_bounce_mib"                 MiB of aligned staging per thread in the disk tier
  *   "host_rows_nt"                    row copies on host threads: 1 = stores that go past the cache (default)
  * Unknown key: KVC_ERR_INVALID_ARG. kvc_reset_tuning puts every knob back to its
@@ -60,17 +61,25 @@ enum {
   KVC_KERNEL_WRITE_ROWS = 1,        /* token per workgroup                          */
   KVC_KERNEL_COPY_TILES = 2,        /* block copy, gather, scatter, direct swap     */
   KVC_KERNEL_WRITE_PLANES = 3,      /* lanes over consecutive tokens of one plane   */
-  KVC_KERNEL_WRITE_RUNS = 4         /* workgroup per chunk of a (block run, plane)  */
+  KVC_KERNEL_WRITE_RUNS = 4,        /* workgroup per chunk of a (block run, plane)  */
+  KVC_KERNEL_ROTATE = 5             /* rotation, alone or with the K/V write        */
 };
 enum {
   KVC_LAUNCH_KERNEL = 0,       /* one of KVC_KERNEL_*                               */
   KVC_LAUNCH_VEC_BYTES = 1,    /* bytes per load/store instruction per lane         */
-  KVC_LAUNCH_PER_LANE = 2,     /* vectors (or planes) in flight per lane            */
+  KVC_LAUNCH_PER_LANE = 2,     /* vectors (or planes) in flight per lane; rotation: a kvc_rope_form */
   KVC_LAUNCH_THREADS = 3,      /* lanes per workgroup                               */
   KVC_LAUNCH_GRID = 4,         /* workgroups                                        */
-  KVC_LAUNCH_NON_TEMPORAL = 5, /* bit 0 stores, bit 1 loads (tile kernel: both = 1) */
+  KVC_LAUNCH_NON_TEMPORAL = 5, /* bit 0 stores, bit 1 loads (tile kernel: both = 1; rotation: loads, as "rope_nt") */
   KVC_LAUNCH_PIPE = 6,         /* write kernels: 1 = a lane waits for each of its loads */
   KVC_LAUNCH_SWAP_MODE = 7     /* the kvc_swap_mode this thread's last swap call ran in  */
+};
+enum kvc_rope_form {
+  KVC_ROPE_ELEMENTS = 0,  /* an element pair per lane                             */
+  KVC_ROPE_PAIRS = 1,     /* a pair of vectors per lane                           */
+  KVC_ROPE_ROWS = 2,      /* the same vector of two heads per lane                */
+  KVC_ROPE_OWNER = 3,     /* a pair of vectors, and what else a lane has to carry */
+  KVC_ROPE_OWNER_TAIL = 4
 };
 int64_t kvc_last_launch_info(int what);
 

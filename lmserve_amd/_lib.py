@@ -42,6 +42,8 @@ KVC_KERNEL_WRITE_ROWS = 1
 KVC_KERNEL_COPY_TILES = 2
 KVC_KERNEL_WRITE_PLANES = 3
 KVC_KERNEL_WRITE_RUNS = 4
+KVC_KERNEL_ROTATE = 5
+KVC_ROPE_ELEMENTS, KVC_ROPE_PAIRS, KVC_ROPE_ROWS, KVC_ROPE_OWNER, KVC_ROPE_OWNER_TAIL = range(5)
 KVC_LAUNCH_KERNEL = 0
 KVC_LAUNCH_VEC_BYTES = 1
 KVC_LAUNCH_PER_LANE = 2

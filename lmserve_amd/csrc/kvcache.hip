@@ -2433,6 +2433,10 @@ int scratch_of_current_device(int64_t** out) {
 }  // namespace
 
 namespace kvc {
+void record_rotation(int vec, int form, int threads, int64_t grid, int nt) {
+  g_last = LastLaunch{KVC_KERNEL_ROTATE, vec, form, threads, grid, nt};
+}
+
 int launch_resolve_slots(const char* fn, const int32_t* batch_indices, const int32_t* positions,
                          const int32_t* kv_indices, const int32_t* kv_indptr, int64_t batch_size,
                          int64_t num_kv_indices, int64_t page_size, int64_t nnz, int64_t* slots,

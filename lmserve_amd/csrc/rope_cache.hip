@@ -208,7 +208,10 @@ struct RopeLayer {
 enum Addressing : int { kNoCache, kSlots, kPages };
 
 // The kernels of rows of aligned 16-byte vectors, and the one of all other rows
-enum VectorForm { kElements, kPairs, kRows, kOwner, kOwnerTail };
+enum VectorForm {
+  kElements = KVC_ROPE_ELEMENTS, kPairs = KVC_ROPE_PAIRS, kRows = KVC_ROPE_ROWS, kOwner = KVC_ROPE_OWNER,
+  kOwnerTail = KVC_ROPE_OWNER_TAIL
+};
 
 template <Addressing ADDR> struct LeanOf { using type = RopeLean; };
 template <> struct LeanOf<kPages> { using type = RopeLeanPages; };
@@ -789,6 +792,7 @@ int launch_rope(RopeArgs a, int64_t num_tokens, VectorForm form, int ntl, unsign
     else if (a.batch_indices) launch_element<T, kPages>(a, grid, block, s);
     else launch_element<T, kSlots>(a, grid, block, s);
     KVC_HIP(hipGetLastError());
+    kvc::record_rotation(T::kBytes, form, (int)threads, grid.x, 0);
     return KVC_OK;
   }
   constexpr int64_t kMaxY = 65535;  // tokens of one launch
@@ -799,6 +803,8 @@ int launch_rope(RopeArgs a, int64_t num_tokens, VectorForm form, int ntl, unsign
     else if (a.batch_indices) launch_vector<T, kPages>(a, form, ntl, grid, block, s);
     else launch_vector<T, kSlots>(a, form, ntl, grid, block, s);
     KVC_HIP(hipGetLastError());
+    kvc::record_rotation(16, form, (int)threads, (int64_t)grid.x * grid.y,
+                         form == kOwner || form == kOwnerTail ? 0 : ntl);
     a.query += kMaxY * a.q_token_stride;
     a.key += kMaxY * a.k_token_stride;
     if (a.value) a.value += kMaxY * a.v_token_stride;
@@ -831,6 +837,7 @@ int launch_rope_layers(RopeArgs a, const RopeLayer* layers, int64_t num_layers, 
     else if (form == kOwner) kvc::launch((rope_layers_kernel<T, kOwner>), grid, block, 0, s, args);
     else kvc::launch((rope_layers_kernel<T, kOwnerTail>), grid, block, 0, s, args);
     KVC_HIP(hipGetLastError());
+    kvc::record_rotation(16, form, (int)threads, (int64_t)grid.x * grid.y * grid.z, form == kPairs && nt ? 3 : 0);
   }
   return KVC_OK;
 }
@@ -1052,7 +1059,7 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
     // 2048 (24 MiB)                    9.3 and 10.9; 18.1 and 18.0; 24.6 and 24.1
     // Steps of the rows form lose by it (8192 tokens x 24 layers, 32 + 8 heads x 80, 32 rotated, 570 and 587 us; 16 layers
     // of 32 + 8 x 64 323 and 330), and so does a rotation without the cache (5000 x 32 + 8 x 128, 954 and 961).
-    if (!ntl && form == kPairs && c && g.num_tokens * (heads + g.num_kv_heads) * g.head_dim * E >= (int64_t(40) << 20))
+    if (!kvc::g_rope_tune.nt && form == kPairs && c && g.num_tokens * (heads + g.num_kv_heads) * g.head_dim * E >= (int64_t(40) << 20))
       ntl = 3;
     if (form != kRows) {
       a.split = a.pairs_per_head;

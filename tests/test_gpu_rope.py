@@ -818,3 +818,23 @@ def test_as_many_layers_as_one_launch_names(gpu, L):
     got_q, got_pool = torch.zeros_like(want_q), torch.zeros_like(want_pool)
     assert plan.run_layers(qs, ks, vs, list(got_pool), list(got_q))
     assert torch.equal(got_q, want_q) and torch.equal(got_pool, want_pool)
+
+
+def test_load_policy_of_the_rotation_by_size_and_by_request(gpu):
+    """Non-temporal loads from 40 MiB of rows on; `rope_nt` 4 keeps plain ones there, as 0 does below."""
+    Hq, Hkv, D, bs, dtype = 32, 8, 128, 16, torch.bfloat16
+    cs = rotary.make_cos_sin_cache(D, 4096, 500000.0, dtype=dtype, device=gpu)
+    for T, by_size in ((3413, 0), (3414, 3)):
+        qkv = torch.randn(T, (Hq + 2 * Hkv) * D, dtype=dtype, device=gpu)
+        q, k, v = qkv.split([Hq * D, Hkv * D, Hkv * D], dim=1)
+        pos = torch.arange(T, dtype=torch.int32, device=gpu)
+        slots = torch.arange(T, device=gpu)
+        outs = []
+        for asked, ran in ((0, by_size), (4, 0), (1, 1), (2, 2), (3, 3)):
+            _lib.set_tuning("rope_nt", asked)
+            pool = torch.zeros(T // bs + 1, 2, bs, Hkv, D, dtype=dtype, device=gpu)
+            q_out, _ = kvc.rotary_pos_emb_and_cache(q, k, v, pos, cs, D, pool, slots, return_key=False)
+            last = _lib.last_launch()
+            assert (last["kernel"], last["per_lane"], last["non_temporal"]) == (_lib.KVC_KERNEL_ROTATE, _lib.KVC_ROPE_PAIRS, ran)
+            outs.append((q_out, pool))
+        assert all(torch.equal(a, b) for o in outs[1:] for a, b in zip(outs[0], o))

@@ -72,7 +72,9 @@ enum {
   KVC_LAUNCH_GRID = 4,         /* workgroups                                        */
   KVC_LAUNCH_NON_TEMPORAL = 5, /* bit 0 stores, bit 1 loads (tile kernel: both = 1; rotation: loads, as "rope_nt") */
   KVC_LAUNCH_PIPE = 6,         /* write kernels: 1 = a lane waits for each of its loads */
-  KVC_LAUNCH_SWAP_MODE = 7     /* the kvc_swap_mode this thread's last swap call ran in  */
+  KVC_LAUNCH_SWAP_MODE = 7,    /* the kvc_swap_mode this thread's last swap call ran in  */
+  KVC_LAUNCH_ORDER = 8,        /* block copies: 1 = all blocks of a layer before the next layer */
+  KVC_LAUNCH_RUN = 9           /* large block copies: neighbouring chunks that go to one XCD */
 };
 enum kvc_rope_form {
   KVC_ROPE_ELEMENTS = 0,  /* an element pair per lane                             */

@@ -52,6 +52,8 @@ KVC_LAUNCH_GRID = 4
 KVC_LAUNCH_NON_TEMPORAL = 5
 KVC_LAUNCH_PIPE = 6
 KVC_LAUNCH_SWAP_MODE = 7
+KVC_LAUNCH_ORDER = 8
+KVC_LAUNCH_RUN = 9
 
 KVC_ABI_VERSION = 6
 FAST_INTERFACE = 2      # names and arguments of the `_kvc_fast` extension's functions
@@ -292,4 +294,6 @@ def last_launch() -> dict:
             "threads": L.kvc_last_launch_info(KVC_LAUNCH_THREADS),
             "grid": L.kvc_last_launch_info(KVC_LAUNCH_GRID),
             "non_temporal": L.kvc_last_launch_info(KVC_LAUNCH_NON_TEMPORAL),
-            "pipe": L.kvc_last_launch_info(KVC_LAUNCH_PIPE)}
+            "pipe": L.kvc_last_launch_info(KVC_LAUNCH_PIPE),
+            "order": L.kvc_last_launch_info(KVC_LAUNCH_ORDER),
+            "run": L.kvc_last_launch_info(KVC_LAUNCH_RUN)}

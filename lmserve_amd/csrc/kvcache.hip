@@ -176,7 +176,7 @@ Knob* find_knob(const char* key) {
 
 // What the most recent kernel launch of this thread looked like (kvc_last_launch_info).
 struct LastLaunch {
-  int64_t kernel = KVC_KERNEL_NONE, vec = 0, per_lane = 0, threads = 0, grid = 0, nt = 0, pipe = 0;
+  int64_t kernel = KVC_KERNEL_NONE, vec = 0, per_lane = 0, threads = 0, grid = 0, nt = 0, pipe = 0, order = 0, run = 0;
 };
 thread_local LastLaunch g_last;
 thread_local int g_last_swap_mode = -1;  // the mode this thread's most recent swap call ran in
@@ -657,12 +657,15 @@ struct StreamArgs {
 struct StreamPlace {
   uint32_t i, layer, chunk;
 };
+// TURN: an XCD takes the next run of every next span, not the same one of all.
+template <bool TURN = false>
 __device__ __forceinline__ StreamPlace stream_place(const StreamArgs& a) {
   uint32_t w = blockIdx.x;
   const uint32_t span = 8 * a.xcd_run;
   const uint32_t in_span = w % span;
   // a span that the launch does not fill stays in grid order
-  if (w - in_span + span <= a.total_chunks) w = w - in_span + (in_span & 7u) * a.xcd_run + (in_span >> 3);
+  if (w - in_span + span <= a.total_chunks)
+    w = w - in_span + ((in_span + (TURN ? w / span : 0)) & 7u) * a.xcd_run + (in_span >> 3);
   const uint32_t tile = w / a.chunks_per_tile;
   const uint32_t chunk = w - tile * a.chunks_per_tile;
   if (a.layer_slowest) {
@@ -714,6 +717,11 @@ __global__ __launch_bounds__(kThreads) void stream_pairs_kernel(StreamArgs a, Pa
 // throughout, then this, us: 64 x 2 x 32 of 64 KiB 73.3 and 64.7, 30 x 2 x 80 85.7 and 74.6, 200 x
 // 2 x 28 of 32 KiB 106 and 93, 1500 x 2 x 12 of 18 KiB 199 and 190, 2000 x 2 x 80 of 8 KiB 726 and 715; 600 x 3 x 32 of 64
 // KiB 871 and 850, 60 x 3 x 24 of 40 KiB 47.9 and 43.2.
+// Items differ in their destinations, and often by turns: four copies of a block are an item of three and one of one. In
+// layer order a tile of 64 KiB is one run, and the XCDs that got the threes wrote three times what the others did. So
+// the XCDs' places move by a run from span to span (the earlier form, blocks in order; layers without the turn; with it,
+// us: 266 x 4 x 12 of 64 KiB 231, 249, 213; 43 x 4 x 12 of 128 KiB 74, 80, 70; 60 x 80 of 64 KiB, every third to four
+// blocks and the others to one, 197, 215, 167). Not in the larger workgroups: 0 to 1 % slower.
 // The list holds FAN + 1 words an item, its source and its destinations (-1: none), so
 // that one scalar load brings an item's ids: with a table of offsets and a loop over the
 // destinations each id is a dependent load of its own (6 x 2 8.7).
@@ -724,7 +732,7 @@ struct FanList {
 
 template <int THREADS, int UNROLL, int FAN>
 __device__ __forceinline__ void fan_tile_chunk(const StreamArgs& a, const int32_t* list) {
-  const auto [i, layer, chunk] = stream_place(a);
+  const auto [i, layer, chunk] = stream_place<THREADS == 64>(a);
   int32_t id[FAN + 1];
 #pragma unroll
   for (int d = 0; d <= FAN; ++d) id[d] = list[(FAN + 1) * i + d];
@@ -1788,7 +1796,7 @@ int launch_stream(const TileArgs& t, TileSides sides, int64_t n, hipStream_t s, 
   else if (plain_load) kvc::launch((stream_tiles_kernel<256, 2, false, true>), grid, block, five_per_cu, s, a);
   else kvc::launch((stream_tiles_kernel<256, 2, true, true>), grid, block, five_per_cu, s, a);
   g_last = LastLaunch{KVC_KERNEL_COPY_TILES, 16, (int64_t)unroll, (int64_t)threads, (int64_t)a.total_chunks,
-                      plain_load || plain_store ? 0 : 1};
+                      plain_load || plain_store ? 0 : 1, 0, a.layer_slowest, a.xcd_run};
   KVC_HIP(hipGetLastError());
   return KVC_OK;
 }
@@ -1870,7 +1878,7 @@ int launch_tiles_vec(TileArgs a, int unroll, int max_wgs, hipStream_t s, bool nt
     case 8: launch_tiles_nt<VEC, 8>(a, (unsigned)grid, s, nt); break;
     default: launch_tiles_nt<VEC, 16>(a, (unsigned)grid, s, nt); break;
   }
-  g_last = LastLaunch{KVC_KERNEL_COPY_TILES, VEC, unroll, kThreads, (int64_t)grid, nt ? 1 : 0};
+  g_last = LastLaunch{KVC_KERNEL_COPY_TILES, VEC, unroll, kThreads, (int64_t)grid, nt ? 1 : 0, 0, a.layer_slowest, 1};
   KVC_HIP(hipGetLastError());
   return KVC_OK;
 }
@@ -1921,7 +1929,8 @@ int launch_fan_copy(StreamArgs a, FanShape shape, int fan, int64_t pairs, const 
     case 4: launch_fan<kThreads, 4>(a, fan, list, device_list, lds, s); break;
     default: launch_fan<kThreads, 8>(a, fan, list, device_list, lds, s); break;
   }
-  g_last = LastLaunch{KVC_KERNEL_COPY_TILES, 16, shape.unroll, (int64_t)threads, (int64_t)a.total_chunks, 1};
+  g_last = LastLaunch{KVC_KERNEL_COPY_TILES, 16, shape.unroll, (int64_t)threads, (int64_t)a.total_chunks, 1, 0,
+                      a.layer_slowest, a.xcd_run};
   KVC_HIP(hipGetLastError());
   return KVC_OK;
 }
@@ -2503,6 +2512,8 @@ int64_t kvc_last_launch_info(int what) {
     case KVC_LAUNCH_NON_TEMPORAL: return g_last.nt;
     case KVC_LAUNCH_PIPE: return g_last.pipe;
     case KVC_LAUNCH_SWAP_MODE: return g_last_swap_mode;
+    case KVC_LAUNCH_ORDER: return g_last.order;
+    case KVC_LAUNCH_RUN: return g_last.run;
     default: return KVC_ERR_INVALID_ARG;
   }
 }

@@ -439,3 +439,28 @@ def test_order_of_large_copies(gpu, tile_bytes, n):
     want[:, ids[n:2 * n]] = pool[:, ids[:n]]
     kvc.copy_blocks(pool, torch.stack([ids[:n], ids[n:2 * n]], 1).flatten().contiguous())
     assert torch.equal(pool, want)
+
+
+@pytest.mark.parametrize("tile_bytes,L,fans,threads", [
+    (65536, 28, (4,) * 19, 64),            # items of three and one by turns, a tile to a run
+    (65536, 28, (4, 1, 1) * 10, 64), (131088, 12, (1, 7) * 11, 64), (49152, 28, (4, 2) * 18, 64),
+    (65536, 28, (5, 6, 7) * 16, 256), (65552, 9, (3, 2, 3) * 30, 256),
+    (65536, 28, (2,) * 37 + (3,), 64),     # a last span that is not full
+])
+def test_large_forks_of_uneven_items(gpu, tile_bytes, L, fans, threads):
+    """Items of few and of many destinations by turns, which the XCDs share out between them: against NumPy."""
+    n = sum(fans)
+    nb = n + len(fans) + 1
+    pool = random_pool((L, nb, tile_bytes // 2), seed=n)
+    dpool = to_bf16(pool, gpu)
+    ids = np.random.default_rng(n).permutation(nb).tolist()
+    d, at = {}, len(fans)
+    for src, fan in zip(ids, fans):
+        d[src] = ids[at:at + fan]
+        at += fan
+    for src, dsts in d.items():
+        pool[:, dsts] = pool[:, src:src + 1]
+    kvc.copy_blocks(dpool, d)
+    ran = _lib.last_launch()
+    assert (ran["per_lane"], ran["threads"], ran["order"]) == (1, threads, 1)
+    assert np.array_equal(bits_of(dpool), pool)

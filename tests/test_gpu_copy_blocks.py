@@ -445,7 +445,7 @@ def test_order_of_large_copies(gpu, tile_bytes, n):
     (65536, 28, (4,) * 19, 64),            # items of three and one by turns, a tile to a run
     (65536, 28, (4, 1, 1) * 10, 64), (131088, 12, (1, 7) * 11, 64), (49152, 28, (4, 2) * 18, 64),
     (65536, 28, (5, 6, 7) * 16, 256), (65552, 9, (3, 2, 3) * 30, 256),
-    (65536, 28, (2,) * 37 + (3,), 64),     # a last span that is not full
+    (65536, 28, (2,) * 37 + (1,), 64),     # a last span that is not full
 ])
 def test_large_forks_of_uneven_items(gpu, tile_bytes, L, fans, threads):
     """Items of few and of many destinations by turns, which the XCDs share out between them: against NumPy."""

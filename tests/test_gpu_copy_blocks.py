@@ -464,3 +464,19 @@ def test_large_forks_of_uneven_items(gpu, tile_bytes, L, fans, threads):
     ran = _lib.last_launch()
     assert (ran["per_lane"], ran["threads"], ran["order"]) == (1, threads, 1)
     assert np.array_equal(bits_of(dpool), pool)
+
+
+@pytest.mark.parametrize("tile_bytes,n,L,run", [
+    (8192, 6143, 1, 64), (8192, 6144, 1, 256), (8208, 1023, 3, 64), (8208, 1024, 3, 256),   # either side of three spans
+])
+def test_runs_of_scatters(gpu, tile_bytes, n, L, run):
+    g = torch.Generator(device=gpu).manual_seed(n)
+    nb = n + 9
+    pool = torch.randint(-2**31, 2**31 - 1, (L, nb, tile_bytes // 4), dtype=torch.int32, device=gpu, generator=g)
+    dense = torch.randint(-2**31, 2**31 - 1, (n, L, tile_bytes // 4), dtype=torch.int32, device=gpu, generator=g)
+    ids = torch.randperm(nb, device=gpu, generator=g)[:n].contiguous()
+    want = pool.clone()
+    want[:, ids] = dense.transpose(0, 1)
+    kvc.scatter_blocks(pool, ids, dense)
+    assert _lib.last_launch()["run"] == run
+    assert torch.equal(pool, want)

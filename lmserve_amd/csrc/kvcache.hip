@@ -1113,9 +1113,13 @@ __global__ __launch_bounds__(kThreads) void upload_kernel(const int4* src, int4*
 
 // The same for the index arrays of a step, with what seq_lens_kernel and batch_indices_positions_kernel make of them:
 // `cu` the new tokens' prefix sums, `indptr` and `last` the block tables', all in the staging buffer. Bound: launches and
-// the link's latency, so the requests' words are asked for ahead of the copy and a wavefront writes a request's tokens.
+// the link's latency, so the requests' words are asked for ahead of the copy and a wavefront writes a request's tokens,
+// the whole workgroup those of a long one.
 // 63 requests, 838 tokens, 6000 block ids, three launches, each behind the one before, and this: the call 13.4 and 7.9 us,
-// with the device's wait 25.5 and 20.0, the device's part of calls that are queued 13.1 and 9.3.
+// with the device's wait 25.5 and 20.0, the device's part of calls that are queued 13.1 and 9.3. Prompts (three launches; a
+// wavefront whatever its request's length; this; us with the wait): 8192 tokens 28.4, 27.2, 23.4, with 255 requests of one
+// 32.0, 30.5, 25.5; 100000 105, 122, 85; 300000 247, 304, 192.
+constexpr int kLongRequest = 256;  // new tokens
 struct UploadIndexArgs {
   const int4* src;
   int4* dst;
@@ -1148,16 +1152,22 @@ __global__ __launch_bounds__(kThreads) void upload_index_kernel(UploadIndexArgs 
     begins[tid] = begin;
     ends[tid] = end;
     firsts[tid] = max(pages, 0) * a.page_size + last - (end - begin);
-    __syncthreads();
+    const auto is_long = [](int64_t from, int64_t to) { return to - from > kLongRequest; };
+    const bool any_long = __syncthreads_or(is_long(begin, end));
     const int count = (int)min(mine - at, (int64_t)kThreads);
-    for (int i = tid >> 6; i < count; i += kThreads / 64) {
-      const int32_t from = begins[i], to = ends[i], first = firsts[i];
+    const auto write = [&](int i, int lane, int lanes) {
+      const int32_t from = begins[i], first = firsts[i];
       const int32_t request = (int32_t)(blockIdx.x + (at + i) * a.grid);
-      for (int64_t j = max(from, 0) + (tid & 63); j < min((int64_t)to, a.nnz); j += 64) {
+      for (int64_t j = max(from, 0) + lane; j < min((int64_t)ends[i], a.nnz); j += lanes) {
         a.batch_indices[j] = request;
         a.positions[j] = first + (int32_t)(j - from);
       }
-    }
+    };
+    for (int i = tid >> 6; i < count; i += kThreads / 64)
+      if (!is_long(begins[i], ends[i])) write(i, tid & 63, 64);
+    if (any_long)
+      for (int i = 0; i < count; ++i)
+        if (is_long(begins[i], ends[i])) write(i, tid, kThreads);
   }
   tell_host(a.read_flags, a.flag_value);
 }

@@ -368,3 +368,26 @@ def test_upload_of_index_arrays_refuses_what_lies_outside(gpu):
         rc = lib.kvc_staging_upload_index(dst.data_ptr(), bytes_, cu, ptr, last, batch, 16, 4, out.data_ptr(),
                                           out.data_ptr(), torch.cuda.current_stream().cuda_stream)
         assert rc == _lib.KVC_ERR_INVALID_ARG
+
+
+@pytest.mark.parametrize("sizes", [
+    [256], [257], [1, 256, 257, 0, 512, 255], [70001, 3],
+    [1] * 33000 + [300, 2, 258],       # in the second round of a workgroup's lanes
+])
+def test_long_requests_uploaded_in_one_launch(gpu, sizes):
+    """Requests of more tokens than a workgroup has lanes, among short ones, in the order given."""
+    sizes = np.asarray(sizes)
+    rng = np.random.default_rng(len(sizes))
+    filled = rng.integers(1, 40, len(sizes))
+    blocks = (filled + sizes + 15) // 16
+    i32 = lambda a: np.asarray(a, dtype=np.int32)
+    cu, indptr = i32(np.concatenate([[0], np.cumsum(sizes)])), i32(np.concatenate([[0], np.cumsum(blocks)]))
+    requests = np.repeat(np.arange(len(sizes)), sizes)
+    positions = np.arange(cu[-1]) - cu[requests] + filled[requests]
+    host = kvc.KVIndexInputs(i32(positions), cu, 0, i32(rng.integers(0, 1000, indptr[-1])), indptr,
+                             i32((filled + sizes - 1) % 16 + 1), i32(requests), i32(positions),
+                             positions.astype(np.int64), list(range(len(sizes))))
+    got = kvc.to_device(host, 16, gpu)
+    for name in ("batch_indices", "positions", "position_ids", "cu_seqlens_q", "kv_block_indices", "kv_block_indptrs",
+                 "kv_last_block_lens", "slot_mapping"):
+        assert np.array_equal(getattr(got, name).cpu().numpy(), getattr(host, name)), name

@@ -263,9 +263,9 @@ struct WriteArgs {
 
 // What a launch of one layer needs of it, in less than the 128 bytes at which a launch begins to cost the host more: a
 // write per layer at decode sizes is bound by that. WriteArgs, with the 256 bytes of launch geometry that reading blockDim
-// adds, and this, us a launch and us a step, by slot and by page table alike (medians of 16 runs, the host in its slower
-// state; in its faster one both take 2.45): 32 layers of 256 tokens x 8 heads x 128 3.3 to 3.9 and 3.2 to 3.4, 125 to 148
-// and 126 to 131; 24 of 838 x 8 x 80 3.4 to 3.9 and 3.3 to 3.5; 16 of 2 x 8 x 64 3.2 to 3.9 and 3.3 to 3.6.
+// adds, and this, us a launch and us a step, by slot and by page table alike (medians of 16 runs in turn, ranges of a few
+// hundredths; where the host is in its faster state both take 2.45 a launch): 32 layers of 256 tokens x 8 heads x 128
+// 3.26 and 3.17, 105.5 and 102.8; 24 of 838 x 8 x 80 3.29 and 3.18, 80.3 and 77.7; 16 of 2 x 8 x 64 3.27 and 3.18, 53.8 and 52.2.
 struct WriteLean {
   const char *key, *value;
   char *key_cache, *value_cache;
@@ -1299,10 +1299,14 @@ struct WriteLaunch {
   bool ntl;  // non-temporal loads
 };
 
-// The lean arguments of a launch of one layer, if they hold it. Page-table counts are compared with 32-bit indices:
+// The lean arguments of a launch of one layer, if they hold it and it is one that gains. By page table, where what they fold
+// away stands ahead of three steps of loads, larger launches lose more on the device than the host saves (WriteArgs and
+// WriteLean, us: 8192 tokens x 8 heads x 128 13.1 and 13.6, 13107 x 8 x 80 13.5 and 14.2; from 120 MiB on up to 15 % at
+// rows of 576 bytes; below 12 MiB of K and V rows within 1 %). Page-table counts are compared with 32-bit indices:
 // beyond every such index they are all the same.
 bool lean_of(const WriteArgs& a, bool paged, uint32_t num_groups, WriteLean* l) {
   const auto u32 = [](int64_t v) { return v >= 0 && v <= (int64_t)UINT32_MAX; };
+  if (paged && (int64_t)a.num_tokens * a.items_per_token * 16 > (int64_t(12) << 20)) return false;
   if (a.items_per_token != 2 * a.vecs_per_row || a.bs_shift < 0 || !u32(a.key_token_stride) || !u32(a.value_token_stride) ||
       !u32(a.cache_block_stride) || !u32(a.cache_slot_stride) || !u32(a.num_cache_blocks))
     return false;

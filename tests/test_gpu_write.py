@@ -756,3 +756,25 @@ def test_many_narrow_rows(gpu, T, L, by):
         want[:, slots // bs, 0, slots % bs] = k
         want[:, slots // bs, 1, slots % bs] = v
         assert torch.equal(pool.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("T,H,D", [(4915, 8, 80), (4916, 8, 80), (3072, 8, 128), (3073, 8, 128), (10922, 3, 96), (10923, 3, 96)])
+def test_page_table_writes_of_one_layer_around_12_mib(gpu, T, H, D):
+    """Either side of where page-table launches take other arguments, against PyTorch."""
+    bs = 16
+    g = torch.Generator(device=gpu).manual_seed(T)
+    k, v = (torch.randint(-2**15, 2**15, (T, H, D), dtype=torch.int16, device=gpu, generator=g).view(torch.bfloat16)
+            for _ in range(2))
+    nb = T // bs + 4
+    table = torch.randperm(nb, device=gpu, generator=g)
+    requests = (torch.arange(T, device=gpu) >= 1000).int()      # two, of which the second starts at page 70
+    pos = torch.arange(T, device=gpu)
+    pos[1000:] -= 1000
+    page = pos // bs + torch.where(requests == 1, 70, 0)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=gpu)
+    pool = torch.zeros(nb + 8, 2, bs, H, D, dtype=torch.bfloat16, device=gpu)
+    want = torch.zeros_like(pool)
+    keep = page < nb                                            # pages past the table's end are skipped
+    want[table[page[keep]], 0, pos[keep] % bs], want[table[page[keep]], 1, pos[keep] % bs] = k[keep], v[keep]
+    kvc.append_paged_kv_cache(k, v, requests, pos.int(), pool, table.int(), i32([0, 70, nb]), i32([bs, bs]))
+    assert torch.equal(pool.view(torch.int16), want.view(torch.int16))

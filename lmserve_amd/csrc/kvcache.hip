@@ -1563,11 +1563,18 @@ int run_write(const char* fn, const void* key, const void* value, void* kc, void
     a.tokens_per_wg = l.threads / a.vecs_per_row;
     a.num_planes = (uint32_t)num_planes;
     l.nt = (g_tune.write_nt & 1) != 0;
-    // Many narrow rows: stores go through the L2 as well, from 24 MiB of K and V rows on (at one or two planes per lane), and from 128 MiB on, which the
-    // last-level cache does not hold beside what is written, the loads are non-temporal (before, the stores, both; us,
-    // three sets of rows in turn, 80 layers of 256 bytes by slot: 1700 tokens 23.3, 22.5, 28.5; 2600 (102 MiB) 41.0, 39.6,
-    // 39.4 and, one set that is still in cache, 3001 (117 MiB) 41.3, 40.0, 48.0; 8000 115.2, 110.1, 109.8; by page table 700 tokens 12.5, 12.4, 11.8; 2300 35.4, 34.8, 38.0; 3001 49.6, 48.9,
-    // 49.1; 8000 121.5, 118.5, 116.3, and with a kernel in front that writes the rows 239, 236, 208)
+    // Many narrow rows, at one or two planes per lane (with several layers: from 64 MiB of K and V rows on). Stores go
+    // through the L2 as well, which pays by slot and is even by page table. From 128 MiB on, with what is written
+    // beside them more than the last-level cache holds, the loads are non-temporal: ahead where the rows were just written, or
+    // others came between, and behind where the same rows, unchanged, are read again while the cache holds them.
+    // 80 layers of 256 bytes, us, before | stores through the L2 | and non-temporal loads; one set of rows again and again;
+    // three in turn; one behind a kernel that writes it (its time included):
+    //   by slot, 66 MiB     22.5 21.1 -       22.2 20.8 -       45.1 43.7 -
+    //     160 MiB           54.3 51.0 55.8    59.6 56.7 56.0    106.4 104.4 102.3
+    //     300 MiB           108 102 100       109 104 102       218 217 195
+    //   by pages, 126 MiB   40.8 41.6 -       48.9 48.1 -       80.8 82.1 -
+    //     160 MiB           49.7 50.5 57.2    61.8 60.8 59.0    102.9 104.0 100.8
+    //     300 MiB           112 110 106       113 110 108       227 226 201
     const int64_t rows_bytes = g.num_tokens * num_planes * g.row_elems * E;
     if (narrow && l.vpt <= 2 && !a.through && rows_bytes >= (int64_t(24) << 20)) a.through = 2;
     l.ntl = (g_tune.write_nt & 2) != 0 && (!narrow || rows_bytes >= (int64_t(128) << 20));

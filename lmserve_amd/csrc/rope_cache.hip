@@ -885,6 +885,17 @@ bool layers_depend(const RopeLayer* layers, int64_t n, const LayerExtents& e) {
   return false;
 }
 
+// Layers whose rows are not those of a layer before
+int64_t distinct_rows(const RopeLayer* layers, int64_t n) {
+  int64_t distinct = 0;
+  for (int64_t i = 0; i < n; ++i) {
+    int64_t j = 0;
+    while (j < i && layers[j].query != layers[i].query) ++j;
+    distinct += j == i;
+  }
+  return distinct;
+}
+
 // Does a row that a layer writes meet a Q or K row that it reads? (V passes through, vector by vector.) Bytes.
 bool writes_its_input(const RopeLayer& p, const RopeGeom& g, const CacheGeom* c, int64_t E) {
   typedef __int128 Wide;  // a cache may be said to have any number of blocks
@@ -1048,18 +1059,28 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
     else if (whole && pairs) form = kPairs;
     else if (!in_place || !g.rotary_dim) form = kRows;
     else form = extras > v_items || v_items > pair_lanes ? kOwnerTail : kOwner;
-    // From 40 MiB of Q, K and V rows on the pair form's loads are non-temporal. Plain ones allocate in caches that no longer
-    // hold the rows anyway, and push out the dirty lines of whatever ran before, the projection that wrote these rows
-    // first of all. Smaller rows are still in the last-level cache, from where plain loads are faster. Plain and
-    // non-temporal, us a launch: four sets of rows in turn; the rows just written; those and query_out read behind it:
-    // 8192 tokens x 64 + 8 heads x 128 59.5 and 56.1; 114.9 and 105.9; 163.5 and 147.1
-    // 5500 x 32 + 8 (64 MiB)           26.3 and 25.1; 48.4 and 44.0; 61.7 and 58.4
-    // 3500 of those (41 MiB)           17.9 and 16.0; 30.1 and 28.9; 40.7 and 39.1
-    // 3000 (35 MiB)                    13.7 and 14.3; 25.2 and 24.8; 35.8 and 33.9
-    // 2048 (24 MiB)                    9.3 and 10.9; 18.1 and 18.0; 24.6 and 24.1
+    // From 40 MiB of Q, K and V rows on the pair form's loads are non-temporal. Beside what the launch writes and what ran
+    // before it, the projection that wrote these rows first of all, the last-level cache no longer holds them well, and
+    // plain loads push out dirty lines. us a launch, plain and non-temporal: the same rows again and again, unchanged; four sets
+    // in turn; rows just written by a kernel in front (its time included); with a copy of query_out behind it as well.
+    // The first is not how rows come, and loses from 64 MiB on:
+    //   32 + 8 heads x 128, 30 MiB   9.9 11.6    11.1 12.5    21.8 21.9    28.9 28.8
+    //     36 MiB                     12.9 13.0   13.5 14.1    25.2 25.4    33.1 33.4
+    //     41 MiB                     14.8 14.1   16.9 15.6    28.2 28.2    36.9 37.0
+    //     64 MiB                     22.0 22.9   25.7 23.2    41.8 42.0    57.6 56.0
+    //     100 MiB                    33.3 34.8   38.1 35.8    65.6 65.8    96.0 88.1
+    //   64 + 8, 41 MiB               14.5 14.1   17.0 15.7    28.0 28.3    38.8 38.9
+    //     64 MiB                     21.7 21.0   25.8 22.7    41.5 41.9    62.5 58.4
+    //     128 MiB                    41.3 45.8   47.9 45.8    89.3 84.4    145.6 125.5
+    // Several layers in one launch: from 128 MiB of rows on that are not those of another layer as well (us a launch, plain and
+    // non-temporal; all layers' rows their own, 28 x 28 + 4 heads x 128: 24 MiB 8.9 11.6, 64 15.2 15.7, 128 42.2 42.3, 200
+    // 75.3 62.5, 400 149 139, 800 300 283; 32 x 32 + 8: 128 43.3 42.0, 260 96.8 80.6, 800 290 276; four sets of rows
+    // that the layers take in turn: 28 x 7.1 MiB 45.6 62.0, 28 x 28.6 284 286, 28 x 57 603 580, 80 x 20 478 584).
     // Steps of the rows form lose by it (8192 tokens x 24 layers, 32 + 8 heads x 80, 32 rotated, 570 and 587 us; 16 layers
-    // of 32 + 8 x 64 323 and 330), and so does a rotation without the cache (5000 x 32 + 8 x 128, 954 and 961).
-    if (!kvc::g_rope_tune.nt && form == kPairs && c && g.num_tokens * (heads + g.num_kv_heads) * g.head_dim * E >= (int64_t(40) << 20))
+    // of 32 + 8 x 64 323 and 330), and so does a rotation without the cache (5000 x 32 + 8 x 128, 32 layers, 954 and 961).
+    const int64_t layer_bytes = g.num_tokens * (heads + g.num_kv_heads) * g.head_dim * E;
+    if (!kvc::g_rope_tune.nt && form == kPairs && c &&
+        (layers ? layer_bytes * distinct_rows(layers, num_layers) >= (int64_t(128) << 20) : layer_bytes >= (int64_t(40) << 20)))
       ntl = 3;
     if (form != kRows) {
       a.split = a.pairs_per_head;

@@ -838,3 +838,32 @@ def test_load_policy_of_the_rotation_by_size_and_by_request(gpu):
             assert (last["kernel"], last["per_lane"], last["non_temporal"]) == (_lib.KVC_KERNEL_ROTATE, _lib.KVC_ROPE_PAIRS, ran)
             outs.append((q_out, pool))
         assert all(torch.equal(a, b) for o in outs[1:] for a, b in zip(outs[0], o))
+
+
+@pytest.mark.parametrize("rows,T,nt", [
+    ("own", 420, 0), ("own", 427, 3),             # either side of 128 MiB over 26 layers
+    ("one", 3500, 0),                             # 41 MiB, the same for every layer
+    ("four", 2600, 0), ("four", 2731, 3),         # either side of 128 MiB over four sets that the layers take in turn
+])
+def test_load_policy_of_several_layers_in_one_launch(gpu, rows, T, nt):
+    """Non-temporal loads where the rows that the launch reads once are many, against plain ones."""
+    L, Hq, Hkv, D, bs, dtype = 26, 32, 8, 128, 16, torch.bfloat16
+    sets = {"own": L, "one": 1, "four": 4}[rows]
+    g = torch.Generator(device=gpu).manual_seed(T)
+    qkv = torch.randn(sets, T, (Hq + 2 * Hkv) * D, dtype=dtype, device=gpu, generator=g)
+    q, k, v = ([t[l % sets] for l in range(L)] for t in qkv.split([Hq * D, Hkv * D, Hkv * D], dim=2))
+    pos = torch.arange(T, dtype=torch.int32, device=gpu)
+    none = torch.zeros(T, dtype=torch.int32, device=gpu)
+    slots = torch.randperm(T + bs, device=gpu, generator=g)[:T].contiguous()
+    cs = rotary.make_cos_sin_cache(D, 4096, 500000.0, dtype=dtype, device=gpu)
+    plan = kvc.PagedRotaryWritePlan(none, pos, none[:1], torch.tensor([0, 1], dtype=torch.int32, device=gpu),
+                                    none[:1], cs, Hq, Hkv, D, bs, slots=slots)
+    got = []
+    for asked, ran in ((0, nt), (4, 0)):
+        _lib.set_tuning("rope_nt", asked)
+        pool = torch.zeros(L, (T + bs) // bs + 1, 2, bs, Hkv, D, dtype=dtype, device=gpu)
+        out = torch.zeros(L, T, Hq * D, dtype=dtype, device=gpu)
+        assert plan.run_layers(q, k, v, list(pool), list(out))
+        assert _lib.last_launch()["non_temporal"] == ran
+        got.append((out, pool))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])

@@ -74,7 +74,8 @@ enum {
   KVC_LAUNCH_PIPE = 6,         /* write kernels: 1 = a lane waits for each of its loads */
   KVC_LAUNCH_SWAP_MODE = 7,    /* the kvc_swap_mode this thread's last swap call ran in  */
   KVC_LAUNCH_ORDER = 8,        /* block copies: 1 = all blocks of a layer before the next layer */
-  KVC_LAUNCH_RUN = 9           /* large block copies: neighbouring chunks that go to one XCD */
+  KVC_LAUNCH_RUN = 9,          /* large block copies: neighbouring chunks that go to one XCD */
+  KVC_LAUNCH_THROUGH = 10      /* write kernels: 1 = rows stored at device scope, 2 = and non-temporal */
 };
 enum kvc_rope_form {
   KVC_ROPE_ELEMENTS = 0,  /* an element pair per lane                             */

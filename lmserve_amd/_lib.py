@@ -54,6 +54,7 @@ KVC_LAUNCH_PIPE = 6
 KVC_LAUNCH_SWAP_MODE = 7
 KVC_LAUNCH_ORDER = 8
 KVC_LAUNCH_RUN = 9
+KVC_LAUNCH_THROUGH = 10
 
 KVC_ABI_VERSION = 6
 FAST_INTERFACE = 2      # names and arguments of the `_kvc_fast` extension's functions
@@ -296,4 +297,5 @@ def last_launch() -> dict:
             "non_temporal": L.kvc_last_launch_info(KVC_LAUNCH_NON_TEMPORAL),
             "pipe": L.kvc_last_launch_info(KVC_LAUNCH_PIPE),
             "order": L.kvc_last_launch_info(KVC_LAUNCH_ORDER),
-            "run": L.kvc_last_launch_info(KVC_LAUNCH_RUN)}
+            "run": L.kvc_last_launch_info(KVC_LAUNCH_RUN),
+            "through": L.kvc_last_launch_info(KVC_LAUNCH_THROUGH)}

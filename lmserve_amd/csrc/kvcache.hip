@@ -176,7 +176,7 @@ Knob* find_knob(const char* key) {
 
 // What the most recent kernel launch of this thread looked like (kvc_last_launch_info).
 struct LastLaunch {
-  int64_t kernel = KVC_KERNEL_NONE, vec = 0, per_lane = 0, threads = 0, grid = 0, nt = 0, pipe = 0, order = 0, run = 0;
+  int64_t kernel = KVC_KERNEL_NONE, vec = 0, per_lane = 0, threads = 0, grid = 0, nt = 0, pipe = 0, order = 0, run = 0, through = 0;
 };
 thread_local LastLaunch g_last;
 thread_local int g_last_swap_mode = -1;  // the mode this thread's most recent swap call ran in
@@ -1598,7 +1598,8 @@ int run_write(const char* fn, const void* key, const void* value, void* kc, void
       }
       KVC_HIP(hipGetLastError());
     }
-    g_last = LastLaunch{KVC_KERNEL_WRITE_PLANES, 16, l.vpt, l.threads, (int64_t)l.grid * l.grid_y, (l.nt ? 1 : 0) | (l.ntl ? 2 : 0), a.pipe};
+    g_last = LastLaunch{KVC_KERNEL_WRITE_PLANES, 16, l.vpt, l.threads, (int64_t)l.grid * l.grid_y, (l.nt ? 1 : 0) | (l.ntl ? 2 : 0), a.pipe,
+                        0, 0, a.through};
     return KVC_OK;
   }
 
@@ -1662,7 +1663,8 @@ int run_write(const char* fn, const void* key, const void* value, void* kc, void
     }
     KVC_HIP(hipGetLastError());
   }
-  g_last = LastLaunch{KVC_KERNEL_WRITE_ROWS, vec, l.vpt, l.threads, l.grid, (l.nt ? 1 : 0) | (l.ntl ? 2 : 0), a.pipe};
+  g_last = LastLaunch{KVC_KERNEL_WRITE_ROWS, vec, l.vpt, l.threads, l.grid, (l.nt ? 1 : 0) | (l.ntl ? 2 : 0), a.pipe,
+                      0, 0, a.through};
   return KVC_OK;
 }
 
@@ -2540,6 +2542,7 @@ int64_t kvc_last_launch_info(int what) {
     case KVC_LAUNCH_SWAP_MODE: return g_last_swap_mode;
     case KVC_LAUNCH_ORDER: return g_last.order;
     case KVC_LAUNCH_RUN: return g_last.run;
+    case KVC_LAUNCH_THROUGH: return g_last.through;
     default: return KVC_ERR_INVALID_ARG;
   }
 }

@@ -428,8 +428,8 @@ def test_large_copies_with_two_destinations_a_block(gpu, tile_bytes, L, fans, th
     assert np.array_equal(bits_of(dpool), pool)
 
 
-@pytest.mark.parametrize("tile_bytes,n", [(65536, 1023), (65536, 1024), (65552, 1024)])
-def test_order_of_large_copies(gpu, tile_bytes, n):
+@pytest.mark.parametrize("tile_bytes,n,order", [(65536, 1023, 1), (65536, 1024, 0), (65552, 1024, 0), (65520, 1025, 1)])
+def test_order_of_large_copies(gpu, tile_bytes, n, order):
     """Tiles of 64 KiB and more: below 64 MiB a layer the launch walks layers, from there on blocks."""
     L = 2
     g = torch.Generator(device=gpu).manual_seed(n)
@@ -438,6 +438,7 @@ def test_order_of_large_copies(gpu, tile_bytes, n):
     want = pool.clone()
     want[:, ids[n:2 * n]] = pool[:, ids[:n]]
     kvc.copy_blocks(pool, torch.stack([ids[:n], ids[n:2 * n]], 1).flatten().contiguous())
+    assert _lib.last_launch()["order"] == order
     assert torch.equal(pool, want)
 
 

@@ -734,11 +734,12 @@ def test_layers_of_a_plan_in_one_launch_equal_layer_by_layer(gpu, L, T, Hq, Hkv,
         plan.run_layers(q, k[1:], v, caches, outs)
 
 
-@pytest.mark.parametrize("T,Hq,Hkv,D,rd,dtype", [
-    (3413, 32, 8, 128, 128, torch.bfloat16), (3414, 32, 8, 128, 128, torch.bfloat16),     # either side of 40 MiB
-    (5470, 32, 8, 80, 32, torch.float16), (5826, 12, 3, 98, 98, torch.float32),           # rows form; elements
+@pytest.mark.parametrize("T,Hq,Hkv,D,rd,dtype,form,nt", [
+    (3413, 32, 8, 128, 128, torch.bfloat16, _lib.KVC_ROPE_PAIRS, 0),     # either side of 40 MiB
+    (3414, 32, 8, 128, 128, torch.bfloat16, _lib.KVC_ROPE_PAIRS, 3),
+    (5470, 32, 8, 80, 32, torch.float16, _lib.KVC_ROPE_ROWS, 0), (5826, 12, 3, 98, 98, torch.float32, _lib.KVC_ROPE_ELEMENTS, 0),
 ])
-def test_loads_of_many_rows_give_the_bits_of_the_same_rows_in_parts(gpu, T, Hq, Hkv, D, rd, dtype):
+def test_loads_of_many_rows_give_the_bits_of_the_same_rows_in_parts(gpu, T, Hq, Hkv, D, rd, dtype, form, nt):
     """From 40 MiB of rows on the loads are of another kind: a call, and two layers in one launch, against calls
     on a third of the tokens each, which stay below."""
     bs, L = 16, 2
@@ -766,6 +767,7 @@ def test_loads_of_many_rows_give_the_bits_of_the_same_rows_in_parts(gpu, T, Hq, 
         else:
             for l in range(L):
                 plan.run(q[l], k[l], v[l], got_pool[l], query_out=got_q[l])
+                assert (_lib.last_launch()["per_lane"], _lib.last_launch()["non_temporal"]) == (form, nt)
         assert torch.equal(got_q, want_q) and torch.equal(got_pool, want_pool)
 
 
@@ -787,6 +789,12 @@ def test_sizes_beyond_the_short_launch_arguments(gpu, what, D, rd):
     plan.run(q, k, v, pool, query_out=want)
     _check_rotation(want.cpu(), q.cpu(), pos.cpu(), cs.cpu(), D, dtype, "query")
     if what == "head":
+        _, want_k = kvc.rotary_pos_emb(q, k, pos, cs, D)
+        _check_rotation(want_k.cpu(), k.cpu(), pos.cpu(), cs.cpu(), D, dtype, "key")
+        want_pool = torch.zeros_like(pool)
+        want_pool[slots // bs, 0, slots % bs] = want_k.view(T, Hkv, D)
+        want_pool[slots // bs, 1, slots % bs] = v.view(T, Hkv, D)
+        assert torch.equal(pool, want_pool)
         return
     far = torch.empty(((2 << 30) + 4096) * (1 if what == "pages" else 2) + (1 << 20), dtype=dtype, device=gpu)
     got, got_pool = torch.empty_like(q), torch.zeros_like(pool)

@@ -732,12 +732,16 @@ def test_strides_beyond_the_short_launch_arguments(gpu, what, planes, by):
     assert torch.equal(cache, want)
 
 
-@pytest.mark.parametrize("T,L", [(1026, 48), (5462, 48), (1024, 49)])   # 24 and 128 MiB of K and V rows, and more
+@pytest.mark.parametrize("T,L,through,non_temporal", [
+    (1026, 48, (0, 0), (1, 1)),             # 24 MiB of K and V rows in 4 planes a lane or more: stores stay as they are
+    (49152, 1, (0, 2), (1, 1)),             # 24 MiB in one or two
+    (2732, 48, (2, 2), (1, 1)), (5462, 48, (2, 2), (1, 3)), (5352, 49, (2, 2), (1, 3)),    # 64; either side of 128 MiB
+])
 @pytest.mark.parametrize("by", ["slots", "pages"])
-def test_many_narrow_rows(gpu, T, L, by):
+def test_many_narrow_rows(gpu, T, L, through, non_temporal, by):
     """Rows of 256 bytes of all layers in one launch, either side of where its stores and loads change."""
     H, D, bs = 1, 128, 16
-    for tokens in (T - 3, T):
+    for tokens, stores, bits in zip((T - 3, T), through, non_temporal):
         g = torch.Generator(device=gpu).manual_seed(tokens)
         k, v = (torch.randint(-2**15, 2**15, (L, tokens, H, D), dtype=torch.int16, device=gpu, generator=g)
                 .view(torch.bfloat16) for _ in range(2))
@@ -752,6 +756,8 @@ def test_many_narrow_rows(gpu, T, L, by):
             i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=gpu)
             kvc.append_paged_kv_cache_layers(k, v, torch.zeros(tokens, dtype=torch.int32, device=gpu), pos.int(), pool,
                                              table.int(), i32([0, nb]), i32([bs]))
+        ran = _lib.last_launch()
+        assert (ran["kernel"], ran["through"], ran["non_temporal"]) == (_PLANE, stores, bits)
         want = torch.zeros_like(pool)
         want[:, slots // bs, 0, slots % bs] = k
         want[:, slots // bs, 1, slots % bs] = v

@@ -609,7 +609,11 @@ __global__ __launch_bounds__(kThreads) void rope_owner_kernel(typename LeanOf<AD
   const RopeArgs a = from_lean<T, ADDR, TAIL ? kOwnerTail : kOwner>(l);
   rope_owner_lane<T, ADDR, true, TAIL>(a, only_layer(a));
 }
-// Other index types, block sizes, and sizes that RopeLean does not hold
+// Other index types, block sizes, and sizes that RopeLean does not hold; pairs: those sizes, and large page-table launches
+template <typename T, Addressing ADDR, int NTL>
+__global__ __launch_bounds__(kThreads) void rope_pairs_general_kernel(RopeArgs a) {
+  rope_pairs_lane<T, ADDR, NTL>(a, only_layer(a));
+}
 template <typename T, Addressing ADDR, int NTL>
 __global__ __launch_bounds__(kThreads) void rope_rows_general_kernel(RopeArgs a) {
   rope_rows_lane<T, ADDR, false, NTL>(a, only_layer(a));
@@ -762,7 +766,12 @@ typename LeanOf<ADDR>::type lean_of(const RopeArgs& a, int64_t E) {
 
 template <typename T, Addressing ADDR, int NTL>
 void launch_vector(const RopeArgs& a, VectorForm form, bool lean, dim3 grid, dim3 block, hipStream_t s) {
-  if (form == kPairs) kvc::launch((rope_pairs_kernel<T, ADDR, NTL>), grid, block, 0, s, lean_of<ADDR>(a, T::kBytes));
+  // By page table what RopeLeanPages folds away stands ahead of three steps of loads. Up to 4 MiB of rows the host's share
+  // of a launch is the longer one; beyond, the device's (us, RopeArgs and this: 700 tokens x 32 + 8 heads x 128 4.2 and 4.4,
+  // 256 x 64 + 8 in fp32 4.8 and 5.2, 1500 x 32 + 8 x 64 4.3 and 4.5; 1 % over all sizes).
+  const bool large = ADDR == kPages && (int64_t)grid.y * (a.num_heads + 2 * a.num_kv_heads) * a.head_dim * T::kBytes > (4 << 20);
+  if (form == kPairs && (!lean || large)) kvc::launch((rope_pairs_general_kernel<T, ADDR, NTL>), grid, block, 0, s, a);
+  else if (form == kPairs) kvc::launch((rope_pairs_kernel<T, ADDR, NTL>), grid, block, 0, s, lean_of<ADDR>(a, T::kBytes));
   else if (lean) kvc::launch((rope_rows_kernel<T, ADDR, NTL>), grid, block, 0, s, lean_of<ADDR>(a, T::kBytes));
   else kvc::launch((rope_rows_general_kernel<T, ADDR, NTL>), grid, block, 0, s, a);
 }
@@ -1027,7 +1036,7 @@ int run_rope(const char* fn, const void* query, const void* key, const void* val
   const bool fixed = threads == 64 || threads == 128 || threads == 192 || threads == 256;
   if (vector) {
     const int64_t half = (g.rotary_dim / 2) * E, v_items = c ? g.num_kv_heads * g.head_dim / ev : 0;
-    const bool fast = lean_fits(a, E) && (!c ? fast_index<kNoCache>(a) : a.batch_indices ? fast_index<kPages>(a) : fast_index<kSlots>(a));
+    const bool fast = !c ? fast_index<kNoCache>(a) : a.batch_indices ? fast_index<kPages>(a) : fast_index<kSlots>(a);
     a.v_items = (uint32_t)v_items;
     a.cache_nt = g.num_tokens * v_items * 32 > (int64_t(3) << 20);
     a.pairs_per_head = (uint32_t)((g.rotary_dim / 2) / ev);

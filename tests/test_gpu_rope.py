@@ -875,3 +875,56 @@ def test_load_policy_of_several_layers_in_one_launch(gpu, rows, T, nt):
         assert _lib.last_launch()["non_temporal"] == ran
         got.append((out, pool))
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("what", ["pages", "query"])
+def test_whole_heads_at_far_rows_stay_pairs(gpu, what):
+    """Strides of 4 GiB and more, which the short launch arguments do not hold, by slot and by page table, against the same
+    call on dense rows."""
+    T, Hq, Hkv, D, bs, nb, dtype = 4, 32, 8, 128, 16, 2, torch.bfloat16
+    q, k, v, pos, cs = (t.to(gpu) for t in _case(gpu, T, Hq, Hkv, D, D, dtype))
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=gpu)
+    pos = i32([17, 18, 3, 0])
+    slots = torch.tensor([1, 2, 19, 16], device=gpu)
+    requests, table, indptr = i32([0, 0, 1, 1]), i32([1, 0, 1]), i32([0, 2, 3])
+    stride = (2 << 30) + 4096                       # elements of two bytes
+    far = torch.empty(nb * stride if what == "pages" else T * stride, dtype=dtype, device=gpu)
+    for by in ("slots", "pages"):
+        plan = kvc.PagedRotaryWritePlan(requests, pos, table, indptr, i32([3, 4]), cs, Hq, Hkv, D, bs,
+                                        slots=slots if by == "slots" else None)
+        pool = torch.zeros(nb, 2, bs, Hkv, D, dtype=dtype, device=gpu)
+        want, got = torch.empty_like(q), torch.empty_like(q)
+        plan.run(q, k, v, pool, query_out=want)
+        got_pool, far_q = torch.zeros_like(pool), q
+        if what == "pages":
+            got_pool = far.as_strided(pool.shape, (stride, *pool.stride()[1:]))
+            got_pool.zero_()
+        else:
+            far_q = far.as_strided(q.shape, (stride, 1)).copy_(q)
+        plan.run(far_q, k, v, got_pool, query_out=got)
+        assert _lib.last_launch()["per_lane"] == _lib.KVC_ROPE_PAIRS
+        assert torch.equal(got, want) and torch.equal(got_pool, pool)
+
+
+@pytest.mark.parametrize("T", [341, 342])           # 4 MiB of rows and less
+@pytest.mark.parametrize("nt", [0, 1, 2, 3])
+def test_page_table_rotation_of_whole_heads_either_side_of_4_mib(gpu, T, nt):
+    Hq, Hkv, D, bs, dtype = 32, 8, 128, 16, torch.bfloat16
+    q, k, v, pos, cs = (t.to(gpu) for t in _case(gpu, T, Hq, Hkv, D, D, dtype, seed=T))
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=gpu)
+    pos = torch.arange(T, dtype=torch.int32, device=gpu)
+    nb = T // bs + 1
+    table = torch.randperm(nb, device=gpu)
+    slots = table[pos.long() // bs] * bs + pos.long() % bs
+    none = torch.zeros(T, dtype=torch.int32, device=gpu)
+    _lib.set_tuning("rope_nt", nt)
+    got = []
+    for s in (slots.contiguous(), None):
+        plan = kvc.PagedRotaryWritePlan(none, pos, table.int(), i32([0, nb]), i32([T - nb * bs + bs]), cs, Hq, Hkv, D, bs, slots=s)
+        pool = torch.zeros(nb, 2, bs, Hkv, D, dtype=dtype, device=gpu)
+        out = torch.empty_like(q)
+        plan.run(q, k, v, pool, query_out=out)
+        assert _lib.last_launch()["per_lane"] == _lib.KVC_ROPE_PAIRS
+        got.append((out, pool))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    _check_rotation(got[0][0].cpu(), q.cpu(), pos.cpu(), cs.cpu(), D, dtype, "query")

@@ -1803,9 +1803,10 @@ int launch_stream(const TileArgs& t, TileSides sides, int64_t n, hipStream_t s, 
   a.num_items = (uint32_t)n;
   // Copies walk a layer at a time: with the layers of a block as neighbours a run touches as many far-apart pages, and
   // what is in flight as many layers (blocks in order and layers in order, us: 400 x 16 layers of 32 KiB 82 and 72, 600 x
-  // 24 of 40 KiB 213 and 202, 64 x 32 of 64 KiB 45.8 and 43.3). Where much of a layer is copied, that alone keeps
-  // neighbours together (1024 x 32 of 64 KiB, 64 MiB a layer, 686 both ways, 2048 1370 and 1385). A dense side wants
-  // its own order (gather 6.2 -> 5.1 TB/s).
+  // 24 of 40 KiB 213 and 202, 64 x 32 of 64 KiB 45.8 and 43.3). Where much of a layer is copied in large tiles, that alone
+  // keeps neighbours together (1024 x 32 of 64 KiB, 64 MiB a layer, 686 both ways, 2048 1370 and 1385); tiles below 64 KiB
+  // gain by layers there too (earlier form, blocks in order, and this: 5333 x 12 of 32 KiB, 167 MiB a layer, 842 and 814, 4266
+  // x 12 of 40 KiB 786 and 773, 9481 x 12 of 18 KiB 848 and 833). A dense side wants its own order (gather 6.2 -> 5.1 TB/s).
   a.layer_slowest = sides == TileSides::kPools && (t.tile_bytes < (64 << 10) || n * t.tile_bytes < (int64_t(64) << 20));
   // Runs of 2 MiB leave what does not fill a span of 16 MiB in grid order, so scatters below three spans take 512 KiB
   // (scatter right behind the gather of the same buffer, 2 MiB and 512 KiB, us for both: 17.5 MiB, 80 layers of 16 KiB, 22.1

@@ -171,11 +171,12 @@ struct RopeArgs {
 
 // The same in 128 bytes, for the kernels that take the index build's types and rows of aligned vectors; byte strides
 // and counts that do not fit send a call to the general form. A launch's arguments are written to memory beyond the
-// host link, and what that costs the host has a step at 128 bytes: launches back to back, us each, of 16 to 128
-// bytes 2.9 to 3.1, of 136 to 352 3.3 to 3.8, of 528 (RopeArgs, and the 256 bytes of launch geometry that a kernel
-// takes along once it reads blockDim) 3.9. Per-layer launches at decode sizes are bound by that: with RopeArgs and with
-// these, us a launch and us a step, 16 layers of 2 tokens x 32 + 8 heads x 64 4.5 and 4.0, 95 and 88; 28 of 64 x 28 + 4 x
-// 128 4.5 and 3.8, 149 and 130; 32 of 256 x 32 + 8 4.4 and 3.6, 163 and 140; 32 of 838 4.4 and 3.6, 182 and 160.
+// host link. What that costs the host hangs on a state of the host that changes from machine to machine and within
+// minutes. Launches of one layer back to back, RopeArgs with the 256 bytes of launch geometry that a kernel takes along once
+// it reads blockDim, and these, us each (32 layers of 256 tokens x 32 + 8 heads x 128; medians of 16 runs in turn): 4.4 and
+// 3.6 where the step at 128 bytes showed most, 4.12 and 4.15, 3.18 and 3.14, and 2.45 both. On the device by slot the short
+// form is 1 % ahead (rows form 3 to 5), and several layers in one launch gain most (64 tokens x 28 layers of 28 + 4 x 128 4.56
+// and 4.30, 256 x 16 of 32 + 8 x 64 6.4 and 5.9, 256 x 80 of 8 + 1 x 128, which takes one launch instead of two, 16.8 and 12.8).
 struct RopeLean {
   const char *query, *key, *value;
   char *query_out, *key_out, *key_cache, *value_cache;

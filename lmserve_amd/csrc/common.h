@@ -23,7 +23,8 @@ inline int log2_exact(int64_t x) {
 // Launch shape of the rotation kernel, set through kvc_set_tuning
 // ("rope_threads": 64/128/192/256 lanes per workgroup, 0 = by size; "rope_nt":
 // non-temporal loads, bit 0 the K and V rows, bit 1 the Q rows, 4 = plain loads,
-// 0 = by size: both for whole heads from 40 MiB of rows on). A forward pass hands the kernel rows its projection has
+// 0 = by size: both for whole heads from 40 MiB of rows on, of several layers in one
+// launch from 128 MiB on). A forward pass hands the kernel rows its projection has
 // just written; while these are still in cache, non-temporal loads make a 2048-token
 // chunk 36 % slower (8.51 against 6.25 us) and leave a decode launch unchanged.
 struct RopeTuning {
